@@ -27,6 +27,7 @@
 #include "hip_check.h"
 #include "attn_device.h"
 #include "kv_step.h"
+#include "step_resident.h"
 #include "launch.h"
 
 #include <algorithm>
@@ -717,6 +718,7 @@ void kv_step_slice(const blt_kv_attn_cache *cache, const float *q_rows, size_t q
 void blt_kv_arm_device_error_check() { g_unchecked_steps.fetch_add(1, std::memory_order_relaxed); }
 
 void blt_kv_check_device_errors() {
+    kv_step_resident_check();
     if (g_unchecked_steps.exchange(0, std::memory_order_relaxed) == 0) return;
     uint32_t word = 0;
     HIP_CHECK(hipMemcpy(&word, statics().error(), sizeof(word), hipMemcpyDeviceToHost));

@@ -18,6 +18,7 @@
 #include "matmul.h"
 #include "cross_rows_device.h"
 #include "rope_device.h"
+#include "step_resident.h"
 
 #include <algorithm>
 #include <cmath>
@@ -446,17 +447,42 @@ void check_vec(const blt_tensor &t, size_t dim, const char *what) {
                 "%s", what);
 }
 
+/* every weight the step reads, before anything is issued */
+void check_layers(const blt_local_decoder *dec, size_t E) {
+    for (size_t l = 0; l < dec->config.num_layers; l++) {
+        const blt_local_layer_storage *s = &dec->layers[l];
+        if (cross_fires(&dec->config, l)) {
+            check_vec(s->cross_norm_weight, E, "blt_kv_decode_step: cross_norm_weight must be [embed_dim] FP32");
+            check_weight(&s->cross_weight_q, E, E, "blt_kv_decode_step: cross_weight_q must be [embed_dim, embed_dim]");
+            check_weight(&s->cross_weight_proj, E, E,
+                         "blt_kv_decode_step: cross_weight_proj must be [embed_dim, embed_dim]");
+        }
+        check_vec(s->norm1_weight, E, "blt_kv_decode_layer: norm weights must be [embed_dim]");
+        check_vec(s->norm2_weight, E, "blt_kv_decode_layer: norm weights must be [embed_dim]");
+        check_weight(&s->attn_qkv_w, E, 3 * E, "blt_kv_decode_layer: attn_qkv_w must be [embed_dim, 3*embed_dim]");
+        check_weight(&s->attn_proj_w, E, E, "blt_kv_decode_layer: attn_proj_w must be [embed_dim, embed_dim]");
+        BLT_REQUIRE(s->ffn_up_w.ndim == 2, "blt_kv_decode_layer: ffn_up_w must be 2D");
+        const size_t hidden = s->ffn_up_w.shape[1];
+        check_weight(&s->ffn_up_w, E, hidden, "blt_kv_decode_layer: ffn_up_w must be [embed_dim, hidden_dim]");
+        check_weight(&s->ffn_gate_w, E, hidden, "blt_kv_decode_layer: ffn_gate_w must be [embed_dim, hidden_dim]");
+        check_weight(&s->ffn_down_w, hidden, E, "blt_kv_decode_layer: ffn_down_w must be [hidden_dim, embed_dim]");
+    }
+}
+
 /* The step for `batch` sequences with n new rows each: base[b] is sequence b's
  * valid length, group[b*n + r] the latent patch of its row r.  Lengths and
  * group ranges travel to the device in one staged copy. */
 /* step_kind / window: BLT_KV_STEP_CAUSAL with the decoder's local window for the incremental step;
  * the diffusion forward runs its clean rows causally without a window and its block rows as
- * BLT_KV_STEP_BLOCK.  positions (host, [batch*n]) when a row's rotary position is not base + r. */
+ * BLT_KV_STEP_BLOCK.  positions (host, [batch*n]) when a row's rotary position is not base + r.
+ * d0_index (host, [batch*n]): the input rows are these rows of d0_rows, the decoder's D_0 table. */
 void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const size_t *base, const size_t *group,
                      const float *d0_rows, float *logits, blt_arena *arena, int step_kind = BLT_KV_STEP_CAUSAL,
-                     size_t window = SIZE_MAX, const size_t *positions = nullptr) {
+                     size_t window = SIZE_MAX, const size_t *positions = nullptr,
+                     const uint32_t *d0_index = nullptr) {
     const blt_local_decoder *dec = cache->decoder;
     const blt_local_decoder_config *cfg = &dec->config;
+    const size_t d0_shape[2] = {batch * n, cache->embed_dim};
     const size_t E = cache->embed_dim, L = cfg->num_layers, H = cfg->num_heads, XH = cfg->cross_attn_heads;
     const size_t V = cfg->vocab_size, rows = batch * n, hd = E / H, xhd = E / XH;
     BLT_REQUIRE(xhd <= 256, "blt_kv_decode_step: cross-attention heads wider than 256 columns are not supported");
@@ -474,6 +500,29 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
                 BLT_REQUIRE(positions[b * n + r] < cfg->max_seq_len, "rope_position_gather: position index out of range");
                 own_positions = own_positions || positions[b * n + r] != base[b] + r;
             }
+    if (step_tolerant()) {
+        check_layers(dec, E);
+        bool crosses[64];
+        StepResident st;
+        std::memset(&st, 0, sizeof(st));
+        st.cache = cache, st.batch = batch, st.n = n, st.base = base, st.latent = group;
+        st.d0_rows = d0_rows, st.row_index = d0_index;
+        st.positions = own_positions ? positions : nullptr;
+        st.crosses = crosses, st.logits = logits;
+        st.window = window == SIZE_MAX ? cfg->local_window : window;
+        st.block_kind = step_kind == BLT_KV_STEP_BLOCK;
+        bool fits = L <= 64;
+        for (size_t l = 0; l < L && fits; l++) crosses[l] = cross_fires(cfg, l);
+        if (fits && kv_step_resident(st)) {
+            HIP_CHECK_LAUNCH("blt_kv_decode_step");
+            return;
+        }
+    }
+    if (d0_index != nullptr) { /* the rows of the table as an array of their own */
+        blt_tensor gathered = blt_tensor_create_uninit(arena, d0_shape, 2, BLT_DTYPE_FP32);
+        blt_embedding_lookup_hip(&dec->d0_embed_weight, d0_index, &gathered);
+        d0_rows = (const float *)gathered.data;
+    }
     std::vector<uint32_t> host(batch + 2 * rows + (own_positions ? rows : 0));
     if (own_positions)
         for (size_t i = 0; i < rows; i++) host[batch + 2 * rows + i] = (uint32_t)positions[i];
@@ -770,23 +819,6 @@ extern "C" void blt_kv_decode_step_batched_hip(blt_kv_cache *cache, size_t *self
 /* ===================================================================== */
 namespace {
 
-/* D_0 rows of the block section (block_diffusion.c:137-146): zeros, or row tokens[r] of the
- * learned table (csrc/ops/gather_scatter_cpu.c:7-29). */
-const float *block_d0_rows(const blt_local_decoder *dec, const blt_block_batch *batch, blt_d0_mode d0_mode,
-                           blt_arena *arena) {
-    const size_t E = dec->config.embed_dim, R = batch->n_block_rows;
-    const size_t shape[2] = {R, E};
-    if (d0_mode != BLT_D0_LEARNED) {
-        blt_tensor zeros = blt_tensor_create(arena, shape, 2, BLT_DTYPE_FP32); /* zero-filled */
-        return (const float *)zeros.data;
-    }
-    BLT_REQUIRE(batch->tokens != NULL, "forward_diffusion_infer: batch->tokens cannot be NULL with the learned D_0 table");
-    BLT_REQUIRE(dec->d0_embed_weight.data != NULL, "forward_diffusion_infer: the decoder has no learned D_0 table");
-    blt_tensor out = blt_tensor_create_uninit(arena, shape, 2, BLT_DTYPE_FP32);
-    blt_embedding_lookup_hip(&dec->d0_embed_weight, batch->tokens, &out);
-    return (const float *)out.data;
-}
-
 void check_block_batch(const blt_block_batch *batch, const char *fn) {
     BLT_REQUIRE(batch != NULL, "%s: arguments cannot be NULL", fn);
     BLT_REQUIRE(batch->n_block_rows >= 1 && batch->positions != NULL && batch->groups != NULL,
@@ -803,8 +835,26 @@ void block_step_run(const blt_kv_cache *cache, size_t num_patches, const blt_blo
     const size_t base = batch->num_clean, R = batch->n_block_rows;
     for (size_t r = 0; r < R; r++)
         BLT_REQUIRE(batch->groups[r] < num_patches, "forward_diffusion_infer: a block row's latent group is out of range");
-    const float *d0 = block_d0_rows(cache->decoder, batch, d0_mode, arena);
-    decode_step_run(cache, 1, R, &base, batch->groups, d0, logits, arena, BLT_KV_STEP_BLOCK, 0, batch->positions);
+    /* D_0 rows of the block section (block_diffusion.c:137-146): zeros, or row tokens[r] of the learned
+     * table (csrc/ops/gather_scatter_cpu.c:7-29), which the step reads in place */
+    const blt_local_decoder *dec = cache->decoder;
+    if (d0_mode != BLT_D0_LEARNED) {
+        const size_t shape[2] = {R, dec->config.embed_dim};
+        blt_tensor zeros = blt_tensor_create(arena, shape, 2, BLT_DTYPE_FP32); /* zero-filled */
+        decode_step_run(cache, 1, R, &base, batch->groups, (const float *)zeros.data, logits, arena, BLT_KV_STEP_BLOCK, 0,
+                        batch->positions);
+        return;
+    }
+    BLT_REQUIRE(batch->tokens != NULL, "forward_diffusion_infer: batch->tokens cannot be NULL with the learned D_0 table");
+    const blt_tensor *table = &dec->d0_embed_weight;
+    BLT_REQUIRE(table->data != NULL, "forward_diffusion_infer: the decoder has no learned D_0 table");
+    BLT_REQUIRE(table->ndim == 2 && table->shape[1] == dec->config.embed_dim && table->dtype == BLT_DTYPE_FP32 &&
+                    table->backend == BLT_BACKEND_HIP,
+                "blt_embedding_lookup: the D_0 table must be a [vocab, embed_dim] FP32 tensor in device memory");
+    for (size_t r = 0; r < R; r++)
+        BLT_REQUIRE(batch->tokens[r] < table->shape[0], "blt_embedding_lookup: id out of range");
+    decode_step_run(cache, 1, R, &base, batch->groups, (const float *)table->data, logits, arena, BLT_KV_STEP_BLOCK, 0,
+                    batch->positions, batch->tokens);
 }
 
 } // namespace

@@ -1702,6 +1702,25 @@ def test_kv_decode_step_batched(batch, n, case, oracle, dev):
         lib.blt_arena_destroy(arena)
 
 
+RESIDENT_CASES = [
+    dict(E=64, H=2, XH=2, L=8, hidden=32, V=16, max_len=160, k=1, window=0, all_layers=True, placement=0),
+    dict(E=64, H=1, XH=1, L=1, hidden=160, V=48, max_len=300, k=2, window=0, all_layers=True, placement=0),
+    dict(E=128, H=4, XH=4, L=2, hidden=1024, V=256, max_len=300, k=1, window=100, all_layers=False, placement=0),
+    dict(E=128, H=2, XH=2, L=2, hidden=512, V=64, max_len=300, k=3, window=0, all_layers=True, placement=0),
+    dict(E=256, H=8, XH=8, L=2, hidden=1024, V=256, max_len=150, k=2, window=40, all_layers=True, placement=0),
+    dict(E=256, H=4, XH=4, L=1, hidden=992, V=272, max_len=300, k=1, window=0, all_layers=True, placement=0),
+]
+
+
+@pytest.mark.parametrize("batch,n,case", [(1, 32, 0), (8, 17, 0), (33, 1, 0), (1, 1, 1), (32, 1, 1),   # rows of a group 1 ... 32,
+                                          (1, 17, 2), (1, 1, 2), (9, 8, 2), (17, 1, 3),               # one and two shares of the
+                                          (1, 32, 4), (8, 16, 4), (64, 1, 4), (1, 1, 5), (30, 1, 5)])   # keys, heads of 32 and 64
+def test_kv_decode_step_in_one_launch(batch, n, case, oracle, dev, monkeypatch):
+    """The one-launch form of the step at the edges of its shapes, against the restated step."""
+    monkeypatch.setitem(globals(), "STEP_CASES", RESIDENT_CASES)
+    test_kv_decode_step_batched(batch, n, case, oracle, dev)
+
+
 def test_graph_replay_of_a_plan_and_a_decode_layer(oracle, dev):
     """Library launches recorded into a HIP graph: every replay, with eager work and
     synchronisations in between, gives the eager result."""
