@@ -396,10 +396,13 @@ void plan_build(blt_attention_plan &pl, const blt_attention_problem *problems, s
         if (b.whole) b.fam = FAM_FINE;
         else if (choose_once(pl.host.data() + b.base, b.count, b.span)) b.fam = FAM_ONCE;
         else if (choose_fine(pl.host.data() + b.base, b.count, b.affine, b.span, b.tall)) b.fam = FAM_FINE;
-        else if (choose_wide(pl.host.data() + b.base, b.count)) b.fam = FAM_WIDE;
+        else if (choose_wide(pl.host.data() + b.base, b.count)) {
+            b.fam = FAM_WIDE;
+            b.tall = attn_wide_tall(pl.host.data() + b.base, b.count);
+        }
         if (b.affine) continue; /* no descriptor or tile memory needed */
         b.tile_base = (uint32_t)pl.tiles.size();
-        if (b.fam == FAM_WIDE) attn_wide_make_tiles(pl.host.data(), b.base, b.count, pl.tiles);
+        if (b.fam == FAM_WIDE) attn_wide_make_tiles(pl.host.data(), b.base, b.count, b.tall, pl.tiles);
         else if (b.fam == FAM_FINE) attn_fine_make_tiles(pl.host.data(), b.base, b.count, pl.tiles);
         else if (b.fam == FAM_ONCE) attn_once_make_tiles(pl.host.data(), b.base, b.count, pl.tiles);
         else attn_mfma_make_tiles(pl.host.data(), b.base, b.count, pl.tiles);
@@ -425,9 +428,9 @@ void plan_launch(const blt_attention_plan &pl, const AttnProb *dev, const AttnTi
         else if (b.fam == FAM_ONCE)
             attn_once_launch(dev, dev_tiles + b.tile_base, b.tiles, b.hd, b.span, b.dense, 0);
         else if (b.fam == FAM_WIDE && b.affine)
-            attn_wide_launch_affine(b.aff, 0);
+            attn_wide_launch_affine(b.aff, b.tall, 0);
         else if (b.fam == FAM_WIDE)
-            attn_wide_launch(dev, dev_tiles + b.tile_base, b.tiles, b.hd, b.dense, 0);
+            attn_wide_launch(dev, dev_tiles + b.tile_base, b.tiles, b.hd, b.dense, b.tall, 0);
         else if (b.fam == FAM_FINE && b.whole)
             attn_whole_launch_affine(b.aff, 0);
         else if (b.fam == FAM_FINE && b.affine)

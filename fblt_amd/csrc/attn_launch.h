@@ -50,11 +50,12 @@ void attn_mfma_launch_affine(const AttnAffine &aff, hipStream_t s);
  * = two 16-bit group indices) */
 bool attn_wide_can(const AttnProb &d);
 uint32_t attn_wide_groups(const AttnProb &d);
-void attn_wide_make_tiles(const AttnProb *host, uint32_t base, uint32_t count, std::vector<AttnTile> &tiles);
-void attn_wide_launch(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t ntiles, uint32_t hd, bool dense,
+bool attn_wide_tall(const AttnProb *probs, uint32_t count);
+void attn_wide_make_tiles(const AttnProb *host, uint32_t base, uint32_t count, bool tall, std::vector<AttnTile> &tiles);
+void attn_wide_launch(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t ntiles, uint32_t hd, bool dense, bool tall,
                       hipStream_t s);
 void attn_wide_launch_single(const AttnProb &single, hipStream_t s);
-void attn_wide_launch_affine(const AttnAffine &aff, hipStream_t s);
+void attn_wide_launch_affine(const AttnAffine &aff, bool tall, hipStream_t s);
 
 /* fine family: 32-row tiles cut into 16 x 16 units over eight waves, K/V rows of a tile shared
  * through LDS; `span` = keys the longest tile of the launch needs */

@@ -3,12 +3,12 @@
  * enough to fill the chip several times over, where throughput matters and
  * per-launch latency does not.
  *
- * Work item = 128 consecutive query rows of one (sequence, head) problem.
- * The four wavefronts of the workgroup own one 32-row query tile each and
+ * Work item = 128 (or 256) consecutive query rows of one (sequence, head) problem.
+ * The wavefronts of the workgroup own one 32-row query tile each and
  * walk the key tiles (32 keys) TOGETHER: every K and V tile is brought from
- * global memory once per workgroup, with fully coalesced 16-byte loads, into
- * a double-buffered LDS area and read from there by all four waves as MFMA
- * fragments.  Nothing is split along the keys, so there is no merge: a wave
+ * global memory once per workgroup, taken apart into three bf16 parts
+ * (split_bf16.h), parked in a double-buffered LDS area and read from there by all
+ * waves as MFMA fragments.  Nothing is split along the keys, so there is no merge: a wave
  * keeps its own running (max, sum, output) from the first key tile to the
  * last and writes its 32 output rows itself.  Against the latency-oriented
  * kernel in attn_mfma.hip this removes the per-tile query load, the
@@ -29,50 +29,54 @@
  * every workgroup of a problem does the same amount of work.
  *
  * Non-finite scores (the reference drops such keys) are handled
- * optimistically: the key loop runs without per-element finiteness tests --
- * on gfx950 the fp32 matrix instructions and the vector ALU share issue
- * cycles, so every VALU instruction saved is matrix time gained -- and a NaN
- * or +inf score necessarily leaves a non-finite row sum behind; a workgroup
- * that finds one re-runs its group with the tests compiled in.
+ * optimistically: the key loop runs without per-element finiteness tests, and
+ * a NaN or infinity in Q, K or V necessarily leaves a row sum or an output that is not finite;
+ * a workgroup that finds one runs its group again on the fp32 instructions with the tests in.
  *
  * Shapes: head_dim 32 or 64 exactly, 16-byte aligned rows, no weights
- * output, any visibility except per-row ranges.  Bound: MFMA (HD MFMAs of 64
- * cycles per 32x32 tile pair against ~500 VALU cycles of softmax that a
- * second resident wave hides).
+ * output, any visibility except per-row ranges.
+ *
+ * Bound: vector ALU and matrix unit together.  A 32x32 tile of heads of 32 is 768 cycles of bf16 matrix
+ * instructions and about 210 vector instructions (5.5 per value to take apart weights, K and V, three per
+ * weight for the softmax); vector instructions of other waves, and of the same wave where the two are mixed, run
+ * beside the matrix instructions but not for free (twelve matrix instructions 175 ns, with 192 fused multiply-adds in
+ * between 391, those alone 326).  On fp32 matrix instructions the same tile took 2048 cycles
+ * that nothing ran beside.  Causal self-attention, 32 problems of 4096 rows: 322 -> 200 us for heads of 32
+ * (107 -> 172 TFLOP/s); 48 problems of 2048 rows, heads of 64: 301 -> 178.
  */
 #include "attn_device.h"
 #include "attn_launch.h"
 #include "attn_tile.h"
 #include "hip_check.h"
+#include "lane_ops.h"
 #include "launch.h"
+#include "split_bf16.h"
 
 #include <algorithm>
 
 namespace {
 
-/* One 128-row group of problem p.  CHECK: test every score for finiteness.
- * Returns (to every thread of the workgroup that asks) whether this lane's
- * row ended with a non-finite sum, which only happens when !CHECK let a
- * non-finite score through; nothing is stored in that case. */
-template <int HD, bool DENSE, bool CHECK>
-__device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, float (&sm_k)[2][32 * (HD + 4)],
-                                           float (&sm_v)[2][32 * (HD + 4)]) {
+/* One group of 32 WV rows of problem p on the fp32 matrix instructions, every score tested for finiteness: the
+ * second run of a group whose first run met something that is not finite. */
+template <int HD, int WV, bool DENSE>
+__device__ __forceinline__ void wide_group_checked(const AttnProb &p, uint32_t group, float (*sm_k)[32 * (HD + 4)],
+                                                float (*sm_v)[32 * (HD + 4)]) {
     constexpr int HALF = HD / 2;
     constexpr int DB = HD / 32;
     constexpr int ROW = HD + 4;
     constexpr int LPR = HD / 4;            /* 16-byte pieces per row               */
-    constexpr int PIECES = 32 * LPR / 256; /* pieces of one tile per thread        */
+    constexpr int PIECES = HD / 32;        /* pieces of one tile per thread of the first four waves */
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t h = lane >> 5;
     const uint32_t c = lane & 31u;
 
-    const uint32_t g0 = group * 128u;       /* first row of the workgroup */
-    /* which of the four query tiles a wave owns rotates with the group index:
+    const uint32_t g0 = group * (32u * WV); /* first row of the workgroup */
+    /* which of the query tiles a wave owns rotates with the group index:
      * under a causal mask the later tiles are longer, and waves with the same
      * index tend to share a SIMD across resident workgroups */
-    const uint32_t q0 = g0 + ((wave + group) & 3u) * 32u; /* first row of this wave */
+    const uint32_t q0 = g0 + ((wave + group) % WV) * 32u; /* first row of this wave */
     const uint32_t row = q0 + c;
     const bool live = row < p.nq;
     const uint32_t i = live ? row : p.nq - 1u;
@@ -83,7 +87,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, fl
 
     /* key spans of the workgroup and of this wave, in tiles; all wave-uniform */
     uint32_t glo, ghi, wlo = 0xFFFFFFFFu, whi = 0u, flo = 0u, fhi = 0u, dummy0, dummy1;
-    span_key_bounds(p, g0, min(g0 + 127u, p.nq - 1u), glo, ghi, dummy0, dummy1);
+    span_key_bounds(p, g0, min(g0 + 32u * WV - 1u, p.nq - 1u), glo, ghi, dummy0, dummy1);
     if (q0 < p.nq) span_key_bounds(p, q0, min(q0 + 31u, p.nq - 1u), wlo, whi, flo, fhi);
     const bool g_any = ghi > glo, w_any = whi > wlo;
     const uint32_t gt_lo = __builtin_amdgcn_readfirstlane(g_any ? glo / 32u : 0u);
@@ -118,9 +122,10 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, fl
         for (int r = 0; r < 16; r++) oacc[b][r] = 0.f;
     float m = neg_inf(), l = 0.f;
 
-    /* ---- tile movement: thread t carries pieces t, t+256, ... of K and of V ---- */
+    /* ---- tile movement: of the first four waves, thread t carries pieces t, t+256, ... of K and of V ---- */
     float pk[4 * PIECES], pv[4 * PIECES];
     auto request = [&](uint32_t kt) __attribute__((always_inline)) {
+        if (wave >= 4u) return;
 #pragma unroll
         for (int u = 0; u < PIECES; u++) {
             const uint32_t e = threadIdx.x + 256u * u;
@@ -132,6 +137,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, fl
         }
     };
     auto park = [&](uint32_t buf) __attribute__((always_inline)) {
+        if (wave >= 4u) return;
 #pragma unroll
         for (int u = 0; u < PIECES; u++) {
             const uint32_t e = threadIdx.x + 256u * u;
@@ -200,7 +206,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, fl
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const float t = sacc[r];
-                    x[r] = (!CHECK || isfinite(t)) ? t : neg_inf();
+                    x[r] = isfinite(t) ? t : neg_inf();
                     mt = fmaxf(mt, x[r]);
                 }
             } else {
@@ -209,7 +215,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, fl
                 for (int r = 0; r < 16; r++) {
                     float t = sacc[r];
                     if (DENSE) t += mk[r] * LOG2E;
-                    const bool vis = (rel + (8u * (r >> 2) + (r & 3u)) < len) & (!CHECK || isfinite(t));
+                    const bool vis = (rel + (8u * (r >> 2) + (r & 3u)) < len) & isfinite(t);
                     x[r] = vis ? t : neg_inf();
                     mt = fmaxf(mt, x[r]);
                 }
@@ -250,8 +256,290 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, fl
 
     /* both halves of a column carry the same m, their sums add */
     l += __shfl_xor(l, 32, 64);
-    if (!CHECK && !isfinite(l)) return true;
-    if (!live) return false;
+    if (!live) return;
+
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    float *orow = p.out + (size_t)i * p.out_stride;
+#pragma unroll
+    for (int b = 0; b < DB; b++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            *reinterpret_cast<float4 *>(orow + b * 32 + 8 * g + 4 * h) =
+                make_float4(oacc[b][4 * g + 0] * inv, oacc[b][4 * g + 1] * inv, oacc[b][4 * g + 2] * inv,
+                            oacc[b][4 * g + 3] * inv);
+    if (h == 0 && p.lse) {
+        p.lse[2 * (size_t)i + 0] = m * LN2; /* back to natural units */
+        p.lse[2 * (size_t)i + 1] = l;
+    }
+}
+
+/* Bytes of LDS of one buffer: three parts of a K tile, rows of HD (+ 8) values; three of a V tile, a row of 32 (+ 8) keys
+ * per column.  The padding puts the 16-byte reads of eight consecutive rows into different banks. */
+template <int HD>
+struct WideTiles {
+    static constexpr int KROW = HD + 8, VROW = 32 + 8;
+    static constexpr int KPART = 32 * KROW, VPART = HD * VROW;
+    __bf16 k[3][KPART], v[3][VPART];
+};
+
+/* One group of 32 WV rows of problem p, WV waves.  Returns whether this lane's row met something that is not finite;
+ * nothing of the row is stored then.
+ *
+ * The keys of a V tile lie in the order in which a lane half holds its scores (accumulator register r of half h
+ * is key acc_key(r, h)): position 16 j + 8 h + i is the key of register 8 j + i, so the weights of a lane are the
+ * second operand as they are. */
+template <int HD, int WV, bool DENSE>
+__device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, WideTiles<HD> (&sm)[2]) {
+    using Tiles = WideTiles<HD>;
+    constexpr int KS = HD / 16;  /* steps of a score's contraction */
+    constexpr int DB = HD / 32;
+    constexpr int EPT = HD / 8;  /* values of K and of V a thread carries per tile */
+    typedef __bf16 piece __attribute__((ext_vector_type(EPT)));
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63u;
+    const uint32_t wave = tid >> 6;
+    const uint32_t h = lane >> 5;
+    const uint32_t c = lane & 31u;
+
+    const uint32_t g0 = group * (32u * WV); /* first row of the workgroup */
+    /* which of the query tiles a wave owns rotates with the group index:
+     * under a causal mask the later tiles are longer, and waves with the same
+     * index tend to share a SIMD across resident workgroups */
+    const uint32_t q0 = g0 + ((wave + group) % WV) * 32u; /* first row of this wave */
+    const uint32_t row = q0 + c;
+    const bool live = row < p.nq;
+    const uint32_t i = live ? row : p.nq - 1u;
+
+    uint32_t lo, hi;
+    row_key_range(p, i, lo, hi);
+    if (!live) hi = lo;
+
+    /* key spans of the workgroup and of this wave, in tiles; all wave-uniform */
+    uint32_t glo, ghi, wlo = 0xFFFFFFFFu, whi = 0u, flo = 0u, fhi = 0u, dummy0, dummy1;
+    span_key_bounds(p, g0, min(g0 + 32u * WV - 1u, p.nq - 1u), glo, ghi, dummy0, dummy1);
+    if (q0 < p.nq) span_key_bounds(p, q0, min(q0 + 31u, p.nq - 1u), wlo, whi, flo, fhi);
+    const bool g_any = ghi > glo, w_any = whi > wlo;
+    const uint32_t gt_lo = __builtin_amdgcn_readfirstlane(g_any ? glo / 32u : 0u);
+    const uint32_t gt_hi = __builtin_amdgcn_readfirstlane(g_any ? (ghi + 31u) / 32u : 0u);
+    const uint32_t kt_lo = __builtin_amdgcn_readfirstlane(w_any ? wlo / 32u : 0u);
+    const uint32_t kt_hi = __builtin_amdgcn_readfirstlane(w_any ? (whi + 31u) / 32u : 0u);
+    flo = __builtin_amdgcn_readfirstlane(flo);
+    fhi = __builtin_amdgcn_readfirstlane(fhi);
+
+    const float scale2 = p.scale * LOG2E;
+    const float *mrow = DENSE ? p.mask + (size_t)i * p.nk : nullptr;
+    const bool mvec = DENSE && (p.nk % 4u == 0u) && ((reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0u);
+
+    /* ---- query fragment: row c, floats 16 s + 8 h ..., pre-scaled ---- */
+    bf16x8 qf[KS][3];
+    {
+        const float *qrow = p.q + (size_t)i * p.q_stride + 8u * h;
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            const float4 a = *reinterpret_cast<const float4 *>(qrow + 16 * s), b = *reinterpret_cast<const float4 *>(qrow + 16 * s + 4);
+            const float x[8] = {a.x * scale2, a.y * scale2, a.z * scale2, a.w * scale2,
+                                b.x * scale2, b.y * scale2, b.z * scale2, b.w * scale2};
+            split_bf16<8>(x, qf[s][0], qf[s][1], qf[s][2]);
+        }
+    }
+
+    floatx16 oacc[DB];
+#pragma unroll
+    for (int b = 0; b < DB; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) oacc[b][r] = 0.f;
+    float m = neg_inf(), l = 0.f;
+
+    /* ---- tile movement: 256 threads carry EPT values of one K row each, 256 EPT keys of one V column each (of eight
+     * waves the first four K and the others V) ---- */
+    const bool for_k = WV == 4 || wave < 4u, for_v = WV == 4 || wave >= 4u;
+    const uint32_t carrier = tid & 255u;
+    const uint32_t krow = carrier >> 3, kcol = (carrier & 7u) * EPT;
+    const uint32_t vcol = carrier % HD, vgrp = carrier / HD; /* HD = 64: eight positions, one wave; HD = 32: four */
+    const uint32_t vkey = HD == 64 ? 16u * (vgrp >> 1) + 4u * (vgrp & 1u) : 16u * (vgrp >> 2) + 4u * ((vgrp >> 1) & 1u) + 8u * (vgrp & 1u);
+    uint32_t koff = 4u * (krow * p.k_stride + kcol), voff[EPT]; /* bytes within a tile */
+#pragma unroll
+    for (int u = 0; u < EPT; u++) voff[u] = 4u * ((vkey + (uint32_t)(u < 4 ? u : u + 4)) * p.v_stride + vcol);
+    const uint32_t last_tile = (p.nk - 1u) / 32u;
+    float pk[EPT], pv[EPT];
+    /* K tile kk and V tile kv; past the last tile: the last one again, past the last row: that row again */
+    auto request = [&](uint32_t kk, uint32_t kv) __attribute__((always_inline)) {
+        kk = min(kk, last_tile), kv = min(kv, last_tile);
+        if (for_k) {
+            const char *base = reinterpret_cast<const char *>(p.k + (size_t)(kk * 32u) * p.k_stride);
+            if (kk * 32u + 32u > p.nk) koff = 4u * (min(krow, p.nk - 1u - kk * 32u) * p.k_stride + kcol);
+#pragma unroll
+            for (int u = 0; u < EPT; u += 4) {
+                const float4 a = *reinterpret_cast<const float4 *>(base + koff + 4 * u);
+                pk[u + 0] = a.x, pk[u + 1] = a.y, pk[u + 2] = a.z, pk[u + 3] = a.w;
+            }
+        }
+        if (for_v) {
+            const char *base = reinterpret_cast<const char *>(p.v + (size_t)(kv * 32u) * p.v_stride);
+            if (kv * 32u + 32u > p.nk) {
+#pragma unroll
+                for (int u = 0; u < EPT; u++)
+                    voff[u] = 4u * (min(vkey + (uint32_t)(u < 4 ? u : u + 4), p.nk - 1u - kv * 32u) * p.v_stride + vcol);
+            }
+#pragma unroll
+            for (int u = 0; u < EPT; u++) pv[u] = *reinterpret_cast<const float *>(base + voff[u]);
+        }
+    };
+    /* pieces of K to buffer kbuf, of V to buffer vbuf */
+    auto park = [&](uint32_t kbuf, uint32_t vbuf, bool k_too, bool v_too) __attribute__((always_inline)) {
+        if (WV == 8) { /* the same instructions for either: two addresses and a choice */
+            piece a[3];
+            float x[EPT];
+#pragma unroll
+            for (int u = 0; u < EPT; u++) x[u] = for_k ? pk[u] : pv[u];
+            split_bf16<EPT>(x, a[0], a[1], a[2]);
+            __bf16 *to = for_k ? &sm[kbuf].k[0][krow * Tiles::KROW + kcol] : &sm[vbuf].v[0][vcol * Tiles::VROW + vgrp * EPT];
+            const uint32_t part = for_k ? Tiles::KPART : Tiles::VPART;
+            if (for_k ? k_too : v_too) {
+#pragma unroll
+                for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(to + part * t) = a[t];
+            }
+            return;
+        }
+        piece a[3];
+        if (k_too) {
+            split_bf16<EPT>(pk, a[0], a[1], a[2]);
+#pragma unroll
+            for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&sm[kbuf].k[t][krow * Tiles::KROW + kcol]) = a[t];
+        }
+        if (v_too) {
+            split_bf16<EPT>(pv, a[0], a[1], a[2]);
+#pragma unroll
+            for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&sm[vbuf].v[t][vcol * Tiles::VROW + vgrp * EPT]) = a[t];
+        }
+    };
+    /* ---- S^T = K Q^T ---- */
+    auto scores = [&](uint32_t buf) __attribute__((always_inline)) {
+        floatx16 s;
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; k++) {
+            bf16x8 kf[3];
+#pragma unroll
+            for (int t = 0; t < 3; t++) kf[t] = *reinterpret_cast<const bf16x8 *>(&sm[buf].k[t][c * Tiles::KROW + 16 * k + 8 * h]);
+            s = mfma_split(kf, qf[k], s);
+        }
+        return s;
+    };
+
+    /* The loop runs one score tile ahead: while tile kt's weights are made and applied, the matrix unit has the
+     * scores of tile kt + 1 to work on.  K is in LDS one tile ahead of V. */
+    floatx16 sacc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) sacc[r] = 0.f;
+    if (gt_lo < gt_hi) {
+        request(gt_lo, gt_lo);
+        park(0, 0, true, true);
+        request(gt_lo + 1u, gt_lo);
+        park(1, 0, true, false);
+        __syncthreads();
+        if (gt_lo == kt_lo) sacc = scores(0);
+        __syncthreads();
+    }
+
+    for (uint32_t kt = gt_lo; kt < gt_hi; kt++) {
+        const uint32_t buf = (kt - gt_lo) & 1u;
+        request(kt + 2u, kt + 1u); /* travels while this tile is worked on */
+
+        if (kt >= kt_lo && kt < kt_hi) {
+            const uint32_t k0 = kt * 32u;
+
+            /* ---- mask, tile maximum ----
+             * Interior tiles (no row masks any key) take the scores as they
+             * are; edge tiles compare the key's offset into the row's range
+             * with one unsigned test.  No per-element branches. */
+            float mt = neg_inf();
+            const bool all_seen = !DENSE && k0 >= flo && k0 + 32u <= fhi; /* wave-uniform */
+            if (!all_seen) {
+                float mk[16];
+                if (DENSE) {
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const uint32_t j0 = k0 + 8u * g + 4u * h;
+                        if (mvec) {
+                            float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+                            if (j0 < p.nk) t = *reinterpret_cast<const float4 *>(mrow + j0);
+                            mk[4 * g + 0] = t.x, mk[4 * g + 1] = t.y, mk[4 * g + 2] = t.z, mk[4 * g + 3] = t.w;
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; e++) mk[4 * g + e] = mrow[min(j0 + e, p.nk - 1u)];
+                        }
+                    }
+                }
+                const uint32_t rel = k0 + 4u * h - lo, len = hi - lo;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    if (DENSE) sacc[r] += mk[r] * LOG2E;
+                    sacc[r] = rel + (8u * (r >> 2) + (r & 3u)) < len ? sacc[r] : neg_inf();
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) mt = fmaxf(mt, sacc[r]);
+            mt = swap32(mt, OpMax());
+            const float mn = fmaxf(m, mt);
+            const float ms = mn == neg_inf() ? 0.f : mn; /* nothing seen yet: keep the differences finite */
+            if (__any(mn > m)) {
+                const float alpha = fast_exp2(m - ms);
+                l *= alpha;
+#pragma unroll
+                for (int b = 0; b < DB; b++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) oacc[b][r] *= alpha;
+                m = mn;
+            }
+            const floatx16 ahead = scores(buf ^ 1u); /* past the wave's last tile: not used */
+
+            /* ---- O^T += V^T P^T ---- */
+            float ps = 0.f;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                float x[8];
+#pragma unroll
+                for (int r = 0; r < 8; r++) {
+                    x[r] = fast_exp2(sacc[8 * j + r] - ms);
+                    ps += x[r];
+                }
+                bf16x8 pf[3];
+                split_bf16<8>(x, pf[0], pf[1], pf[2]);
+#pragma unroll
+                for (int b = 0; b < DB; b++) {
+                    bf16x8 vf[3];
+#pragma unroll
+                    for (int t = 0; t < 3; t++)
+                        vf[t] = *reinterpret_cast<const bf16x8 *>(&sm[buf].v[t][(32 * b + c) * Tiles::VROW + 16 * j + 8 * h]);
+                    oacc[b] = mfma_split(vf, pf, oacc[b]);
+                }
+            }
+            l += ps;
+            sacc = ahead;
+            park(buf, buf ^ 1u, true, true);
+#pragma unroll
+            for (int n = 0; n < 6 * KS + 12 * DB; n++) { /* a matrix instruction, its time in vector instructions */
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, HD == 32 ? 6 : 4, 0);
+            }
+        } else {
+            if (kt + 1u == kt_lo) sacc = scores(buf ^ 1u);
+            park(buf, buf ^ 1u, true, true);
+        }
+        __syncthreads();
+    }
+
+    /* both halves of a column carry the same m, their sums add */
+    l = swap32(l, OpSum());
+    bool bad = !isfinite(l);
+#pragma unroll
+    for (int b = 0; b < DB; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) bad |= !isfinite(oacc[b][r]);
+    if (bad || !live) return bad;
 
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     float *orow = p.out + (size_t)i * p.out_stride;
@@ -279,12 +567,12 @@ __device__ __forceinline__ void wide_pair(uint32_t t, uint32_t G, uint32_t &ga, 
     gb = t < ga ? t : WIDE_NO_GROUP;
 }
 
-template <int HD, int SRC, bool DENSE>
-__global__ __launch_bounds__(256, 2) void attn_wide_kernel(const AttnProb *__restrict__ probs,
+template <int HD, int WV, int SRC, bool DENSE>
+__global__ __launch_bounds__(64 * WV, 2) void attn_wide_kernel(const AttnProb *__restrict__ probs,
                                                            const AttnTile *__restrict__ tiles, AttnAffine aff) {
     constexpr int TILE = 32 * (HD + 4);
-    __shared__ __attribute__((aligned(16))) float sm_k[2][TILE];
-    __shared__ __attribute__((aligned(16))) float sm_v[2][TILE];
+    constexpr int CHECKED = 4 * TILE * 4, SPLIT = 2 * sizeof(WideTiles<HD>);
+    __shared__ __attribute__((aligned(16))) unsigned char sm[CHECKED > SPLIT ? CHECKED : SPLIT];
 
     uint32_t ga, gb = WIDE_NO_GROUP;
     AttnProb p;
@@ -309,23 +597,43 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(const AttnProb *__res
     for (int pass = 0; pass < 2; pass++) {
         const uint32_t group = pass == 0 ? ga : gb;
         if (group == WIDE_NO_GROUP) break;
-        const bool bad = wide_group<HD, DENSE, false>(p, group, sm_k, sm_v);
-        if (__syncthreads_or(bad)) wide_group<HD, DENSE, true>(p, group, sm_k, sm_v);
+        const bool bad = wide_group<HD, WV, DENSE>(p, group, *reinterpret_cast<WideTiles<HD>(*)[2]>(sm));
+        if (__syncthreads_or(bad)) {
+            float (*const tiles32)[TILE] = reinterpret_cast<float (*)[TILE]>(sm);
+            wide_group_checked<HD, WV, DENSE>(p, group, tiles32, tiles32 + 2);
+        }
     }
 }
 
 template <int SRC>
 void launch_wide(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nblocks, const AttnAffine &aff, uint32_t hd,
-                 bool dense, hipStream_t s) {
+                 bool dense, bool tall, hipStream_t s) {
     const dim3 grid(nblocks), block(256);
     if (hd == 32u && dense)
-        blt_launch("attn_wide", attn_wide_kernel<32, SRC, true>, grid, block, 0, s, dprobs, dtiles, aff);
+        blt_launch("attn_wide", attn_wide_kernel<32, 4, SRC, true>, grid, block, 0, s, dprobs, dtiles, aff);
+    else if (hd == 32u && tall)
+        blt_launch("attn_wide", attn_wide_kernel<32, 8, SRC, false>, grid, dim3(512), 0, s, dprobs, dtiles, aff);
     else if (hd == 32u)
-        blt_launch("attn_wide", attn_wide_kernel<32, SRC, false>, grid, block, 0, s, dprobs, dtiles, aff);
+        blt_launch("attn_wide", attn_wide_kernel<32, 4, SRC, false>, grid, block, 0, s, dprobs, dtiles, aff);
     else if (dense)
-        blt_launch("attn_wide", attn_wide_kernel<64, SRC, true>, grid, block, 0, s, dprobs, dtiles, aff);
+        blt_launch("attn_wide", attn_wide_kernel<64, 4, SRC, true>, grid, block, 0, s, dprobs, dtiles, aff);
     else
-        blt_launch("attn_wide", attn_wide_kernel<64, SRC, false>, grid, block, 0, s, dprobs, dtiles, aff);
+        blt_launch("attn_wide", attn_wide_kernel<64, 4, SRC, false>, grid, block, 0, s, dprobs, dtiles, aff);
+}
+
+/* groups of 128 rows, of 256 if tall */
+uint32_t groups_of(const AttnProb &d, bool tall) { return tall ? (d.nq + 255u) / 256u : (d.nq + 127u) / 128u; }
+
+/* Causal problems without a window: group g sees ~g+1 times the keys of group
+ * 0, so groups are run in pairs (g, G-1-g) of equal total work.  Short
+ * problems keep single groups: their imbalance is bounded by a few tiles and
+ * twice the workgroups hide more latency. */
+bool in_pairs(const AttnProb &d) { return d.vis == ATTN_VIS_CAUSAL && d.window == 0u && attn_wide_groups(d) >= 8u; }
+
+/* work items of one problem */
+uint32_t items_of(const AttnProb &d, bool tall) {
+    const uint32_t G = groups_of(d, tall);
+    return in_pairs(d) ? (G + 1u) / 2u : G;
 }
 
 } // namespace
@@ -336,35 +644,35 @@ bool attn_wide_can(const AttnProb &d) {
            d.vis != ATTN_VIS_RANGE && d.nk >= 1u && d.nq >= 1u && d.nq <= 0xFFFEu * 128u; /* group indices travel in 16 bits */
 }
 
-uint32_t attn_wide_groups(const AttnProb &d) { return (d.nq + 127u) / 128u; }
+uint32_t attn_wide_groups(const AttnProb &d) { return groups_of(d, false); }
 
-/* Causal problems without a window: group g sees ~g+1 times the keys of group
- * 0, so groups are run in pairs (g, G-1-g) of equal total work.  Short
- * problems keep single groups: their imbalance is bounded by a few tiles and
- * twice the workgroups hide more latency. */
-bool attn_wide_pairs(const AttnProb &d) {
-    return d.vis == ATTN_VIS_CAUSAL && d.window == 0u && attn_wide_groups(d) >= 8u;
-}
-
-/* work items of one problem */
-uint32_t attn_wide_items(const AttnProb &d) {
-    const uint32_t G = attn_wide_groups(d);
-    return attn_wide_pairs(d) ? (G + 1u) / 2u : G;
+/* Eight waves instead of four?  Halves what a wave spends on splitting the K and V tiles, which counts for heads of 32 (the
+ * split is a fifth of a tile's vector instructions; heads of 64 have twice the matrix work per score).  Rows of
+ * paired problems only, so that no 256-row group is mostly empty, and enough items for every compute unit:
+ * 32 problems of 4096 rows 204 -> 195 us, 320 problems of 300 rows without this rule 40 -> 42 us. */
+bool attn_wide_tall(const AttnProb *probs, uint32_t count) {
+    uint64_t items = 0;
+    for (uint32_t i = 0; i < count; i++) {
+        if (probs[i].hd != 32u || !in_pairs(probs[i])) return false;
+        items += items_of(probs[i], true);
+    }
+    return items >= 256u;
 }
 
 /* Work items for problems [base, base+count), longest first. */
-void attn_wide_make_tiles(const AttnProb *host, uint32_t base, uint32_t count, std::vector<AttnTile> &tiles) {
+void attn_wide_make_tiles(const AttnProb *host, uint32_t base, uint32_t count, bool tall, std::vector<AttnTile> &tiles) {
     struct Item {
         AttnTile t;
         uint32_t work;
     };
-    auto key_tiles = [](const AttnProb &d, uint32_t g) -> uint32_t {
+    const uint32_t rows = tall ? 256u : 128u;
+    auto key_tiles = [rows](const AttnProb &d, uint32_t g) -> uint32_t {
         uint64_t hi = d.nk, lo = 0;
         if (d.vis == ATTN_VIS_CAUSAL) {
-            const uint64_t last = std::min<uint64_t>((uint64_t)g * 128u + 127u, d.nq - 1u) + d.causal_off;
+            const uint64_t last = std::min<uint64_t>((uint64_t)g * rows + rows - 1u, d.nq - 1u) + d.causal_off;
             hi = std::min<uint64_t>(hi, last + 1u);
             if (d.window > 0) {
-                const uint64_t first = (uint64_t)g * 128u + d.causal_off;
+                const uint64_t first = (uint64_t)g * rows + d.causal_off;
                 lo = first + 1u > d.window ? first + 1u - d.window : 0u;
             }
         }
@@ -373,9 +681,9 @@ void attn_wide_make_tiles(const AttnProb *host, uint32_t base, uint32_t count, s
     std::vector<Item> items;
     for (uint32_t n = 0; n < count; n++) {
         const AttnProb &d = host[base + n];
-        const uint32_t G = attn_wide_groups(d);
-        const bool pairs = attn_wide_pairs(d);
-        const uint32_t n_items = attn_wide_items(d);
+        const uint32_t G = groups_of(d, tall);
+        const bool pairs = in_pairs(d);
+        const uint32_t n_items = items_of(d, tall);
         for (uint32_t t = 0; t < n_items; t++) {
             const uint32_t ga = pairs ? G - 1u - t : t;
             const uint32_t gb = pairs && t < ga ? t : 0xFFFFu;
@@ -390,30 +698,31 @@ void attn_wide_make_tiles(const AttnProb *host, uint32_t base, uint32_t count, s
     for (const Item &it : items) tiles.push_back(it.t);
 }
 
-void attn_wide_launch(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t ntiles, uint32_t hd, bool dense,
+void attn_wide_launch(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t ntiles, uint32_t hd, bool dense, bool tall,
                       hipStream_t s) {
     if (ntiles == 0) return;
     AttnAffine none;
     __builtin_memset(&none, 0, sizeof(none));
-    launch_wide<SRC_TILES>(dprobs, dtiles, ntiles, none, hd, dense, s);
+    launch_wide<SRC_TILES>(dprobs, dtiles, ntiles, none, hd, dense, tall, s);
 }
 
 void attn_wide_launch_single(const AttnProb &single, hipStream_t s) {
     AttnAffine a;
     __builtin_memset(&a, 0, sizeof(a));
+    const bool tall = attn_wide_tall(&single, 1);
     a.first = single;
-    a.nqt = attn_wide_groups(single);
-    a.reserved = attn_wide_pairs(single) ? 1u : 0u;
-    launch_wide<SRC_SINGLE>(nullptr, nullptr, attn_wide_items(single), a, single.hd, single.vis == ATTN_VIS_DENSE, s);
+    a.nqt = groups_of(single, tall);
+    a.reserved = in_pairs(single) ? 1u : 0u;
+    launch_wide<SRC_SINGLE>(nullptr, nullptr, items_of(single, tall), a, single.hd, single.vis == ATTN_VIS_DENSE, tall, s);
 }
 
 /* The batch descriptor of the mfma family, re-read for this kernel: `nqt`
- * counts 128-row groups and `reserved` says whether groups run in pairs. */
-void attn_wide_launch_affine(const AttnAffine &aff_in, hipStream_t s) {
+ * counts groups of 128 rows (256 if tall) and `reserved` says whether they run in pairs. */
+void attn_wide_launch_affine(const AttnAffine &aff_in, bool tall, hipStream_t s) {
     AttnAffine aff = aff_in;
-    aff.nqt = attn_wide_groups(aff.first);
-    aff.reserved = attn_wide_pairs(aff.first) ? 1u : 0u;
-    const uint32_t blocks = aff.count * attn_wide_items(aff.first);
+    aff.nqt = groups_of(aff.first, tall);
+    aff.reserved = in_pairs(aff.first) ? 1u : 0u;
+    const uint32_t blocks = aff.count * items_of(aff.first, tall);
     if (blocks == 0) return;
-    launch_wide<SRC_AFFINE>(nullptr, nullptr, blocks, aff, aff.first.hd, aff.first.vis == ATTN_VIS_DENSE, s);
+    launch_wide<SRC_AFFINE>(nullptr, nullptr, blocks, aff, aff.first.hd, aff.first.vis == ATTN_VIS_DENSE, tall, s);
 }

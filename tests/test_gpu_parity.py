@@ -780,6 +780,58 @@ def test_attention_kernel_families(family):
         assert ("attn_whole" in launched) == (shape == "fine128"), launched
 
 
+@pytest.mark.parametrize("batch,H,hd,nq,nk,window", [
+    (24, 4, 32, 1025, 1025, 0), (24, 4, 32, 1281, 1313, 0),    # eight waves: a group of one row, an offset diagonal
+    (32, 5, 32, 520, 520, 0), (64, 2, 64, 513, 600, 40),       # four waves: ragged last group; windows shorter than a tile
+    (24, 8, 64, 300, 300, 0)])
+def test_attention_on_split_operands(batch, H, hd, nq, nk, window, dev):
+    """The wide kernel on bf16 parts against float64, then with values that are not finite in one problem: a key with
+    such a score leaves the softmax, the other columns of a bad value row and all other problems stay as they were."""
+    import torch
+    w = workloads.offset_causal(batch=batch, nq=nq, nk=nk, H=H, hd=hd, window=window)
+    d = dev.DeviceWorkload(w)
+    lib = api.load()
+    E = H * hd
+    i, j = torch.arange(nq, device="cuda")[:, None], torch.arange(nk, device="cuda")[None, :]
+    seen = j <= i + nk - nq
+    if window:
+        seen &= j > i + nk - nq - window
+
+    def run():
+        d.zero_outputs()
+        plan = d.make_plan("descriptor")
+        assert lib.blt_attention_plan_kernel_hip(plan) == b"wide"
+        lib.blt_attention_plan_run_hip(plan)
+        lib.blt_backend_pass_sync_hip()
+        lib.blt_attention_plan_destroy_hip(plan)
+        return torch.from_numpy(d.output("out").copy()).cuda().view(batch, nq, H, hd)
+
+    def want(b, head, dropped=None):
+        q, k, v = (d.dev[n].view(batch, -1, H, hd)[b, :, head].double() for n in ("q", "k", "v"))
+        s = (q @ k.T.contiguous()) * w.heads[0].scale
+        keep = seen if dropped is None else seen & (j != dropped)
+        p = torch.softmax(s.masked_fill(~keep, float("-inf")), dim=1)
+        return (p @ v.nan_to_num(0.0, 0.0, 0.0)).float()
+
+    try:
+        first = run()
+        for b, head in ((0, 0), (batch - 1, H - 1), (batch // 2, H // 2)):
+            assert_close(first[b, :, head].cpu().numpy(), want(b, head).cpu().numpy(), "problem %d/%d" % (b, head))
+        d.dev["k"].view(batch, nk, H, hd)[1, 7, 1, 3] = float("nan")
+        d.dev["v"].view(batch, nk, H, hd)[2, 40, 0, 5] = float("inf")
+        torch.cuda.synchronize()
+        got = run()
+        assert_close(got[1, :, 1].cpu().numpy(), want(1, 1, dropped=7).cpu().numpy(), "a key that is not finite")
+        rows = seen[:, 40]
+        assert torch.isinf(got[2, rows, 0, 5]).all() and (got[2, rows, 0, 5] > 0).all()
+        others = [c for c in range(hd) if c != 5]
+        assert_close(got[2, :, 0][:, others].cpu().numpy(), want(2, 0)[:, others].cpu().numpy(), "columns beside the bad one")
+        got[1, :, 1], got[2, :, 0] = first[1, :, 1], first[2, :, 0]
+        assert torch.equal(got, first)
+    finally:
+        d.close()
+
+
 @pytest.mark.parametrize("family", ["auto", "rows", "mfma", "wide", "fine", "fine16", "fine128", "once"])
 def test_attention_random_shapes(family):
     """72 randomly shaped strided batches per routing (automatic, and every family / workgroup shape
