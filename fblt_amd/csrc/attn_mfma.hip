@@ -1,6 +1,7 @@
 /*
- * "mfma" kernel family: fused QK^T -> online softmax -> PV on the fp32 matrix
- * cores of gfx950 (v_mfma_f32_32x32x2_f32), for prefill and block shapes.
+ * "mfma" kernel family: fused QK^T -> online softmax -> PV on the matrix
+ * cores of gfx950, for prefill and block shapes.  Both contractions run on three
+ * bf16 parts of their fp32 operands (split_bf16.h), each lane taking its own fragments apart.
  *
  * Work item = one tile of 32 query rows of one (sequence, head) problem, run
  * by a workgroup of four wavefronts (eight when the launch has about as
@@ -30,15 +31,19 @@
  * workgroup (they work on different keys), so there is nothing to stage in
  * LDS; LDS only carries the final merge.
  *
- * Bound: MFMA for long rows (2*HD/2 + 2*HD/2 ... = HD MFMAs of 64 cycles per
- * 32x32 tile against ~8*HD bytes of K/V), launch/latency for the small
- * shapes.
+ * Bound: the vector ALU for long rows (a 32x32 tile of heads of 64: 1536 cycles of matrix instructions beside
+ * about 650 vector instructions, most of them splitting K, V and the weights, which the waves do not
+ * share; on the fp32 matrix instructions it was 4096 cycles with nothing beside them), launch/latency for
+ * the small shapes.  Causal self-attention, fp32 instructions -> parts: 8 heads of 64 over 4096 rows 202 -> 139 us,
+ * over 1024 rows 26.3 -> 22.9; 8 heads of 32 over 4096 rows 108 -> 82.
  */
 #include "attn_device.h"
 #include "attn_launch.h"
 #include "attn_tile.h"
 #include "hip_check.h"
+#include "lane_ops.h"
 #include "launch.h"
+#include "split_bf16.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -238,9 +243,14 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
     float kg[HD / 2]; /* one 32-row tile spread over the wave, 16 bytes per lane and step */
     float *my_k = sm_body + (STAGE ? wave * 32 * ROW : 0);
 
-    float qf[HALF];
+    constexpr int QS = HALF / 8; /* steps of a score's contraction */
+    bf16x8 qf[QS][3];
     float kf[HALF];
     float vf[DB][16];
+    auto query_row = [&](float (&q)[HALF]) __attribute__((always_inline)) {
+        if constexpr (STAGE) frag_from_lds<HD>(q, sm_q, h, c);
+        else load_half_row<HALF, EXACT>(q, p.q + (size_t)i * p.q_stride, h * HALF, p.hd, vec4);
+    };
 
     if (STAGE) {
         /* the query tile is shared by the waves: each brings its share */
@@ -259,8 +269,6 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         } else {
             tile_to_lds_slow<HD>(sm_q, p.q, p.q_stride, q0, p.nq, p.hd, threadIdx.x, NT);
         }
-    } else {
-        load_half_row<HALF, EXACT>(qf, p.q + (size_t)i * p.q_stride, h * HALF, p.hd, vec4);
     }
 
     /* K tile kt: global -> (registers ->) this wave's LDS area, in two steps
@@ -297,13 +305,52 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         K_REQUEST(kt);
         fetch_v(kt);
     }
-    if (STAGE) {
-        __syncthreads(); /* query tile complete */
-        frag_from_lds<HD>(qf, sm_q, h, c);
-        if (kt < kt_hi) K_PARK(kt);
+    if (STAGE) __syncthreads(); /* query tile complete */
+    {
+        float q[HALF];
+        query_row(q);
+#pragma unroll
+        for (int s = 0; s < QS; s++) split_bf16_at<8>(q, 8 * s, qf[s]);
     }
+    if (STAGE && kt < kt_hi) K_PARK(kt);
+    bool bad = false; /* met a score that is not finite */
+    /* ---- scale, mask, running maximum: scores of tile kt -> weights ---- */
+    auto weigh = [&](const floatx16 &sacc, uint32_t tile, float (&x)[16]) __attribute__((always_inline)) {
+        const uint32_t k0 = tile * 32u;
+        float mt = neg_inf();
+        const bool all_seen = !DENSE && k0 >= flo && k0 + 32u <= fhi; /* uniform: no row masks any key */
+        /* lo <= j < hi as one unsigned compare, widened to "always" on tiles every row sees whole:
+         * written with && the sixteen tests become sixteen pairs of branches */
+        const uint32_t vlo = all_seen ? 0u : lo;
+        const uint32_t vlen = all_seen ? 0xFFFFFFFFu : (hi > lo ? hi - lo : 0u);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const uint32_t j = k0 + acc_key(r, h);
+            float t;
+            if (DENSE) t = (sacc[r] * p.scale + mrow[min(j, p.nk - 1u)]) * LOG2E;
+            else t = sacc[r] * scale2;
+            const bool fin = isfinite(t);
+            const bool vis = ((j - vlo) < vlen) & fin;
+            bad |= DENSE ? !isfinite(sacc[r]) : !fin;
+            x[r] = vis ? t : neg_inf();
+            mt = fmaxf(mt, x[r]);
+        }
+        mt = swap32(mt, OpMax());
+        const float mn = fmaxf(m, mt);
+        const float ms = mn == neg_inf() ? 0.f : mn; /* nothing seen yet: keep the differences finite */
+        const float alpha = fast_exp2(m - ms);
+        float ps = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            x[r] = fast_exp2(x[r] - ms);
+            ps += x[r];
+        }
+        l = l * alpha + ps;
+        m = mn;
+        return alpha;
+    };
+    /* The contractions run on three bf16 parts of their operands. */
     while (kt < kt_hi) {
-        const uint32_t k0 = kt * 32u;
         const uint32_t ktn = kt + NW;
 
         if (STAGE) {
@@ -317,54 +364,70 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
 #pragma unroll
         for (int r = 0; r < 16; r++) sacc[r] = 0.f;
 #pragma unroll
-        for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s], qf[s], sacc, 0, 0, 0);
+        for (int s = 0; s < QS; s++) {
+            bf16x8 parts[3];
+            split_bf16_at<8>(kf, 8 * s, parts);
+            sacc = mfma_split(parts, qf[s], sacc);
+        }
         if (!STAGE && ktn < kt_hi) K_REQUEST(ktn);
 
-        /* ---- scale, mask, tile maximum ---- */
         float x[16];
-        float mt = neg_inf();
-        const bool all_seen = !DENSE && k0 >= flo && k0 + 32u <= fhi; /* uniform: no row masks any key */
-        /* lo <= j < hi as one unsigned compare, widened to "always" on tiles every row sees whole:
-         * written with && the sixteen tests become sixteen pairs of branches */
-        const uint32_t vlo = all_seen ? 0u : lo;
-        const uint32_t vlen = all_seen ? 0xFFFFFFFFu : (hi > lo ? hi - lo : 0u);
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const uint32_t j = k0 + acc_key(r, h);
-            float t;
-            if (DENSE) t = (sacc[r] * p.scale + mrow[min(j, p.nk - 1u)]) * LOG2E;
-            else t = sacc[r] * scale2;
-            const bool vis = ((j - vlo) < vlen) & isfinite(t);
-            x[r] = vis ? t : neg_inf();
-            mt = fmaxf(mt, x[r]);
-        }
-        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-        const float mn = fmaxf(m, mt);
-        const float ms = mn == neg_inf() ? 0.f : mn; /* nothing seen yet: keep the differences finite */
-        const float alpha = fast_exp2(m - ms);
-        float ps = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            x[r] = fast_exp2(x[r] - ms);
-            ps += x[r];
-        }
-        l = l * alpha + ps;
-        m = mn;
+        const float alpha = weigh(sacc, kt, x);
 
         /* ---- O^T = O^T * alpha + V^T P^T ---- */
 #pragma unroll
-        for (int b = 0; b < DB; b++) {
+        for (int b = 0; b < DB; b++)
 #pragma unroll
             for (int r = 0; r < 16; r++) oacc[b][r] *= alpha;
 #pragma unroll
-            for (int s = 0; s < 16; s++)
-                oacc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[b][s], x[s], oacc[b], 0, 0, 0);
+        for (int j = 0; j < 2; j++) {
+            bf16x8 pp[3], vp[3];
+            split_bf16_at<8>(x, 8 * j, pp);
+#pragma unroll
+            for (int b = 0; b < DB; b++) {
+                split_bf16_at<8>(vf[b], 8 * j, vp);
+                oacc[b] = mfma_split(vp, pp, oacc[b]);
+            }
         }
         if (ktn < kt_hi) {
             fetch_v(ktn);
             K_PARK(ktn);
         }
         kt = ktn;
+    }
+#pragma unroll
+    for (int b = 0; b < DB; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) bad |= !isfinite(oacc[b][r]);
+    if (__any(bad)) {
+        /* something is not finite: this wave's tiles once more on the fp32 instructions, which tell infinities from NaN */
+        m = neg_inf(), l = 0.f;
+#pragma unroll
+        for (int b = 0; b < DB; b++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) oacc[b][r] = 0.f;
+        for (kt = kt_lo + wave; kt < kt_hi; kt += NW) {
+            K_REQUEST(kt);
+            K_PARK(kt);
+            if (STAGE) frag_from_lds<HD>(kf, my_k, h, c);
+            float q[HALF], x[16];
+            query_row(q);
+            floatx16 sacc;
+#pragma unroll
+            for (int r = 0; r < 16; r++) sacc[r] = 0.f;
+#pragma unroll
+            for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s], q[s], sacc, 0, 0, 0);
+            const float alpha = weigh(sacc, kt, x);
+            fetch_v(kt);
+#pragma unroll
+            for (int b = 0; b < DB; b++) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) oacc[b][r] *= alpha;
+#pragma unroll
+                for (int s = 0; s < 16; s++)
+                    oacc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[b][s], x[s], oacc[b], 0, 0, 0);
+            }
+        }
     }
 
     /* both halves of a column carry the same m, their sums add */
@@ -481,6 +544,8 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
     float *wrow = p.weights + (size_t)i * p.nk;
     const bool wvec = (p.nk % 4u == 0u) && ((reinterpret_cast<uintptr_t>(p.weights) & 15u) == 0u);
     const uint32_t nkt = (p.nk + 31u) / 32u;
+    float q[HALF];
+    query_row(q);
     for (uint32_t wt = wave; wt < nkt; wt += NW) {
         const uint32_t k0 = wt * 32u;
         float w[16];
@@ -496,7 +561,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
 #pragma unroll
             for (int r = 0; r < 16; r++) sacc[r] = 0.f;
 #pragma unroll
-            for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s], qf[s], sacc, 0, 0, 0);
+            for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s], q[s], sacc, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const uint32_t j = k0 + acc_key(r, h);

@@ -42,6 +42,15 @@ __device__ __forceinline__ void split_bf16(const float (&x)[N], Vec &high, Vec &
     }
 }
 
+/* ... of N consecutive ones of a register array */
+template <int N, int M>
+__device__ __forceinline__ void split_bf16_at(const float (&x)[M], int first, bf16x8 (&parts)[3]) {
+    float y[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) y[i] = x[first + i];
+    split_bf16<N>(y, parts[0], parts[1], parts[2]);
+}
+
 /* acc += A B over 16 of K, smallest partial products first */
 template <typename Acc>
 __device__ __forceinline__ Acc mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b)[3], Acc acc) {

@@ -780,12 +780,14 @@ def test_attention_kernel_families(family):
         assert ("attn_whole" in launched) == (shape == "fine128"), launched
 
 
-@pytest.mark.parametrize("batch,H,hd,nq,nk,window", [
-    (24, 4, 32, 1025, 1025, 0), (24, 4, 32, 1281, 1313, 0),    # eight waves: a group of one row, an offset diagonal
-    (32, 5, 32, 520, 520, 0), (64, 2, 64, 513, 600, 40),       # four waves: ragged last group; windows shorter than a tile
-    (24, 8, 64, 300, 300, 0)])
-def test_attention_on_split_operands(batch, H, hd, nq, nk, window, dev):
-    """The wide kernel on bf16 parts against float64, then with values that are not finite in one problem: a key with
+@pytest.mark.parametrize("kernel,batch,H,hd,nq,nk,window", [
+    ("wide", 24, 4, 32, 1025, 1025, 0), ("wide", 24, 4, 32, 1281, 1313, 0),   # eight waves: a group of one row, an offset diagonal
+    ("wide", 32, 5, 32, 520, 520, 0), ("wide", 64, 2, 64, 513, 600, 40),      # four waves: ragged last group; short windows
+    ("wide", 24, 8, 64, 300, 300, 0),
+    ("mfma", 3, 2, 32, 777, 777, 0), ("mfma", 3, 4, 64, 801, 801, 100), ("mfma", 3, 2, 128, 225, 300, 0),
+    ("mfma", 3, 2, 40, 130, 130, 0)])                                          # heads of 40: elements with a guard
+def test_attention_on_split_operands(kernel, batch, H, hd, nq, nk, window, dev):
+    """The kernels that work on bf16 parts against float64, then with values that are not finite in one problem: a key with
     such a score leaves the softmax, the other columns of a bad value row and all other problems stay as they were."""
     import torch
     w = workloads.offset_causal(batch=batch, nq=nq, nk=nk, H=H, hd=hd, window=window)
@@ -800,7 +802,7 @@ def test_attention_on_split_operands(batch, H, hd, nq, nk, window, dev):
     def run():
         d.zero_outputs()
         plan = d.make_plan("descriptor")
-        assert lib.blt_attention_plan_kernel_hip(plan) == b"wide"
+        assert lib.blt_attention_plan_kernel_hip(plan) == kernel.encode()
         lib.blt_attention_plan_run_hip(plan)
         lib.blt_backend_pass_sync_hip()
         lib.blt_attention_plan_destroy_hip(plan)
