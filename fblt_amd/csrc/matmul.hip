@@ -12,10 +12,10 @@
  *    sum -- k ascending, product and sum rounded separately -- so this path
  *    is bit-identical to blt_matmul_cpu.
  *
- *  - "mfma" (everything else): 64x64 output tiles per workgroup of four
- *    wavefronts (128x128, four MFMA tiles per wavefront, once there are 512
- *    such tiles), K in steps of 32 (16) through double-buffered LDS tiles,
- *    v_mfma_f32_32x32x2_f32 accumulation.  The product is accumulated
+ *  - "mfma" (everything else): 64x64 or 128x128 output tiles per workgroup of eight
+ *    wavefronts, K in steps of 32 through double-buffered LDS tiles, on the bf16
+ *    matrix instructions with both operands taken apart into three exact parts on the
+ *    way to LDS (split_bf16.h).  The product is accumulated
  *    TRANSPOSED (MFMA A operand = b tile, B operand = a tile), which puts one
  *    output ROW in each lane with four consecutive columns per register
  *    group: rows are stored with 16-byte stores, and an optional epilogue can
@@ -23,6 +23,11 @@
  *    embedding of the Q and K blocks of a packed QKV projection
  *    (csrc/models/attention.c:76-90) -- without a second pass over the
  *    result.  Summation order differs from the reference's (fp32 tolerance).
+ *    Bound: matrix and vector instructions share the time about evenly for the 64x64 tile
+ *    (384 and 470 cycles of a step), the matrix ones for the 128x128 tile, at the clock that
+ *    load leaves.  On fp32 instructions -> on parts: 2048 x 512 . 512 x 2048 46.5 -> 31.2 us,
+ *    2048 x 2048 . 2048 x 512 49 -> 41, 8192 x 512 . 512 x 512 43.9 -> 29.5,
+ *    4096 x 1024 . 1024 x 4096 273 -> 195 (176 TFLOP/s).
  *
  *  - "splitk" (outputs too small to give every compute unit a 64x64 tile,
  *    e.g. 512x128 * 128x384): one 32x32 output tile per workgroup, its four
@@ -37,6 +42,7 @@
 #include "hip_check.h"
 #include "launch.h"
 #include "matmul.h"
+#include "split_bf16.h"
 #include "cross_rows_device.h"
 
 #include <stdint.h>
@@ -83,97 +89,72 @@ __device__ __forceinline__ void store4(const MatmulArgs &g, uint32_t row, uint32
     }
 }
 
-/* One (64*WT)x(64*WT) output tile per workgroup of four wavefronts; each wave owns a quadrant of
- * WT x WT MFMA tiles.  WT = 2 is for products large enough to give every compute unit several
- * 128x128 tiles: a fragment read from LDS then feeds two matrix instructions, the four
- * accumulators of a wave are independent, and operands come from L2 half as often.
- * K in steps of 32/WT through double-buffered LDS tiles.
- * VEC: a, b 16-byte aligned with lda, ldb, K, N multiples of 4, so a 16-byte
- * piece is either entirely inside or entirely outside the matrices.
- * ROPE: rotate pairs of the first g.rope_cols columns in the epilogue. */
-template <int WT, int NW>
+/* One (64*WT)x(64*WT) output tile per workgroup of eight wavefronts: four quadrants of WT x WT MFMA tiles, and for each
+ * quadrant two waves that take half of every K step (16 of 32); their sums meet in LDS at the end.  The
+ * operands are taken apart into three bf16 parts (split_bf16.h) once per workgroup, on the way from registers
+ * to the double-buffered LDS tiles: rows of a as [row][k], columns of b as [column][k], so that a fragment is one
+ * 16-byte read.  WT = 2 halves the split and the LDS reads per output.
+ * VEC: a 16-byte aligned with lda and K multiples of 4.  ROPE: rotate pairs of the first g.rope_cols columns in
+ * the epilogue. */
+template <int WT>
 struct MfmaShape {
-    static constexpr int BM = TM * WT, BN = TN * WT, BK = TK / WT, THREADS = 64 * NW;
-    static constexpr int AP = BK + 4; /* floats per LDS row of the a tile: 16-byte fragment reads of 32 rows hit all banks */
-    static constexpr int BP = BN + 4;
-    static constexpr int NP = BM * BK / 4 / THREADS; /* 16-byte pieces of each tile a thread moves per step */
-    static constexpr int KW = BK / 2 / (NW / 4);     /* k values of a step per half of a wave */
-    static constexpr size_t LDS_BYTES = (2 * BM * AP + 2 * BK * BP) * sizeof(float);
-    static_assert(BM * BK == BK * BN && NP * 4 * THREADS == BM * BK, "a thread moves the same number of pieces of both tiles");
-    static_assert(NW == 4 || (NW == 8 && WT == 1), "eight waves: the small tile only");
-    static_assert(NW == 4 || 4 * 16 * 64 * sizeof(float) <= LDS_BYTES, "the second group's sums pass through the tile buffers");
+    static constexpr int BT = 64 * WT;          /* rows and columns of the tile */
+    static constexpr int EPT = 4 * WT;          /* values of each operand a thread carries per step */
+    static constexpr int LP = TK + 8;           /* LDS row: 16-byte reads of eight consecutive rows hit different banks */
+    static constexpr int PART = BT * LP;
+    struct Tiles {
+        __bf16 a[3][PART], b[3][PART];
+    };
+    static constexpr size_t LDS_BYTES = 2 * sizeof(Tiles);
+    static_assert(4 * WT * WT * 16 * 64 * sizeof(float) <= LDS_BYTES, "the second waves' sums pass through the tile buffers");
 };
 
-/* NW = 8 (small tile): a second group of four waves takes the other half of every K step, so each
- * SIMD holds two waves of the workgroup and one's waits (LDS, memory, barrier) fall into the
- * other's matrix instructions; with one workgroup per compute unit and four waves those waits
- * left the matrix cores idle 46 % of the time.  The groups' sums meet in LDS at the end. */
-template <bool VEC, bool ROPE, int WT, int NW = 4>
-__global__ __launch_bounds__(64 * NW, 2) void matmul_mfma_kernel(MatmulArgs g) {
-    using Shape = MfmaShape<WT, NW>;
-    constexpr int BM = Shape::BM, BN = Shape::BN, BK = Shape::BK, KW = Shape::KW, NP = Shape::NP;
-    constexpr int AP = Shape::AP, BP = Shape::BP, THREADS = Shape::THREADS;
-    extern __shared__ __attribute__((aligned(16))) float mm_lds[];
-    float (*sa)[BM * AP] = reinterpret_cast<float (*)[BM * AP]>(mm_lds);
-    float (*sb)[BK * BP] = reinterpret_cast<float (*)[BK * BP]>(mm_lds + 2 * BM * AP);
+template <bool VEC, bool ROPE, int WT>
+__global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
+    using Shape = MfmaShape<WT>;
+    constexpr int BT = Shape::BT, EPT = Shape::EPT, LP = Shape::LP;
+    typedef __bf16 piece __attribute__((ext_vector_type(EPT)));
+    extern __shared__ __attribute__((aligned(16))) unsigned char mm_lds[];
+    auto *tiles = reinterpret_cast<typename Shape::Tiles *>(mm_lds);
 
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t h = lane >> 5, c = lane & 31u;
     const uint32_t wr = (wave & 3u) >> 1, wc = wave & 1u; /* wave's quadrant of the tile */
-    const uint32_t kg = wave >> 2;                         /* its half of a K step (eight waves) */
-    const uint32_t row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
+    const uint32_t kg = wave >> 2;                         /* its half of a K step */
+    const uint32_t row0 = blockIdx.y * BT, col0 = blockIdx.x * BT;
 
-    /* pieces of 4 floats this thread moves per K step: NP of the a tile, NP of the b tile.
-     * Loads go to clamped addresses and land in registers untouched; pieces outside the matrices
-     * are zeroed only when they are parked in LDS, after the step's matrix instructions, so that
-     * nothing between the requests and those instructions waits for memory. */
-    auto request = [&](float (&pa)[NP][4], float (&pb)[NP][4], uint32_t k0) __attribute__((always_inline)) {
+    /* this thread's values of a step: EPT consecutive k of one row of a, of one column of b; rows and columns past the end
+     * repeat the last one (their results are not stored), k past the end is zeroed on the way to LDS */
+    const uint32_t a_row = tid / (TK / EPT), a_k = (tid % (TK / EPT)) * EPT;
+    const uint32_t b_col = tid % BT, b_k = (tid / BT) * EPT;
+    const float *const arow = g.a + (size_t)min(row0 + a_row, g.m - 1u) * g.lda;
+    uint32_t b_off[EPT]; /* bytes within a step's rows of b */
 #pragma unroll
-        for (int u = 0; u < NP; u++) {
-            const uint32_t e = threadIdx.x + (uint32_t)THREADS * u;
-            {
-                const uint32_t r = row0 + e / (BK / 4), k = k0 + 4u * (e % (BK / 4));
-                const float *src = g.a + (size_t)min(r, g.m - 1u) * g.lda;
-                if (VEC) {
-                    const float4 t = *reinterpret_cast<const float4 *>(src + min(k, g.k - 4u));
-                    pa[u][0] = t.x, pa[u][1] = t.y, pa[u][2] = t.z, pa[u][3] = t.w;
-                } else {
+    for (int i = 0; i < EPT; i++) b_off[i] = 4u * ((b_k + i) * g.ldb + min(col0 + b_col, g.n - 1u));
+    auto request = [&](float (&pa)[EPT], float (&pb)[EPT], uint32_t k0) __attribute__((always_inline)) {
+        const char *base = reinterpret_cast<const char *>(g.b + (size_t)k0 * g.ldb);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) pa[u][i] = src[min(k + i, g.k - 1u)];
-                }
-            }
-            {
-                const uint32_t k = k0 + e / (BN / 4), col = col0 + 4u * (e % (BN / 4));
-                const float *src = g.b + (size_t)min(k, g.k - 1u) * g.ldb;
-                if (VEC) {
-                    const float4 t = *reinterpret_cast<const float4 *>(src + min(col, g.n - 4u));
-                    pb[u][0] = t.x, pb[u][1] = t.y, pb[u][2] = t.z, pb[u][3] = t.w;
-                } else {
+        for (int i = 0; i < EPT; i++) pb[i] = *reinterpret_cast<const float *>(base + b_off[i]);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) pb[u][i] = src[min(col + i, g.n - 1u)];
-                }
+        for (int i = 0; i < EPT; i += 4) {
+            if (VEC) {
+                const float4 t = *reinterpret_cast<const float4 *>(arow + k0 + a_k + i);
+                pa[i] = t.x, pa[i + 1] = t.y, pa[i + 2] = t.z, pa[i + 3] = t.w;
+            } else {
+                pa[i] = arow[k0 + a_k + i], pa[i + 1] = arow[k0 + a_k + i + 1];
+                pa[i + 2] = arow[k0 + a_k + i + 2], pa[i + 3] = arow[k0 + a_k + i + 3];
             }
         }
     };
-    auto park = [&](const float (&pa)[NP][4], const float (&pb)[NP][4], uint32_t buf, uint32_t k0)
-                    __attribute__((always_inline)) {
+    auto park = [&](const float (&pa)[EPT], const float (&pb)[EPT], uint32_t buf) __attribute__((always_inline)) {
+        piece parts[3];
+        split_bf16<EPT>(pa, parts[0], parts[1], parts[2]);
 #pragma unroll
-        for (int u = 0; u < NP; u++) {
-            const uint32_t e = threadIdx.x + (uint32_t)THREADS * u;
-            const uint32_t ka = k0 + 4u * (e % (BK / 4));
-            const uint32_t kb = k0 + e / (BN / 4), col = col0 + 4u * (e % (BN / 4));
-            float va[4], vb[4];
+        for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&tiles[buf].a[t][a_row * LP + a_k]) = parts[t];
+        split_bf16<EPT>(pb, parts[0], parts[1], parts[2]);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                va[i] = (VEC ? ka : ka + i) < g.k ? pa[u][i] : 0.f;
-                vb[i] = (kb < g.k && (VEC ? col : col + i) < g.n) ? pb[u][i] : 0.f;
-            }
-            *reinterpret_cast<float4 *>(&sa[buf][(e / (BK / 4)) * AP + 4u * (e % (BK / 4))]) =
-                make_float4(va[0], va[1], va[2], va[3]);
-            *reinterpret_cast<float4 *>(&sb[buf][(e / (BN / 4)) * BP + 4u * (e % (BN / 4))]) =
-                make_float4(vb[0], vb[1], vb[2], vb[3]);
-        }
+        for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&tiles[buf].b[t][b_col * LP + b_k]) = parts[t];
     };
 
     floatx16 acc[WT][WT];
@@ -184,75 +165,109 @@ __global__ __launch_bounds__(64 * NW, 2) void matmul_mfma_kernel(MatmulArgs g) {
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
 
-    /* Two register sets take turns: the pieces of step s+1 and s+2 are on their way while step s
-     * runs, so a request has two steps of matrix work to arrive in (one step is less than the
-     * memory latency when a wave is alone on its SIMD).  Requests and parks are unconditional --
-     * addresses are clamped, pieces past K parked as zeros -- so that no load sits behind a branch
-     * and no wait has to assume the worst at a join. */
-    const uint32_t steps = (g.k + BK - 1u) / BK;
-    float pa0[NP][4], pb0[NP][4], pa1[NP][4], pb1[NP][4];
-    request(pa0, pb0, 0);
-    request(pa1, pb1, BK);
-    /* the requests keep the order they have in the loop (one whole set after the other): the wait
-     * counts inside the loop are the worst case of both ways into it */
-    __builtin_amdgcn_sched_barrier(0);
-    park(pa0, pb0, 0, 0);
-    request(pa0, pb0, 2u * BK);
-    __syncthreads();
-    auto step = [&](uint32_t s, float (&pa)[NP][4], float (&pb)[NP][4]) __attribute__((always_inline)) {
-        /* (pa, pb) hold the pieces of step s+1 */
-        const uint32_t buf = s & 1u;
-        /* MFMA A operand (rows of D = output columns): b[k][col], k = KW*(2*kg + h) + t
-         * MFMA B operand (columns of D = output rows):  a[row][k]                       */
-        const float *ar = &sa[buf][(wr * (32u * WT) + c) * AP + KW * (2u * kg + h)];
-        const float *bc = &sb[buf][(KW * (2u * kg + h)) * BP + wc * (32u * WT) + c];
-        /* every fragment of the step is requested from LDS before its first matrix instruction:
-         * read just in time, each pair of instructions waited for the next read */
-        float av[WT][KW], bv[WT][KW];
+    struct Fragments {
+        bf16x8 a[WT][3], b[WT][3];
+    };
+    auto read = [&](uint32_t buf, Fragments &f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t4 = 0; t4 < KW; t4 += 4) {
+        for (int t = 0; t < 3; t++)
 #pragma unroll
             for (int i = 0; i < WT; i++) {
-                const float4 t = *reinterpret_cast<const float4 *>(ar + 32 * i * AP + t4);
-                av[i][t4 + 0] = t.x, av[i][t4 + 1] = t.y, av[i][t4 + 2] = t.z, av[i][t4 + 3] = t.w;
+                f.a[i][t] = *reinterpret_cast<const bf16x8 *>(&tiles[buf].a[t][(wr * (32u * WT) + 32u * i + c) * LP + 16u * kg + 8u * h]);
+                f.b[i][t] = *reinterpret_cast<const bf16x8 *>(&tiles[buf].b[t][(wc * (32u * WT) + 32u * i + c) * LP + 16u * kg + 8u * h]);
             }
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int j = 0; j < WT; j++) bv[j][t4 + t] = bc[(t4 + t) * BP + 32 * j];
-        }
-        __builtin_amdgcn_sched_barrier(0); /* the compiler would sink the reads back between the instructions */
-#pragma unroll
-        for (int t = 0; t < KW; t++)
-#pragma unroll
-            for (int i = 0; i < WT; i++)
-#pragma unroll
-                for (int j = 0; j < WT; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[j][t], av[i][t], acc[i][j], 0, 0, 0);
-        park(pa, pb, buf ^ 1u, (s + 1u) * BK); /* past K this parks zeros in the buffer nobody reads again */
-        request(pa, pb, (s + 3u) * BK);
-        __syncthreads();
     };
-    /* steps in pairs, one per register set; an odd count ends with a step over zeros */
-    for (uint32_t s = 0; s < steps; s += 2u) {
-        step(s, pa1, pb1);
-        step(s + 1u, pa0, pb0);
+    auto multiply = [&](const Fragments &f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < WT; i++)
+#pragma unroll
+            for (int j = 0; j < WT; j++) acc[i][j] = mfma_split(f.b[j], f.a[i], acc[i][j]);
+    };
+    /* Whole steps: two register sets take turns, the values of step s+1 and s+2 are on their way while step s
+     * runs, so a request has two steps of matrix work to arrive in.  Past the last one it is requested and
+     * parked again, into the buffer nobody reads: no branch between the matrix instructions and the split. */
+    const uint32_t steps = g.k / TK;
+    if (steps != 0u) {
+        float pa0[EPT], pb0[EPT], pa1[EPT], pb1[EPT];
+        auto of_step = [&](uint32_t s) { return min(s, steps - 1u) * TK; };
+        request(pa0, pb0, 0);
+        request(pa1, pb1, of_step(1u));
+        park(pa0, pb0, 0);
+        request(pa0, pb0, of_step(2u));
+        __syncthreads();
+        auto step = [&](uint32_t s, float (&pa)[EPT], float (&pb)[EPT]) __attribute__((always_inline)) {
+            /* (pa, pb) hold the values of step s+1 */
+            Fragments f;
+            read(s & 1u, f);
+            multiply(f);
+            park(pa, pb, (s & 1u) ^ 1u);
+#pragma unroll
+            for (int n = 0; n < 6 * WT * WT; n++) { /* a matrix instruction, its time in vector instructions */
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, WT == 2 ? 4 : 8, 0);
+            }
+            request(pa, pb, of_step(s + 3u));
+            __syncthreads();
+        };
+        for (uint32_t s = 0; s < steps; s += 2u) {
+            step(s, pa1, pb1);
+            if (s + 1u < steps) step(s + 1u, pa0, pb0);
+        }
+    }
+    if (g.k % TK != 0u) { /* what is left of K, zeros behind it */
+        const uint32_t k0 = steps * TK;
+        float pa[EPT], pb[EPT];
+#pragma unroll
+        for (int i = 0; i < EPT; i++) {
+            const float x = arow[min(k0 + a_k + i, g.k - 1u)];
+            const float y = g.b[(size_t)min(k0 + b_k + i, g.k - 1u) * g.ldb + min(col0 + b_col, g.n - 1u)];
+            pa[i] = k0 + a_k + i < g.k ? x : 0.f, pb[i] = k0 + b_k + i < g.k ? y : 0.f;
+        }
+        park(pa, pb, 0); /* the loop ended on a barrier */
+        __syncthreads();
+        Fragments f;
+        read(0, f);
+        multiply(f);
+        __syncthreads();
     }
 
-    if constexpr (NW == 8) { /* the loop ended on a barrier: the tile buffers are free */
-        float *meet = mm_lds + (wave & 3u) * (16u * 64u);
-        if (kg == 1u) {
+    /* the tile buffers are free */
+    float *meet = reinterpret_cast<float *>(mm_lds) + (wave & 3u) * (WT * WT * 16u * 64u) + lane;
+    if (kg == 1u) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) meet[r * 64 + lane] = acc[0][0][r];
+        for (int i = 0; i < WT * WT; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) meet[(i * 16 + r) * 64] = acc[i / WT][i % WT][r];
+    }
+    __syncthreads();
+    if (kg == 1u) return;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < WT * WT; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            acc[i / WT][i % WT][r] += meet[(i * 16 + r) * 64];
+            bad |= !isfinite(acc[i / WT][i % WT][r]);
         }
-        __syncthreads();
-        if (kg == 1u) return;
+    if (__any(bad)) {
+        /* something is not finite: the quadrant again on the fp32 instructions, which tell infinities from NaN */
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[0][0][r] = acc[0][0][r] + meet[r * 64 + lane];
+        for (int i = 0; i < WT; i++)
+#pragma unroll
+            for (int j = 0; j < WT; j++) {
+                const float *ar = g.a + (size_t)min(row0 + 32u * (WT * wr + i) + c, g.m - 1u) * g.lda;
+                const float *bc = g.b + min(col0 + 32u * (WT * wc + j) + c, g.n - 1u);
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+                for (uint32_t k = h; k < g.k + h; k += 2u) { /* an odd K ends with a product of zeros */
+                    const float x = k < g.k ? ar[k] : 0.f, y = k < g.k ? bc[(size_t)k * g.ldb] : 0.f;
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y, x, acc[i][j], 0, 0, 0);
+                }
+            }
     }
 
     /* lane (h, c) holds out[row0 + 32*(WT*wr + i) + c][col0 + 32*(WT*wc + j) + 8*q + 4*h + 0..3] in acc[i][j][4q..4q+3] */
-    const bool vst = VEC && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(g.out) & 15u) == 0u) &&
+    const bool vst = VEC && g.n % 4u == 0u && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(g.out) & 15u) == 0u) &&
                      ((reinterpret_cast<uintptr_t>(g.residual) & 15u) == 0u);
 #pragma unroll
     for (int i = 0; i < WT; i++) {
@@ -771,21 +786,17 @@ void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStrea
 }
 
 namespace {
-template <bool VEC, bool ROPE, int WT, int NW>
-void launch_mfma_as(dim3 grid, hipStream_t s, const MatmulArgs &g) {
-    constexpr size_t lds = MfmaShape<WT, NW>::LDS_BYTES;
-    static_assert(lds <= 64u * 1024u, "above 64 KB a kernel has to ask for its LDS first");
-    blt_launch("matmul_mfma", matmul_mfma_kernel<VEC, ROPE, WT, NW>, grid, dim3(64 * NW), lds, s, g);
-}
 template <bool VEC, bool ROPE, int WT>
-void launch_mfma(dim3 grid, hipStream_t s, const MatmulArgs &g) {
-    if constexpr (WT == 1) {
-        if (g.k >= 256u) { /* from eight K steps on: below, the meeting of the sums costs what the overlap gains */
-            launch_mfma_as<VEC, ROPE, 1, 8>(grid, s, g);
-            return;
-        }
+void launch_mfma(const MatmulArgs &g, hipStream_t s) {
+    constexpr uint32_t BT = MfmaShape<WT>::BT;
+    const dim3 grid((g.n + BT - 1u) / BT, (g.m + BT - 1u) / BT);
+    constexpr size_t lds = MfmaShape<WT>::LDS_BYTES;
+    if constexpr (lds > 64u * 1024u) { /* above 64 KB a kernel has to ask for its LDS first */
+        static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void *>(matmul_mfma_kernel<VEC, ROPE, WT>),
+                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        HIP_CHECK(asked);
     }
-    launch_mfma_as<VEC, ROPE, WT, 4>(grid, s, g);
+    blt_launch("matmul_mfma", matmul_mfma_kernel<VEC, ROPE, WT>, grid, dim3(512), lds, s, g);
 }
 } // namespace
 
@@ -822,33 +833,28 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
         }
         return;
     }
-    /* 128x128 tiles once there are enough of them to load every compute unit twice over */
-    const uint32_t tx = (g.n + 2 * TN - 1) / (2 * TN), ty = (g.m + 2 * TM - 1) / (2 * TM);
-    constexpr uint64_t big_from = 512u;
-    /* Two large tiles are resident per compute unit, 512 at a time: a last round that fills less
-     * than three eighths of the chip costs more than the large tile gains (576 tiles, 6144 x 512 .
-     * 512 x 1536: 106 us against 92 with the small tile; 640: 106 / 104; 960: 142 / 151) until the
-     * rounds are many. */
-    const uint64_t big_tiles = (uint64_t)tx * ty, last_round = big_tiles % 512u;
-    const bool short_tail = big_tiles < 2048u && last_round != 0u && last_round < 192u;
-    if (big_tiles >= big_from && !short_tail) {
-        const dim3 grid(tx, ty);
+    /* One 128x128 workgroup lives on a compute unit, 256 at a time, and takes 3.3 times as long as a 64x64 one, which
+     * splits and reads twice as much per output: the large tile once its rounds are at least three quarters full
+     * (2048 x 512 . 512 x 1536, 192 tiles: 27.9 us against 28.6; 2048 columns, 256 tiles: 31.2 against 36.9; 1024
+     * columns, 128 tiles of K = 256: 15.2 against 11.4). */
+    const uint64_t big_tiles = (uint64_t)((g.n + 127u) / 128u) * ((g.m + 127u) / 128u);
+    const bool big = big_tiles >= (big_tiles + 255u) / 256u * 192u;
+    if (big) {
         if (rope) {
-            if (vec) launch_mfma<true, true, 2>(grid, s, g);
-            else launch_mfma<false, true, 2>(grid, s, g);
+            if (vec) launch_mfma<true, true, 2>(g, s);
+            else launch_mfma<false, true, 2>(g, s);
         } else {
-            if (vec) launch_mfma<true, false, 2>(grid, s, g);
-            else launch_mfma<false, false, 2>(grid, s, g);
+            if (vec) launch_mfma<true, false, 2>(g, s);
+            else launch_mfma<false, false, 2>(g, s);
         }
         return;
     }
-    const dim3 grid((g.n + TN - 1) / TN, (g.m + TM - 1) / TM);
     if (rope) {
-        if (vec) launch_mfma<true, true, 1>(grid, s, g);
-        else launch_mfma<false, true, 1>(grid, s, g);
+        if (vec) launch_mfma<true, true, 1>(g, s);
+        else launch_mfma<false, true, 1>(g, s);
     } else {
-        if (vec) launch_mfma<true, false, 1>(grid, s, g);
-        else launch_mfma<false, false, 1>(grid, s, g);
+        if (vec) launch_mfma<true, false, 1>(g, s);
+        else launch_mfma<false, false, 1>(g, s);
     }
 }
 

@@ -930,6 +930,35 @@ def test_matmul(m, k, n, exact, oracle, dev):
         assert_close(got, ref, "matmul %dx%dx%d" % (m, k, n))
 
 
+@pytest.mark.parametrize("m,k,n", [(769, 1, 769), (800, 33, 772), (1025, 512, 1540), (2049, 96, 2050), (770, 130, 771)])
+def test_matmul_on_split_operands(m, k, n, dev):
+    """Both tile sizes of the product on bf16 parts at ragged edges against float64, then with values that are not finite:
+    what they take part in is what fp32 sums give, everything else stays."""
+    import torch
+    lib = api.load()
+    a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda") / k ** 0.5
+    out = torch.full((m, n), 7.0, device="cuda")
+
+    def product():
+        va, vb, vo = _dev_tensor(a), _dev_tensor(b), _dev_tensor(out)
+        torch.cuda.synchronize()
+        lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+        lib.blt_backend_pass_sync_hip()
+        return out.clone()
+
+    first = product()
+    assert_close(first.cpu().numpy(), (a.double() @ b.double()).float().cpu().numpy(), "matmul %dx%dx%d" % (m, k, n))
+    a[5, k - 1], a[m - 1, 0], b[0, n - 1] = float("inf"), float("nan"), 3.4e38
+    got = product()
+    inf = (a[5, :, None].cpu() * b.cpu()).sum(dim=0)  # one infinity in each sum: infinite with its sign
+    assert torch.equal(got[5, :n - 1].cpu(), inf[:n - 1]) and torch.isnan(got[m - 1]).all()
+    want = torch.outer(a[:, 0].cpu(), b[0, n - 1:].cpu())[:, 0] if k == 1 else (a.cpu() @ b[:, n - 1].cpu())
+    big = [i for i in range(m) if i not in (5, m - 1)]
+    last = got[big, n - 1].cpu()
+    assert torch.equal(torch.isinf(last), torch.isinf(want[big])) and torch.equal(torch.sign(last), torch.sign(want[big]))
+    assert_close(got[big][:, :n - 1].cpu().numpy(), first[big][:, :n - 1].cpu().numpy(), "beside the bad values")
+
+
 @pytest.mark.parametrize("T,H,hd,docs", [(200, 2, 32, [0, 7, 90, 150]), (512, 4, 32, [0, 300]), (128, 8, 64, [0]),
                                          (96, 2, 64, [0, 20, 40, 60, 80])])
 def test_document_causal_ranges_take_the_matrix_cores(T, H, hd, docs, oracle, dev):
