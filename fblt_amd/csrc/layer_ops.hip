@@ -340,7 +340,6 @@ void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_wei
     float *qkv = (float *)blt_arena_alloc(arena, rows * 3 * E * sizeof(float), 64);
     float *combined = (float *)blt_arena_alloc(arena, rows * E * sizeof(float), 64);
     float *resid1 = (float *)blt_arena_alloc(arena, rows * E * sizeof(float), 64);
-    float *up = (float *)blt_arena_alloc(arena, rows * Hd * sizeof(float), 64);
     float *gate = (float *)blt_arena_alloc(arena, rows * Hd * sizeof(float), 64);
 
     MatmulArgs probe;
@@ -381,14 +380,9 @@ void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_wei
     probe.n = (uint32_t)Hd;
     if (matmul_takes_norm(probe)) { /* RMSNorm, up, gate and SwiGLU in one pass */
         gemm(resid1, f32(w->ffn_up_w), gate, rows, E, Hd, nullptr, f32(w->ffn_gate_w), f32(w->norm2_weight));
-    } else if (matmul_takes_gated(probe)) {
-        rmsnorm_launch(resid1, f32(w->norm2_weight), normed, rows, E);
-        gemm(normed, f32(w->ffn_up_w), gate, rows, E, Hd, nullptr, f32(w->ffn_gate_w)); /* up, gate, SwiGLU */
     } else {
         rmsnorm_launch(resid1, f32(w->norm2_weight), normed, rows, E);
-        gemm(normed, f32(w->ffn_up_w), up, rows, E, Hd);
-        gemm(normed, f32(w->ffn_gate_w), gate, rows, E, Hd);
-        swiglu_launch(gate, up, gate, rows * Hd);
+        gemm(normed, f32(w->ffn_up_w), gate, rows, E, Hd, nullptr, f32(w->ffn_gate_w)); /* up, gate, SwiGLU */
     }
     gemm(gate, f32(w->ffn_down_w), rows_out, rows, Hd, E, resid1); /* projection + residual */
     HIP_CHECK_LAUNCH("blt_kv_decode_layer");
@@ -657,15 +651,7 @@ void refresh_cross_seq(blt_kv_cache *cache, size_t seq, const blt_tensor *patch_
         g.b2 = (const float *)s->cross_weight_v.data;
         g.out2 = (float *)cache->cross_v[l].data + row0 * E;
         g.tolerant = step_tolerant();
-        if (matmul_takes_gated(g)) { /* K and V in one pass over the patch rows */
-            matmul_f32_launch(g, 0);
-        } else {
-            g.b2 = nullptr, g.out2 = nullptr;
-            matmul_f32_launch(g, 0);
-            g.b = (const float *)s->cross_weight_v.data;
-            g.out = (float *)cache->cross_v[l].data + row0 * E;
-            matmul_f32_launch(g, 0);
-        }
+        matmul_f32_launch(g, 0); /* K and V in one pass over the patch rows */
     }
     std::memcpy(&cache->cached_patches[seq * cache->max_seq_len + from_patch], &patches[from_patch],
                 (num_patches - from_patch) * sizeof(blt_patch_info)); /* kv_cache.c:154-157 */

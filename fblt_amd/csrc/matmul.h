@@ -63,8 +63,6 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s);
 /* g0 (plain) and g1 (two weight matrices, two outputs) in one launch; only when matmul_pair_ok says so */
 bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1);
 void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStream_t s);
-/* b2 is only implemented by the kernels for small outputs; false = run the two products and the activation apart */
-bool matmul_takes_gated(const MatmulArgs &g);
 /* the cross-attention epilogue for this shape and g.cross_head_dim, no other epilogue set */
 bool matmul_takes_cross(const MatmulArgs &g);
 /* norm_w likewise */

@@ -95,7 +95,13 @@ __device__ __forceinline__ void store4(const MatmulArgs &g, uint32_t row, uint32
  * to the double-buffered LDS tiles: rows of a as [row][k], columns of b as [column][k], so that a fragment is one
  * 16-byte read.  WT = 2 halves the split and the LDS reads per output.
  * VEC: a 16-byte aligned with lda and K multiples of 4.  ROPE: rotate pairs of the first g.rope_cols columns in
- * the epilogue. */
+ * the epilogue.
+ * NORM: the row statistic comes from the values on their way to LDS, the norm weight is multiplied in there, the row's
+ * scale after the product: two vector instructions per value of a against a pass over a of its own (2048 rows of
+ * 512: 14 us with sums in the reference's order).
+ * GATED: the left quadrants are columns of a*b, the right ones the same columns of a*b2; the gates pass through LDS to
+ * the waves that hold the other factor (2048 x 512 . 512 x (2 x 2048): two products and the activation 71 us,
+ * this way 63). */
 template <int WT>
 struct MfmaShape {
     static constexpr int BT = 64 * WT;          /* rows and columns of the tile */
@@ -109,45 +115,71 @@ struct MfmaShape {
     static_assert(4 * WT * WT * 16 * 64 * sizeof(float) <= LDS_BYTES, "the second waves' sums pass through the tile buffers");
 };
 
-template <bool VEC, bool ROPE, int WT>
+template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED>
 __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
     using Shape = MfmaShape<WT>;
     constexpr int BT = Shape::BT, EPT = Shape::EPT, LP = Shape::LP;
     typedef __bf16 piece __attribute__((ext_vector_type(EPT)));
     extern __shared__ __attribute__((aligned(16))) unsigned char mm_lds[];
     auto *tiles = reinterpret_cast<typename Shape::Tiles *>(mm_lds);
+    __shared__ float row_ss[NORM ? BT : 1];
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t h = lane >> 5, c = lane & 31u;
     const uint32_t wr = (wave & 3u) >> 1, wc = wave & 1u; /* wave's quadrant of the tile */
     const uint32_t kg = wave >> 2;                         /* its half of a K step */
-    const uint32_t row0 = blockIdx.y * BT, col0 = blockIdx.x * BT;
+    constexpr uint32_t COLS = GATED ? BT / 2 : BT; /* columns of a product */
+    const uint32_t row0 = blockIdx.y * BT, col0 = blockIdx.x * COLS;
 
     /* this thread's values of a step: EPT consecutive k of one row of a, of one column of b; rows and columns past the end
      * repeat the last one (their results are not stored), k past the end is zeroed on the way to LDS */
     const uint32_t a_row = tid / (TK / EPT), a_k = (tid % (TK / EPT)) * EPT;
     const uint32_t b_col = tid % BT, b_k = (tid / BT) * EPT;
     const float *const arow = g.a + (size_t)min(row0 + a_row, g.m - 1u) * g.lda;
+    /* b or b2: one of them per wave, for the small tile per half of a wave */
+    const float *const bmat = GATED && (WT == 2 ? (wave & 1u) != 0u : b_col >= COLS) ? g.b2 : g.b;
+    const uint32_t b_at = min(col0 + b_col % COLS, g.n - 1u);
     uint32_t b_off[EPT]; /* bytes within a step's rows of b */
 #pragma unroll
-    for (int i = 0; i < EPT; i++) b_off[i] = 4u * ((b_k + i) * g.ldb + min(col0 + b_col, g.n - 1u));
-    auto request = [&](float (&pa)[EPT], float (&pb)[EPT], uint32_t k0) __attribute__((always_inline)) {
-        const char *base = reinterpret_cast<const char *>(g.b + (size_t)k0 * g.ldb);
+    for (int i = 0; i < EPT; i++) b_off[i] = 4u * ((b_k + i) * g.ldb + b_at);
+    struct Values {
+        float a[EPT], b[EPT], w[NORM ? EPT : 1];
+    };
+    auto request = [&](Values &v, uint32_t k0) __attribute__((always_inline)) {
+        const char *base = reinterpret_cast<const char *>(bmat + (size_t)k0 * g.ldb);
 #pragma unroll
-        for (int i = 0; i < EPT; i++) pb[i] = *reinterpret_cast<const float *>(base + b_off[i]);
+        for (int i = 0; i < EPT; i++) v.b[i] = *reinterpret_cast<const float *>(base + b_off[i]);
 #pragma unroll
         for (int i = 0; i < EPT; i += 4) {
             if (VEC) {
                 const float4 t = *reinterpret_cast<const float4 *>(arow + k0 + a_k + i);
-                pa[i] = t.x, pa[i + 1] = t.y, pa[i + 2] = t.z, pa[i + 3] = t.w;
+                v.a[i] = t.x, v.a[i + 1] = t.y, v.a[i + 2] = t.z, v.a[i + 3] = t.w;
             } else {
-                pa[i] = arow[k0 + a_k + i], pa[i + 1] = arow[k0 + a_k + i + 1];
-                pa[i + 2] = arow[k0 + a_k + i + 2], pa[i + 3] = arow[k0 + a_k + i + 3];
+                v.a[i] = arow[k0 + a_k + i], v.a[i + 1] = arow[k0 + a_k + i + 1];
+                v.a[i + 2] = arow[k0 + a_k + i + 2], v.a[i + 3] = arow[k0 + a_k + i + 3];
+            }
+            if constexpr (NORM) {
+                const float *w = g.norm_w + k0 + a_k + i;
+                if (VEC) {
+                    const float4 t = *reinterpret_cast<const float4 *>(w);
+                    v.w[i] = t.x, v.w[i + 1] = t.y, v.w[i + 2] = t.z, v.w[i + 3] = t.w;
+                } else {
+                    v.w[i] = w[0], v.w[i + 1] = w[1], v.w[i + 2] = w[2], v.w[i + 3] = w[3];
+                }
             }
         }
     };
-    auto park = [&](const float (&pa)[EPT], const float (&pb)[EPT], uint32_t buf) __attribute__((always_inline)) {
+    float ss = 0.f; /* this thread's share of its row's sum of squares */
+    auto park = [&](const Values &v, uint32_t buf, bool counts) __attribute__((always_inline)) {
+        float pa[EPT], pb[EPT], squares = 0.f;
+#pragma unroll
+        for (int i = 0; i < EPT; i++) {
+            if constexpr (NORM) squares = fmaf(v.a[i], v.a[i], squares), pa[i] = v.a[i] * v.w[i];
+            else pa[i] = v.a[i];
+            pb[i] = v.b[i];
+        }
+        if constexpr (NORM) ss += counts ? squares : 0.f;
         piece parts[3];
         split_bf16<EPT>(pa, parts[0], parts[1], parts[2]);
 #pragma unroll
@@ -188,47 +220,53 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
      * parked again, into the buffer nobody reads: no branch between the matrix instructions and the split. */
     const uint32_t steps = g.k / TK;
     if (steps != 0u) {
-        float pa0[EPT], pb0[EPT], pa1[EPT], pb1[EPT];
+        Values v0, v1;
         auto of_step = [&](uint32_t s) { return min(s, steps - 1u) * TK; };
-        request(pa0, pb0, 0);
-        request(pa1, pb1, of_step(1u));
-        park(pa0, pb0, 0);
-        request(pa0, pb0, of_step(2u));
+        request(v0, 0);
+        request(v1, of_step(1u));
+        park(v0, 0, true);
+        request(v0, of_step(2u));
         __syncthreads();
-        auto step = [&](uint32_t s, float (&pa)[EPT], float (&pb)[EPT]) __attribute__((always_inline)) {
-            /* (pa, pb) hold the values of step s+1 */
+        auto step = [&](uint32_t s, Values &v) __attribute__((always_inline)) {
+            /* v holds the values of step s+1 */
             Fragments f;
             read(s & 1u, f);
             multiply(f);
-            park(pa, pb, (s & 1u) ^ 1u);
+            park(v, (s & 1u) ^ 1u, s + 1u < steps);
 #pragma unroll
             for (int n = 0; n < 6 * WT * WT; n++) { /* a matrix instruction, its time in vector instructions */
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, WT == 2 ? 4 : 8, 0);
             }
-            request(pa, pb, of_step(s + 3u));
+            request(v, of_step(s + 3u));
             __syncthreads();
         };
         for (uint32_t s = 0; s < steps; s += 2u) {
-            step(s, pa1, pb1);
-            if (s + 1u < steps) step(s + 1u, pa0, pb0);
+            step(s, v1);
+            if (s + 1u < steps) step(s + 1u, v0);
         }
     }
     if (g.k % TK != 0u) { /* what is left of K, zeros behind it */
         const uint32_t k0 = steps * TK;
-        float pa[EPT], pb[EPT];
+        Values v;
 #pragma unroll
         for (int i = 0; i < EPT; i++) {
-            const float x = arow[min(k0 + a_k + i, g.k - 1u)];
-            const float y = g.b[(size_t)min(k0 + b_k + i, g.k - 1u) * g.ldb + min(col0 + b_col, g.n - 1u)];
-            pa[i] = k0 + a_k + i < g.k ? x : 0.f, pb[i] = k0 + b_k + i < g.k ? y : 0.f;
+            const uint32_t ka = min(k0 + a_k + i, g.k - 1u), kb = min(k0 + b_k + i, g.k - 1u);
+            const float x = arow[ka], y = bmat[(size_t)kb * g.ldb + b_at];
+            v.a[i] = k0 + a_k + i < g.k ? x : 0.f, v.b[i] = k0 + b_k + i < g.k ? y : 0.f;
+            if constexpr (NORM) v.w[i] = g.norm_w[ka];
         }
-        park(pa, pb, 0); /* the loop ended on a barrier */
+        park(v, 0, true); /* the loop ended on a barrier */
         __syncthreads();
         Fragments f;
         read(0, f);
         multiply(f);
         __syncthreads();
+    }
+    if constexpr (NORM) { /* the threads of a row are neighbours */
+#pragma unroll
+        for (uint32_t d = 1u; d < TK / EPT; d *= 2u) ss += __shfl_xor(ss, (int)d, 64);
+        if (tid % (TK / EPT) == 0u) row_ss[a_row] = ss;
     }
 
     /* the tile buffers are free */
@@ -249,6 +287,8 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
             acc[i / WT][i % WT][r] += meet[(i * 16 + r) * 64];
             bad |= !isfinite(acc[i / WT][i % WT][r]);
         }
+    const bool gate_wave = GATED && wc == 1u;
+    const uint32_t wave_col = col0 + (GATED ? 0u : wc * (32u * WT));
     if (__any(bad)) {
         /* something is not finite: the quadrant again on the fp32 instructions, which tell infinities from NaN */
 #pragma unroll
@@ -256,19 +296,51 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
 #pragma unroll
             for (int j = 0; j < WT; j++) {
                 const float *ar = g.a + (size_t)min(row0 + 32u * (WT * wr + i) + c, g.m - 1u) * g.lda;
-                const float *bc = g.b + min(col0 + 32u * (WT * wc + j) + c, g.n - 1u);
+                const float *bc = (gate_wave ? g.b2 : g.b) + min(wave_col + 32u * j + c, g.n - 1u);
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
                 for (uint32_t k = h; k < g.k + h; k += 2u) { /* an odd K ends with a product of zeros */
-                    const float x = k < g.k ? ar[k] : 0.f, y = k < g.k ? bc[(size_t)k * g.ldb] : 0.f;
+                    float x = k < g.k ? ar[k] : 0.f;
+                    const float y = k < g.k ? bc[(size_t)k * g.ldb] : 0.f;
+                    if (NORM && k < g.k) x *= g.norm_w[k];
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y, x, acc[i][j], 0, 0, 0);
                 }
             }
     }
+    if constexpr (NORM) {
+#pragma unroll
+        for (int i = 0; i < WT; i++) {
+            const float scale = 1.0f / sqrtf(row_ss[32u * (WT * wr + i) + c] / (float)g.k + 1e-6f); /* reductions_cpu.c:345-346 */
+#pragma unroll
+            for (int j = 0; j < WT; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] *= scale;
+        }
+    }
+    MatmulArgs to = g;
+    if constexpr (GATED) {
+        if (g.out2 == nullptr) { /* the waves of the second group have left: these four meet */
+            if (gate_wave) {
+#pragma unroll
+                for (int i = 0; i < WT * WT; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) meet[(i * 16 + r) * 64] = acc[i / WT][i % WT][r];
+            }
+            __syncthreads();
+            if (gate_wave) return;
+            const float *gates = meet + WT * WT * 16u * 64u; /* of the wave to the right */
+#pragma unroll
+            for (int i = 0; i < WT * WT; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i / WT][i % WT][r] = silu_times(gates[(i * 16 + r) * 64], acc[i / WT][i % WT][r]);
+        } else if (gate_wave) {
+            to.out = g.out2, to.residual = nullptr;
+        }
+    }
 
-    /* lane (h, c) holds out[row0 + 32*(WT*wr + i) + c][col0 + 32*(WT*wc + j) + 8*q + 4*h + 0..3] in acc[i][j][4q..4q+3] */
-    const bool vst = VEC && g.n % 4u == 0u && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(g.out) & 15u) == 0u) &&
-                     ((reinterpret_cast<uintptr_t>(g.residual) & 15u) == 0u);
+    /* lane (h, c) holds out[row0 + 32*(WT*wr + i) + c][wave_col + 32*j + 8*q + 4*h + 0..3] in acc[i][j][4q..4q+3] */
+    const bool vst = VEC && g.n % 4u == 0u && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(to.out) & 15u) == 0u) &&
+                     ((reinterpret_cast<uintptr_t>(to.residual) & 15u) == 0u);
 #pragma unroll
     for (int i = 0; i < WT; i++) {
         const uint32_t row = row0 + 32u * (WT * wr + i) + c;
@@ -277,7 +349,7 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
         for (int j = 0; j < WT; j++)
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                store4<ROPE>(g, row, col0 + 32u * (WT * wc + j) + 8u * q + 4u * h,
+                store4<ROPE>(to, row, wave_col + 32u * j + 8u * q + 4u * h,
                              make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
                                          acc[i][j][4 * q + 3]),
                              vst);
@@ -746,7 +818,6 @@ void launch_splitk(const MatmulArgs &g_in, dim3 grid, hipStream_t s) {
 
 } // namespace
 
-bool matmul_takes_gated(const MatmulArgs &g) { return choose_path(g) != PATH_MFMA; }
 bool matmul_takes_cross(const MatmulArgs &g) {
     if (g.b2 || g.residual || (g.rope_cos != nullptr && g.rope_cols > 0) || g.cross_head_dim == 0u ||
         g.n % g.cross_head_dim != 0u)
@@ -755,14 +826,11 @@ bool matmul_takes_cross(const MatmulArgs &g) {
     if (path == PATH_SKINNY) return g.n <= 256u && g.cross_head_dim <= 256u;
     return path == PATH_SPLITK && g.cross_head_dim == 32u && g.n % 32u == 0u && g.k % 4u == 0u;
 }
-bool matmul_takes_norm(const MatmulArgs &g) {
-    const Path path = choose_path(g);
-    return path == PATH_SPLITK || (path == PATH_SKINNY && g.k <= SKINNY_KC);
-}
+bool matmul_takes_norm(const MatmulArgs &g) { return choose_path(g) != PATH_SKINNY || g.k <= SKINNY_KC; }
 
 namespace {
 bool vec_ok(const MatmulArgs &g) {
-    return aligned16(g.a) && aligned16(g.b) && g.lda % 4u == 0 && g.ldb % 4u == 0 && g.k % 4u == 0 && g.n % 4u == 0;
+    return aligned16(g.a) && aligned16(g.b) && aligned16(g.norm_w) && g.lda % 4u == 0 && g.ldb % 4u == 0 && g.k % 4u == 0 && g.n % 4u == 0;
 }
 } // namespace
 
@@ -786,17 +854,31 @@ void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStrea
 }
 
 namespace {
-template <bool VEC, bool ROPE, int WT>
-void launch_mfma(const MatmulArgs &g, hipStream_t s) {
-    constexpr uint32_t BT = MfmaShape<WT>::BT;
-    const dim3 grid((g.n + BT - 1u) / BT, (g.m + BT - 1u) / BT);
+template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED>
+void launch_mfma_as(const MatmulArgs &g, hipStream_t s) {
+    constexpr uint32_t BT = MfmaShape<WT>::BT, COLS = GATED ? BT / 2u : BT;
+    const dim3 grid((g.n + COLS - 1u) / COLS, (g.m + BT - 1u) / BT);
     constexpr size_t lds = MfmaShape<WT>::LDS_BYTES;
-    if constexpr (lds > 64u * 1024u) { /* above 64 KB a kernel has to ask for its LDS first */
-        static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void *>(matmul_mfma_kernel<VEC, ROPE, WT>),
-                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const auto kernel = matmul_mfma_kernel<VEC, ROPE, WT, NORM, GATED>;
+    if constexpr (lds > 64u * 1024u - 512u) { /* from 64 KB on a kernel has to ask for its LDS first */
+        static const hipError_t asked =
+            hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         HIP_CHECK(asked);
     }
-    blt_launch("matmul_mfma", matmul_mfma_kernel<VEC, ROPE, WT>, grid, dim3(512), lds, s, g);
+    blt_launch("matmul_mfma", kernel, grid, dim3(512), lds, s, g);
+}
+template <bool VEC, int WT>
+void launch_mfma(const MatmulArgs &g, bool rope, hipStream_t s) {
+    if (g.b2) {
+        if (g.norm_w) launch_mfma_as<VEC, false, WT, true, true>(g, s);
+        else launch_mfma_as<VEC, false, WT, false, true>(g, s);
+    } else if (rope) {
+        if (g.norm_w) launch_mfma_as<VEC, true, WT, true, false>(g, s);
+        else launch_mfma_as<VEC, true, WT, false, false>(g, s);
+    } else {
+        if (g.norm_w) launch_mfma_as<VEC, false, WT, true, false>(g, s);
+        else launch_mfma_as<VEC, false, WT, false, false>(g, s);
+    }
 }
 } // namespace
 
@@ -804,7 +886,7 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
     if (g.m == 0 || g.n == 0) return;
     const bool rope = g.rope_cos != nullptr && g.rope_cols > 0;
     const Path path = choose_path(g);
-    BLT_REQUIRE(g.b2 == nullptr || path != PATH_MFMA, "matmul: the gated product is not available for this shape");
+    BLT_REQUIRE(g.b2 == nullptr || !rope, "matmul: a gated product is not rotated");
     BLT_REQUIRE(g.norm_w == nullptr || matmul_takes_norm(g), "matmul: the fused row norm is not available for this shape");
     if (path == PATH_SKINNY) {
         BLT_REQUIRE(g.cross_k == nullptr || (matmul_takes_cross(g) && g.cross_v && g.cross_out && g.cross_lo &&
@@ -837,24 +919,15 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
      * splits and reads twice as much per output: the large tile once its rounds are at least three quarters full
      * (2048 x 512 . 512 x 1536, 192 tiles: 27.9 us against 28.6; 2048 columns, 256 tiles: 31.2 against 36.9; 1024
      * columns, 128 tiles of K = 256: 15.2 against 11.4). */
-    const uint64_t big_tiles = (uint64_t)((g.n + 127u) / 128u) * ((g.m + 127u) / 128u);
+    const uint32_t big_cols = g.b2 ? 64u : 128u;
+    const uint64_t big_tiles = (uint64_t)((g.n + big_cols - 1u) / big_cols) * ((g.m + 127u) / 128u);
     const bool big = big_tiles >= (big_tiles + 255u) / 256u * 192u;
     if (big) {
-        if (rope) {
-            if (vec) launch_mfma<true, true, 2>(g, s);
-            else launch_mfma<false, true, 2>(g, s);
-        } else {
-            if (vec) launch_mfma<true, false, 2>(g, s);
-            else launch_mfma<false, false, 2>(g, s);
-        }
-        return;
-    }
-    if (rope) {
-        if (vec) launch_mfma<true, true, 1>(g, s);
-        else launch_mfma<false, true, 1>(g, s);
+        if (vec) launch_mfma<true, 2>(g, rope, s);
+        else launch_mfma<false, 2>(g, rope, s);
     } else {
-        if (vec) launch_mfma<true, false, 1>(g, s);
-        else launch_mfma<false, false, 1>(g, s);
+        if (vec) launch_mfma<true, 1>(g, rope, s);
+        else launch_mfma<false, 1>(g, rope, s);
     }
 }
 

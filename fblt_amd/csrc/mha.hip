@@ -303,25 +303,15 @@ extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_t
     g.out = (float *)act.data;
     g.m = (uint32_t)T, g.k = (uint32_t)E, g.n = (uint32_t)hidden;
     g.lda = (uint32_t)E, g.ldb = g.ldo = (uint32_t)hidden;
-    if (matmul_takes_gated(g) && matmul_takes_norm(g)) { /* norm, up, gate and the activation in one pass */
-        g.b2 = (const float *)w->ffn_gate_w->data;
+    g.b2 = (const float *)w->ffn_gate_w->data;
+    if (matmul_takes_norm(g)) { /* norm, up, gate and the activation in one pass */
         g.norm_w = (const float *)w->norm2_weight->data;
-        matmul_f32_launch(g, 0);
     } else {
         blt_tensor normed = blt_tensor_create_uninit(arena, embed_shape, 2, BLT_DTYPE_FP32);
         blt_rmsnorm_forward_hip(&attn_residual, w->norm2_weight, &normed);
         g.a = (const float *)normed.data;
-        if (matmul_takes_gated(g)) {
-            g.b2 = (const float *)w->ffn_gate_w->data;
-            matmul_f32_launch(g, 0);
-        } else {
-            blt_tensor gate = blt_tensor_create_uninit(arena, hidden_shape, 2, BLT_DTYPE_FP32);
-            matmul_f32_launch(g, 0);
-            g.b = (const float *)w->ffn_gate_w->data, g.out = (float *)gate.data;
-            matmul_f32_launch(g, 0);
-            blt_swiglu_forward_hip(&gate, &act, &act);
-        }
     }
+    matmul_f32_launch(g, 0);
     std::memset(&g, 0, sizeof(g));
     g.a = (const float *)act.data;
     g.b = (const float *)w->ffn_down_w->data;
@@ -342,8 +332,7 @@ extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_t
  *
  *   1. q = query_in * weight_q;
  *   2. k = kv_in * weight_k and v = kv_in * weight_v in one pass over kv_in
- *      (two launches when the product is large enough for the 64x64 kernel;
- *      at small sizes 1 and 2 share one launch);
+ *      (at small sizes 1 and 2 share one launch);
  *   3. all heads in one attention launch.  The mask configuration is reduced
  *      on the host to one key range per query row (a patch sees the bytes of
  *      its own group, which are contiguous) and uploaded as 8 bytes per row;
@@ -418,15 +407,7 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
         matmul_f32_launch_pair(g, gkv, 0); /* all three in one launch */
     } else {
         matmul_f32_launch(g, 0);
-        if (T != 0 && matmul_takes_gated(gkv)) {
-            matmul_f32_launch(gkv, 0);
-        } else if (T != 0) {
-            gkv.b2 = nullptr, gkv.out2 = nullptr;
-            matmul_f32_launch(gkv, 0);
-            gkv.b = (const float *)weights->weight_v->data;
-            gkv.out = v;
-            matmul_f32_launch(gkv, 0);
-        }
+        if (T != 0) matmul_f32_launch(gkv, 0);
     }
 
     /* 3. mask as row ranges when it reduces, then every head in one launch */
