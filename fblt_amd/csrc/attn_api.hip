@@ -457,6 +457,7 @@ void plan_launch(const blt_attention_plan &pl, const AttnProb *dev, const AttnTi
  * thread's ring of buffers (blt_upload_staged). */
 struct Staging {
     blt_attention_plan plan;
+    std::vector<unsigned char> both; /* descriptors and tiles */
     void *device = nullptr;
     size_t capacity = 0;
 
@@ -485,8 +486,10 @@ struct Staging {
         /* the device copy is rewritten in stream order, behind the kernels of the previous call that
          * read it; the host side goes through the ring of pinned buffers, so consecutive calls do
          * not wait for each other */
-        blt_upload_staged(device, plan.host.data(), pbytes);
-        if (tbytes) blt_upload_staged(static_cast<char *>(device) + pbytes, plan.tiles.data(), tbytes);
+        both.resize(need); /* one upload, not two */
+        __builtin_memcpy(both.data(), plan.host.data(), pbytes);
+        if (tbytes) __builtin_memcpy(both.data() + pbytes, plan.tiles.data(), tbytes);
+        blt_upload_staged(device, both.data(), need);
         plan_launch(plan, static_cast<const AttnProb *>(device),
                     reinterpret_cast<const AttnTile *>(static_cast<const char *>(device) + pbytes));
     }

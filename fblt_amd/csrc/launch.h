@@ -22,8 +22,8 @@ bool blt_stream_capturing();
  * the stream the thread was on when it began (the one the graph will be replayed on). */
 hipStream_t blt_stream_key();
 /* Host-to-device copy that returns at once and lets the caller reuse `src`
- * right away: the bytes go through a small ring of pinned buffers owned by
- * the calling thread (memory.hip).  Not usable while a graph is captured. */
+ * right away: a few kilobytes travel in kernel arguments, more goes through a small ring of
+ * pinned buffers owned by the calling thread (memory.hip).  Not usable while a graph is captured. */
 void blt_upload_staged(void *dst, const void *src, size_t bytes);
 /* Turns a sticky error the KV step kernels raised on the device (a sequence outgrew what its
  * launch, slab or rotation tables hold) into the fatal error; costs one 4-byte read-back, and
