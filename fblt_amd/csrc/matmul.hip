@@ -742,10 +742,11 @@ Path choose_path(const MatmulArgs &g) {
      * (bit-identical results) */
     constexpr uint32_t exact_rows = 32u;
     if (g.m <= exact_rows && !rope && !g.tolerant) return PATH_SKINNY;
-    /* up to 143 64x64 tiles (a bit over half the compute units): quarter tiles, K split over the
-     * waves.  Measured at K = 512 ... 4096: a fifth faster than the 64x64 kernel at 128 tiles, level
-     * with it at 144 ... 192, a quarter slower at 256 */
-    constexpr uint64_t splitk_below = 144u;
+    /* up to 111 64x64 tiles (a bit under half the compute units), 79 of a pair of products: quarter tiles, K split
+     * over the waves.  Measured in whole blocks: 108 tiles of K = 128 a tenth of a product faster than on the tile kernel,
+     * 128 ... 132 tiles of K = 256 ... 1024 a tenth slower; pairs of 72 tiles of K = 128 faster, of 80 and 128
+     * tiles of K = 256 and 512 slower (block of 200 rows of 512: 54.8 -> 49.7 us on the tile kernel). */
+    const uint64_t splitk_below = g.b2 ? 80u : 112u;
     if ((uint64_t)((g.n + TN - 1) / TN) * ((g.m + TM - 1) / TM) < splitk_below) return PATH_SPLITK;
     return PATH_MFMA;
 }
