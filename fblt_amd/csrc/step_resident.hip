@@ -874,11 +874,11 @@ bool kv_step_resident(const StepResident &st) {
     if (group_rows > MAX_GROUP_ROWS || st.batch > MAX_ROWS) return false;
     /* Where the launches win, measured over E, heads, layers, rows and lengths (us, launches -> resident, four
      * layers).  Up to 16 rows a group and heads of 32: everywhere (E = 64: 113 -> 50 at one row, 133 -> 82 at 96;
-     * E = 256: 155 -> 93, 254 -> 231 at 64 rows of 900 keys).  17 to 32 rows: one sequence (E = 128: 222 -> 208)
-     * or narrow (E = 64: 140 -> 126); eight groups of wide rows have 256 compute units' worth of product in the
-     * launches (E = 256: 229 -> 282).  Heads of 64 have half the keys per wave in flight: single rows of few
+     * E = 256: 155 -> 93, 254 -> 231 at 64 rows of 900 keys).  17 to 32 rows: narrow models only (E = 64: 140 ->
+     * 126), the products of wide ones have all compute units in the launches (E = 256: 25 rows 227 -> 247, eight
+     * groups of 32 rows 229 -> 282).  Heads of 64 have half the keys per wave in flight: single rows of few
      * sequences a group (E = 256, 20 sequences: 187 -> 162; 64 of 900 keys: 251 -> 343). */
-    if (group_rows > 16 && st.batch > 1 && E > 64) return false;
+    if (group_rows > 16 && E > 64) return false;
     if (hd == 64 && (st.n > 1 || per_group > 4)) return false;
     if (st.row_index != nullptr && st.batch != 1) return false;
     const size_t hidden = dec->layers[0].ffn_up_w.shape[1];
