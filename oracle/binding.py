@@ -25,7 +25,7 @@ _sp = C.POINTER(C.c_size_t)
 def build(ref=True):
     """Compile the checker (and the reference build when its sources exist)."""
     subprocess.check_call(["make", "-s", "-B", "-C", HERE, "all"])
-    if ref and os.path.isdir(os.environ.get("REF_ROOT", "/root/reference")):
+    if ref and os.path.isdir(os.path.join(os.environ.get("REF_ROOT", "/root/reference"), "csrc")):
         subprocess.check_call(["make", "-s", "-B", "-C", HERE, "ref"])
         if os.path.exists(os.path.join(HERE, "..", "fblt_amd", "lib", "libfblt_hip.so")):
             subprocess.check_call(["make", "-s", "-C", HERE, "callers", "stack_callers", "model_callers", "model_driver"])
