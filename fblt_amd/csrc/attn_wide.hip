@@ -636,12 +636,16 @@ uint32_t items_of(const AttnProb &d, bool tall) {
     return in_pairs(d) ? (G + 1u) / 2u : G;
 }
 
+/* the 32 rows of a K or V tile are reached by 32-bit byte offsets */
+constexpr uint32_t WIDE_MAX_STRIDE = 0xFFFFFFFFu / 4u / 32u - 64u;
+
 } // namespace
 
 /* shapes the kernel is able to run */
 bool attn_wide_can(const AttnProb &d) {
     return (d.hd == 32u || d.hd == 64u) && (d.flags & ATTN_FLAG_VEC4) != 0 && d.weights == nullptr &&
-           d.vis != ATTN_VIS_RANGE && d.nk >= 1u && d.nq >= 1u && d.nq <= 0xFFFEu * 128u; /* group indices travel in 16 bits */
+           d.vis != ATTN_VIS_RANGE && d.nk >= 1u && d.nq >= 1u && d.nq <= 0xFFFEu * 128u && /* group indices travel in 16 bits */
+           d.k_stride <= WIDE_MAX_STRIDE && d.v_stride <= WIDE_MAX_STRIDE;
 }
 
 uint32_t attn_wide_groups(const AttnProb &d) { return groups_of(d, false); }

@@ -747,6 +747,8 @@ Path choose_path(const MatmulArgs &g) {
      * 128 ... 132 tiles of K = 256 ... 1024 a tenth slower; pairs of 72 tiles of K = 128 faster, of 80 and 128
      * tiles of K = 256 and 512 slower (block of 200 rows of 512: 54.8 -> 49.7 us on the tile kernel). */
     const uint64_t splitk_below = g.b2 ? 80u : 112u;
+    /* the tile kernel reaches the 32 rows of b of a step by 32-bit byte offsets, this one computes addresses in 64 bits */
+    if (g.ldb > 0xFFFFFFFFu / 4u / TK) return PATH_SPLITK;
     if ((uint64_t)((g.n + TN - 1) / TN) * ((g.m + TM - 1) / TM) < splitk_below) return PATH_SPLITK;
     return PATH_MFMA;
 }
@@ -793,10 +795,11 @@ bool slice_scratch(MatmulArgs &g, size_t tiles, hipStream_t s) {
  * to about 256 workgroups, and more made it slower again. */
 uint32_t slices_for(const MatmulArgs &g, dim3 grid, bool eight) {
     if (g.b2 || g.cross_k || g.norm_w) return 1u;
-    const uint32_t chunks = (g.k + 31u) / 32u, tiles = grid.x * grid.y;
+    const uint32_t chunks = (g.k + 31u) / 32u;
+    const uint64_t tiles = (uint64_t)grid.x * grid.y;
     const uint32_t room = chunks / (eight ? 8u : 4u);
     if (chunks < 32u || tiles > 128u) return 1u;
-    return std::max(1u, std::min(room, 256u / tiles));
+    return std::max(1u, std::min(room, 256u / (uint32_t)tiles));
 }
 
 template <bool VEC, bool ROPE>
@@ -956,6 +959,12 @@ extern "C" void blt_matmul_hip(const blt_tensor *a, const blt_tensor *b, blt_ten
     g.out = (float *)out->data;
     g.m = (uint32_t)m, g.k = (uint32_t)k, g.n = (uint32_t)n;
     g.lda = (uint32_t)k, g.ldb = (uint32_t)n, g.ldo = (uint32_t)n;
-    matmul_f32_launch(g, 0);
+    /* a grid holds fewer than 2^32 threads in x, up to sixteen of them a column */
+    constexpr uint32_t most = 1u << 27;
+    for (size_t at = 0; at < n; at += most) {
+        g.b = (const float *)b->data + at, g.out = (float *)out->data + at;
+        g.n = (uint32_t)std::min<size_t>(n - at, most);
+        matmul_f32_launch(g, 0);
+    }
     HIP_CHECK_LAUNCH("blt_matmul");
 }

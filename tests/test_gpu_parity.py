@@ -959,6 +959,46 @@ def test_matmul_on_split_operands(m, k, n, dev):
     assert_close(got[big][:, :n - 1].cpu().numpy(), first[big][:, :n - 1].cpu().numpy(), "beside the bad values")
 
 
+@pytest.mark.parametrize("m,k,n", [(40, 33, (1 << 25) + 64), (33, 1, (1 << 27) + 5)])
+def test_matmul_of_very_wide_matrices(m, k, n, dev):
+    """More than 2^25 columns: the rows of b of one K step lie more than 2^32 bytes apart; more than 2^27: the columns
+    go in several launches.  A sample of columns, the first and the last against float64."""
+    import torch
+    lib = api.load()
+    a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
+    out = torch.full((m, n), 7.0, device="cuda")
+    va, vb, vo = _dev_tensor(a), _dev_tensor(b), _dev_tensor(out)
+    torch.cuda.synchronize()
+    lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    lib.blt_backend_pass_sync_hip()
+    cols = torch.cat([torch.arange(64), torch.randint(0, n, (4096,)), (1 << 25) + torch.arange(-64, 64),
+                      torch.arange(n - 64, n)]).clamp_(0, n - 1).cuda()
+    assert_close(out[:, cols].cpu().numpy(), (a.double() @ b[:, cols].double()).cpu().numpy(), "matmul %dx%dx%d" % (m, k, n))
+
+
+def test_attention_over_rows_far_apart(dev):
+    """Batches large enough for the throughput kernel whose K and V rows are more than 2^27 bytes apart (a tile of 32 rows
+    spans more than 2^32)."""
+    import torch
+    lib = api.load()
+    nq, nk, hd, count, stride = 160, 40, 32, 330, (1 << 25) + 4
+    slab = torch.empty(nk * stride, device="cuda")
+    rows = slab.view(nk, stride)[:, :2 * hd]
+    rows.copy_(torch.randn(nk, 2 * hd, device="cuda"))
+    q, out = torch.randn(count, nq, hd, device="cuda"), torch.full((count, nq, hd), 7.0, device="cuda")
+    scale = float(hd) ** -0.5
+    probs = [api.problem(api.head_args(q[i].data_ptr(), slab.data_ptr(), slab.data_ptr() + 4 * hd, out[i].data_ptr(), nq, nk, hd,
+                                       scale, hd, stride, stride, hd, 0, lse=None), api.BLT_ATTN_MASK_CAUSAL)
+             for i in range(count)]
+    torch.cuda.synchronize()
+    lib.blt_attention_batch_hip(api.problem_array(probs), count)
+    lib.blt_backend_pass_sync_hip()
+    k, v = rows[:, :hd].double().cpu(), rows[:, hd:].double().cpu()
+    s = (q.double().cpu() @ k.T) * scale
+    s.masked_fill_(torch.triu(torch.ones(nq, nk, dtype=torch.bool), 1), -float("inf"))
+    assert_close(out.cpu().numpy(), (torch.softmax(s, -1) @ v).numpy(), "rows far apart")
+
+
 @pytest.mark.parametrize("T,H,hd,docs", [(200, 2, 32, [0, 7, 90, 150]), (512, 4, 32, [0, 300]), (128, 8, 64, [0]),
                                          (96, 2, 64, [0, 20, 40, 60, 80])])
 def test_document_causal_ranges_take_the_matrix_cores(T, H, hd, docs, oracle, dev):
