@@ -315,7 +315,8 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
     if (STAGE && kt < kt_hi) K_PARK(kt);
     bool bad = false; /* met a score that is not finite */
     /* ---- scale, mask, running maximum: scores of tile kt -> weights ---- */
-    auto weigh = [&](const floatx16 &sacc, uint32_t tile, float (&x)[16]) __attribute__((always_inline)) {
+    /* unit: of the score registers */
+    auto weigh = [&](const floatx16 &sacc, float unit, uint32_t tile, float (&x)[16]) __attribute__((always_inline)) {
         const uint32_t k0 = tile * 32u;
         float mt = neg_inf();
         const bool all_seen = !DENSE && k0 >= flo && k0 + 32u <= fhi; /* uniform: no row masks any key */
@@ -327,8 +328,8 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         for (int r = 0; r < 16; r++) {
             const uint32_t j = k0 + acc_key(r, h);
             float t;
-            if (DENSE) t = (sacc[r] * p.scale + mrow[min(j, p.nk - 1u)]) * LOG2E;
-            else t = sacc[r] * scale2;
+            if (DENSE) t = (sacc[r] * (p.scale * unit) + mrow[min(j, p.nk - 1u)]) * LOG2E;
+            else t = sacc[r] * (scale2 * unit);
             const bool fin = isfinite(t);
             const bool vis = ((j - vlo) < vlen) & fin;
             bad |= DENSE ? !isfinite(sacc[r]) : !fin;
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         if (!STAGE && ktn < kt_hi) K_REQUEST(ktn);
 
         float x[16];
-        const float alpha = weigh(sacc, kt, x);
+        const float alpha = weigh(sacc, SPLIT_DOWN, kt, x);
 
         /* ---- O^T = O^T * alpha + V^T P^T ---- */
 #pragma unroll
@@ -398,9 +399,12 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
 #pragma unroll
     for (int b = 0; b < DB; b++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) bad |= !isfinite(oacc[b][r]);
+        for (int r = 0; r < 16; r++) {
+            bad |= !isfinite(oacc[b][r]);
+            oacc[b][r] *= SPLIT_DOWN;
+        }
     if (__any(bad)) {
-        /* something is not finite: this wave's tiles once more on the fp32 instructions, which tell infinities from NaN */
+        /* something is not finite, or too large for the scaled sums: this wave's tiles once more on the fp32 instructions, which tell infinities from NaN */
         m = neg_inf(), l = 0.f;
 #pragma unroll
         for (int b = 0; b < DB; b++)
@@ -417,7 +421,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
             for (int r = 0; r < 16; r++) sacc[r] = 0.f;
 #pragma unroll
             for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s], q[s], sacc, 0, 0, 0);
-            const float alpha = weigh(sacc, kt, x);
+            const float alpha = weigh(sacc, 1.0f, kt, x);
             fetch_v(kt);
 #pragma unroll
             for (int b = 0; b < DB; b++) {

@@ -327,7 +327,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
     flo = __builtin_amdgcn_readfirstlane(flo);
     fhi = __builtin_amdgcn_readfirstlane(fhi);
 
-    const float scale2 = p.scale * LOG2E;
+    const float scale2 = p.scale * LOG2E * SPLIT_UP;
     const float *mrow = DENSE ? p.mask + (size_t)i * p.nk : nullptr;
     const bool mvec = DENSE && (p.nk % 4u == 0u) && ((reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0u);
 
@@ -340,7 +340,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
             const float4 a = *reinterpret_cast<const float4 *>(qrow + 16 * s), b = *reinterpret_cast<const float4 *>(qrow + 16 * s + 4);
             const float x[8] = {a.x * scale2, a.y * scale2, a.z * scale2, a.w * scale2,
                                 b.x * scale2, b.y * scale2, b.z * scale2, b.w * scale2};
-            split_bf16<8>(x, qf[s][0], qf[s][1], qf[s][2]);
+            split_bf16_scaled<8>(x, qf[s][0], qf[s][1], qf[s][2]);
         }
     }
 
@@ -350,6 +350,8 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
 #pragma unroll
         for (int r = 0; r < 16; r++) oacc[b][r] = 0.f;
     float m = neg_inf(), l = 0.f;
+    bool bad = false;
+    constexpr float unit = DENSE ? 1.0f : SPLIT_DOWN; /* of the score registers */
 
     /* ---- tile movement: 256 threads carry EPT values of one K row each, 256 EPT keys of one V column each (of eight
      * waves the first four K and the others V) ---- */
@@ -476,13 +478,16 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
                 const uint32_t rel = k0 + 4u * h - lo, len = hi - lo;
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    if (DENSE) sacc[r] += mk[r] * LOG2E;
+                    if (DENSE) {
+                        bad |= !isfinite(sacc[r]); /* behind the mask a score that overflowed downwards looks masked */
+                        sacc[r] = sacc[r] * SPLIT_DOWN + mk[r] * LOG2E;
+                    }
                     sacc[r] = rel + (8u * (r >> 2) + (r & 3u)) < len ? sacc[r] : neg_inf();
                 }
             }
 #pragma unroll
             for (int r = 0; r < 16; r++) mt = fmaxf(mt, sacc[r]);
-            mt = swap32(mt, OpMax());
+            mt = swap32(mt, OpMax()) * unit;
             const float mn = fmaxf(m, mt);
             const float ms = mn == neg_inf() ? 0.f : mn; /* nothing seen yet: keep the differences finite */
             if (__any(mn > m)) {
@@ -503,7 +508,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
                 float x[8];
 #pragma unroll
                 for (int r = 0; r < 8; r++) {
-                    x[r] = fast_exp2(sacc[8 * j + r] - ms);
+                    x[r] = fast_exp2(sacc[8 * j + r] * unit - ms);
                     ps += x[r];
                 }
                 bf16x8 pf[3];
@@ -534,14 +539,15 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
 
     /* both halves of a column carry the same m, their sums add */
     l = swap32(l, OpSum());
-    bool bad = !isfinite(l);
+    /* no weight at all on keys that a row sees: its scores are not finite, or overflowed downwards */
+    bad |= !isfinite(l) || (!DENSE && l == 0.f && hi > lo);
 #pragma unroll
     for (int b = 0; b < DB; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) bad |= !isfinite(oacc[b][r]);
     if (bad || !live) return bad;
 
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const float inv = l > 0.f ? SPLIT_DOWN / l : 0.f;
     float *orow = p.out + (size_t)i * p.out_stride;
 #pragma unroll
     for (int b = 0; b < DB; b++)

@@ -1,8 +1,14 @@
 /*
- * fp32 contractions on the bf16 matrix instructions.
+ * fp32 contractions on the bf16 matrix instructions: the operands as sums of lower-precision terms, the
+ * products of the leading terms added in fp32 (the splitting of Dekker 1971, as used for matrix units by
+ * Markidis et al. 2018 and Henry, Tang and Heinecke 2019, "Leveraging the bfloat16 artificial intelligence
+ * datatype for higher-precision computations").
  *
- * An fp32 value is the exact sum of three bf16 values (each rounded to nearest from what the ones
- * before leave; 8 significant bits each, 24 in all).  A product of two such sums is taken as the six
+ * SPLIT_UP times an fp32 value is the exact sum of three bf16 values (each rounded to nearest from what the ones
+ * before leave; 8 significant bits each, 24 in all).  The factor keeps that true down to the smallest subnormal:
+ * the last bit of any fp32 value is a multiple of 2^-149, the smallest bf16 subnormal 2^-133 (the matrix
+ * instructions take bf16 subnormals as they are).  Unscaled, operands of 1e-36 had a relative error of 2.7e-5, of
+ * 1e-38 of 2.7e-3.  Results come out SPLIT_UP^2 times as large; SPLIT_DOWN takes that back.  A product of two such sums is taken as the six
  * partial products that are at least 2^-18 of it,
  *     x y = h h' + (h m' + m h') + (h l' + l h' + m m')  (+ m l' + l m' + l l', below 2^-25)
  * accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  Against float64 the result is a little closer than
@@ -11,8 +17,9 @@
  * Six bf16 instructions take 192 cycles of the matrix unit where the fp32 ones take 512, and they leave
  * the vector ALU free, which the fp32 ones do not.
  *
- * A value that is not finite, or rounds to infinity in bf16 (above 3.39e38), leaves NaN in the lower parts
- * and so in every result it takes part in: the caller looks for results that are not finite.
+ * A value that is not finite, or is above 5.1e33 and rounds to infinity in bf16 once scaled, leaves NaN in the lower
+ * parts and so in every result it takes part in; a result above 7.9e28 overflows before it is scaled back.  The
+ * caller looks for results that are not finite and computes those on the fp32 instructions.
  */
 #ifndef FBLT_AMD_SPLIT_BF16_H
 #define FBLT_AMD_SPLIT_BF16_H
@@ -23,11 +30,13 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-/* N values -> their three parts.  (v_dot2_f32_bf16 would take a part off in one instruction instead of a shift or mask and
+constexpr float SPLIT_UP = 0x1p16f, SPLIT_DOWN = 0x1p-32f;
+
+/* N values, SPLIT_UP times what they stand for -> their three parts.  (v_dot2_f32_bf16 would take a part off in one instruction instead of a shift or mask and
  * a subtraction, but it runs in the matrix unit's place: twelve matrix instructions with eight of each in
  * between take 228 ns with conversions, 211 with shifts, 394 with it.) */
 template <int N, typename Vec>
-__device__ __forceinline__ void split_bf16(const float (&x)[N], Vec &high, Vec &mid, Vec &low) {
+__device__ __forceinline__ void split_bf16_scaled(const float (&x)[N], Vec &high, Vec &mid, Vec &low) {
     uint32_t *const out[3] = {reinterpret_cast<uint32_t *>(&high), reinterpret_cast<uint32_t *>(&mid), reinterpret_cast<uint32_t *>(&low)};
 #pragma unroll
     for (int i = 0; i < N; i += 2) {
@@ -42,6 +51,15 @@ __device__ __forceinline__ void split_bf16(const float (&x)[N], Vec &high, Vec &
     }
 }
 
+/* ... of plain values */
+template <int N, typename Vec>
+__device__ __forceinline__ void split_bf16(const float (&x)[N], Vec &high, Vec &mid, Vec &low) {
+    float y[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) y[i] = x[i] * SPLIT_UP;
+    split_bf16_scaled<N>(y, high, mid, low);
+}
+
 /* ... of N consecutive ones of a register array */
 template <int N, int M>
 __device__ __forceinline__ void split_bf16_at(const float (&x)[M], int first, bf16x8 (&parts)[3]) {
@@ -51,7 +69,7 @@ __device__ __forceinline__ void split_bf16_at(const float (&x)[M], int first, bf
     split_bf16<N>(y, parts[0], parts[1], parts[2]);
 }
 
-/* acc += A B over 16 of K, smallest partial products first */
+/* acc += SPLIT_UP^2 A B over 16 of K, smallest partial products first */
 template <typename Acc>
 __device__ __forceinline__ Acc mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b)[3], Acc acc) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], acc, 0, 0, 0);

@@ -959,6 +959,59 @@ def test_matmul_on_split_operands(m, k, n, dev):
     assert_close(got[big][:, :n - 1].cpu().numpy(), first[big][:, :n - 1].cpu().numpy(), "beside the bad values")
 
 
+def _relative(got, ref):
+    return float((got.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-36, 1.0), (1.0, 1e-38), (1e-40, 1e33), (1e-37, 1e30), (1e16, 1e16)])
+@pytest.mark.parametrize("m,k,n", [(1024, 6, 1024), (1030, 512, 1026), (2048, 33, 2048)])
+def test_matmul_over_the_range_of_fp32(m, k, n, scale_a, scale_b, dev):
+    """Products on bf16 parts hold their operands in all 24 bits down to subnormals, and results too large for the
+    scaled sums are as close: within what a chain of k fp32 additions gives (2^-24 sqrt(k) and a factor of three for
+    the roundings of the operands' products)."""
+    import torch
+    lib = api.load()
+    a, b = torch.randn(m, k, device="cuda") * scale_a, torch.randn(k, n, device="cuda") * scale_b
+    out = torch.full((m, n), 7.0, device="cuda")
+    va, vb, vo = _dev_tensor(a), _dev_tensor(b), _dev_tensor(out)
+    torch.cuda.synchronize()
+    lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    lib.blt_backend_pass_sync_hip()
+    assert _relative(out, a.double() @ b.double()) <= 3 * 2.0 ** -24 * max(k, 4) ** 0.5
+
+
+@pytest.mark.parametrize("scale_q,scale_k,scale_v", [(1.0, 1.0, 1.0), (1.0, 1.0, 1e-36), (1e-33, 1e33, 1.0), (1e-36, 1e36, 1.0),
+                                                     (1e36, 1e-36, 1.0), (1.0, 1.0, 1e33), (0.0, 0.0, 1.0)])
+@pytest.mark.parametrize("T,H,hd,batch", [(300, 1, 48, 1), (300, 1, 128, 1), (256, 4, 32, 80), (256, 4, 64, 80), (2304, 4, 32, 16)])
+def test_attention_over_the_range_of_fp32(T, H, hd, batch, scale_q, scale_k, scale_v, dev):
+    """Attention on bf16 parts (the latency kernel, the throughput kernel with four and eight waves) with tiny and huge
+    operands, outputs and scores too large for the scaled sums: within ten times 2^-24 sqrt(hd), the rounding of a score of
+    a few units.  Scale 0: all scores -1e30, every visible key weighs the same."""
+    import torch
+    lib = api.load()
+    qkv = [torch.randn(batch, H, T, hd, device="cuda") * s for s in (scale_q, scale_k, scale_v)]
+    if scale_q == 0.0:
+        qkv[0].fill_(1e15)
+        qkv[1].fill_(-1e15)
+    q, k, v = qkv
+    out = torch.full_like(q, 7.0)
+    scale = float(np.float32(hd) ** np.float32(-0.5))
+    probs = [api.problem(api.head_args(*(t[b, h].data_ptr() for t in (q, k, v, out)), T, T, hd, scale, hd, hd, hd, hd, 0),
+                         api.BLT_ATTN_MASK_CAUSAL) for b in range(batch) for h in range(H)]
+    plan = lib.blt_attention_plan_create_hip(api.problem_array(probs), len(probs))
+    name = lib.blt_attention_plan_kernel_hip(plan).decode()
+    torch.cuda.synchronize()
+    lib.blt_attention_plan_run_hip(plan)
+    lib.blt_backend_pass_sync_hip()
+    lib.blt_attention_plan_destroy_hip(plan)
+    assert ("mfma" if batch == 1 else "wide") in name, name
+    hidden = torch.triu(torch.ones(T, T, dtype=torch.bool, device="cuda"), 1)
+    for b in range(0, batch, 15):
+        s = (q[b].double() @ k[b].double().transpose(1, 2).contiguous()) * scale
+        ref = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ v[b].double()
+        assert _relative(out[b], ref) <= 10 * 2.0 ** -24 * hd ** 0.5, (b, name)
+
+
 @pytest.mark.parametrize("m,k,n", [(40, 33, (1 << 25) + 64), (33, 1, (1 << 27) + 5)])
 def test_matmul_of_very_wide_matrices(m, k, n, dev):
     """More than 2^25 columns: the rows of b of one K step lie more than 2^32 bytes apart; more than 2^27: the columns
