@@ -313,7 +313,10 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         for (int s = 0; s < QS; s++) split_bf16_at<8>(q, 8 * s, qf[s]);
     }
     if (STAGE && kt < kt_hi) K_PARK(kt);
-    bool bad = false; /* met a score that is not finite */
+    /* Scores of one or two products are closer on the fp32 instructions (as the products of matmul.hip; heads of one, error
+     * of the output against float64 1.4 ... 2.6e-7 on parts, 1.0 ... 2.0e-7): only the second run below */
+    const bool few = !EXACT && p.hd < 3u;
+    bool bad = few; /* met a score that is not finite */
     /* ---- scale, mask, running maximum: scores of tile kt -> weights ---- */
     /* unit: of the score registers */
     auto weigh = [&](const floatx16 &sacc, float unit, uint32_t tile, float (&x)[16]) __attribute__((always_inline)) {
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         return alpha;
     };
     /* The contractions run on three bf16 parts of their operands. */
-    while (kt < kt_hi) {
+    while (kt < kt_hi && !few) {
         const uint32_t ktn = kt + NW;
 
         if (STAGE) {

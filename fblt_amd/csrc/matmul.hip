@@ -757,6 +757,9 @@ Path choose_path(const MatmulArgs &g) {
     const uint64_t splitk_below = g.b2 ? 80u : 112u;
     /* the tile kernel reaches the 32 rows of b of a step by 32-bit byte offsets, this one computes addresses in 64 bits */
     if (g.ldb > 0xFFFFFFFFu / 4u / TK) return PATH_SPLITK;
+    /* one or two products an element: three parts drop the bits that fp32 rounds them to (error against float64 3.5e-8
+     * and 3.4e-8, on the fp32 instructions 2.5e-8 and 3.1e-8; from three on the parts are closer, 3.3e-8 against 3.6e-8) */
+    if (g.k < 3u) return PATH_SPLITK;
     if ((uint64_t)((g.n + TN - 1) / TN) * ((g.m + TM - 1) / TM) < splitk_below) return PATH_SPLITK;
     return PATH_MFMA;
 }
@@ -962,17 +965,16 @@ extern "C" void blt_matmul_hip(const blt_tensor *a, const blt_tensor *b, blt_ten
     BLT_REQUIRE(m <= 0x7FFFFFFFu && k <= 0x7FFFFFFFu && n <= 0x7FFFFFFFu, "matmul: dimensions exceed 2^31-1");
     MatmulArgs g;
     __builtin_memset(&g, 0, sizeof(g));
-    g.a = (const float *)a->data;
-    g.b = (const float *)b->data;
-    g.out = (float *)out->data;
-    g.m = (uint32_t)m, g.k = (uint32_t)k, g.n = (uint32_t)n;
+    g.k = (uint32_t)k;
     g.lda = (uint32_t)k, g.ldb = (uint32_t)n, g.ldo = (uint32_t)n;
-    /* a grid holds fewer than 2^32 threads in x, up to sixteen of them a column */
-    constexpr uint32_t most = 1u << 27;
-    for (size_t at = 0; at < n; at += most) {
-        g.b = (const float *)b->data + at, g.out = (float *)out->data + at;
-        g.n = (uint32_t)std::min<size_t>(n - at, most);
-        matmul_f32_launch(g, 0);
-    }
+    /* a grid holds fewer than 2^32 threads in x, up to sixteen of them a column, and 65535 workgroups in y, of 32 rows and more */
+    constexpr size_t most_cols = 1u << 27, most_rows = 1u << 20;
+    for (size_t row = 0; row < m; row += most_rows)
+        for (size_t col = 0; col < n; col += most_cols) {
+            g.a = (const float *)a->data + row * k, g.b = (const float *)b->data + col;
+            g.out = (float *)out->data + row * n + col;
+            g.m = (uint32_t)std::min(m - row, most_rows), g.n = (uint32_t)std::min(n - col, most_cols);
+            matmul_f32_launch(g, 0);
+        }
     HIP_CHECK_LAUNCH("blt_matmul");
 }

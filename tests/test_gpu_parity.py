@@ -980,9 +980,27 @@ def test_matmul_over_the_range_of_fp32(m, k, n, scale_a, scale_b, dev):
     assert _relative(out, a.double() @ b.double()) <= 3 * 2.0 ** -24 * max(k, 4) ** 0.5
 
 
+@pytest.mark.parametrize("m,k,n", [(1024, 1, 1024), (1500, 2, 700), (2048, 3, 2048), (1024, 4, 1024)])
+def test_matmul_of_few_products(m, k, n, dev):
+    """One and two products an element are as close as fp32 makes them: a single one correctly rounded (uniform rounding
+    errors have a root mean square of 2^-24 / sqrt(12) of the power of two below the value, less over random values: 2.6e-8
+    is what correct rounding of a normal product gives), two 3.2e-8; three and four on parts no worse than two roundings."""
+    import torch
+    lib = api.load()
+    a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
+    out = torch.full((m, n), 7.0, device="cuda")
+    va, vb, vo = _dev_tensor(a), _dev_tensor(b), _dev_tensor(out)
+    torch.cuda.synchronize()
+    lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    lib.blt_backend_pass_sync_hip()
+    if k == 1:
+        assert torch.equal(out, a * b)
+    assert _relative(out, a.double() @ b.double()) <= (2.6e-8 if k == 1 else 3.2e-8 if k == 2 else 3.6e-8)
+
+
 @pytest.mark.parametrize("scale_q,scale_k,scale_v", [(1.0, 1.0, 1.0), (1.0, 1.0, 1e-36), (1e-33, 1e33, 1.0), (1e-36, 1e36, 1.0),
                                                      (1e36, 1e-36, 1.0), (1.0, 1.0, 1e33), (0.0, 0.0, 1.0)])
-@pytest.mark.parametrize("T,H,hd,batch", [(300, 1, 48, 1), (300, 1, 128, 1), (256, 4, 32, 80), (256, 4, 64, 80), (2304, 4, 32, 16)])
+@pytest.mark.parametrize("T,H,hd,batch", [(300, 1, 1, 1), (300, 1, 2, 1), (300, 1, 48, 1), (300, 1, 128, 1), (256, 4, 32, 80), (256, 4, 64, 80), (2304, 4, 32, 16)])
 def test_attention_over_the_range_of_fp32(T, H, hd, batch, scale_q, scale_k, scale_v, dev):
     """Attention on bf16 parts (the latency kernel, the throughput kernel with four and eight waves) with tiny and huge
     operands, outputs and scores too large for the scaled sums: within ten times 2^-24 sqrt(hd), the rounding of a score of
@@ -1012,10 +1030,11 @@ def test_attention_over_the_range_of_fp32(T, H, hd, batch, scale_q, scale_k, sca
         assert _relative(out[b], ref) <= 10 * 2.0 ** -24 * hd ** 0.5, (b, name)
 
 
-@pytest.mark.parametrize("m,k,n", [(40, 33, (1 << 25) + 64), (33, 1, (1 << 27) + 5)])
+@pytest.mark.parametrize("m,k,n", [(40, 33, (1 << 25) + 64), (33, 1, (1 << 27) + 5), (40, 5, (1 << 27) + 5),
+                                   ((1 << 22) + 70, 2, 64)])
 def test_matmul_of_very_wide_matrices(m, k, n, dev):
-    """More than 2^25 columns: the rows of b of one K step lie more than 2^32 bytes apart; more than 2^27: the columns
-    go in several launches.  A sample of columns, the first and the last against float64."""
+    """More than 2^25 columns: the rows of b of one K step lie more than 2^32 bytes apart; more than 2^27 columns or 2^20
+    rows go in several launches.  A sample of columns, the first and the last against float64."""
     import torch
     lib = api.load()
     a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
@@ -1025,7 +1044,7 @@ def test_matmul_of_very_wide_matrices(m, k, n, dev):
     lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
     lib.blt_backend_pass_sync_hip()
     cols = torch.cat([torch.arange(64), torch.randint(0, n, (4096,)), (1 << 25) + torch.arange(-64, 64),
-                      torch.arange(n - 64, n)]).clamp_(0, n - 1).cuda()
+                      torch.arange(n - 64, n)]).clamp_(0, n - 1).unique().cuda()
     assert_close(out[:, cols].cpu().numpy(), (a.double() @ b[:, cols].double()).cpu().numpy(), "matmul %dx%dx%d" % (m, k, n))
 
 
