@@ -406,7 +406,12 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
             bad |= !isfinite(oacc[b][r]);
             oacc[b][r] *= SPLIT_DOWN;
         }
-    if (__any(bad)) {
+    /* Weights come from the scores their maximum and sum were taken from, by the same instructions: with weights the
+     * waves decide together, and the query is at hand after the output may have been stored in its place. */
+    const bool again = p.weights ? __syncthreads_or(bad) != 0 : __any(bad) != 0;
+    float q[HALF];
+    if (again) {
+        query_row(q);
         /* something is not finite, or too large for the scaled sums: this wave's tiles once more on the fp32 instructions, which tell infinities from NaN */
         m = neg_inf(), l = 0.f;
 #pragma unroll
@@ -417,8 +422,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
             K_REQUEST(kt);
             K_PARK(kt);
             if (STAGE) frag_from_lds<HD>(kf, my_k, h, c);
-            float q[HALF], x[16];
-            query_row(q);
+            float x[16];
             floatx16 sacc;
 #pragma unroll
             for (int r = 0; r < 16; r++) sacc[r] = 0.f;
@@ -551,8 +555,13 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
     float *wrow = p.weights + (size_t)i * p.nk;
     const bool wvec = (p.nk % 4u == 0u) && ((reinterpret_cast<uintptr_t>(p.weights) & 15u) == 0u);
     const uint32_t nkt = (p.nk + 31u) / 32u;
-    float q[HALF];
-    query_row(q);
+    if constexpr (STAGE) { /* from LDS, instead of keeping it in registers */
+        query_row(q);
+        if (!again) {
+#pragma unroll
+            for (int s = 0; s < QS; s++) split_bf16_at<8>(q, 8 * s, qf[s]);
+        }
+    }
     for (uint32_t wt = wave; wt < nkt; wt += NW) {
         const uint32_t k0 = wt * 32u;
         float w[16];
@@ -567,14 +576,24 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
             floatx16 sacc;
 #pragma unroll
             for (int r = 0; r < 16; r++) sacc[r] = 0.f;
+            if (again) {
 #pragma unroll
-            for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s], q[s], sacc, 0, 0, 0);
+                for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s], q[s], sacc, 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int s = 0; s < QS; s++) {
+                    bf16x8 parts[3];
+                    split_bf16_at<8>(kf, 8 * s, parts);
+                    sacc = mfma_split(parts, qf[s], sacc);
+                }
+            }
+            const float unit = again ? 1.0f : SPLIT_DOWN;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const uint32_t j = k0 + acc_key(r, h);
                 float t;
-                if (DENSE) t = (sacc[r] * p.scale + mrow[min(j, p.nk - 1u)]) * LOG2E;
-                else t = sacc[r] * scale2;
+                if (DENSE) t = (sacc[r] * (p.scale * unit) + mrow[min(j, p.nk - 1u)]) * LOG2E;
+                else t = sacc[r] * (scale2 * unit);
                 const bool vis = j >= lo && j < hi && isfinite(t);
                 w[r] = vis ? fast_exp2(t - M) * invL : 0.f;
             }

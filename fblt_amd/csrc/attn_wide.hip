@@ -282,8 +282,8 @@ struct WideTiles {
     __bf16 k[3][KPART], v[3][VPART];
 };
 
-/* One group of 32 WV rows of problem p, WV waves.  Returns whether this lane's row met something that is not finite;
- * nothing of the row is stored then.
+/* One group of 32 WV rows of problem p, WV waves.  Returns whether any of its rows met something that is not finite;
+ * nothing is stored then.
  *
  * The keys of a V tile lie in the order in which a lane half holds its scores (accumulator register r of half h
  * is key acc_key(r, h)): position 16 j + 8 h + i is the key of register 8 j + i, so the weights of a lane are the
@@ -545,7 +545,9 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
     for (int b = 0; b < DB; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) bad |= !isfinite(oacc[b][r]);
-    if (bad || !live) return bad;
+    /* together, before anything is stored: the output may lie in place of the queries, which the second run reads */
+    if (__syncthreads_or(bad)) return true;
+    if (!live) return false;
 
     const float inv = l > 0.f ? SPLIT_DOWN / l : 0.f;
     float *orow = p.out + (size_t)i * p.out_stride;
@@ -603,8 +605,7 @@ __global__ __launch_bounds__(64 * WV, 2) void attn_wide_kernel(const AttnProb *_
     for (int pass = 0; pass < 2; pass++) {
         const uint32_t group = pass == 0 ? ga : gb;
         if (group == WIDE_NO_GROUP) break;
-        const bool bad = wide_group<HD, WV, DENSE>(p, group, *reinterpret_cast<WideTiles<HD>(*)[2]>(sm));
-        if (__syncthreads_or(bad)) {
+        if (wide_group<HD, WV, DENSE>(p, group, *reinterpret_cast<WideTiles<HD>(*)[2]>(sm))) {
             float (*const tiles32)[TILE] = reinterpret_cast<float (*)[TILE]>(sm);
             wide_group_checked<HD, WV, DENSE>(p, group, tiles32, tiles32 + 2);
         }

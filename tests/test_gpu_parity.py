@@ -959,6 +959,51 @@ def test_matmul_on_split_operands(m, k, n, dev):
     assert_close(got[big][:, :n - 1].cpu().numpy(), first[big][:, :n - 1].cpu().numpy(), "beside the bad values")
 
 
+@pytest.mark.parametrize("T,hd,dense", [(300, 48, False), (300, 128, False), (1200, 32, True), (1200, 64, False), (130, 2, False)])
+def test_weights_and_output_share_their_scores(T, hd, dense, dev):
+    """Weights taken after the output: they sum to one even where scores are large (a score of a thousand has a rounding
+    error of 6e-5, which cancels only if maximum, sum and weight use the same score), and an output stored in place of the
+    queries does not change them."""
+    import torch
+    lib = api.load()
+    q, k, v = (torch.randn(T, hd, device="cuda") * s for s in (30.0, 3.0, 1.0))
+    out, weights = torch.full_like(q, 7.0), torch.full((2, T, T), 7.0, device="cuda")
+    mask = torch.triu(torch.full((T, T), -float("inf"), device="cuda"), 1) if dense else None
+    scale = float(hd) ** -0.5
+
+    def run(to, w):
+        a = api.head_args(q.data_ptr(), k.data_ptr(), v.data_ptr(), to.data_ptr(), T, T, hd, scale, hd, hd, hd, hd, 0,
+                          weights=w.data_ptr(), mask=mask.data_ptr() if dense else None, causal=not dense)
+        torch.cuda.synchronize()
+        lib.blt_attention_head_core(abi.BLT_BACKEND_HIP, C.byref(a))
+        lib.blt_backend_pass_sync_hip()
+
+    run(out, weights[0])
+    # nk roundings of 2^-24 of weights that sum to one, at random, and the exponentials' own
+    assert float((weights[0].double().sum(-1) - 1).abs().max()) <= 6e-7
+    run(q, weights[1])
+    assert torch.equal(weights[0], weights[1]) and torch.equal(out, q)
+
+
+@pytest.mark.parametrize("T,H,hd,batch", [(256, 4, 32, 80), (256, 4, 64, 80), (2304, 4, 32, 16), (300, 1, 128, 1)])
+def test_second_run_reads_queries_in_place_of_the_output(T, H, hd, batch, dev):
+    """One query row that is not finite sends its group through the kernels' second run; with the output in place of the
+    queries it gives what it gives beside them."""
+    import torch
+    lib = api.load()
+    q, k, v = (torch.randn(batch, H, T, hd, device="cuda") for _ in range(3))
+    q[0, 0, T // 2 + 3, 1] = float("inf")
+    got = []
+    for to in (torch.full_like(q, 7.0), q):
+        probs = [api.problem(api.head_args(*(t[b, h].data_ptr() for t in (q, k, v, to)), T, T, hd, float(hd) ** -0.5, hd, hd, hd,
+                                           hd, 0), api.BLT_ATTN_MASK_CAUSAL) for b in range(batch) for h in range(H)]
+        torch.cuda.synchronize()
+        lib.blt_attention_batch_hip(api.problem_array(probs), len(probs))
+        lib.blt_backend_pass_sync_hip()
+        got.append(to)
+    assert torch.equal(got[0], got[1]) and bool(torch.isfinite(got[0]).all())
+
+
 def _relative(got, ref):
     return float((got.double() - ref).norm() / ref.norm())
 
