@@ -294,8 +294,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
             const float4 x = *reinterpret_cast<const float4 *>(&part_ss[buf][row][v]);
             s += (x.x + x.y) + (x.z + x.w);
         }
-        const float x = s * (1.0f / (float)E) + 1e-6f, y = __builtin_amdgcn_rsqf(x); /* reductions_cpu.c:345-346 */
-        return y * (1.5f - 0.5f * x * y * y); /* one Newton step on the unit's estimate: an exact root and division are 40 instructions */
+        return 1.0f / sqrtf(s * (1.0f / (float)E) + 1e-6f); /* reductions_cpu.c:345-346 */
     };
     using All = std::integral_constant<uint32_t, WAVES>;
     using One = std::integral_constant<int, 1>;
@@ -326,9 +325,8 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
                 const float *s0 = all, *s1 = all + KB, *st0 = all + 2 * KB, *st1 = all + 2 * KB + 2;
                 const float M = fmaxf(st0[0], st1[0]), Ms = M == neg_inf() ? 0.f : M;
                 const float f0 = fast_exp2(st0[0] - Ms), f1 = fast_exp2(st1[0] - Ms), Lt = st0[1] * f0 + st1[1] * f1;
-                const float inv = Lt > 0.f ? 1.0f / Lt : 0.f;
 #pragma unroll
-                for (int i = 0; i < KB; i++) av[rt][i] = (s0[i] * f0 + s1[i] * f1) * inv;
+                for (int i = 0; i < KB; i++) av[rt][i] = Lt > 0.f ? (s0[i] * f0 + s1[i] * f1) / Lt : 0.f;
             }
         } else {
             operand(Steps(), src, KB * wave, tag, av);

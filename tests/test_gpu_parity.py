@@ -1871,18 +1871,15 @@ def test_kv_decode_step_long_prefill(window, oracle, dev):
         lib.blt_arena_destroy(arena)
 
 
-@pytest.mark.parametrize("batch,n,case", [(8, 1, 0), (64, 1, 2), (16, 4, 1), (5, 3, 3), (64, 8, 2),
-                                          (3, 40, 4), (5, 33, 5)])   # chunks of more than 32 rows per sequence
-def test_kv_decode_step_batched(batch, n, case, oracle, dev):
-    """blt_kv_decode_step_batched_hip: every sequence of a batched cache in one pass, against the
-    restated step run sequence by sequence; two steps in a row."""
+def _decode_steps(batch, n, c, seed, oracle, row_scale=1.0):
+    """Two steps of a batched cache against the restated step run sequence by sequence; the kernels each step launched."""
     import torch
     from fblt_amd import decoder
     lib = api.load()
-    c = STEP_CASES[case]
+    launched = []
     E, V, k, L, max_len = c["E"], c["V"], c["k"], c["L"], c["max_len"]
     rs = np.random.RandomState(500 + batch + n)
-    host, device = _decoders(oracle, c, 600 + case)
+    host, device = _decoders(oracle, c, seed)
     mine = decoder.HostCache(host, max_len, batch)
     arena = lib.blt_arena_create(256 << 20, abi.BLT_BACKEND_HIP)
     try:
@@ -1916,7 +1913,7 @@ def test_kv_decode_step_batched(batch, n, case, oracle, dev):
         num = abi.size_array(counts)
         for step in range(2):
             closed = (C.c_int * batch)(*([0] * batch if step == 0 else rs.randint(0, 2, size=batch).tolist()))
-            rows = rs.randn(batch * n, E).astype(np.float32)
+            rows = (rs.randn(batch * n, E) * row_scale).astype(np.float32)
             ref = np.zeros((batch * n, V), dtype=np.float32)
             for b in range(batch):
                 r = np.ascontiguousarray(rows[b * n:(b + 1) * n])
@@ -1929,10 +1926,13 @@ def test_kv_decode_step_batched(batch, n, case, oracle, dev):
             tl = torch.full((batch * n, V), 7.0, dtype=torch.float32, device="cuda")
             vd, vl = _dev_tensor(td), _dev_tensor(tl)
             arena.contents.offset = mark
+            lib.blt_hip_profile_begin()
             lib.blt_kv_decode_step_batched_hip(cache, self_len, table_ptrs, num, closed, C.byref(vd), C.byref(vl), arena)
+            launched.append(sorted(api.profile_end()))
             lib.blt_backend_pass_sync_hip()
             assert [self_len[b] for b in range(batch)] == (lens + (step + 1) * n).tolist()
-            assert_close(tl.cpu().numpy(), ref, "batched step %d logits" % step)
+            # the absolute term of the tolerance is for rows of order one
+            assert_close(tl.cpu().numpy() / np.float32(row_scale), ref / np.float32(row_scale), "batched step %d logits" % step)
             for name in ("self_k", "self_v", "cross_k", "cross_v"):
                 for l in range(L):
                     assert_close(_tier(lib, cache, name, l, batch * max_len, E), mine.tiers[name][l],
@@ -1940,6 +1940,15 @@ def test_kv_decode_step_batched(batch, n, case, oracle, dev):
         lib.blt_kv_cache_destroy(cache)
     finally:
         lib.blt_arena_destroy(arena)
+    return launched
+
+
+@pytest.mark.parametrize("batch,n,case", [(8, 1, 0), (64, 1, 2), (16, 4, 1), (5, 3, 3), (64, 8, 2),
+                                          (3, 40, 4), (5, 33, 5)])   # chunks of more than 32 rows per sequence
+def test_kv_decode_step_batched(batch, n, case, oracle, dev):
+    """blt_kv_decode_step_batched_hip: every sequence of a batched cache in one pass, against the
+    restated step run sequence by sequence; two steps in a row."""
+    _decode_steps(batch, n, STEP_CASES[case], 600 + case, oracle)
 
 
 RESIDENT_CASES = [
@@ -1952,13 +1961,29 @@ RESIDENT_CASES = [
 ]
 
 
-@pytest.mark.parametrize("batch,n,case", [(1, 32, 0), (8, 17, 0), (33, 1, 0), (1, 1, 1), (32, 1, 1),   # rows of a group 1 ... 32,
-                                          (1, 17, 2), (1, 1, 2), (9, 8, 2), (17, 1, 3),               # one and two shares of the
-                                          (1, 32, 4), (8, 16, 4), (64, 1, 4), (1, 1, 5), (30, 1, 5)])   # keys, heads of 32 and 64
-def test_kv_decode_step_in_one_launch(batch, n, case, oracle, dev, monkeypatch):
+ONE_LAUNCH = ["kv_step_resident"]
+
+
+@pytest.mark.parametrize("batch,n,case", [(1, 32, 0), (8, 17, 0), (33, 1, 0), (1, 1, 1), (32, 1, 1),   # rows of a group 1 ... 32 at
+                                          (1, 16, 2), (1, 1, 2), (9, 8, 2), (17, 1, 3),               # 64 columns, 1 ... 16 at 128 and
+                                          (1, 11, 4), (8, 16, 4), (64, 1, 4), (1, 1, 5), (30, 1, 5)])   # 256, heads of 32 and 64
+def test_kv_decode_step_in_one_launch(batch, n, case, oracle, dev):
     """The one-launch form of the step at the edges of its shapes, against the restated step."""
-    monkeypatch.setitem(globals(), "STEP_CASES", RESIDENT_CASES)
-    test_kv_decode_step_batched(batch, n, case, oracle, dev)
+    assert _decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle) == [ONE_LAUNCH] * 2
+
+
+@pytest.mark.parametrize("batch,n,case", [(1, 17, 2), (1, 32, 4), (9, 2, 3), (40, 1, 5), (9, 17, 0)])
+def test_kv_decode_step_past_one_launch(batch, n, case, oracle, dev):
+    """One row more than the one-launch form takes: the launches, against the restated step."""
+    launched = _decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle)
+    assert all("kv_step_resident" not in names for names in launched), launched
+
+
+@pytest.mark.parametrize("batch,n,case", [(1, 1, 2), (9, 8, 2), (33, 1, 0)])
+def test_kv_decode_step_of_rows_whose_norm_overflows(batch, n, case, oracle, dev):
+    """Input rows of 1e20: their sum of squares is infinite and the normalised row zero, in the one-launch form as in
+    the restated step."""
+    assert _decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle, row_scale=1e20) == [ONE_LAUNCH] * 2
 
 
 def test_graph_replay_of_a_plan_and_a_decode_layer(oracle, dev):
