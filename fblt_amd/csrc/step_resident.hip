@@ -838,17 +838,20 @@ std::atomic<bool> g_launched{false};
 
 template <int E, int HD>
 void launch_resident(uint32_t row_tiles, uint32_t blocks, hipStream_t s, const ResidentArgs &a) {
-    if (row_tiles == 1u) blt_launch("kv_step_resident", kv_step_resident_kernel<E, HD, 1>, dim3(blocks), dim3(64 * WAVES), 0, s, a);
-    else blt_launch("kv_step_resident", kv_step_resident_kernel<E, HD, 2>, dim3(blocks), dim3(64 * WAVES), 0, s, a);
+    if constexpr (E == 64 && HD == 32) { /* the only shape that takes more than 16 rows a group */
+        if (row_tiles == 2u) {
+            blt_launch("kv_step_resident", kv_step_resident_kernel<E, HD, 2>, dim3(blocks), dim3(64 * WAVES), 0, s, a);
+            return;
+        }
+    }
+    blt_launch("kv_step_resident", kv_step_resident_kernel<E, HD, 1>, dim3(blocks), dim3(64 * WAVES), 0, s, a);
 }
 uint32_t group_words(uint32_t E, uint32_t row_tiles, uint32_t hidden) {
     switch (E * 4u + row_tiles) {
     case 64 * 4 + 1: return Regions<64, 1>::total(hidden);
     case 64 * 4 + 2: return Regions<64, 2>::total(hidden);
     case 128 * 4 + 1: return Regions<128, 1>::total(hidden);
-    case 128 * 4 + 2: return Regions<128, 2>::total(hidden);
-    case 256 * 4 + 1: return Regions<256, 1>::total(hidden);
-    default: return Regions<256, 2>::total(hidden);
+    default: return Regions<256, 1>::total(hidden);
     }
 }
 
