@@ -32,10 +32,17 @@
  * fragments through the wave's LDS tile, exact online softmax per wave, waves merged through LDS, shares merged by the
  * reader.
  *
- * Every wait is bounded (SPIN_LIMIT polls, then the wave raises a word in pinned host memory, stops
- * waiting for the rest of the launch and runs to its end; the host turns the word into a fatal error).  The
- * launcher never lets two of these launches run at the same time on one device, and a launch is at
- * most 512 workgroups that fit two per compute unit, so all of its workgroups become resident.
+ * Who waits.  A launch is up to 512 workgroups, two per compute unit, and nothing promises that they all become
+ * resident: another kernel may keep its place for as long as it likes, another process may run this very step.  So
+ * nobody waits for a workgroup that has not started.  The workgroups of a group call the roll first: each has a word
+ * in which it signs in, and who finds the time up before everybody has signs the others out.  If all are in, each has the
+ * role its index gives it.  Else those that are in take all the work among them, stage by stage in the same order (any
+ * number can: the first unfinished stage waits for nothing unfinished), and who finds itself signed out leaves.  The
+ * fewer are in, the longer it is worth waiting: 20 us for the last one, 1.3 ms for the second.
+ *
+ * Every wait is bounded all the same (SPIN_LIMIT polls, then the wave raises a word in pinned host memory, stops
+ * waiting for the rest of the launch, takes NaN for what it did not get and runs to its end; the host turns the word
+ * into a fatal error at its next look).
  *
  * Measured, launches -> this kernel: one row, two layers of 128 columns, 300 keys 69 -> 37 us; 64 such rows 78 ->
  * 60 us; 16 draft rows of one sequence 80 -> 61 us.  What is left is the chain: a hand-over takes about 1 us from
@@ -52,9 +59,13 @@
 #include "rope_device.h"
 #include "step_resident.h"
 
+#include <unistd.h>
+
 #include <algorithm>
 #include <atomic>
-#include <mutex>
+#include <cstdlib>
+#include <cstring>
+#include <map>
 
 namespace {
 
@@ -67,6 +78,7 @@ constexpr uint32_t MAX_GROUP_ROWS = 32;
 constexpr uint32_t MAX_ROWS = GROUPS * MAX_GROUP_ROWS;
 constexpr uint32_t MAX_SPLITS_R = 2; /* shares of a (sequence, head)'s keys */
 constexpr uint32_t SPIN_LIMIT = 1u << 22; /* polls, about half a microsecond each */
+constexpr uint32_t ROLL_LIMIT = 2000; /* ticks of 10 ns */
 constexpr uint32_t MAX_HIDDEN = 1024;
 
 struct ResidentLayer {
@@ -83,15 +95,16 @@ struct ResidentArgs {
     float *logits;
     const float *cos, *sin;
     uint64_t *words;   /* hand-over words, group_words per group */
+    uint64_t *rolls;   /* a word per workgroup, 2 WORKERS per group */
     uint32_t *timeout; /* pinned host word */
     uint64_t group_words;
     uint64_t max_seq, slab_x; /* rows per sequence of the tier-1 / tier-2 slabs */
     uint32_t L, E, H, hidden, V;
     uint32_t batch, n, per_group; /* sequences, rows per sequence, sequences per group */
     uint32_t splits;              /* shares of the keys */
-    uint32_t attn_workers;        /* workgroups per group for the self-attention, after WORKERS for the products */
     uint32_t subtokens, window, block_kind;
     uint32_t tag; /* tag of layer 0; layer l uses tag + l */
+    uint32_t roll_limit, spin_limit;
     uint32_t indexed; /* rows come from d0 + row_index[r] * E and sit at position[r] (one sequence) */
     float scale;      /* log2(e) / sqrt(head_dim) */
     float xscale;     /* 1 / sqrt(head_dim) */
@@ -131,8 +144,10 @@ __device__ __forceinline__ uint32_t operand_at(uint32_t row, uint32_t k) {
 /* A wave's waiting state: once one wait has run out, none of the wave's later ones wait. */
 struct Waiter {
     uint32_t *timeout;
+    uint32_t limit;
     bool expired;
 };
+__device__ __forceinline__ float not_there() { return __builtin_nanf(""); }
 
 /* N words per lane, the one number i at(i), until every lane that is not `pad` has them all.  A wave that
  * misses some looks again after a sleep: at all of them while they are few, else at the last one only
@@ -156,18 +171,22 @@ __device__ __forceinline__ void await_at(Waiter &wt, At at, bool pad, uint32_t t
                 __builtin_amdgcn_s_sleep(1);
                 missing = ((uint32_t)(word_load(at(N - 1)) >> 32) != tag) & !pad;
                 spin++;
-            } while (__any(missing) && spin < SPIN_LIMIT);
+            } while (__any(missing) && spin < wt.limit);
         } else {
             __builtin_amdgcn_s_sleep(1);
         }
         __builtin_amdgcn_s_setprio(2);
-        if (spin >= SPIN_LIMIT) {
+        if (spin >= wt.limit) {
             wt.expired = true;
             __hip_atomic_store(wt.timeout, (blockIdx.x << 16) | line, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 #pragma unroll
     for (int i = 0; i < N; i++) out[i] = __uint_as_float((uint32_t)t[i]); /* pad lanes: anything */
+    if (wt.expired) {
+#pragma unroll
+        for (int i = 0; i < N; i++) out[i] = not_there();
+    }
 }
 /* word `index` of a region: a uniform base and a 32-bit byte offset per lane, which the load takes as they are */
 __device__ __forceinline__ const uint64_t *word_of(const uint64_t *base, uint32_t index) {
@@ -203,18 +222,33 @@ struct ResidentShape {
     static constexpr int AREA = 2 * PART > ATTN ? 2 * PART : ATTN;
 };
 
-constexpr uint32_t WORKERS = 32; /* product workgroups of a group: one per compute unit of a die */
+constexpr uint32_t WORKERS = 32; /* workgroups of a group for the products, and as many for the self-attention: one of each per compute unit of a die */
 /* Tile 0 of a stage goes to this worker, tile 1 to the next: consecutive stages on different workgroups, so
  * that the ones of a stage have its weights in registers and are looking for its operand when the stage before
  * finishes. */
 constexpr uint32_t FIRST_XQ = 24, FIRST_XPROJ = 0, FIRST_QKV = 8, FIRST_PROJ = 0, FIRST_UPGATE = 16, FIRST_DOWN = 8, FIRST_LM = 16;
 
+/* Stages of a layer in their order, and the LM head behind the last layer */
+enum Stage : uint32_t { STAGE_XQ, STAGE_XPROJ, STAGE_QKV, STAGE_ATTN, STAGE_PROJ, STAGE_UPGATE, STAGE_DOWN, STAGES, STAGE_LM = STAGES };
+/* What a call of a role works on: everything, or one stage (STAGES of layer L: the LM head). */
+struct WholeStep {
+    __device__ __forceinline__ uint32_t begin() const { return 0u; }
+    __device__ __forceinline__ uint32_t end(uint32_t L) const { return L; }
+    __device__ __forceinline__ bool has(Stage) const { return true; }
+};
+struct OneStage {
+    uint32_t layer, stage;
+    __device__ __forceinline__ uint32_t begin() const { return layer; }
+    __device__ __forceinline__ uint32_t end(uint32_t L) const { return min(layer + 1u, L); }
+    __device__ __forceinline__ bool has(Stage st) const { return st == stage; }
+};
+
 /* The workgroups that run the products: every stage but the self-attention.  A stage of a worker: its weights,
  * the operand as soon as it is there, the product over the wave's share of K, the waves' partial tiles through
  * LDS, the results of 256 threads per row tile. */
-template <int E, int HD, int RT>
-__device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, float *area, float (*part_ss)[16 * RT][WAVES],
-                                             float (*xquery)[HD]) {
+template <int E, int HD, int RT, typename Share>
+__device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, const Share sh, float *area,
+                                             float (*part_ss)[16 * RT][WAVES], float (*xquery)[HD]) {
     using At = Regions<E, RT>;
     using Shape = ResidentShape<HD, RT>;
     constexpr int QD = HD / 4, DT = HD / 16, H = E / HD;
@@ -236,7 +270,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
     };
     fresh_lane();
     uint64_t *const words = gv.words;
-    Waiter wt{args->timeout, false};
+    Waiter wt{args->timeout, args->spin_limit, false};
     uint32_t buf = 0;
 
     /* the left operand of this wave's KBN steps from step kb_lo on */
@@ -326,7 +360,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
                 const float M = fmaxf(st0[0], st1[0]), Ms = M == neg_inf() ? 0.f : M;
                 const float f0 = fast_exp2(st0[0] - Ms), f1 = fast_exp2(st1[0] - Ms), Lt = st0[1] * f0 + st1[1] * f1;
 #pragma unroll
-                for (int i = 0; i < KB; i++) av[rt][i] = Lt > 0.f ? (s0[i] * f0 + s1[i] * f1) / Lt : 0.f;
+                for (int i = 0; i < KB; i++) av[rt][i] = Lt == 0.f ? 0.f : (s0[i] * f0 + s1[i] * f1) / Lt;
             }
         } else {
             operand(Steps(), src, KB * wave, tag, av);
@@ -351,13 +385,13 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
     auto first = [&](uint32_t at) { return (gv.worker - at) & (WORKERS - 1u); };
 
     const uint32_t L = args->L;
-    for (uint32_t layer = 0; layer < L; layer++) {
+    for (uint32_t layer = sh.begin(); layer < sh.end(L); layer++) {
         ArgsPtr ap = hidden_args(args);
         const uint32_t tag = ap->tag + layer;
         const bool crossed = ap->layer[layer].xq != nullptr, plain = layer == 0u;
         const uint32_t in = At::input(layer);
 
-        if (crossed && first(FIRST_XQ) < (uint32_t)H) { /* ---- query projection of one cross head, its rows' cross attention ---- */
+        if (crossed && sh.has(STAGE_XQ) && first(FIRST_XQ) < (uint32_t)H) { /* ---- query projection of one cross head, its rows' cross attention ---- */
             fresh_lane();
             const uint32_t head = first(FIRST_XQ), kpart = wave % XKS, tpart = wave / XKS;
             float b[2][XKB], av[RT][XKB], ss[RT];
@@ -435,11 +469,11 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
             }
             buf ^= 1u;
         }
-        if (crossed && first(FIRST_XPROJ) < (uint32_t)E / 16u)
+        if (crossed && sh.has(STAGE_XPROJ) && first(FIRST_XPROJ) < (uint32_t)E / 16u)
             square(ap, ap->layer[layer].xproj, At::xcomb, false, tag, plain, in, tag - 1u, At::mid, first(FIRST_XPROJ));
 
         ap = hidden_args(args);
-        for (uint32_t t = first(FIRST_QKV); t < 3u * E / 16u; t += WORKERS) { /* ---- QKV: rotated, keys and values written through ---- */
+        for (uint32_t t = first(FIRST_QKV); sh.has(STAGE_QKV) && t < 3u * E / 16u; t += WORKERS) { /* ---- QKV: rotated, keys and values written through ---- */
             fresh_lane();
             float b[KB], av[RT][KB], ss[RT], cs = 0.f, sn = 0.f;
             const float *w = ap->layer[layer].qkv + (4u * KB * wave + g) * (3u * E) + t * 16u + c;
@@ -489,14 +523,14 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
         }
 
         ap = hidden_args(args);
-        if (first(FIRST_PROJ) < (uint32_t)E / 16u)
+        if (sh.has(STAGE_PROJ) && first(FIRST_PROJ) < (uint32_t)E / 16u)
             square(ap, ap->layer[layer].proj, At::comb, ap->splits > 1u, tag, plain && !crossed, crossed ? At::mid : in,
                    crossed ? tag : tag - 1u, At::resid, first(FIRST_PROJ));
 
         ap = hidden_args(args);
         fresh_lane();
         const uint32_t hidden = ap->hidden, steps = hidden / 32u; /* steps: of a wave in the down projection */
-        const bool down_here = first(FIRST_DOWN) < (uint32_t)E / 16u;
+        const bool down_here = sh.has(STAGE_DOWN) && first(FIRST_DOWN) < (uint32_t)E / 16u;
         constexpr int CH = RT == 1 ? 16 : 8; /* its steps in flight together */
         float bd[CH];
         const float *wd = ap->layer[layer].down + (4u * steps * wave + g) * E + first(FIRST_DOWN) * 16u + c;
@@ -504,7 +538,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
 #pragma unroll
             for (int i = 0; i < CH; i++) bd[i] = (uint32_t)i < steps ? wd[i * 4u * E] : 0.f;
         }
-        for (uint32_t t = first(FIRST_UPGATE); t < hidden / 16u; t += WORKERS) { /* ---- up, gate, activation ---- */
+        for (uint32_t t = first(FIRST_UPGATE); sh.has(STAGE_UPGATE) && t < hidden / 16u; t += WORKERS) { /* ---- up, gate, activation ---- */
             fresh_lane();
             float b[2][KB], av[RT][KB], ss[RT];
             const uint32_t off = (4u * KB * wave + g) * hidden + t * 16u + c;
@@ -569,6 +603,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
         }
     }
 
+    if (!sh.has(STAGE_LM)) return;
     ArgsPtr ap = hidden_args(args);
     const uint32_t V = ap->V;
     for (uint32_t t = first(FIRST_LM); t < V / 16u; t += WORKERS) { /* ---- LM head ---- */
@@ -593,22 +628,22 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, f
 
 /* The workgroups that run the self-attention stages: units of one (sequence, head, share of the keys).  The first
  * key and value tiles of a wave are requested and turned into fragments before the query is there. */
-template <int E, int HD, int RT>
-__device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv, float *area) {
+template <int E, int HD, int RT, typename Share>
+__device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv, const Share sh, float *area) {
     using At = Regions<E, RT>;
     constexpr int QD = HD / 4, NV = QD / 4, DT = HD / 16, ROW = HD + 4, H = E / HD;
     constexpr int LPR = HD / 4, RPI = 64 / LPR;
     constexpr int T = HD == 32 ? 2 : 1; /* key tiles a wave has in registers */
     const uint32_t tid = threadIdx.x, wave = gv.wave;
     uint64_t *const words = gv.words;
-    Waiter wt{args->timeout, false};
+    Waiter wt{args->timeout, args->spin_limit, false};
     float *const sm_max = area, *const sm_sum = area + 16 * WAVES;
     float *const tiles = area + 2 * 16 * WAVES;
     float *const tile = tiles + wave * (16 * ROW);
-    const uint32_t splits = args->splits, units = gv.ns * (uint32_t)H * splits, workers = args->attn_workers, n = args->n;
+    const uint32_t splits = args->splits, units = gv.ns * (uint32_t)H * splits, n = args->n;
 
-    for (uint32_t layer = 0; layer < args->L; layer++)
-    for (uint32_t u = gv.worker; u < units; u += workers) {
+    for (uint32_t layer = sh.begin(); layer < sh.end(args->L); layer++)
+    for (uint32_t u = gv.worker; u < units; u += WORKERS) {
         const ArgsPtr ap = hidden_args(args);
         uint32_t lane = tid & 63u;
         asm volatile("" : "+v"(lane));
@@ -749,6 +784,7 @@ __device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv,
                 }
             }
             lsum = swap32(swap16(lsum, OpSum()), OpSum());
+            if (wt.expired) lsum = not_there(); /* scores that are not finite would just weigh nothing */
             if (g == 0) sm_max[c * WAVES + wave] = mx, sm_sum[c * WAVES + wave] = lsum;
             /* lane (g, c) holds columns DT (4g + r) + dd of query row c */
 #pragma unroll
@@ -784,11 +820,37 @@ __device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv,
                     word_store(words + At::comb + split * At::M + operand_at<RT>(R, col), sum, tag);
                     if (mc < 2u) word_store(words + At::stat + (split * H + head) * (32u * RT) + R * 2u + mc, mc == 0u ? M : Lt, tag);
                 } else {
-                    word_store(words + At::comb + operand_at<RT>(R, col), Lt > 0.f ? sum / Lt : 0.f, tag);
+                    word_store(words + At::comb + operand_at<RT>(R, col), Lt == 0.f ? 0.f : sum / Lt, tag);
                 }
             }
             __syncthreads(); /* the area may be written again */
         }
+    }
+}
+
+struct Standing {
+    uint32_t rank, members; /* members == 0: the work is others' */
+};
+/* The roll call of a group, by one wave of each of its workgroups; lane i looks at workgroup i's word: 2 tag = in, 2 tag + 1 =
+ * out, less = not decided yet.  Words only grow and each is decided once, so everybody comes to the same list. */
+__device__ __forceinline__ Standing call_roll(uint64_t *roll, uint32_t index, uint32_t tag, uint32_t limit) {
+    static_assert(2u * WORKERS == 64u, "a lane per workgroup");
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t in = 2ull * tag;
+    if (lane == 0u) __hip_atomic_fetch_max(roll + index, in, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t begin = wall_clock64();
+    for (;;) {
+        uint64_t word = __hip_atomic_load(roll + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t present = __ballot(word == in);
+        if (__all(word >= in)) {
+            if ((present >> index & 1ull) == 0ull) return {0u, 0u};
+            return {(uint32_t)__popcll(present & ((1ull << index) - 1ull)), (uint32_t)__popcll(present)};
+        }
+        /* only who is in for good signs others out: somebody always is */
+        if ((present >> index & 1ull) != 0ull && (wall_clock64() - begin) * __popcll(present) >= 64ull * limit && word < in)
+            __hip_atomic_compare_exchange_strong(roll + lane, &word, in + 1ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_sleep(1);
     }
 }
 
@@ -797,21 +859,37 @@ __global__ __launch_bounds__(64 * WAVES, 4) void kv_step_resident_kernel(Residen
     __shared__ __attribute__((aligned(16))) float area[ResidentShape<HD, RT>::AREA];
     __shared__ __attribute__((aligned(16))) float part_ss[2][16 * RT][WAVES];
     __shared__ float xquery[16 * RT][HD];
+    __shared__ Standing standing;
     GroupView gv;
-    const uint32_t group = blockIdx.x % GROUPS;
-    gv.worker = blockIdx.x / GROUPS;
+    const uint32_t group = blockIdx.x % GROUPS, index = blockIdx.x / GROUPS;
     gv.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     gv.seq0 = group * a.per_group;
     if (gv.seq0 >= a.batch) return;
+    if (gv.wave == 0u) {
+        const Standing st = call_roll(a.rolls + group * (2u * WORKERS), index, a.tag, a.roll_limit);
+        if (threadIdx.x == 0u) standing = st;
+    }
+    __syncthreads();
+    const uint32_t rank = __builtin_amdgcn_readfirstlane(standing.rank), members = __builtin_amdgcn_readfirstlane(standing.members);
     gv.ns = min(a.per_group, a.batch - gv.seq0);
     gv.rows = gv.ns * a.n, gv.row0 = gv.seq0 * a.n;
     gv.words = a.words + (size_t)group * a.group_words;
     const ArgsPtr ap = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
-    if (gv.worker < WORKERS) {
-        product_role<E, HD, RT>(ap, gv, area, part_ss, xquery);
-    } else {
-        gv.worker -= WORKERS;
-        attention_role<E, HD, RT>(ap, gv, area);
+    if (members == 2u * WORKERS) {
+        gv.worker = index & (WORKERS - 1u);
+        if (index < WORKERS) product_role<E, HD, RT>(ap, gv, WholeStep(), area, part_ss, xquery);
+        else attention_role<E, HD, RT>(ap, gv, WholeStep(), area);
+        return;
+    }
+    const uint32_t stride = min(members, WORKERS);
+    if (rank >= stride) return;
+    for (uint32_t stage = 0; stage <= a.L * STAGES; stage++) {
+        const OneStage one{stage / STAGES, stage < a.L * STAGES ? stage % STAGES : (uint32_t)STAGE_LM};
+        for (gv.worker = rank; gv.worker < WORKERS; gv.worker += stride) {
+            if (one.stage == STAGE_ATTN) attention_role<E, HD, RT>(ap, gv, one, area);
+            else product_role<E, HD, RT>(ap, gv, one, area, part_ss, xquery);
+            __syncthreads(); /* the shared areas may be written again */
+        }
     }
 }
 
@@ -820,47 +898,94 @@ __global__ void clear_hand_over_kernel(uint64_t *w, size_t n) {
     if (i < n) w[i] = 0u;
 }
 
-/* Hand-over words of one device (launches follow each other, see below: one set serves all streams).  Tags of
- * successive launches differ, so the words are cleared only when they are new or the tags have run through. */
-struct DeviceState {
+typedef void (*ResidentKernel)(ResidentArgs);
+ResidentKernel kernel_of(size_t E, size_t hd, uint32_t row_tiles) {
+    if (E == 64 && hd == 32) return row_tiles == 2u ? kv_step_resident_kernel<64, 32, 2> : kv_step_resident_kernel<64, 32, 1>;
+    if (E == 64) return kv_step_resident_kernel<64, 64, 1>;
+    if (E == 128) return hd == 32 ? kv_step_resident_kernel<128, 32, 1> : kv_step_resident_kernel<128, 64, 1>;
+    return hd == 32 ? kv_step_resident_kernel<256, 32, 1> : kv_step_resident_kernel<256, 64, 1>;
+}
+constexpr uint32_t group_words(size_t E, uint32_t row_tiles, uint32_t hidden) {
+    return (E == 64 ? row_tiles == 2u ? Regions<64, 2>::total(hidden) : Regions<64, 1>::total(hidden)
+                    : E == 128 ? Regions<128, 1>::total(hidden) : Regions<256, 1>::total(hidden)) + 63u & ~63u;
+}
+
+/* Hand-over words and roll calls of one (thread, stream), like the library's other scratch: launches on one stream follow
+ * each other, launches on two streams never share them.  Tags of successive launches differ, so the words are cleared
+ * only when they are new or the tags have run through.  Sized for every shape the kernel takes (3.7 MB). */
+struct HandOver {
+    static constexpr size_t WORDS = GROUPS * (size_t)std::max(group_words(64, 2, MAX_HIDDEN), group_words(256, 1, MAX_HIDDEN));
+    static constexpr size_t COUNT = WORDS + GROUPS * 2u * WORKERS; /* and the roll calls */
     uint64_t *words = nullptr;
-    size_t count = 0;
-    uint32_t next_tag = 1;
-    bool used = false, several = false; /* launched at all; from more than one stream */
-    hipStream_t last = nullptr;
-    hipEvent_t done = nullptr; /* end of the last launch, recorded once several streams launch */
+    uint32_t next_tag = 0;
+};
+struct HandOvers {
+    std::map<std::pair<int, hipStream_t>, HandOver> by_stream;
+    ~HandOvers() { /* a thread that ends gives them back; when the process does, the runtime may have ended first */
+        if (gettid() != getpid())
+            for (auto &entry : by_stream) (void)hipFree(entry.second.words); /* waits for what still uses them */
+    }
 };
 
-std::mutex g_lock;
-DeviceState g_devices[64];
-uint32_t *g_timeout = nullptr; /* pinned, written by a kernel whose waits ran out */
+/* pinned, written by a kernel whose waits ran out */
+uint32_t *timeout_word() {
+    static uint32_t *const word = [] {
+        uint32_t *w = nullptr;
+        HIP_CHECK(hipHostMalloc((void **)&w, 64, hipHostMallocPortable));
+        *w = 0u;
+        return w;
+    }();
+    return word;
+}
 std::atomic<bool> g_launched{false};
 
-template <int E, int HD>
-void launch_resident(uint32_t row_tiles, uint32_t blocks, hipStream_t s, const ResidentArgs &a) {
-    if constexpr (E == 64 && HD == 32) { /* the only shape that takes more than 16 rows a group */
-        if (row_tiles == 2u) {
-            blt_launch("kv_step_resident", kv_step_resident_kernel<E, HD, 2>, dim3(blocks), dim3(64 * WAVES), 0, s, a);
-            return;
-        }
-    }
-    blt_launch("kv_step_resident", kv_step_resident_kernel<E, HD, 1>, dim3(blocks), dim3(64 * WAVES), 0, s, a);
+/* BLT_HIP_STEP_TEST=team|giveup|wrap (test hook): who looks signs out whoever is not in yet / no wait lasts
+ * / the tags run through at the third launch of a stream */
+enum TestPin { TEST_NONE, TEST_TEAM, TEST_GIVEUP, TEST_WRAP };
+TestPin test_pin() {
+    static const TestPin pin = [] {
+        const char *e = getenv("BLT_HIP_STEP_TEST");
+        if (e && std::strcmp(e, "team") == 0) return TEST_TEAM;
+        if (e && std::strcmp(e, "giveup") == 0) return TEST_GIVEUP;
+        if (e && std::strcmp(e, "wrap") == 0) return TEST_WRAP;
+        return TEST_NONE;
+    }();
+    return pin;
 }
-uint32_t group_words(uint32_t E, uint32_t row_tiles, uint32_t hidden) {
-    switch (E * 4u + row_tiles) {
-    case 64 * 4 + 1: return Regions<64, 1>::total(hidden);
-    case 64 * 4 + 2: return Regions<64, 2>::total(hidden);
-    case 128 * 4 + 1: return Regions<128, 1>::total(hidden);
-    default: return Regions<256, 1>::total(hidden);
+
+/* Do `blocks` workgroups of the kernel fit the compute units this stream may use, all at once?  The launch would be right
+ * otherwise too (see the roll call), but the launches would be faster. */
+bool can_be_resident(ResidentKernel kernel, uint32_t blocks, int dev, hipStream_t s) {
+    struct Known {
+        ResidentKernel kernel;
+        int dev;
+        uint32_t per_unit, units;
+    };
+    static thread_local Known known{nullptr, 0, 0u, 0u};
+    if (known.kernel != kernel || known.dev != dev) {
+        int per_unit = 0, units = 0;
+        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_unit, reinterpret_cast<const void *>(kernel), 64 * WAVES, 0));
+        HIP_CHECK(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev));
+        known = Known{kernel, dev, (uint32_t)per_unit, (uint32_t)units};
     }
+    uint32_t mask[32], open = 0;
+    const uint32_t mask_words = (known.units + 31u) / 32u;
+    if (mask_words > 32u) return false;
+    if (hipExtStreamGetCUMask(s, mask_words, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    for (uint32_t i = 0; i < mask_words; i++) open += (uint32_t)__builtin_popcount(mask[i]);
+    return (uint64_t)known.per_unit * std::min(open, known.units) >= blocks;
 }
 
 } // namespace
 
 void kv_step_resident_check() {
-    if (g_launched.load(std::memory_order_relaxed) && __atomic_load_n(g_timeout, __ATOMIC_RELAXED) != 0u)
-        BLT_FATAL("blt_kv_decode_step: workgroup %u of the resident step gave up waiting (step_resident.hip:%u)", *g_timeout >> 16,
-                  *g_timeout & 0xFFFFu);
+    if (!g_launched.load(std::memory_order_relaxed)) return;
+    const uint32_t word = __atomic_load_n(timeout_word(), __ATOMIC_RELAXED);
+    if (word != 0u)
+        BLT_FATAL("blt_kv_decode_step: workgroup %u of the resident step gave up waiting (step_resident.hip:%u)", word >> 16, word & 0xFFFFu);
 }
 
 bool kv_step_resident(const StepResident &st) {
@@ -935,60 +1060,38 @@ bool kv_step_resident(const StepResident &st) {
     /* Workgroups per group: one per compute unit of a die; the widest stage (hidden / 16 tiles) fills them.
      * Keys are shared out while there are workgroups without a (sequence, head) and a share keeps every
      * wave of a workgroup a tile. */
-    a.attn_workers = 32u;
     const uint32_t pairs = (uint32_t)(per_group * H);
     a.splits = 1u;
     if (hd % (E / 8) == 0)
-        while (a.splits < MAX_SPLITS_R && pairs * a.splits * 2u <= a.attn_workers && longest >= 128u * a.splits) a.splits *= 2u;
+        while (a.splits < MAX_SPLITS_R && pairs * a.splits * 2u <= WORKERS && longest >= 128u * a.splits) a.splits *= 2u;
     const uint32_t rt = group_rows > 16 ? 2u : 1u;
-    a.group_words = (group_words(a.E, rt, a.hidden) + 63u) / 64u * 64u;
+    a.group_words = group_words(E, rt, a.hidden);
 
     int dev = 0;
     HIP_CHECK(hipGetDevice(&dev));
-    BLT_REQUIRE(dev >= 0 && dev < 64, "device index %d out of range", dev);
-    std::lock_guard<std::mutex> hold(g_lock);
-    if (!g_timeout) {
-        HIP_CHECK(hipHostMalloc((void **)&g_timeout, 64, hipHostMallocDefault));
-        *g_timeout = 0u;
-    }
-    kv_step_resident_check();
     const hipStream_t s = blt_stream();
-    DeviceState &ds = g_devices[dev];
-    /* Two launches at once could each hold compute units the other's last workgroups wait for: launches
-     * from different streams follow each other.  Events only once a second stream has appeared. */
-    if (ds.used && ds.last != s) {
-        if (!ds.several) {
-            HIP_CHECK(hipDeviceSynchronize());
-            HIP_CHECK(hipEventCreateWithFlags(&ds.done, hipEventDisableTiming));
-            ds.several = true;
-        } else {
-            HIP_CHECK(hipStreamWaitEvent(s, ds.done, 0));
-        }
+    const ResidentKernel kernel = kernel_of(E, hd, rt);
+    const uint32_t groups = (uint32_t)((st.batch + per_group - 1) / per_group);
+    if (!can_be_resident(kernel, groups * 2u * WORKERS, dev, s)) return false;
+    kv_step_resident_check();
+    static thread_local HandOvers hand_overs;
+    HandOver &ho = hand_overs.by_stream[{dev, s}];
+    const TestPin pin = test_pin();
+    if (ho.next_tag == 0u || ho.next_tag > 0xFFFFFFFFu - 2u * MAX_LAYERS) {
+        const bool fresh = ho.words == nullptr;
+        if (fresh) HIP_CHECK(hipMalloc((void **)&ho.words, HandOver::COUNT * sizeof(uint64_t)));
+        blt_launch("kv_step_clear", clear_hand_over_kernel, dim3((unsigned)((HandOver::COUNT + 255) / 256)), dim3(256), 0, s, ho.words,
+                   HandOver::COUNT);
+        ho.next_tag = fresh && pin == TEST_WRAP ? 0xFFFFFFFFu - 2u * MAX_LAYERS - (uint32_t)L : 1u;
     }
-    const size_t need = (size_t)GROUPS * a.group_words;
-    if (need > ds.count || ds.next_tag > 0xFFFFFFFFu - 2u * MAX_LAYERS) {
-        if (need > ds.count) {
-            if (ds.words) HIP_CHECK(hipFree(ds.words)); /* waits for the launch that may still use them */
-            ds.count = std::max(need, 2 * ds.count);
-            HIP_CHECK(hipMalloc((void **)&ds.words, ds.count * sizeof(uint64_t)));
-        }
-        hipLaunchKernelGGL(clear_hand_over_kernel, dim3((unsigned)((ds.count + 255) / 256)), dim3(256), 0, s, ds.words, ds.count);
-        ds.next_tag = 1;
-    }
-    a.words = ds.words;
-    a.timeout = g_timeout;
-    a.tag = ds.next_tag;
-    ds.next_tag += (uint32_t)L;
-
-    const uint32_t blocks = GROUPS * (WORKERS + a.attn_workers);
-    if (E == 64 && hd == 32) launch_resident<64, 32>(rt, blocks, s, a);
-    else if (E == 64) launch_resident<64, 64>(rt, blocks, s, a);
-    else if (E == 128 && hd == 32) launch_resident<128, 32>(rt, blocks, s, a);
-    else if (E == 128) launch_resident<128, 64>(rt, blocks, s, a);
-    else if (hd == 32) launch_resident<256, 32>(rt, blocks, s, a);
-    else launch_resident<256, 64>(rt, blocks, s, a);
-    if (ds.several) HIP_CHECK(hipEventRecord(ds.done, s));
-    ds.used = true, ds.last = s;
+    a.words = ho.words;
+    a.rolls = ho.words + HandOver::WORDS;
+    a.timeout = timeout_word();
+    a.roll_limit = pin == TEST_TEAM ? 0u : ROLL_LIMIT;
+    a.spin_limit = pin == TEST_GIVEUP ? 0u : SPIN_LIMIT;
+    a.tag = ho.next_tag;
+    ho.next_tag += (uint32_t)L;
+    blt_launch("kv_step_resident", kernel, dim3(GROUPS * 2u * WORKERS), dim3(64 * WAVES), 0, s, a);
     g_launched.store(true, std::memory_order_relaxed);
     return true;
 }

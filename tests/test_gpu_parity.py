@@ -1871,8 +1871,9 @@ def test_kv_decode_step_long_prefill(window, oracle, dev):
         lib.blt_arena_destroy(arena)
 
 
-def _decode_steps(batch, n, c, seed, oracle, row_scale=1.0):
-    """Two steps of a batched cache against the restated step run sequence by sequence; the kernels each step launched."""
+def _decode_steps(batch, n, c, seed, oracle, row_scale=1.0, before_sync=None):
+    """Two steps of a batched cache against the restated step run sequence by sequence; the kernels each step launched.
+    before_sync(logits): called after each step, before the library synchronises."""
     import torch
     from fblt_amd import decoder
     lib = api.load()
@@ -1929,6 +1930,8 @@ def _decode_steps(batch, n, c, seed, oracle, row_scale=1.0):
             lib.blt_hip_profile_begin()
             lib.blt_kv_decode_step_batched_hip(cache, self_len, table_ptrs, num, closed, C.byref(vd), C.byref(vl), arena)
             launched.append(sorted(api.profile_end()))
+            if before_sync:
+                before_sync(tl)
             lib.blt_backend_pass_sync_hip()
             assert [self_len[b] for b in range(batch)] == (lens + (step + 1) * n).tolist()
             # the absolute term of the tolerance is for rows of order one
@@ -1961,7 +1964,9 @@ RESIDENT_CASES = [
 ]
 
 
-ONE_LAUNCH = ["kv_step_resident"]
+def in_one_launch(launched):
+    """Every step the resident kernel and nothing else (the first one of a stream clears its words)."""
+    return all(names in (["kv_step_resident"], ["kv_step_clear", "kv_step_resident"]) for names in launched)
 
 
 @pytest.mark.parametrize("batch,n,case", [(1, 32, 0), (8, 17, 0), (33, 1, 0), (1, 1, 1), (32, 1, 1),   # rows of a group 1 ... 32 at
@@ -1969,7 +1974,7 @@ ONE_LAUNCH = ["kv_step_resident"]
                                           (1, 11, 4), (8, 16, 4), (64, 1, 4), (1, 1, 5), (30, 1, 5)])   # 256, heads of 32 and 64
 def test_kv_decode_step_in_one_launch(batch, n, case, oracle, dev):
     """The one-launch form of the step at the edges of its shapes, against the restated step."""
-    assert _decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle) == [ONE_LAUNCH] * 2
+    assert in_one_launch(_decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle))
 
 
 @pytest.mark.parametrize("batch,n,case", [(1, 17, 2), (1, 32, 4), (9, 2, 3), (40, 1, 5), (9, 17, 0)])
@@ -1983,7 +1988,105 @@ def test_kv_decode_step_past_one_launch(batch, n, case, oracle, dev):
 def test_kv_decode_step_of_rows_whose_norm_overflows(batch, n, case, oracle, dev):
     """Input rows of 1e20: their sum of squares is infinite and the normalised row zero, in the one-launch form as in
     the restated step."""
-    assert _decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle, row_scale=1e20) == [ONE_LAUNCH] * 2
+    assert in_one_launch(_decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle, row_scale=1e20))
+
+
+@pytest.mark.parametrize("mode", ["team", "wrap", "giveup"])
+def test_one_launch_step_under_adverse_conditions(mode):
+    """Workgroups that are not all resident, tags that run through, waits that run out: see step_pin_case.py."""
+    import os
+    import subprocess
+    import sys
+    script = os.path.join(os.path.dirname(os.path.abspath(__file__)), "step_pin_case.py")
+    p = subprocess.run([sys.executable, "-u", script, mode], capture_output=True, text=True, timeout=100)
+    assert "CHECKED" in p.stdout, (p.stdout[-2000:], p.stderr[-2000:])
+    assert "NOT REACHED" not in p.stdout
+    if mode == "giveup":
+        assert p.returncode == 1 and "gave up waiting" in p.stderr, (p.returncode, p.stderr[-500:])
+    else:
+        assert p.returncode == 0, (p.returncode, p.stderr[-500:])
+
+
+class _StepOnStream:
+    """A batch of sequences whose next step can be issued over and over, each time from the same lengths."""
+
+    def __init__(self, lib, oracle, c, seed, batch, repeats):
+        import torch
+        from fblt_amd import decoder
+        rs = np.random.RandomState(seed)
+        self.lib, self.c, self.batch = lib, c, batch
+        self.device = _decoders(oracle, c, seed)[1]
+        self.arena = lib.blt_arena_create(256 << 20, abi.BLT_BACKEND_HIP)
+        self.cache = lib.blt_kv_cache_create_batched(self.arena, self.device.ptr, c["max_len"], batch)
+        self.mark = self.arena.contents.offset
+        self.lens = rs.randint(1, c["max_len"] - 2, size=batch).tolist()
+        tables = [decoder.patch_table([n + 1]) for n in self.lens]
+        pin = torch.from_numpy(rs.randn(1, c["k"] * c["E"]).astype(np.float32)).cuda()
+        for b in range(batch):
+            vp = _dev_tensor(pin)
+            lib.blt_kv_cache_refresh_cross_seq_hip(self.cache, b, C.byref(vp), tables[b], 1, 0, self.arena)
+        for name in ("self_k", "self_v"):
+            for l in range(c["L"]):
+                slab = rs.randn(batch * c["max_len"], c["E"]).astype(np.float32)
+                lib.blt_hip_memcpy_h2d(getattr(self.cache.contents, name)[l].data, slab.ctypes.data, slab.nbytes)
+        lib.blt_backend_pass_sync_hip()
+        self.rows = torch.from_numpy(rs.randn(batch, c["E"]).astype(np.float32)).cuda()
+        self.logits = torch.full((repeats, batch, c["V"]), 7.0, device="cuda")
+        self.ptrs = (C.POINTER(abi.BltPatchInfo) * batch)(*(C.cast(t, C.POINTER(abi.BltPatchInfo)) for t in tables))
+        self.num, self.keep = abi.size_array([1] * batch), (tables, pin)
+
+    def step(self, i):
+        self.arena.contents.offset = self.mark
+        lens, closed = abi.size_array(self.lens), (C.c_int * self.batch)()
+        vd, vl = _dev_tensor(self.rows), _dev_tensor(self.logits[i])
+        self.lib.blt_kv_decode_step_batched_hip(self.cache, lens, self.ptrs, self.num, closed, C.byref(vd), C.byref(vl), self.arena)
+
+    def close(self):
+        self.lib.blt_kv_cache_destroy(self.cache)
+        self.lib.blt_arena_destroy(self.arena)
+
+
+@pytest.mark.parametrize("threads", [False, True])
+def test_one_launch_steps_on_two_streams(threads, oracle, dev):
+    """Steps issued on two streams without waiting for each other, from one thread on two streams of its own and from two
+    threads on hipStreamPerThread (one handle, two streams): every one gives what the step alone gives, bit for bit."""
+    import threading
+
+    import torch
+    lib = api.load()
+    repeats = 40
+    work = [_StepOnStream(lib, oracle, RESIDENT_CASES[i], 900 + i, b, repeats + 1) for i, b in ((2, 16), (4, 64))]
+    try:
+        for w in work:
+            w.step(repeats)
+        lib.blt_backend_pass_sync_hip()
+        if threads:
+            def issue(w):
+                lib.blt_hip_set_stream(2)   # hipStreamPerThread
+                for i in range(repeats):
+                    w.step(i)
+                lib.blt_backend_pass_sync_hip()
+            pool = [threading.Thread(target=issue, args=(w,)) for w in work]
+            for t in pool:
+                t.start()
+            for t in pool:
+                t.join()
+        else:
+            streams = [torch.cuda.Stream() for _ in work]
+            for i in range(repeats):
+                for w, s in zip(work, streams):
+                    lib.blt_hip_set_stream(s.cuda_stream)
+                    w.step(i)
+            lib.blt_hip_set_stream(None)
+        lib.blt_backend_pass_sync_hip()
+        for w in work:
+            got = w.logits.cpu().numpy()
+            assert np.isfinite(got).all()
+            assert all(got[i].tobytes() == got[repeats].tobytes() for i in range(repeats))
+    finally:
+        lib.blt_hip_set_stream(None)
+        for w in work:
+            w.close()
 
 
 def test_graph_replay_of_a_plan_and_a_decode_layer(oracle, dev):
