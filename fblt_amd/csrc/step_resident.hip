@@ -1070,6 +1070,11 @@ bool kv_step_resident(const StepResident &st) {
     int dev = 0;
     HIP_CHECK(hipGetDevice(&dev));
     const hipStream_t s = blt_stream();
+    /* recorded by the caller's own capture of the stream, a replay would find the words of the launch before it under its
+     * own tag */
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (s != nullptr) HIP_CHECK(hipStreamIsCapturing(s, &capture));
+    if (capture != hipStreamCaptureStatusNone) return false;
     const ResidentKernel kernel = kernel_of(E, hd, rt);
     const uint32_t groups = (uint32_t)((st.batch + per_group - 1) / per_group);
     if (!can_be_resident(kernel, groups * 2u * WORKERS, dev, s)) return false;

@@ -2089,6 +2089,31 @@ def test_one_launch_steps_on_two_streams(threads, oracle, dev):
             w.close()
 
 
+def test_step_in_a_capture_of_the_callers_own(oracle, dev):
+    """A step recorded by the caller's capture of its stream, which the library does not see begin, goes in launches:
+    every replay gives what the step gives."""
+    import torch
+    lib = api.load()
+    w = _StepOnStream(lib, oracle, RESIDENT_CASES[2], 950, 16, 2)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    try:
+        lib.blt_hip_set_stream(stream.cuda_stream)
+        w.step(0)
+        lib.blt_backend_pass_sync_hip()
+        want = w.logits[0].cpu().numpy()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+            w.step(1)
+        for _ in range(3):
+            w.logits[1].fill_(7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_close(w.logits[1].cpu().numpy(), want, "replayed step")
+    finally:
+        lib.blt_hip_set_stream(None)
+        w.close()
+
+
 def test_graph_replay_of_a_plan_and_a_decode_layer(oracle, dev):
     """Library launches recorded into a HIP graph: every replay, with eager work and
     synchronisations in between, gives the eager result."""
