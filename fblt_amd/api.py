@@ -294,7 +294,7 @@ def profile_end_list(capacity=1 << 16):
 
 def profile_end():
     """Close the open profile: {kernel tag: (launches, total_ms, min_ms, max_ms)}."""
-    rows = (BltHipKernelTime * 16)()
-    n = load().blt_hip_profile_end(rows, 16)
+    rows = (BltHipKernelTime * 64)()
+    n = load().blt_hip_profile_end(rows, 64)
     return {rows[i].name.decode(): (int(rows[i].launches), rows[i].total_ms, rows[i].min_ms, rows[i].max_ms)
-            for i in range(min(n, 16))}
+            for i in range(min(n, 64))}

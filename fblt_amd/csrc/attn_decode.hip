@@ -516,8 +516,8 @@ void acquire_scratch(StepArgs &a, size_t floats, size_t batch, bool static_scrat
         if (sc.tickets) g.retired.push_back(sc.tickets);
         sc.ticket_count = std::max<size_t>(2 * batch, 1024);
         HIP_CHECK(hipMalloc((void **)&sc.tickets, sc.ticket_count * sizeof(uint32_t)));
-        hipLaunchKernelGGL(kv_clear_words_kernel, dim3((unsigned)((sc.ticket_count + 255) / 256)), dim3(256), 0,
-                           blt_stream(), sc.tickets, sc.ticket_count);
+        blt_launch("kv_clear_words", kv_clear_words_kernel, dim3((unsigned)((sc.ticket_count + 255) / 256)), dim3(256), 0,
+                   blt_stream(), sc.tickets, sc.ticket_count);
     }
     a.partial = sc.partial;
     a.tickets = sc.tickets;

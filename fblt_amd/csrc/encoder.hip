@@ -145,9 +145,9 @@ void pool_launch(const float *h, size_t seq_len, size_t embed_dim, const blt_pat
             BLT_REQUIRE(pi.start_idx + pi.length <= seq_len, "patch_pool: patch out of range");
             c.start[j] = (uint32_t)pi.start_idx, c.len[j] = (uint32_t)pi.length;
         }
-        hipLaunchKernelGGL(patch_pool_kernel, dim3((unsigned)n), dim3(256), 0, blt_stream(), h, out + j0 * out_stride,
-                           (uint32_t)embed_dim, (uint32_t)out_stride, (uint32_t)copies,
-                           pool_type == BLT_POOL_MAX ? 1 : 0, c);
+        blt_launch("patch_pool", patch_pool_kernel, dim3((unsigned)n), dim3(256), 0, blt_stream(), h, out + j0 * out_stride,
+                   (uint32_t)embed_dim, (uint32_t)out_stride, (uint32_t)copies,
+                   pool_type == BLT_POOL_MAX ? 1 : 0, c);
         HIP_CHECK_LAUNCH("blt_patch_pool_forward");
     }
 }
@@ -191,8 +191,8 @@ extern "C" void blt_indexed_row_accumulate_hip(const blt_tensor *table, const ui
             BLT_REQUIRE(c.v[i] == BLT_IDX_SENTINEL || c.v[i] < table->shape[0],
                         "blt_indexed_row_accumulate: index out of range");
         }
-        hipLaunchKernelGGL(rows_accumulate_kernel, dim3((unsigned)n), dim3(256), 0, blt_stream(),
-                           (const float *)table->data, (float *)io->data + r0 * embed_dim, (uint64_t)embed_dim, c);
+        blt_launch("rows_accumulate", rows_accumulate_kernel, dim3((unsigned)n), dim3(256), 0, blt_stream(),
+                   (const float *)table->data, (float *)io->data + r0 * embed_dim, (uint64_t)embed_dim, c);
         HIP_CHECK_LAUNCH("blt_indexed_row_accumulate");
     }
 }
@@ -204,8 +204,8 @@ extern "C" void blt_scale_hip(blt_tensor *t, float scalar) {
     BLT_REQUIRE(t->backend == BLT_BACKEND_HIP, "blt_scale: HIP implementation called with non-HIP backend");
     if (t->numel == 0) return;
     const unsigned blocks = (unsigned)std::min<size_t>((t->numel + 255u) / 256u, 4096u);
-    hipLaunchKernelGGL(scale_kernel, dim3(blocks), dim3(256), 0, blt_stream(), (float *)t->data, (uint64_t)t->numel,
-                       scalar);
+    blt_launch("scale", scale_kernel, dim3(blocks), dim3(256), 0, blt_stream(), (float *)t->data, (uint64_t)t->numel,
+               scalar);
     HIP_CHECK_LAUNCH("blt_scale");
 }
 
@@ -284,9 +284,9 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
 
     const size_t byte_shape[2] = {seq_len, E}, patch_shape[2] = {num_patches, patch_dim};
     blt_tensor h = blt_tensor_create_uninit(arena, byte_shape, 2, BLT_DTYPE_FP32);
-    hipLaunchKernelGGL(embed_sum_kernel, dim3((unsigned)seq_len), dim3(256), 0, blt_stream(),
-                       (const float *)model->byte_embedding_weight.data, (const uint32_t *)dev_idx, (float *)h.data,
-                       (uint32_t)E, tables, ng.normalize ? 1 : 0, 1.0f / (float)(ng.num_ngram_sizes + 1));
+    blt_launch("embed_sum", embed_sum_kernel, dim3((unsigned)seq_len), dim3(256), 0, blt_stream(),
+               (const float *)model->byte_embedding_weight.data, (const uint32_t *)dev_idx, (float *)h.data,
+               (uint32_t)E, tables, ng.normalize ? 1 : 0, 1.0f / (float)(ng.num_ngram_sizes + 1));
     HIP_CHECK_LAUNCH("blt_local_encoder_forward: embedding");
 
     /* ---- P_0: pooled rows in every sub-token column block (local_encoder.c:237-245) ---- */

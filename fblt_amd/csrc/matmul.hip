@@ -791,8 +791,8 @@ bool slice_scratch(MatmulArgs &g, size_t tiles, hipStream_t s) {
         sc.ticket_count = std::max<size_t>(2 * tiles, 1024);
         HIP_CHECK(hipMalloc((void **)&sc.tickets, sc.ticket_count * sizeof(uint32_t)));
         /* a fill kernel, not a memset, on the stream the launches follow */
-        hipLaunchKernelGGL(clear_words_kernel, dim3((unsigned)((sc.ticket_count + 255) / 256)), dim3(256), 0,
-                           s ? s : blt_stream(), sc.tickets, sc.ticket_count);
+        blt_launch("matmul_clear_words", clear_words_kernel, dim3((unsigned)((sc.ticket_count + 255) / 256)), dim3(256), 0,
+                   s ? s : blt_stream(), sc.tickets, sc.ticket_count);
     }
     g.slice_sums = sc.sums;
     g.slice_tickets = sc.tickets;

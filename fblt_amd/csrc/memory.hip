@@ -56,8 +56,8 @@ extern "C" void blt_hip_memset(void *dst, int value, size_t bytes) {
     const size_t body16 = (bytes - head) / 16u;
     const unsigned int b = (unsigned int)(value & 0xFF), pattern = b | (b << 8) | (b << 16) | (b << 24);
     const unsigned blocks = (unsigned)std::min<size_t>(2048, std::max<size_t>(1, (body16 + 255) / 256));
-    hipLaunchKernelGGL(fill_bytes_kernel, dim3(blocks), dim3(256), 0, blt_stream(), static_cast<unsigned char *>(dst),
-                       pattern, head, body16, bytes);
+    blt_launch("fill_bytes", fill_bytes_kernel, dim3(blocks), dim3(256), 0, blt_stream(), static_cast<unsigned char *>(dst),
+               pattern, head, body16, bytes);
     HIP_CHECK_LAUNCH("blt_hip_memset");
 }
 
@@ -117,7 +117,7 @@ bool upload_in_arguments(void *dst, const void *src, size_t bytes) {
         } else {
             __builtin_memcpy(a.words, from + at, 4u * a.count);
         }
-        hipLaunchKernelGGL(upload_words_kernel, dim3((a.count + 255u) / 256u), dim3(256), 0, blt_stream(), a);
+        blt_launch("upload_words", upload_words_kernel, dim3((a.count + 255u) / 256u), dim3(256), 0, blt_stream(), a);
     }
     HIP_CHECK_LAUNCH("upload_words");
     return true;

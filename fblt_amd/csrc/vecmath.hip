@@ -125,11 +125,11 @@ extern "C" void blt_strided_copy_hip(blt_backend backend, float *dst, size_t dst
     const uint64_t work = rows * (vec ? cols / 4 : cols);
     const unsigned blocks = (unsigned)((work + 255u) / 256u < 4096u ? (work + 255u) / 256u : 4096u);
     if (vec)
-        hipLaunchKernelGGL(strided_copy_kernel<true>, dim3(blocks), dim3(256), 0, blt_stream(), dst, (uint64_t)dst_stride, src,
-                           (uint64_t)src_stride, (uint64_t)rows, (uint64_t)cols);
+        blt_launch("strided_copy", strided_copy_kernel<true>, dim3(blocks), dim3(256), 0, blt_stream(), dst, (uint64_t)dst_stride, src,
+                   (uint64_t)src_stride, (uint64_t)rows, (uint64_t)cols);
     else
-        hipLaunchKernelGGL(strided_copy_kernel<false>, dim3(blocks), dim3(256), 0, blt_stream(), dst, (uint64_t)dst_stride, src,
-                           (uint64_t)src_stride, (uint64_t)rows, (uint64_t)cols);
+        blt_launch("strided_copy", strided_copy_kernel<false>, dim3(blocks), dim3(256), 0, blt_stream(), dst, (uint64_t)dst_stride, src,
+                   (uint64_t)src_stride, (uint64_t)rows, (uint64_t)cols);
     HIP_CHECK_LAUNCH("blt_strided_copy");
 }
 
@@ -154,11 +154,11 @@ extern "C" void blt_rows_gather_hip(const blt_tensor *src, const size_t *pos_hos
         GatherRows g;
         for (size_t i = 0; i < (size_t)GATHER_ROWS; i++) g.pos[i] = i < n ? pos_host[r0 + i] : 0;
         if (vec)
-            hipLaunchKernelGGL(rows_gather_kernel<true>, dim3((unsigned)n), dim3(256), 0, blt_stream(), s,
-                               d + r0 * row_len, (uint64_t)row_len, g);
+            blt_launch("rows_gather", rows_gather_kernel<true>, dim3((unsigned)n), dim3(256), 0, blt_stream(), s,
+                       d + r0 * row_len, (uint64_t)row_len, g);
         else
-            hipLaunchKernelGGL(rows_gather_kernel<false>, dim3((unsigned)n), dim3(256), 0, blt_stream(), s,
-                               d + r0 * row_len, (uint64_t)row_len, g);
+            blt_launch("rows_gather", rows_gather_kernel<false>, dim3((unsigned)n), dim3(256), 0, blt_stream(), s,
+                       d + r0 * row_len, (uint64_t)row_len, g);
         HIP_CHECK_LAUNCH("blt_rows_gather");
     }
 }
@@ -188,8 +188,8 @@ extern "C" void blt_softmax_masked_row_inplace_hip(blt_backend backend, float *r
                 "blt_softmax_masked_row_inplace: HIP implementation called with non-HIP backend");
     if (row_len == 0) return;
     BLT_REQUIRE(row != NULL, "blt_softmax_masked_row_inplace: row must not be NULL");
-    hipLaunchKernelGGL(softmax_row_kernel, dim3(1), dim3(256), 0, blt_stream(), row, (uint64_t)row_len, (uint64_t)row_idx,
-                       is_causal ? 1 : 0, mask_row, scale);
+    blt_launch("softmax_row", softmax_row_kernel, dim3(1), dim3(256), 0, blt_stream(), row, (uint64_t)row_len, (uint64_t)row_idx,
+               is_causal ? 1 : 0, mask_row, scale);
     HIP_CHECK_LAUNCH("blt_softmax_masked_row_inplace");
 }
 
@@ -199,7 +199,7 @@ extern "C" float blt_vec_dot_hip(blt_backend backend, const float *a, const floa
     BLT_REQUIRE(a != NULL && b != NULL, "blt_vec_dot: buffers must not be NULL");
     static thread_local float *slot = nullptr;
     if (!slot) HIP_CHECK(hipMalloc((void **)&slot, sizeof(float)));
-    hipLaunchKernelGGL(dot_kernel, dim3(1), dim3(256), 0, blt_stream(), a, b, (uint64_t)n, slot);
+    blt_launch("dot", dot_kernel, dim3(1), dim3(256), 0, blt_stream(), a, b, (uint64_t)n, slot);
     HIP_CHECK_LAUNCH("blt_vec_dot");
     float r = 0.f;
     HIP_CHECK(hipMemcpyAsync(&r, slot, sizeof(float), hipMemcpyDeviceToHost, blt_stream()));

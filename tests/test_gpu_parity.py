@@ -2114,6 +2114,22 @@ def test_step_in_a_capture_of_the_callers_own(oracle, dev):
         w.close()
 
 
+def test_profile_holds_every_launch(dev):
+    """Uploads that travel in kernel arguments and the small kernels beside the main path are in the kernel-time profile."""
+    import torch
+    lib = api.load()
+    qkv, out = torch.randn(3, 40, 32, device="cuda"), torch.zeros(3, 40, 32, device="cuda")
+    probs = [api.problem(api.head_args(qkv.data_ptr(), qkv.data_ptr(), qkv.data_ptr(), out[i].data_ptr(), 20 + i * i, 40, 32, 0.2, 32, 32,
+                                       32, 32, 0), api.BLT_ATTN_MASK_CAUSAL) for i in range(3)]   # three sizes: no strided batch
+    vd, vs = _dev_tensor(out[0]), _dev_tensor(qkv[0])
+    torch.cuda.synchronize()
+    lib.blt_hip_profile_begin()
+    lib.blt_attention_batch_hip(api.problem_array(probs), 3)
+    lib.blt_rows_gather(C.byref(vs), (C.c_size_t * 40)(*range(40)), C.byref(vd))
+    launched = api.profile_end()
+    assert launched["upload_words"][0] >= 1 and launched["rows_gather"][0] == 1, launched
+
+
 def test_graph_replay_of_a_plan_and_a_decode_layer(oracle, dev):
     """Library launches recorded into a HIP graph: every replay, with eager work and
     synchronisations in between, gives the eager result."""
