@@ -56,217 +56,75 @@
 
 namespace {
 
-/* One group of 32 WV rows of problem p on the fp32 matrix instructions, every score tested for finiteness: the
- * second run of a group whose first run met something that is not finite. */
+/* The rows of a group once more on the fp32 matrix instructions, every score tested for finiteness: the second run of a
+ * group whose first run met something that is not finite.  Seldom, so without any of the machinery of the first: a wave
+ * per 32 rows by itself, operands straight from memory. */
 template <int HD, int WV, bool DENSE>
-__device__ __forceinline__ void wide_group_checked(const AttnProb &p, uint32_t group, float (*sm_k)[32 * (HD + 4)],
-                                                float (*sm_v)[32 * (HD + 4)]) {
+__device__ __forceinline__ void wide_group_checked(const AttnProb &p, uint32_t group) {
     constexpr int HALF = HD / 2;
     constexpr int DB = HD / 32;
-    constexpr int ROW = HD + 4;
-    constexpr int LPR = HD / 4;            /* 16-byte pieces per row               */
-    constexpr int PIECES = HD / 32;        /* pieces of one tile per thread of the first four waves */
-
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
-    const uint32_t h = lane >> 5;
-    const uint32_t c = lane & 31u;
-
-    const uint32_t g0 = group * (32u * WV); /* first row of the workgroup */
-    /* which of the query tiles a wave owns rotates with the group index:
-     * under a causal mask the later tiles are longer, and waves with the same
-     * index tend to share a SIMD across resident workgroups */
-    const uint32_t q0 = g0 + ((wave + group) % WV) * 32u; /* first row of this wave */
-    const uint32_t row = q0 + c;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t h = lane >> 5, c = lane & 31u;
+    const uint32_t q0 = group * (32u * WV) + wave * 32u, row = q0 + c;
+    if (q0 >= p.nq) return;
     const bool live = row < p.nq;
     const uint32_t i = live ? row : p.nq - 1u;
-
-    uint32_t lo, hi;
+    uint32_t lo, hi, wlo, whi, flo, fhi;
     row_key_range(p, i, lo, hi);
-    if (!live) hi = lo;
+    span_key_bounds(p, q0, min(q0 + 31u, p.nq - 1u), wlo, whi, flo, fhi);
 
-    /* key spans of the workgroup and of this wave, in tiles; all wave-uniform */
-    uint32_t glo, ghi, wlo = 0xFFFFFFFFu, whi = 0u, flo = 0u, fhi = 0u, dummy0, dummy1;
-    span_key_bounds(p, g0, min(g0 + 32u * WV - 1u, p.nq - 1u), glo, ghi, dummy0, dummy1);
-    if (q0 < p.nq) span_key_bounds(p, q0, min(q0 + 31u, p.nq - 1u), wlo, whi, flo, fhi);
-    const bool g_any = ghi > glo, w_any = whi > wlo;
-    const uint32_t gt_lo = __builtin_amdgcn_readfirstlane(g_any ? glo / 32u : 0u);
-    const uint32_t gt_hi = __builtin_amdgcn_readfirstlane(g_any ? (ghi + 31u) / 32u : 0u);
-    const uint32_t kt_lo = __builtin_amdgcn_readfirstlane(w_any ? wlo / 32u : 0u);
-    const uint32_t kt_hi = __builtin_amdgcn_readfirstlane(w_any ? (whi + 31u) / 32u : 0u);
-    flo = __builtin_amdgcn_readfirstlane(flo);
-    fhi = __builtin_amdgcn_readfirstlane(fhi);
-
-    const float scale2 = p.scale * LOG2E;
-    const float *mrow = DENSE ? p.mask + (size_t)i * p.nk : nullptr;
-    const bool mvec = DENSE && (p.nk % 4u == 0u) && ((reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0u);
-
-    /* ---- query fragment: row c, floats [h*HALF, (h+1)*HALF), pre-scaled ---- */
-    float qf[HALF];
-    {
-        const float *qrow = p.q + (size_t)i * p.q_stride + h * HALF;
+    float qf[HALF], m = neg_inf(), l = 0.f;
 #pragma unroll
-        for (int s = 0; s < HALF; s += 4) {
-            const float4 t = *reinterpret_cast<const float4 *>(qrow + s);
-            qf[s + 0] = t.x * scale2;
-            qf[s + 1] = t.y * scale2;
-            qf[s + 2] = t.z * scale2;
-            qf[s + 3] = t.w * scale2;
-        }
-    }
-
+    for (int s = 0; s < HALF; s++) qf[s] = p.q[(size_t)i * p.q_stride + h * HALF + s] * (p.scale * LOG2E);
     floatx16 oacc[DB];
 #pragma unroll
     for (int b = 0; b < DB; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) oacc[b][r] = 0.f;
-    float m = neg_inf(), l = 0.f;
 
-    /* ---- tile movement: of the first four waves, thread t carries pieces t, t+256, ... of K and of V ---- */
-    float pk[4 * PIECES], pv[4 * PIECES];
-    auto request = [&](uint32_t kt) __attribute__((always_inline)) {
-        if (wave >= 4u) return;
+    for (uint32_t k0 = whi > wlo ? wlo / 32u * 32u : whi; k0 < whi; k0 += 32u) {
+        const float *krow = p.k + (size_t)min(k0 + c, p.nk - 1u) * p.k_stride + h * HALF;
+        floatx16 sacc;
 #pragma unroll
-        for (int u = 0; u < PIECES; u++) {
-            const uint32_t e = threadIdx.x + 256u * u;
-            const uint32_t j = min(kt * 32u + e / LPR, p.nk - 1u);
-            const float4 a = *reinterpret_cast<const float4 *>(p.k + (size_t)j * p.k_stride + 4u * (e % LPR));
-            const float4 b = *reinterpret_cast<const float4 *>(p.v + (size_t)j * p.v_stride + 4u * (e % LPR));
-            pk[4 * u + 0] = a.x, pk[4 * u + 1] = a.y, pk[4 * u + 2] = a.z, pk[4 * u + 3] = a.w;
-            pv[4 * u + 0] = b.x, pv[4 * u + 1] = b.y, pv[4 * u + 2] = b.z, pv[4 * u + 3] = b.w;
+        for (int r = 0; r < 16; r++) sacc[r] = 0.f;
+#pragma unroll
+        for (int s = 0; s < HALF; s++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[s], qf[s], sacc, 0, 0, 0);
+        float x[16], mt = neg_inf();
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const uint32_t j = k0 + acc_key(r, h);
+            const float t = DENSE ? sacc[r] + p.mask[(size_t)i * p.nk + min(j, p.nk - 1u)] * LOG2E : sacc[r];
+            x[r] = (j >= lo) & (j < hi) & isfinite(t) ? t : neg_inf();
+            mt = fmaxf(mt, x[r]);
         }
-    };
-    auto park = [&](uint32_t buf) __attribute__((always_inline)) {
-        if (wave >= 4u) return;
+        const float mn = fmaxf(m, swap32(mt, OpMax())), ms = mn == neg_inf() ? 0.f : mn;
+        const float alpha = fast_exp2(m - ms);
+        m = mn, l *= alpha;
 #pragma unroll
-        for (int u = 0; u < PIECES; u++) {
-            const uint32_t e = threadIdx.x + 256u * u;
-            const uint32_t off = (e / LPR) * ROW + 4u * (e % LPR);
-            *reinterpret_cast<float4 *>(&sm_k[buf][off]) =
-                make_float4(pk[4 * u + 0], pk[4 * u + 1], pk[4 * u + 2], pk[4 * u + 3]);
-            *reinterpret_cast<float4 *>(&sm_v[buf][off]) =
-                make_float4(pv[4 * u + 0], pv[4 * u + 1], pv[4 * u + 2], pv[4 * u + 3]);
+        for (int r = 0; r < 16; r++) {
+            x[r] = fast_exp2(x[r] - ms);
+            l += x[r];
         }
-    };
-
-    if (gt_lo < gt_hi) {
-        request(gt_lo);
-        park(0);
-    }
-    __syncthreads();
-
-    for (uint32_t kt = gt_lo; kt < gt_hi; kt++) {
-        const uint32_t buf = (kt - gt_lo) & 1u;
-        const bool more = kt + 1u < gt_hi;
-        if (more) request(kt + 1u); /* travels while this tile is worked on */
-
-        if (kt >= kt_lo && kt < kt_hi) {
-            const uint32_t k0 = kt * 32u;
-            const float *ks = sm_k[buf];
-            const float *vs = sm_v[buf];
-
-            /* dense mask values for this lane's 16 keys: requested before the first contraction */
-            float mk[16];
-            if (DENSE) {
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const uint32_t j0 = k0 + 8u * g + 4u * h;
-                    if (mvec) {
-                        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if (j0 < p.nk) t = *reinterpret_cast<const float4 *>(mrow + j0);
-                        mk[4 * g + 0] = t.x, mk[4 * g + 1] = t.y, mk[4 * g + 2] = t.z, mk[4 * g + 3] = t.w;
-                    } else {
+        for (int b = 0; b < DB; b++) {
 #pragma unroll
-                        for (int e = 0; e < 4; e++) mk[4 * g + e] = mrow[min(j0 + e, p.nk - 1u)];
-                    }
-                }
-            }
-
-            /* ---- S^T = K Q^T ---- */
-            floatx16 sacc;
-#pragma unroll
-            for (int r = 0; r < 16; r++) sacc[r] = 0.f;
-#pragma unroll
-            for (int s4 = 0; s4 < HALF; s4 += 4) {
-                const float4 t = *reinterpret_cast<const float4 *>(ks + c * ROW + h * HALF + s4);
-                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(t.x, qf[s4 + 0], sacc, 0, 0, 0);
-                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(t.y, qf[s4 + 1], sacc, 0, 0, 0);
-                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(t.z, qf[s4 + 2], sacc, 0, 0, 0);
-                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(t.w, qf[s4 + 3], sacc, 0, 0, 0);
-            }
-
-            /* ---- mask, tile maximum ----
-             * Interior tiles (no row masks any key) take the scores as they
-             * are; edge tiles compare the key's offset into the row's range
-             * with one unsigned test.  No per-element branches. */
-            float x[16];
-            float mt = neg_inf();
-            const bool all_seen = !DENSE && k0 >= flo && k0 + 32u <= fhi; /* wave-uniform */
-            if (all_seen) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const float t = sacc[r];
-                    x[r] = isfinite(t) ? t : neg_inf();
-                    mt = fmaxf(mt, x[r]);
-                }
-            } else {
-                const uint32_t rel = k0 + 4u * h - lo, len = hi - lo;
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    float t = sacc[r];
-                    if (DENSE) t += mk[r] * LOG2E;
-                    const bool vis = (rel + (8u * (r >> 2) + (r & 3u)) < len) & isfinite(t);
-                    x[r] = vis ? t : neg_inf();
-                    mt = fmaxf(mt, x[r]);
-                }
-            }
-            mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-            const float mn = fmaxf(m, mt);
-            const float ms = mn == neg_inf() ? 0.f : mn; /* nothing seen yet: keep the differences finite */
-            if (__any(mn > m)) {
-                const float alpha = fast_exp2(m - ms);
-                l *= alpha;
-#pragma unroll
-                for (int b = 0; b < DB; b++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) oacc[b][r] *= alpha;
-                m = mn;
-            }
-            float ps = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                x[r] = fast_exp2(x[r] - ms);
-                ps += x[r];
-            }
-            l += ps;
-
-            /* ---- O^T += V^T P^T ---- */
+            for (int r = 0; r < 16; r++) oacc[b][r] *= alpha;
 #pragma unroll
             for (int s = 0; s < 16; s++) {
-                const float *vrow = vs + acc_key(s, h) * ROW + c;
-#pragma unroll
-                for (int b = 0; b < DB; b++)
-                    oacc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * b], x[s], oacc[b], 0, 0, 0);
+                const float v = p.v[(size_t)min(k0 + acc_key(s, h), p.nk - 1u) * p.v_stride + 32 * b + c];
+                oacc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, x[s], oacc[b], 0, 0, 0);
             }
         }
-
-        if (more) park(buf ^ 1u);
-        __syncthreads();
     }
 
-    /* both halves of a column carry the same m, their sums add */
-    l += __shfl_xor(l, 32, 64);
+    l = swap32(l, OpSum()); /* both halves of a column carry the same m */
     if (!live) return;
-
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     float *orow = p.out + (size_t)i * p.out_stride;
 #pragma unroll
     for (int b = 0; b < DB; b++)
 #pragma unroll
-        for (int g = 0; g < 4; g++)
-            *reinterpret_cast<float4 *>(orow + b * 32 + 8 * g + 4 * h) =
-                make_float4(oacc[b][4 * g + 0] * inv, oacc[b][4 * g + 1] * inv, oacc[b][4 * g + 2] * inv,
-                            oacc[b][4 * g + 3] * inv);
+        for (int r = 0; r < 16; r++) orow[32 * b + acc_key(r, h)] = oacc[b][r] * inv;
     if (h == 0 && p.lse) {
         p.lse[2 * (size_t)i + 0] = m * LN2; /* back to natural units */
         p.lse[2 * (size_t)i + 1] = l;
@@ -578,9 +436,7 @@ __device__ __forceinline__ void wide_pair(uint32_t t, uint32_t G, uint32_t &ga, 
 template <int HD, int WV, int SRC, bool DENSE>
 __global__ __launch_bounds__(64 * WV, 2) void attn_wide_kernel(const AttnProb *__restrict__ probs,
                                                            const AttnTile *__restrict__ tiles, AttnAffine aff) {
-    constexpr int TILE = 32 * (HD + 4);
-    constexpr int CHECKED = 4 * TILE * 4, SPLIT = 2 * sizeof(WideTiles<HD>);
-    __shared__ __attribute__((aligned(16))) unsigned char sm[CHECKED > SPLIT ? CHECKED : SPLIT];
+    __shared__ __attribute__((aligned(16))) WideTiles<HD> sm[2];
 
     uint32_t ga, gb = WIDE_NO_GROUP;
     AttnProb p;
@@ -605,10 +461,7 @@ __global__ __launch_bounds__(64 * WV, 2) void attn_wide_kernel(const AttnProb *_
     for (int pass = 0; pass < 2; pass++) {
         const uint32_t group = pass == 0 ? ga : gb;
         if (group == WIDE_NO_GROUP) break;
-        if (wide_group<HD, WV, DENSE>(p, group, *reinterpret_cast<WideTiles<HD>(*)[2]>(sm))) {
-            float (*const tiles32)[TILE] = reinterpret_cast<float (*)[TILE]>(sm);
-            wide_group_checked<HD, WV, DENSE>(p, group, tiles32, tiles32 + 2);
-        }
+        if (wide_group<HD, WV, DENSE>(p, group, sm)) wide_group_checked<HD, WV, DENSE>(p, group);
     }
 }
 
