@@ -44,8 +44,9 @@
  * waiting for the rest of the launch, takes NaN for what it did not get and runs to its end; the host turns the word
  * into a fatal error at its next look).
  *
- * Measured, launches -> this kernel: one row, two layers of 128 columns, 300 keys 69 -> 37 us; 64 such rows 78 ->
- * 60 us; 16 draft rows of one sequence 80 -> 61 us.  What is left is the chain: a hand-over takes about 1 us from
+ * Measured, launches -> this kernel: one row, two layers of 128 columns, 300 keys 69 -> 38 us; 64 such rows 78 ->
+ * 61 us; 16 draft rows of one sequence 80 -> 61 us.  The roll call is a quarter of a microsecond of that where the first
+ * loads of a workgroup are on their way meanwhile, and 1.5 us in front of everything.  What is left is the chain: a hand-over takes about 1 us from
  * the store to the reader's first use, and a wave that shares its SIMD with three others issues an instruction
  * every nine cycles, so the 100 ... 200 instructions of a stage between its operand and its result are another.
  */
@@ -183,10 +184,7 @@ __device__ __forceinline__ void await_at(Waiter &wt, At at, bool pad, uint32_t t
     }
 #pragma unroll
     for (int i = 0; i < N; i++) out[i] = __uint_as_float((uint32_t)t[i]); /* pad lanes: anything */
-    if (wt.expired) {
-#pragma unroll
-        for (int i = 0; i < N; i++) out[i] = not_there();
-    }
+    out[0] = wt.expired ? not_there() : out[0]; /* one of a row's values is enough to make every sum of it NaN */
 }
 /* word `index` of a region: a uniform base and a 32-bit byte offset per lane, which the load takes as they are */
 __device__ __forceinline__ const uint64_t *word_of(const uint64_t *base, uint32_t index) {
@@ -230,24 +228,70 @@ constexpr uint32_t FIRST_XQ = 24, FIRST_XPROJ = 0, FIRST_QKV = 8, FIRST_PROJ = 0
 
 /* Stages of a layer in their order, and the LM head behind the last layer */
 enum Stage : uint32_t { STAGE_XQ, STAGE_XPROJ, STAGE_QKV, STAGE_ATTN, STAGE_PROJ, STAGE_UPGATE, STAGE_DOWN, STAGES, STAGE_LM = STAGES };
-/* What a call of a role works on: everything, or one stage (STAGES of layer L: the LM head). */
-struct WholeStep {
-    __device__ __forceinline__ uint32_t begin() const { return 0u; }
-    __device__ __forceinline__ uint32_t end(uint32_t L) const { return L; }
-    __device__ __forceinline__ bool has(Stage) const { return true; }
+struct Standing {
+    uint32_t rank, members; /* members == 0: the work is others' */
 };
+/* The roll call of a group.  A word per workgroup: 2 tag = in, 2 tag + 1 = out, less = not decided yet.  Words only grow and
+ * each is decided once, so everybody comes to the same list. */
+__device__ __forceinline__ void sign_in(uint64_t *roll, uint32_t index, uint32_t tag) {
+    __hip_atomic_fetch_max(roll + index, 2ull * tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+/* by one wave of each workgroup; lane i looks at workgroup i's word */
+__device__ __forceinline__ Standing call_roll(uint64_t *roll, uint32_t index, uint32_t tag, uint32_t limit) {
+    static_assert(2u * WORKERS == 64u, "a lane per workgroup");
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t in = 2ull * tag;
+    const uint64_t begin = wall_clock64();
+    for (;;) {
+        uint64_t word = __hip_atomic_load(roll + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t present = __ballot(word == in);
+        if (__all(word >= in)) {
+            if ((present >> index & 1ull) == 0ull) return {0u, 0u};
+            return {(uint32_t)__popcll(present & ((1ull << index) - 1ull)), (uint32_t)__popcll(present)};
+        }
+        /* only who is in for good signs others out: somebody always is */
+        if ((present >> index & 1ull) != 0ull && (wall_clock64() - begin) * __popcll(present) >= 64ull * limit && word < in)
+            __hip_atomic_compare_exchange_strong(roll + lane, &word, in + 1ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+/* What a call of a role works on: one stage (STAGES of layer L: the LM head) ... */
 struct OneStage {
     uint32_t layer, stage;
     __device__ __forceinline__ uint32_t begin() const { return layer; }
     __device__ __forceinline__ uint32_t end(uint32_t L) const { return min(layer + 1u, L); }
     __device__ __forceinline__ bool has(Stage st) const { return st == stage; }
+    __device__ __forceinline__ bool all_here(uint32_t) { return true; }
+};
+/* ... or everything, if all workgroups of the group are there: a role asks before its first wait and its first store, with
+ * its first loads on their way, and returns if not.  All waves of a workgroup ask at the same place. */
+struct WholeStep {
+    ArgsPtr args;
+    uint32_t group, index;
+    Standing *standing; /* in LDS */
+    bool asked;
+    __device__ __forceinline__ uint32_t begin() const { return 0u; }
+    __device__ __forceinline__ uint32_t end(uint32_t L) const { return L; }
+    __device__ __forceinline__ bool has(Stage) const { return true; }
+    __device__ __forceinline__ bool all_here(uint32_t wave) {
+        if (asked) return true;
+        asked = true;
+        if (wave == 0u) {
+            const Standing st = call_roll(args->rolls + group * (2u * WORKERS), index, args->tag, args->roll_limit);
+            if ((threadIdx.x & 63u) == 0u) *standing = st;
+        }
+        __syncthreads();
+        return __builtin_amdgcn_readfirstlane(standing->members) == 2u * WORKERS;
+    }
 };
 
 /* The workgroups that run the products: every stage but the self-attention.  A stage of a worker: its weights,
  * the operand as soon as it is there, the product over the wave's share of K, the waves' partial tiles through
  * LDS, the results of 256 threads per row tile. */
 template <int E, int HD, int RT, typename Share>
-__device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, const Share sh, float *area,
+__device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, Share sh, float *area,
                                              float (*part_ss)[16 * RT][WAVES], float (*xquery)[HD]) {
     using At = Regions<E, RT>;
     using Shape = ResidentShape<HD, RT>;
@@ -345,6 +389,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
         for (int i = 0; i < KB; i++) b[i] = wp[4 * i * E];
         const uint32_t oc = t * 16u + f_col;
         if (f_on && res_plain) r1[0] = plain_row(ap, f_safe)[oc];
+        if (!sh.all_here(wave)) return false;
         if (shares) { /* the shares' sums, weighed with the common maximum and divided by the common sum; a wave's columns are of one head */
             const uint32_t head = 4u * KB * wave / HD;
 #pragma unroll
@@ -381,6 +426,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
         meet(One(), acc, nullptr);
         if (f_on && f_row < rows) word_store(words + to + operand_at<RT>(f_row, oc), r1[0] + total(All(), f_rt, 0), tag);
         buf ^= 1u;
+        return true;
     };
     auto first = [&](uint32_t at) { return (gv.worker - at) & (WORKERS - 1u); };
 
@@ -411,7 +457,8 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
             const size_t cell0 = cell(min(wave * RPW + lane / HD, rows - 1u));
             const float early_k = xk[cell0], early_v = xv[cell0];
             if (plain) operand_plain(std::integral_constant<int, XKB>(), ap, XKB * kpart, av);
-            else operand(std::integral_constant<int, XKB>(), in, XKB * kpart, tag - 1u, av);
+            if (!sh.all_here(wave)) return;
+            if (!plain) operand(std::integral_constant<int, XKB>(), in, XKB * kpart, tag - 1u, av);
             floatx4 acc[RT][2];
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
@@ -469,8 +516,9 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
             }
             buf ^= 1u;
         }
-        if (crossed && sh.has(STAGE_XPROJ) && first(FIRST_XPROJ) < (uint32_t)E / 16u)
-            square(ap, ap->layer[layer].xproj, At::xcomb, false, tag, plain, in, tag - 1u, At::mid, first(FIRST_XPROJ));
+        if (crossed && sh.has(STAGE_XPROJ) && first(FIRST_XPROJ) < (uint32_t)E / 16u &&
+            !square(ap, ap->layer[layer].xproj, At::xcomb, false, tag, plain, in, tag - 1u, At::mid, first(FIRST_XPROJ)))
+            return;
 
         ap = hidden_args(args);
         for (uint32_t t = first(FIRST_QKV); sh.has(STAGE_QKV) && t < 3u * E / 16u; t += WORKERS) { /* ---- QKV: rotated, keys and values written through ---- */
@@ -492,7 +540,8 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
             float *cell = (part_of == 1u ? ap->layer[layer].ck : ap->layer[layer].cv) + ((size_t)(gv.seq0 + sq) * ap->max_seq + slot) * E + cc;
             asm volatile("" : "+v"(to), "+v"(cell)); /* here, not after the wait */
             if (plain && !crossed) operand_plain(Steps(), ap, KB * wave, av);
-            else operand(Steps(), crossed ? At::mid : in, KB * wave, crossed ? tag : tag - 1u, av);
+            if (!sh.all_here(wave)) return;
+            if (!plain || crossed) operand(Steps(), crossed ? At::mid : in, KB * wave, crossed ? tag : tag - 1u, av);
             floatx4 acc[RT][1];
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
@@ -523,9 +572,10 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
         }
 
         ap = hidden_args(args);
-        if (sh.has(STAGE_PROJ) && first(FIRST_PROJ) < (uint32_t)E / 16u)
-            square(ap, ap->layer[layer].proj, At::comb, ap->splits > 1u, tag, plain && !crossed, crossed ? At::mid : in,
-                   crossed ? tag : tag - 1u, At::resid, first(FIRST_PROJ));
+        if (sh.has(STAGE_PROJ) && first(FIRST_PROJ) < (uint32_t)E / 16u &&
+            !square(ap, ap->layer[layer].proj, At::comb, ap->splits > 1u, tag, plain && !crossed, crossed ? At::mid : in,
+                    crossed ? tag : tag - 1u, At::resid, first(FIRST_PROJ)))
+            return;
 
         ap = hidden_args(args);
         fresh_lane();
@@ -549,6 +599,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
                 const float n1 = nw[4 * i];
                 b[0][i] = up[4 * i * hidden] * n1, b[1][i] = gate[4 * i * hidden] * n1;
             }
+            if (!sh.all_here(wave)) return;
             operand(Steps(), At::resid, KB * wave, tag, av);
             floatx4 acc[RT][2];
 #pragma unroll
@@ -572,6 +623,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
 
         ap = hidden_args(args);
         if (down_here) { /* ---- down projection + residual ---- */
+            if (!sh.all_here(wave)) return;
             fresh_lane();
             const uint32_t oc = first(FIRST_DOWN) * 16u + f_col;
             float r1[1] = {0.f};
@@ -612,6 +664,7 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
         const float *w = ap->lm + (size_t)(4u * KB * wave + g) * V + t * 16u + c;
 #pragma unroll
         for (int i = 0; i < KB; i++) b[i] = w[(size_t)(4 * i) * V];
+        if (!sh.all_here(wave)) return;
         operand(Steps(), At::output(L - 1u), KB * wave, ap->tag + L - 1u, av);
         floatx4 acc[RT][1];
 #pragma unroll
@@ -624,12 +677,13 @@ __device__ __forceinline__ void product_role(ArgsPtr args, const GroupView gv, c
         if (f_on && f_row < rows) ap->logits[(size_t)(gv.row0 + f_row) * V + t * 16u + f_col] = total(All(), f_rt, 0);
         buf ^= 1u;
     }
+    (void)sh.all_here(wave); /* a workgroup without any tile may have to stand in for others */
 }
 
 /* The workgroups that run the self-attention stages: units of one (sequence, head, share of the keys).  The first
  * key and value tiles of a wave are requested and turned into fragments before the query is there. */
 template <int E, int HD, int RT, typename Share>
-__device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv, const Share sh, float *area) {
+__device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv, Share sh, float *area) {
     using At = Regions<E, RT>;
     constexpr int QD = HD / 4, NV = QD / 4, DT = HD / 16, ROW = HD + 4, H = E / HD;
     constexpr int LPR = HD / 4, RPI = 64 / LPR;
@@ -641,6 +695,7 @@ __device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv,
     float *const tiles = area + 2 * 16 * WAVES;
     float *const tile = tiles + wave * (16 * ROW);
     const uint32_t splits = args->splits, units = gv.ns * (uint32_t)H * splits, n = args->n;
+    if (!sh.all_here(wave)) return;
 
     for (uint32_t layer = sh.begin(); layer < sh.end(args->L); layer++)
     for (uint32_t u = gv.worker; u < units; u += WORKERS) {
@@ -828,32 +883,6 @@ __device__ __forceinline__ void attention_role(ArgsPtr args, const GroupView gv,
     }
 }
 
-struct Standing {
-    uint32_t rank, members; /* members == 0: the work is others' */
-};
-/* The roll call of a group, by one wave of each of its workgroups; lane i looks at workgroup i's word: 2 tag = in, 2 tag + 1 =
- * out, less = not decided yet.  Words only grow and each is decided once, so everybody comes to the same list. */
-__device__ __forceinline__ Standing call_roll(uint64_t *roll, uint32_t index, uint32_t tag, uint32_t limit) {
-    static_assert(2u * WORKERS == 64u, "a lane per workgroup");
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t in = 2ull * tag;
-    if (lane == 0u) __hip_atomic_fetch_max(roll + index, in, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint64_t begin = wall_clock64();
-    for (;;) {
-        uint64_t word = __hip_atomic_load(roll + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint64_t present = __ballot(word == in);
-        if (__all(word >= in)) {
-            if ((present >> index & 1ull) == 0ull) return {0u, 0u};
-            return {(uint32_t)__popcll(present & ((1ull << index) - 1ull)), (uint32_t)__popcll(present)};
-        }
-        /* only who is in for good signs others out: somebody always is */
-        if ((present >> index & 1ull) != 0ull && (wall_clock64() - begin) * __popcll(present) >= 64ull * limit && word < in)
-            __hip_atomic_compare_exchange_strong(roll + lane, &word, in + 1ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_sleep(1);
-    }
-}
-
 template <int E, int HD, int RT>
 __global__ __launch_bounds__(64 * WAVES, 4) void kv_step_resident_kernel(ResidentArgs a) {
     __shared__ __attribute__((aligned(16))) float area[ResidentShape<HD, RT>::AREA];
@@ -865,22 +894,18 @@ __global__ __launch_bounds__(64 * WAVES, 4) void kv_step_resident_kernel(Residen
     gv.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     gv.seq0 = group * a.per_group;
     if (gv.seq0 >= a.batch) return;
-    if (gv.wave == 0u) {
-        const Standing st = call_roll(a.rolls + group * (2u * WORKERS), index, a.tag, a.roll_limit);
-        if (threadIdx.x == 0u) standing = st;
-    }
-    __syncthreads();
-    const uint32_t rank = __builtin_amdgcn_readfirstlane(standing.rank), members = __builtin_amdgcn_readfirstlane(standing.members);
+    if (threadIdx.x == 0u) sign_in(a.rolls + group * (2u * WORKERS), index, a.tag);
     gv.ns = min(a.per_group, a.batch - gv.seq0);
     gv.rows = gv.ns * a.n, gv.row0 = gv.seq0 * a.n;
     gv.words = a.words + (size_t)group * a.group_words;
     const ArgsPtr ap = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
-    if (members == 2u * WORKERS) {
-        gv.worker = index & (WORKERS - 1u);
-        if (index < WORKERS) product_role<E, HD, RT>(ap, gv, WholeStep(), area, part_ss, xquery);
-        else attention_role<E, HD, RT>(ap, gv, WholeStep(), area);
-        return;
-    }
+    gv.worker = index & (WORKERS - 1u);
+    const WholeStep whole{ap, group, index, &standing, false};
+    if (index < WORKERS) product_role<E, HD, RT>(ap, gv, whole, area, part_ss, xquery);
+    else attention_role<E, HD, RT>(ap, gv, whole, area);
+    const uint32_t rank = __builtin_amdgcn_readfirstlane(standing.rank), members = __builtin_amdgcn_readfirstlane(standing.members);
+    if (members == 2u * WORKERS) return;
+
     const uint32_t stride = min(members, WORKERS);
     if (rank >= stride) return;
     for (uint32_t stage = 0; stage <= a.L * STAGES; stage++) {
