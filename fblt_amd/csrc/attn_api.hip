@@ -134,13 +134,13 @@ Family choose_family(const AttnProb &d) {
     return FAM_ROWS;
 }
 
-/* The wide kernel pays off once its 128-row work items give every compute
- * unit one (short rows: few key tiles per item) or two (long rows: the
- * latency-oriented mfma kernel, which splits the keys of a 32-row tile over
- * its waves, keeps the shorter serial chain for longer) -- measured
- * crossovers: 128..256 items at 128 keys, 256..512 items at 512 keys. */
+/* The wide kernel pays off once its 128-row work items give every compute unit one and a half (rows of up to 512
+ * keys) or two (longer: the latency-oriented mfma kernel, which splits the keys of a 32-row tile over its waves, keeps
+ * the shorter serial chain for longer).  Causal, us, mfma against wide: 256 keys, 256 items of heads of 32 12.9 / 14.1,
+ * of 64 20.4 / 21.3, 384 items 17.2 / 15.2 and 29.0 / 25.0; 512 keys, 384 items 22.4 / 22.9 and 39.7 / 38.9; 768 keys,
+ * 384 items 29.3 / 30.6 and 50.4 / 52.7, 576 items 41.3 / 34.9 and 72.0 / 58.7. */
 uint32_t wide_min_groups(uint32_t max_nk) {
-    return max_nk <= 256u ? 256u : 512u;
+    return max_nk <= 512u ? 384u : 512u;
 }
 
 /* Do problems p[0..n), all routed to the mfma family, go to the wide kernel instead? */
@@ -158,19 +158,20 @@ bool choose_wide(const AttnProb *p, uint32_t n) {
 }
 
 /* Do problems p[0..n), all routed to the mfma family, go to the fine kernel, and in which workgroup
- * shape?  `span` gets the keys its longest 32-row tile needs.  Measured at both head widths (4 heads
- * of 32, 8 heads of 64), 1..128 sequences of 64..2048 rows, against the other two matrix-core
- * kernels:
+ * shape?  `span` gets the keys its longest 32-row tile needs.  Causal, us, at both head widths (4 heads of 32, 8 heads of
+ * 64), against the other matrix-core kernels:
  *   - few long problems (at most 128 tiles of 32 rows, rows of 256 keys and more): workgroups of 16
  *     rows and sixteen waves double the workgroups and halve the chain of matrix instructions on the
- *     busiest SIMD (512 rows x 4 heads: 8.9 -> 8.0 us; 1024 rows: 15.1 -> 11.7 us).  Only strided
- *     batches and single problems have this shape;
- *   - one LDS fill holds every key a tile needs (128 keys at width 64, 256 at 32): ahead unless the
- *     launch is tiny (up to one 4-wave workgroup per compute unit: the mfma kernel's shorter
- *     prologue wins from 128 keys on) or so large that workgroups queue up several deep (the wide
- *     kernel overlaps its fetches with its arithmetic, this one fetches, then computes);
- *   - longer rows when the launch is just what the chip holds at once, two 8-wave workgroups per
- *     compute unit (512 tiles: 10..25 % ahead of the mfma kernel, behind it at 256 and at 1024). */
+ *     busiest SIMD (1024 rows x 4 heads: 11.9, mfma 14.4).  Only strided batches and single problems have this
+ *     shape;
+ *   - rows of up to 128 keys, which one LDS fill holds at either width: ahead unless the launch is tiny (up to one
+ *     4-wave workgroup per compute unit: the mfma kernel's shorter prologue wins from 128 keys on) or so large that
+ *     the wide kernel has its items (64 keys, 384 tiles of heads of 64 7.1, mfma 9.3; 128 keys, 384 groups
+ *     22.1, wide 20.9; 64 keys, 512 groups 12.1, wide 12.9);
+ *   - longer rows, up to 512 keys, when the launch is what the chip holds at once, two 8-wave workgroups per compute
+ *     unit: 288 to 512 tiles while one fill holds them (192 keys of heads of 32: 7.7, mfma 9.2; with 576 tiles 9.7 against
+ *     8.5), 449 to 512 beyond (256 keys of heads of 64: 10.9, mfma 11.5; 512 keys 17.0 / 17.2; 1024 keys are level,
+ *     2048 behind). */
 bool choose_fine(const AttnProb *p, uint32_t n, bool strided, uint32_t &span, bool &tall) {
     /* BLT_HIP_FINE_ROWS=16|32 pins the workgroup shape (tuning and test hook) */
     static const int rows_pinned = [] {
@@ -200,9 +201,10 @@ bool choose_fine(const AttnProb *p, uint32_t n, bool strided, uint32_t &span, bo
         tall = true;
         return true;
     }
-    if (span > attn_fine_fill_max(p[0].hd)) return tiles > 448u && tiles <= 512u;
+    if (span > attn_fine_fill_max(p[0].hd)) return tiles > 448u && tiles <= 512u && max_nk <= 512u;
     if (tiles <= 256u && span > 64u) return false;
-    return groups < (max_nk <= 64u ? 640u : 448u);
+    if (span > 128u) return tiles <= 512u;
+    return groups < (max_nk <= 64u ? 640u : 384u);
 }
 
 /* Do problems p[0..n), all routed to the mfma family, go to the once kernel (16-row tiles whose keys
@@ -219,10 +221,11 @@ bool choose_once(const AttnProb *p, uint32_t n, uint32_t &span) {
         most = std::max(most, attn_once_span_tiles(p[i]));
         tiles += (p[i].nq + 15u) / 16u;
     }
-    /* measured against the other matrix-core kernels (4 heads of 32 over 256 ... 1024 rows, 8 heads of 64
-     * over 128 rows, 1 ... 16 sequences): ahead up to 256 tiles whatever the rows' length (one workgroup
-     * per compute unit), up to 512 tiles while a row has at most 128 keys, behind beyond */
-    if (forced == 0 && tiles > (most <= 8u ? 512u : 256u)) return false;
+    /* Causal, us: one workgroup per compute unit whatever the rows' length (256 tiles of 256 keys, heads of 32: 5.3, mfma
+     * 6.7; of 64: 7.5 / 9.5), two while a row has 65 to 128 keys (512 tiles of 128 keys 5.1, fine 5.2, and 6.9 / 7.2;
+     * of 256 keys 7.1, mfma 6.8, and 11.3 / 9.8).  Two of shorter rows are better off on the fine kernel, which has half the
+     * workgroups (512 tiles of 64 keys 4.8, fine 4.5, and 6.5 / 5.5). */
+    if (forced == 0 && tiles > (most > 4u && most <= 8u ? 512u : 256u)) return false;
     span = most;
     return true;
 }
@@ -241,10 +244,11 @@ bool choose_whole(const AttnProb &d, uint32_t n, bool strided) {
     if (!strided || (forced != 0 && forced != 4) || !attn_whole_can(d)) return false;
     if (rows_pinned != 0) return rows_pinned == 128;
     if (forced != 0 || d.nq < 48u) return false; /* three row halves and fewer leave most of the waves idle */
-    /* measured against the family's other shapes and the wide kernel (8 heads of 64 and 4 heads
-     * of 32): 128 rows ahead from 144 problems on (11.9 against 12.4 us; 12.5 against 15.6 at
-     * 256, 38.7 against 45.5 at 1024, 72.5 against 86 at 2048), 64 rows from 768 on */
-    return n >= (d.nq > 64u ? 144u : 640u);
+    /* Against the family's other shapes and the wide kernel, us, heads of 64 and of 32.  128 rows from 144 problems on: 128
+     * problems 10.5, fine 8.5 (7.3 / 6.4); 192 problems 10.8, fine 14.0 (7.1, mfma 8.8); 1024 35.7, wide 40.0 (20.4 /
+     * 23.5); 2048 64.1 / 73.6.  64 rows from 512 on: 384 problems 11.2, fine 10.3 (7.6, mfma 7.4), 512 11.8 / 12.0
+     * (8.0, wide 8.7); 1024 21.2, fine 23.0 (12.4, wide 14.7) */
+    return n >= (d.nq > 64u ? 144u : 512u);
 }
 
 /* Element distance between two float pointers (either both NULL or both set). */
