@@ -310,13 +310,14 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         float q[HALF];
         query_row(q);
 #pragma unroll
-        for (int s = 0; s < QS; s++) split_bf16_at<8>(q, 8 * s, qf[s]);
+        for (int s = 0; s < QS; s++) split_bf16_at<8>(q, 8 * s, qf[s], SPLIT_FAR);
     }
     if (STAGE && kt < kt_hi) K_PARK(kt);
     /* Scores of one or two products are closer on the fp32 instructions (as the products of matmul.hip; heads of one, error
-     * of the output against float64 1.4 ... 2.6e-7 on parts, 1.0 ... 2.0e-7): only the second run below */
-    const bool few = !EXACT && p.hd < 3u;
-    bool bad = few; /* met a score that is not finite */
+     * of the output against float64 1.4 ... 2.6e-7 on parts, 1.0 ... 2.0e-7): only the second run below.  Likewise where
+     * the scale is so large that the keys' error in a score (split_bf16.h) would count. */
+    const bool fp32_only = (!EXACT && p.hd < 3u) || fabsf(scale2) > 64.0f;
+    bool bad = fp32_only; /* met a score that is not finite */
     /* ---- scale, mask, running maximum: scores of tile kt -> weights ---- */
     /* unit: of the score registers */
     auto weigh = [&](const floatx16 &sacc, float unit, uint32_t tile, float (&x)[16]) __attribute__((always_inline)) {
@@ -354,7 +355,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         return alpha;
     };
     /* The contractions run on three bf16 parts of their operands. */
-    while (kt < kt_hi && !few) {
+    while (kt < kt_hi && !fp32_only) {
         const uint32_t ktn = kt + NW;
 
         if (STAGE) {
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
             split_bf16_at<8>(x, 8 * j, pp);
 #pragma unroll
             for (int b = 0; b < DB; b++) {
-                split_bf16_at<8>(vf[b], 8 * j, vp);
+                split_bf16_at<8>(vf[b], 8 * j, vp, SPLIT_FAR);
                 oacc[b] = mfma_split(vp, pp, oacc[b]);
             }
         }
@@ -559,7 +560,7 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         query_row(q);
         if (!again) {
 #pragma unroll
-            for (int s = 0; s < QS; s++) split_bf16_at<8>(q, 8 * s, qf[s]);
+            for (int s = 0; s < QS; s++) split_bf16_at<8>(q, 8 * s, qf[s], SPLIT_FAR);
         }
     }
     for (uint32_t wt = wave; wt < nkt; wt += NW) {

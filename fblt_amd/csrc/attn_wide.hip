@@ -99,12 +99,13 @@ __device__ __forceinline__ void wide_group_checked(const AttnProb &p, uint32_t g
         }
         const float mn = fmaxf(m, swap32(mt, OpMax())), ms = mn == neg_inf() ? 0.f : mn;
         const float alpha = fast_exp2(m - ms);
-        m = mn, l *= alpha;
+        float ps = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             x[r] = fast_exp2(x[r] - ms);
-            l += x[r];
+            ps += x[r];
         }
+        m = mn, l = l * alpha + ps;
 #pragma unroll
         for (int b = 0; b < DB; b++) {
 #pragma unroll
@@ -185,7 +186,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
     flo = __builtin_amdgcn_readfirstlane(flo);
     fhi = __builtin_amdgcn_readfirstlane(fhi);
 
-    const float scale2 = p.scale * LOG2E * SPLIT_UP;
+    const float scale2 = p.scale * LOG2E * SPLIT_FAR;
     const float *mrow = DENSE ? p.mask + (size_t)i * p.nk : nullptr;
     const bool mvec = DENSE && (p.nk % 4u == 0u) && ((reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0u);
 
@@ -198,7 +199,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
             const float4 a = *reinterpret_cast<const float4 *>(qrow + 16 * s), b = *reinterpret_cast<const float4 *>(qrow + 16 * s + 4);
             const float x[8] = {a.x * scale2, a.y * scale2, a.z * scale2, a.w * scale2,
                                 b.x * scale2, b.y * scale2, b.z * scale2, b.w * scale2};
-            split_bf16_scaled<8>(x, qf[s][0], qf[s][1], qf[s][2]);
+            split_bf16<8>(x, qf[s][0], qf[s][1], qf[s][2]);
         }
     }
 
@@ -252,7 +253,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
             piece a[3];
             float x[EPT];
 #pragma unroll
-            for (int u = 0; u < EPT; u++) x[u] = for_k ? pk[u] : pv[u];
+            for (int u = 0; u < EPT; u++) x[u] = for_k ? pk[u] : pv[u] * SPLIT_FAR;
             split_bf16<EPT>(x, a[0], a[1], a[2]);
             __bf16 *to = for_k ? &sm[kbuf].k[0][krow * Tiles::KROW + kcol] : &sm[vbuf].v[0][vcol * Tiles::VROW + vgrp * EPT];
             const uint32_t part = for_k ? Tiles::KPART : Tiles::VPART;
@@ -269,7 +270,10 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
             for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&sm[kbuf].k[t][krow * Tiles::KROW + kcol]) = a[t];
         }
         if (v_too) {
-            split_bf16<EPT>(pv, a[0], a[1], a[2]);
+            float x[EPT];
+#pragma unroll
+            for (int u = 0; u < EPT; u++) x[u] = pv[u] * SPLIT_FAR;
+            split_bf16<EPT>(x, a[0], a[1], a[2]);
 #pragma unroll
             for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&sm[vbuf].v[t][vcol * Tiles::VROW + vgrp * EPT]) = a[t];
         }

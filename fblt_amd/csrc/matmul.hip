@@ -175,9 +175,9 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
         float pa[EPT], pb[EPT], squares = 0.f;
 #pragma unroll
         for (int i = 0; i < EPT; i++) {
-            if constexpr (NORM) squares = fmaf(v.a[i], v.a[i], squares), pa[i] = v.a[i] * v.w[i];
-            else pa[i] = v.a[i];
-            pb[i] = v.b[i];
+            if constexpr (NORM) squares = fmaf(v.a[i], v.a[i], squares), pa[i] = v.a[i] * v.w[i] * SPLIT_UP;
+            else pa[i] = v.a[i] * SPLIT_UP;
+            pb[i] = v.b[i] * SPLIT_UP;
         }
         if constexpr (NORM) ss += counts ? squares : 0.f;
         piece parts[3];

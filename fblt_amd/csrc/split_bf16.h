@@ -4,11 +4,17 @@
  * Markidis et al. 2018 and Henry, Tang and Heinecke 2019, "Leveraging the bfloat16 artificial intelligence
  * datatype for higher-precision computations").
  *
- * SPLIT_UP times an fp32 value is the exact sum of three bf16 values (each rounded to nearest from what the ones
- * before leave; 8 significant bits each, 24 in all).  The factor keeps that true down to the smallest subnormal:
- * the last bit of any fp32 value is a multiple of 2^-149, the smallest bf16 subnormal 2^-133 (the matrix
- * instructions take bf16 subnormals as they are).  Unscaled, operands of 1e-36 had a relative error of 2.7e-5, of
- * 1e-38 of 2.7e-3.  Results come out SPLIT_UP^2 times as large; SPLIT_DOWN takes that back.  A product of two such sums is taken as the six
+ * An fp32 value is the exact sum of three bf16 values (each rounded to nearest from what the ones before leave; 8
+ * significant bits each, 24 in all), as long as its last bit, a multiple of 2^-149 for any fp32 value, is at least
+ * the smallest bf16 subnormal, 2^-133 (the matrix instructions take bf16 subnormals as they are).  Below 2^-110 the sum
+ * is within 2^-134 only: products of operands of 1e-36 had a relative error of 2.7e-5.  So operands whose relative error
+ * counts are taken times a power of two, and the results come out that much larger:
+ *   - both operands of a plain product times SPLIT_UP, which makes the sum exact for every fp32 value;
+ *   - in an attention the queries and the values times SPLIT_FAR, keys and weights as they are.  A key's error of
+ *     2^-134 meets queries of at most 2^96 (larger ones overflow, see below): at most 2^-31 in a score, where the score's
+ *     absolute error is what counts.  A weight's error of 2^-134 is below the 2^-126 at which the exponential unit cuts
+ *     weights off.
+ * SPLIT_DOWN takes either back.  A product of two such sums is taken as the six
  * partial products that are at least 2^-18 of it,
  *     x y = h h' + (h m' + m h') + (h l' + l h' + m m')  (+ m l' + l m' + l l', below 2^-25)
  * accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  Against float64 the result is a little closer than
@@ -17,7 +23,7 @@
  * Six bf16 instructions take 192 cycles of the matrix unit where the fp32 ones take 512, and they leave
  * the vector ALU free, which the fp32 ones do not.
  *
- * A value that is not finite, or is above 5.1e33 and rounds to infinity in bf16 once scaled, leaves NaN in the lower
+ * A value that is not finite, or rounds to infinity in bf16 (above 3.39e38 with its factor), leaves NaN in the lower
  * parts and so in every result it takes part in; a result above 7.9e28 overflows before it is scaled back.  The
  * caller looks for results that are not finite and computes those on the fp32 instructions.
  */
@@ -30,13 +36,13 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr float SPLIT_UP = 0x1p16f, SPLIT_DOWN = 0x1p-32f;
+constexpr float SPLIT_UP = 0x1p16f, SPLIT_FAR = 0x1p32f, SPLIT_DOWN = 0x1p-32f;
 
-/* N values, SPLIT_UP times what they stand for -> their three parts.  (v_dot2_f32_bf16 would take a part off in one instruction instead of a shift or mask and
+/* N values -> their three parts.  (v_dot2_f32_bf16 would take a part off in one instruction instead of a shift or mask and
  * a subtraction, but it runs in the matrix unit's place: twelve matrix instructions with eight of each in
  * between take 228 ns with conversions, 211 with shifts, 394 with it.) */
 template <int N, typename Vec>
-__device__ __forceinline__ void split_bf16_scaled(const float (&x)[N], Vec &high, Vec &mid, Vec &low) {
+__device__ __forceinline__ void split_bf16(const float (&x)[N], Vec &high, Vec &mid, Vec &low) {
     uint32_t *const out[3] = {reinterpret_cast<uint32_t *>(&high), reinterpret_cast<uint32_t *>(&mid), reinterpret_cast<uint32_t *>(&low)};
 #pragma unroll
     for (int i = 0; i < N; i += 2) {
@@ -51,25 +57,16 @@ __device__ __forceinline__ void split_bf16_scaled(const float (&x)[N], Vec &high
     }
 }
 
-/* ... of plain values */
-template <int N, typename Vec>
-__device__ __forceinline__ void split_bf16(const float (&x)[N], Vec &high, Vec &mid, Vec &low) {
-    float y[N];
-#pragma unroll
-    for (int i = 0; i < N; i++) y[i] = x[i] * SPLIT_UP;
-    split_bf16_scaled<N>(y, high, mid, low);
-}
-
-/* ... of N consecutive ones of a register array */
+/* ... of N consecutive ones of a register array, times `factor` */
 template <int N, int M>
-__device__ __forceinline__ void split_bf16_at(const float (&x)[M], int first, bf16x8 (&parts)[3]) {
+__device__ __forceinline__ void split_bf16_at(const float (&x)[M], int first, bf16x8 (&parts)[3], float factor = 1.0f) {
     float y[N];
 #pragma unroll
-    for (int i = 0; i < N; i++) y[i] = x[first + i];
+    for (int i = 0; i < N; i++) y[i] = x[first + i] * factor;
     split_bf16<N>(y, parts[0], parts[1], parts[2]);
 }
 
-/* acc += SPLIT_UP^2 A B over 16 of K, smallest partial products first */
+/* acc += A B over 16 of K, smallest partial products first */
 template <typename Acc>
 __device__ __forceinline__ Acc mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b)[3], Acc acc) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], acc, 0, 0, 0);

@@ -1044,7 +1044,7 @@ def test_matmul_of_few_products(m, k, n, dev):
 
 
 @pytest.mark.parametrize("scale_q,scale_k,scale_v", [(1.0, 1.0, 1.0), (1.0, 1.0, 1e-36), (1e-33, 1e33, 1.0), (1e-36, 1e36, 1.0),
-                                                     (1e36, 1e-36, 1.0), (1.0, 1.0, 1e33), (0.0, 0.0, 1.0)])
+                                                     (1e36, 1e-36, 1.0), (1e28, 1e-28, 1.0), (1e-40, 1e37, 1e25), (1.0, 1.0, 1e33), (0.0, 0.0, 1.0)])
 @pytest.mark.parametrize("T,H,hd,batch", [(300, 1, 1, 1), (300, 1, 2, 1), (300, 1, 48, 1), (300, 1, 128, 1), (256, 4, 32, 80), (256, 4, 64, 80), (2304, 4, 32, 16)])
 def test_attention_over_the_range_of_fp32(T, H, hd, batch, scale_q, scale_k, scale_v, dev):
     """Attention on bf16 parts (the latency kernel, the throughput kernel with four and eight waves) with tiny and huge
