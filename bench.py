@@ -27,6 +27,9 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix, published
+# fp32 products taken as six bf16 ones (split_bf16.h) on the dense bf16 rate, published 2500
+SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 6.0
+SPLIT_KERNELS = {"wide", "mfma", "attn_wide", "attn_mfma", "matmul_mfma"}
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.md")
 DETAIL_FILE = os.path.join(ROOT, "gpurun_out", "bench_detail.json")
@@ -61,12 +64,13 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def roofline(bound, work, avg_s, traffic=None):
-    """work = algorithmic bytes (hbm) or flops (mfma) per launch."""
+def roofline(bound, work, avg_s, traffic=None, kernel=""):
+    """work = algorithmic bytes (hbm) or flops (mfma) per launch; kernel: the names of what ran, joined by +."""
     if bound == "hbm":
         achieved, peak, unit = work / avg_s / 1e9, HBM_PEAK_GBS, "GB/s"
     else:
-        achieved, peak, unit = work / avg_s / 1e12, FP32_MFMA_PEAK_TFLOPS, "TFLOP/s"
+        peak = SPLIT_MFMA_PEAK_TFLOPS if SPLIT_KERNELS & set(kernel.split("+")) else FP32_MFMA_PEAK_TFLOPS
+        achieved, unit = work / avg_s / 1e12, "TFLOP/s"
     return {"bound": bound, "achieved": achieved, "peak": peak, "unit": unit, "frac": achieved / peak,
             "traffic": traffic}
 
@@ -159,7 +163,7 @@ def bench_dense(make, steps, warmup, bound, mask_mode="descriptor", warm_ms=WARM
         "tokens_per_s_kernel": w.tokens / avg_s,
         "flops": w.flops, "bytes": w.bytes,
         "roofline_hbm": roofline("hbm", w.bytes, avg_s, MEASURED_TRAFFIC_BYTES.get(w.name)),
-        "roofline_mfma": roofline("mfma", w.flops, avg_s),
+        "roofline_mfma": roofline("mfma", w.flops, avg_s, kernel=kernel),
     }
     res["warmup_ms"] = warm_ms
     if caller:
@@ -397,7 +401,7 @@ def bench_block(name, T, E, H, steps, warmup, gemm_only=None, cross=None, warm_m
            "kernel_us_min": min(v[2] for v in prof.values()) * 1e3,
            "per_kernel_us": {k: v[1] * 1e3 / steps for k, v in prof.items()},
            "tokens_per_s": tokens * steps / wall_plain, "tokens_per_s_kernel": tokens / avg_s, "flops": flops,
-           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s)}
+           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s, kernel="+".join(sorted(prof)))}
     if warm_ms:
         res["warmup_ms"] = warm_ms
     res["roofline"] = res["roofline_mfma"]
@@ -570,7 +574,7 @@ def bench_decode_layer(steps, warmup, batch=64, H=4, hd=32, hidden=512, len_hi=5
            "kernel_us_min": min(v[2] for v in prof.values()) * 1e3,
            "per_kernel_us": {k: v[1] * 1e3 / steps for k, v in prof.items()},
            "tokens_per_s": batch * steps / wall_plain, "tokens_per_s_kernel": batch / avg_s, "flops": flops,
-           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s)}
+           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s, kernel="+".join(sorted(prof)))}
     res["roofline"] = res["roofline_hbm"]
     return res
 
@@ -706,7 +710,7 @@ def bench_decode_step(steps, warmup, batch=64, L=2, E=128, H=4, hidden=512, V=25
            "kernel_us_min": min(v[2] for v in prof.values()) * 1e3,
            "per_kernel_us": {k: v[1] * 1e3 / steps for k, v in prof.items()},
            "tokens_per_s": rows * steps / wall_plain, "tokens_per_s_kernel": rows / avg_s, "flops": flops,
-           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s)}
+           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s, kernel="+".join(sorted(prof)))}
     res["roofline"] = res["roofline_hbm"]
     return res
 
@@ -778,7 +782,7 @@ def bench_encoder(steps, warmup, cpu_budget_s):
            "launches_per_step": mine["launches_per_pass"], "tokens_per_step": T, "us_per_step": mine["wall_us_per_pass"],
            "kernel_us_avg": mine["kernel_us_per_pass"], "kernel_us_min": min(mine["per_kernel_us"].values()),
            "per_kernel_us": mine["per_kernel_us"], "tokens_per_s": T / (mine["wall_us_per_pass"] * 1e-6), "flops": flops,
-           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s)}
+           "bytes": nbytes, "roofline_hbm": roofline("hbm", nbytes, avg_s), "roofline_mfma": roofline("mfma", flops, avg_s, kernel="+".join(sorted(mine["per_kernel_us"])))}
     res["roofline"] = res["roofline_mfma"]
     if cpu_budget_s > 0:
         from oracle import binding
@@ -857,7 +861,7 @@ def bench_decoder_forward(steps, warmup, cpu_budget_s, T=512, L=2, E=128, H=4, h
            "launches_per_step": sum(v[0] for v in prof.values()) / steps, "tokens_per_step": T, "us_per_step": wall * 1e6,
            "kernel_us_avg": kernel_us, "kernel_us_min": min(per_kernel.values()), "per_kernel_us": per_kernel,
            "tokens_per_s": T / wall, "flops": flops, "bytes": nbytes,
-           "roofline_hbm": roofline("hbm", nbytes, kernel_us * 1e-6), "roofline_mfma": roofline("mfma", flops, kernel_us * 1e-6)}
+           "roofline_hbm": roofline("hbm", nbytes, kernel_us * 1e-6), "roofline_mfma": roofline("mfma", flops, kernel_us * 1e-6, kernel="+".join(sorted(per_kernel)))}
     res["roofline"] = res["roofline_mfma"]
     if cpu_budget_s > 0:
         from oracle import binding

@@ -34,8 +34,8 @@
  * Bound: the vector ALU for long rows (a 32x32 tile of heads of 64: 1536 cycles of matrix instructions beside
  * about 650 vector instructions, most of them splitting K, V and the weights, which the waves do not
  * share; on the fp32 matrix instructions it was 4096 cycles with nothing beside them), launch/latency for
- * the small shapes.  Causal self-attention, fp32 instructions -> parts: 8 heads of 64 over 4096 rows 202 -> 139 us,
- * over 1024 rows 26.3 -> 22.9; 8 heads of 32 over 4096 rows 108 -> 82.
+ * the small shapes.  Causal self-attention, fp32 instructions -> parts: 8 heads of 64 over 4096 rows 200 -> 146 us,
+ * over 1024 rows 26.6 -> 24.0; 8 heads of 32 over 4096 rows 107 -> 86.
  */
 #include "attn_device.h"
 #include "attn_launch.h"

@@ -37,12 +37,12 @@
  * output, any visibility except per-row ranges.
  *
  * Bound: vector ALU and matrix unit together.  A 32x32 tile of heads of 32 is 768 cycles of bf16 matrix
- * instructions and about 210 vector instructions (5.5 per value to take apart weights, K and V, three per
- * weight for the softmax); vector instructions of other waves, and of the same wave where the two are mixed, run
- * beside the matrix instructions but not for free (twelve matrix instructions 175 ns, with 192 fused multiply-adds in
- * between 391, those alone 326).  On fp32 matrix instructions the same tile took 2048 cycles
- * that nothing ran beside.  Causal self-attention, 32 problems of 4096 rows: 322 -> 200 us for heads of 32
- * (107 -> 172 TFLOP/s); 48 problems of 2048 rows, heads of 64: 301 -> 178.
+ * instructions and about 215 vector instructions (5.5 per value to take apart weights, K and V, three per
+ * weight for the softmax); within a wave the two run side by side where they are mixed (twelve matrix instructions 179 ns,
+ * 192 fused multiply-adds 386, both 384), less so with a second wave on the SIMD (330, 399, 637).  On fp32 matrix
+ * instructions the same tile took 2048 cycles that nothing ran beside.  Causal self-attention, 32 problems of 4096
+ * rows: 323 -> 209 us for heads of 32 (106 -> 164 TFLOP/s; matrix unit busy 0.44 of the time, vector issue 0.60);
+ * 48 problems of 2048 rows, heads of 64: 299 -> 180.
  */
 #include "attn_device.h"
 #include "attn_launch.h"

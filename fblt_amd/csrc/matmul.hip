@@ -12,7 +12,7 @@
  *    sum -- k ascending, product and sum rounded separately -- so this path
  *    is bit-identical to blt_matmul_cpu.
  *
- *  - "mfma" (everything else): 64x64 or 128x128 output tiles per workgroup of eight
+ *  - "mfma" (everything else; from three terms a sum on): 64x64 or 128x128 output tiles per workgroup of eight
  *    wavefronts, K in steps of 32 through double-buffered LDS tiles, on the bf16
  *    matrix instructions with both operands taken apart into three exact parts on the
  *    way to LDS (split_bf16.h).  The product is accumulated
@@ -24,13 +24,13 @@
  *    (csrc/models/attention.c:76-90) -- without a second pass over the
  *    result.  Summation order differs from the reference's (fp32 tolerance).
  *    Bound: matrix and vector instructions share the time about evenly for the 64x64 tile
- *    (384 and 470 cycles of a step), the matrix ones for the 128x128 tile, at the clock that
- *    load leaves.  On fp32 instructions -> on parts: 2048 x 512 . 512 x 2048 46.5 -> 31.2 us,
- *    2048 x 2048 . 2048 x 512 49 -> 41, 8192 x 512 . 512 x 512 43.9 -> 29.5,
- *    4096 x 1024 . 1024 x 4096 273 -> 195 (176 TFLOP/s).
+ *    (384 and about 500 cycles of a step), the matrix ones and the barrier of every step for the 128x128 tile
+ *    (8192 x 512 . 512 x 1536: matrix unit busy 0.40 of the time, vector issue 0.34).  On fp32 instructions -> on
+ *    parts: 2048 x 512 . 512 x 2048 41.0 -> 30.4 us, 2048 x 2048 . 2048 x 512 45.3 -> 37.0, 8192 x 512 . 512 x 512
+ *    42.8 -> 30.2, 4096 x 1024 . 1024 x 4096 274 -> 197 (174 TFLOP/s).
  *
  *  - "splitk" (outputs too small to give every compute unit a 64x64 tile,
- *    e.g. 512x128 * 128x384): one 32x32 output tile per workgroup, its four
+ *    e.g. 512x128 * 128x384; sums of one or two terms; more than 2^25 columns): one 32x32 output tile per workgroup, its four
  *    wavefronts take the 32-wide K chunks round-robin straight from global
  *    memory (no LDS staging, no barrier in the loop) and add their partial
  *    tiles through LDS at the end.  Same accumulator layout and epilogue as

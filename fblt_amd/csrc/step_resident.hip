@@ -46,9 +46,11 @@
  *
  * Measured, launches -> this kernel: one row, two layers of 128 columns, 300 keys 69 -> 38 us; 64 such rows 78 ->
  * 61 us; 16 draft rows of one sequence 80 -> 61 us.  The roll call is a quarter of a microsecond of that where the first
- * loads of a workgroup are on their way meanwhile, and 1.5 us in front of everything.  What is left is the chain: a hand-over takes about 1 us from
- * the store to the reader's first use, and a wave that shares its SIMD with three others issues an instruction
- * every nine cycles, so the 100 ... 200 instructions of a stage between its operand and its result are another.
+ * loads of a workgroup are on their way meanwhile, and 1.5 us in front of everything.  What is left is the chain: a
+ * hand-over takes about 1 us from the store to the reader's first use, and a wave that shares its SIMD with three
+ * others issues an instruction every nine cycles, so the 100 ... 200 instructions of a stage between its operand and
+ * its result are another.  Two workgroups of eight waves on a compute unit leave a wave 128 registers, which do not hold
+ * either role: about 40 are spilled at heads of 32, about 150 at heads of 64, and a reload waits for every load before it.
  */
 #include "blt_hip.h"
 #include "blt_fatal.h"
@@ -1027,8 +1029,9 @@ bool kv_step_resident(const StepResident &st) {
      * layers).  Up to 16 rows a group and heads of 32: everywhere (E = 64: 113 -> 50 at one row, 133 -> 82 at 96;
      * E = 256: 155 -> 93, 254 -> 231 at 64 rows of 900 keys).  17 to 32 rows: narrow models only (E = 64: 140 ->
      * 126), the products of wide ones have all compute units in the launches (E = 256: 25 rows 227 -> 247, eight
-     * groups of 32 rows 229 -> 282).  Heads of 64 have half the keys per wave in flight: single rows of few
-     * sequences a group (E = 256, 20 sequences: 187 -> 162; 64 of 900 keys: 251 -> 343). */
+     * groups of 32 rows 229 -> 282).  Heads of 64 have half the keys per wave in flight and spill four
+     * times as many registers: single rows of few sequences a group (E = 256, 20 sequences: 187 -> 162; 64 of 900 keys: 251
+     * -> 343). */
     if (group_rows > 16 && E > 64) return false;
     if (hd == 64 && (st.n > 1 || per_group > 4)) return false;
     if (st.row_index != nullptr && st.batch != 1) return false;
