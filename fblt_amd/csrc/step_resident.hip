@@ -983,27 +983,26 @@ TestPin test_pin() {
 /* Do `blocks` workgroups of the kernel fit the compute units this stream may use, all at once?  The launch would be right
  * otherwise too (see the roll call), but the launches would be faster. */
 bool can_be_resident(ResidentKernel kernel, uint32_t blocks, int dev, hipStream_t s) {
-    struct Known {
-        ResidentKernel kernel;
-        int dev;
-        uint32_t per_unit, units;
+    struct Fit {
+        uint32_t per_unit = 0, units = 0;
     };
-    static thread_local Known known{nullptr, 0, 0u, 0u};
-    if (known.kernel != kernel || known.dev != dev) {
+    static thread_local std::map<std::pair<ResidentKernel, int>, Fit> fits;
+    Fit &fit = fits[{kernel, dev}];
+    if (fit.units == 0u) {
         int per_unit = 0, units = 0;
         HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_unit, reinterpret_cast<const void *>(kernel), 64 * WAVES, 0));
         HIP_CHECK(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev));
-        known = Known{kernel, dev, (uint32_t)per_unit, (uint32_t)units};
+        fit.per_unit = (uint32_t)per_unit, fit.units = (uint32_t)units;
     }
     uint32_t mask[32], open = 0;
-    const uint32_t mask_words = (known.units + 31u) / 32u;
+    const uint32_t mask_words = (fit.units + 31u) / 32u;
     if (mask_words > 32u) return false;
     if (hipExtStreamGetCUMask(s, mask_words, mask) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
     for (uint32_t i = 0; i < mask_words; i++) open += (uint32_t)__builtin_popcount(mask[i]);
-    return (uint64_t)known.per_unit * std::min(open, known.units) >= blocks;
+    return (uint64_t)fit.per_unit * std::min(open, fit.units) >= blocks;
 }
 
 } // namespace

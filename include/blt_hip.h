@@ -123,9 +123,11 @@ void blt_cross_attention_forward_hip(const blt_tensor *query_in, const blt_tenso
  * copies and per-head calls of the reference are gone, the row groups follow
  * the same latent rule (kv_cache.c:199-213).  A prompt chunk of more than 32
  * rows is staged once (rotation, write-through) and attended by the prefill
- * kernels with the causal diagonal moved by the cached length.  Up to 32 new
- * rows every projection is bit-identical to the CPU reference; attention is
- * within fp32 tolerance. */
+ * kernels with the causal diagonal moved by the cached length.  Steps of few
+ * rows of a decoder of 64, 128 or 256 columns, and draft passes of one, are one
+ * launch.  Results are within fp32 tolerance of the CPU step
+ * (BLT_HIP_EXACT_STEP=1 in the environment: projections of up to 32 new rows
+ * bit-identical). */
 void blt_kv_cache_refresh_cross_hip(blt_kv_cache *cache, const blt_tensor *patch_in, const blt_patch_info *patches,
                                     size_t num_patches, size_t from_patch, blt_arena *arena);
 void blt_kv_decode_step_hip(blt_kv_cache *cache, const blt_tensor *patch_in, const blt_patch_info *patches,
