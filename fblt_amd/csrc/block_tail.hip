@@ -1,0 +1,264 @@
+/*
+ * Everything of a transformer block behind its attention in ONE launch (csrc/models/transformer.c:112-128,
+ * csrc/infer/kv_cache.c:384-414):
+ *
+ *   resid = x + comb * proj
+ *   act   = silu(RMSNorm(resid) * gate) .* (RMSNorm(resid) * up)
+ *   out   = resid + act * down
+ *
+ * As launches these are three products of 4 to 7 us each whatever their size, because each waits for the one before
+ * and for a trip of its own to memory.  All three are row-local, so here a workgroup takes 16 rows from the
+ * attention's output to the block's, and the hidden layer is dealt to several workgroups (grid x): each computes
+ * all of resid -- again, 2 * 16 * E * E operations that would otherwise be a launch --, its own HS hidden columns,
+ * and its share of the last product's sum.  The shares go to a per-stream buffer, the workgroup that draws the last
+ * ticket of its row tile adds them in the order of the slices.  Nobody waits for another workgroup.
+ *
+ * Weights are on their way to registers from the first instruction on, the ones used first first: each is used by one
+ * wave only, so LDS would add a trip and save nothing.  fp32 matrix instructions: under 16 rows, taking a weight apart into
+ * bf16 parts costs more than the matrix time it saves.
+ *
+ * Bound: latency.  E = 128, hidden 512, 512 rows: 10.9 us in the kernel trace, of which (parts left out, one after the other)
+ * an empty launch with all requests 3, the barriers and the partial sums through LDS 2.5 (0 would need a whole row's
+ * product in one wave), fp32 matrix time of the compute unit 2.2, the ticket 1.9.  Whole blocks, three launches -> this: 128 rows
+ * 25.0 -> 17.3 us, 512 rows 29.5 -> 21.6; E = 64 22.7 -> 13.9 and 26.1 -> 17.2; E = 256, 128 rows 31.5 -> 28.4.
+ * Relative error of the block against float64: 1.57e-7 -> 1.45e-7 (E = 128, 128 rows), 1.64e-7 -> 1.47e-7 (256 of 256).
+ */
+#include "blt_hip.h"
+#include "blt_fatal.h"
+#include "hip_check.h"
+#include "lane_ops.h"
+#include "launch.h"
+#include "matmul.h"
+
+#include <cstring>
+
+namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+/* Columns go in groups of 64, a wave per (group, share of the terms): lane (g, c) loads four consecutive columns
+ * 4 c .. 4 c + 3 of row 4 g + t of every block of 16 terms, 16 bytes, and column j of the four is the tile of every fourth
+ * column from j on.  A load instruction costs a compute unit's vector memory path about the same whatever it
+ * brings: with a tile of 16 consecutive columns a wave and 4 bytes a lane the 690 loads of a workgroup were what the launch
+ * waited for. */
+template <int E_, int NW_, bool PROJ_>
+struct TailShape {
+    static constexpr int E = E_, HS = 64, NW = NW_, THREADS = 64 * NW;
+    static constexpr bool PROJ = PROJ_;
+    static constexpr int ROW = E + 4, ACT = HS + 4; /* LDS rows, four banks apart */
+    template <int COLS, int TERMS>
+    struct Product {
+        static constexpr int GROUPS = COLS / 64, SHARES = NW / GROUPS, BLOCKS = TERMS / 16 / SHARES, PITCH = COLS + 4;
+        static constexpr int PART = SHARES * 16 * PITCH; /* floats of the partial tiles */
+        static_assert(GROUPS * SHARES == NW && BLOCKS * SHARES * 16 == TERMS, "waves over groups and shares");
+    };
+    using Proj = Product<E, E>;
+    using Gated = Product<2 * HS, E>; /* the up columns, then the gate columns */
+    using Down = Product<E, HS>;
+    static constexpr int EPT = 16 * E / THREADS; /* of the 16 rows of E, and of HS, a thread finishes */
+    static constexpr int APT = 16 * HS / THREADS;
+    static constexpr int AREA = Proj::PART > Gated::PART ? Proj::PART : Gated::PART;
+};
+
+/* the weights of a wave's product: from `w`, row-major with `ld` columns, rows from term0 on */
+template <int BLOCKS>
+__device__ __forceinline__ void request(floatx4 (&v)[4 * BLOCKS], const float *w, size_t ld, uint32_t term0) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const float *p = w + (size_t)(term0 + 4u * (lane >> 4)) * ld + 4u * (lane & 15u);
+#pragma unroll
+    for (int i = 0; i < 4 * BLOCKS; i++) v[i] = *reinterpret_cast<const floatx4 *>(p + (size_t)(16 * (i / 4) + i % 4) * ld);
+}
+/* the wave's sums over its share of the terms, to rows of PITCH of its part */
+template <int BLOCKS, int PITCH>
+__device__ __forceinline__ void multiply(const float *rows, uint32_t row_pitch, uint32_t term0, const floatx4 (&v)[4 * BLOCKS], float *part) {
+    const uint32_t lane = threadIdx.x & 63u, g = lane >> 4, c = lane & 15u;
+    const float *mine = rows + c * row_pitch + term0 + 4u * g;
+    floatx4 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < BLOCKS; b++) {
+        const floatx4 a = *reinterpret_cast<const floatx4 *>(mine + 16 * b);
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], v[4 * b + t][j], acc[j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        *reinterpret_cast<floatx4 *>(part + (4u * g + r) * PITCH + 4u * c) = floatx4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+}
+/* N consecutive values, the shares' sums added */
+template <int SHARES, int PITCH, int N>
+__device__ __forceinline__ void gather(const float *part, float (&out)[N]) {
+    typedef float values __attribute__((ext_vector_type(N)));
+    values v = *reinterpret_cast<const values *>(part);
+#pragma unroll
+    for (int s = 1; s < SHARES; s++) v += *reinterpret_cast<const values *>(part + s * 16 * PITCH);
+#pragma unroll
+    for (int i = 0; i < N; i++) out[i] = v[i];
+}
+
+template <typename Shape>
+__global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArgs a) {
+    using Proj = typename Shape::Proj;
+    using Gated = typename Shape::Gated;
+    using Down = typename Shape::Down;
+    constexpr int E = Shape::E, HS = Shape::HS, ROW = Shape::ROW, ACT = Shape::ACT, EPT = Shape::EPT, APT = Shape::APT;
+    typedef float rowpart __attribute__((ext_vector_type(EPT)));
+    __shared__ __attribute__((aligned(16))) float rows[16 * ROW], part[Shape::AREA], act[16 * ACT];
+    __shared__ uint32_t ticket;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t slices = gridDim.x, slice = blockIdx.x, row0 = 16u * blockIdx.y;
+    /* what this thread finishes of the 16 rows */
+    constexpr uint32_t TPR = E / EPT; /* threads of a row: neighbours in one wave */
+    static_assert(TPR <= 64, "a row's threads are in one wave");
+    const uint32_t f_row = tid / TPR, f_col = EPT * (tid % TPR);
+    const size_t f_at = (size_t)min(row0 + f_row, a.rows - 1u) * E + f_col;
+
+    floatx4 wp[Shape::PROJ ? 4 * Proj::BLOCKS : 1], wg[4 * Gated::BLOCKS], wd[4 * Down::BLOCKS];
+    const uint32_t p_group = wave % Proj::GROUPS, p_term = wave / Proj::GROUPS * (16 * Proj::BLOCKS);
+    const uint32_t g_group = wave % Gated::GROUPS, g_term = wave / Gated::GROUPS * (16 * Gated::BLOCKS);
+    const uint32_t d_group = wave % Down::GROUPS, d_term = wave / Down::GROUPS * (16 * Down::BLOCKS);
+    rowpart in;
+    if constexpr (Shape::PROJ) in = *reinterpret_cast<const rowpart *>(a.comb + f_at);
+    const rowpart x = *reinterpret_cast<const rowpart *>(a.x + f_at);
+    const rowpart norm_w = *reinterpret_cast<const rowpart *>(a.norm_w + f_col);
+    if constexpr (Shape::PROJ) request<Proj::BLOCKS>(wp, a.proj + 64u * p_group, E, p_term);
+    __builtin_amdgcn_sched_barrier(0); /* requests in the order in which they are used, all before the first wait */
+    const bool is_gate = g_group >= (uint32_t)Gated::GROUPS / 2u;
+    request<Gated::BLOCKS>(wg, (is_gate ? a.gate : a.up) + slice * HS + 64u * (g_group % (Gated::GROUPS / 2)), a.hidden, g_term);
+    request<Down::BLOCKS>(wd, a.down + (size_t)slice * HS * E + 64u * d_group, E, d_term);
+    __builtin_amdgcn_sched_barrier(0);
+
+    float resid[EPT];
+    if constexpr (Shape::PROJ) {
+        *reinterpret_cast<rowpart *>(rows + f_row * ROW + f_col) = in;
+        __syncthreads();
+        multiply<Proj::BLOCKS, Proj::PITCH>(rows, ROW, p_term, wp, part + wave / Proj::GROUPS * (16 * Proj::PITCH) + 64u * p_group);
+        __syncthreads();
+        gather<Proj::SHARES, Proj::PITCH, EPT>(part + f_row * Proj::PITCH + f_col, resid);
+#pragma unroll
+        for (int i = 0; i < EPT; i++) resid[i] = x[i] + resid[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < EPT; i++) resid[i] = x[i];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < EPT; i++) ss += resid[i] * resid[i];
+    ss = key_sum<TPR < 32 ? TPR : 32>(ss);
+    if (TPR == 64) ss = swap32(ss, OpSum());
+    const float scale = 1.0f / sqrtf(ss / (float)E + 1e-6f); /* reductions_cpu.c:345-346 */
+    rowpart n;
+#pragma unroll
+    for (int i = 0; i < EPT; i++) n[i] = resid[i] * scale * norm_w[i];
+    *reinterpret_cast<rowpart *>(rows + f_row * ROW + f_col) = n;
+    __syncthreads();
+    multiply<Gated::BLOCKS, Gated::PITCH>(rows, ROW, g_term, wg, part + wave / Gated::GROUPS * (16 * Gated::PITCH) + 64u * g_group);
+    __syncthreads();
+    {
+        typedef float values __attribute__((ext_vector_type(APT)));
+        const uint32_t h_row = tid / (HS / APT), h_col = APT * (tid % (HS / APT));
+        float up[APT], gate[APT];
+        gather<Gated::SHARES, Gated::PITCH, APT>(part + h_row * Gated::PITCH + h_col, up);
+        gather<Gated::SHARES, Gated::PITCH, APT>(part + h_row * Gated::PITCH + HS + h_col, gate);
+        values v;
+#pragma unroll
+        for (int i = 0; i < APT; i++) v[i] = silu_times(gate[i], up[i]);
+        *reinterpret_cast<values *>(act + h_row * ACT + h_col) = v;
+    }
+    __syncthreads();
+    multiply<Down::BLOCKS, Down::PITCH>(act, ACT, d_term, wd, part + wave / Down::GROUPS * (16 * Down::PITCH) + 64u * d_group);
+    __syncthreads();
+    float sum[EPT];
+    gather<Down::SHARES, Down::PITCH, EPT>(part + f_row * Down::PITCH + f_col, sum);
+
+    if (slices > 1u) {
+        /* device-scope stores and loads, and an explicit wait for the stores' completion before the barrier that
+         * precedes the workgroup's ticket */
+        constexpr uint32_t WORDS = 16 * E / 2; /* a slice's sums, two a word */
+        uint64_t *mine = a.sums + (size_t)blockIdx.y * slices * WORDS + tid;
+#pragma unroll
+        for (int i = 0; i < EPT / 2; i++)
+            __hip_atomic_store(mine + (size_t)slice * WORDS + i * Shape::THREADS,
+                               (uint64_t)__float_as_uint(sum[2 * i + 1]) << 32 | __float_as_uint(sum[2 * i]), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        blt_vector_memory_done();
+        __syncthreads();
+        if (tid == 0u)
+            ticket = __hip_atomic_fetch_add(&a.tickets[blockIdx.y], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (ticket != slices - 1u) return;
+        if (tid == 0u) a.tickets[blockIdx.y] = 0u; /* re-armed for the next launch */
+#pragma unroll
+        for (int i = 0; i < EPT; i++) sum[i] = 0.f;
+        for (uint32_t z = 0; z < slices; z += 8u) { /* slice order, whoever comes last */
+            uint64_t t[8][EPT / 2];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; u++)
+#pragma unroll
+                for (int i = 0; i < EPT / 2; i++)
+                    t[u][i] = __hip_atomic_load(mine + (size_t)min(z + u, slices - 1u) * WORDS + i * Shape::THREADS, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; u++)
+#pragma unroll
+                for (int i = 0; i < EPT; i++)
+                    sum[i] += z + u < slices ? __uint_as_float((uint32_t)(t[u][i / 2] >> (32 * (i % 2)))) : 0.f;
+        }
+    }
+    rowpart out;
+#pragma unroll
+    for (int i = 0; i < EPT; i++) out[i] = resid[i] + sum[i];
+    if (row0 + f_row < a.rows) *reinterpret_cast<rowpart *>(a.out + f_at) = out;
+}
+
+template <typename Shape>
+void launch_tail(const BlockTailArgs &a, dim3 grid, hipStream_t s) {
+    blt_launch("block_tail", block_tail_kernel<Shape>, grid, dim3(Shape::THREADS), 0, s, a);
+}
+
+} // namespace
+
+bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s) {
+    if (a.rows == 0u || a.hidden == 0u || (embed_dim != 64u && embed_dim != 128u && embed_dim != 256u) || a.hidden % 64u != 0u)
+        return false;
+    for (const void *p : {(const void *)a.comb, (const void *)a.x, (const void *)a.proj, (const void *)a.norm_w, (const void *)a.up,
+                          (const void *)a.gate, (const void *)a.down, (const void *)a.out, (const void *)a.resid})
+        if ((reinterpret_cast<uintptr_t>(p) & 15u) != 0u) return false;
+    /* A workgroup's time hardly depends on its load, so the launch takes as many times that as the chip needs rounds, and the
+     * products as launches fill it better.  Whole blocks (projection to output, attention included), launches / this:
+     *   E = 64 (four workgroups of four waves a compute unit): 256 x 4 = 1024 workgroups 68.7 / 61.6 us
+     *   E = 128 (two of eight waves): 512 workgroups 35.2 / 30.1 (1024 rows) and 31.4 / 28.4 (hidden layer of 1024), 768
+     *   workgroups 49.2 / 49.2, 1024 53.8 / 57.3
+     *   E = 256 (one of sixteen waves, the projection a launch of its own): 256 workgroups 34.2 / 33.2; 512 as 256 of twice
+     *   the hidden columns 41.3 / 41.3 */
+    const uint64_t workgroups = (uint64_t)((a.rows + 15u) / 16u) * (a.hidden / 64u);
+    if (workgroups > (embed_dim == 64u ? 1024u : embed_dim == 128u ? 512u : 256u)) return false;
+    /* recorded by the caller's own capture, a replay may run beside later launches that use the same sums and tickets */
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const hipStream_t stream = s ? s : blt_stream();
+    if (!blt_stream_capturing() && stream != nullptr) HIP_CHECK(hipStreamIsCapturing(stream, &capture));
+    if (capture != hipStreamCaptureStatusNone) return false;
+    const uint32_t slices = a.hidden / 64u, tiles = (a.rows + 15u) / 16u;
+    if (slices > 1u && !matmul_slice_scratch((size_t)tiles * slices * 16u * embed_dim, tiles, s, (float **)&a.sums, &a.tickets))
+        return false;
+    const dim3 grid(slices, tiles);
+    if (embed_dim == 64u) {
+        launch_tail<TailShape<64, 4, true>>(a, grid, s);
+    } else if (embed_dim == 128u) {
+        launch_tail<TailShape<128, 8, true>>(a, grid, s);
+    } else { /* 1024 threads leave a wave 128 registers, and its share of proj is 64 of them */
+        MatmulArgs g;
+        std::memset(&g, 0, sizeof(g));
+        g.a = a.comb, g.b = a.proj, g.residual = a.x, g.out = a.resid;
+        g.m = a.rows, g.k = g.n = g.lda = g.ldb = g.ldo = embed_dim;
+        g.tolerant = 1u;
+        matmul_f32_launch(g, s);
+        a.x = a.resid;
+        launch_tail<TailShape<256, 16, false>>(a, grid, s);
+    }
+    return true;
+}

@@ -375,6 +375,17 @@ void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_wei
         blt_kv_rope_attend_step_hip(cache, qkv, 3 * E, qkv + E, 3 * E, qkv + 2 * E, 3 * E, rope_cos, rope_sin,
                                     rope_positions, combined, E, n, step_kind, commit, max_len_hint);
     }
+    if (rows > 32 || step_tolerant()) { /* up to 32 rows the products keep the reference's order of sums unless told otherwise */
+        BlockTailArgs t;
+        std::memset(&t, 0, sizeof(t));
+        t.comb = combined, t.x = rows_in, t.proj = f32(w->attn_proj_w), t.norm_w = f32(w->norm2_weight);
+        t.up = f32(w->ffn_up_w), t.gate = f32(w->ffn_gate_w), t.down = f32(w->ffn_down_w), t.out = rows_out, t.resid = resid1;
+        t.rows = (uint32_t)rows, t.hidden = (uint32_t)Hd;
+        if (rows <= 0xFFFFFFFFu && Hd <= 0xFFFFFFFFu && block_tail_launch(t, (uint32_t)E, 0)) {
+            HIP_CHECK_LAUNCH("blt_kv_decode_layer");
+            return;
+        }
+    }
     gemm(combined, f32(w->attn_proj_w), resid1, rows, E, E, rows_in); /* projection + residual in one pass */
     /* feed-forward block, kv_cache.c:396-414 */
     probe.n = (uint32_t)Hd;

@@ -60,6 +60,25 @@ struct MatmulArgs {
 };
 
 void matmul_f32_launch(const MatmulArgs &g, hipStream_t s);
+__device__ __forceinline__ float silu_times(float gate, float up) {
+    const float silu = gate / (1.0f + expf(-gate));
+    return silu * up;
+}
+/* Room for `floats` partial sums and `count` zeroed tickets of one launch on the stream, per (thread, stream): launches on one
+ * stream follow each other, launches on two never share them.  Every launch leaves its tickets at zero.  false: the
+ * buffers would have to grow while a graph capture is open. */
+bool matmul_slice_scratch(size_t floats, size_t count, hipStream_t s, float **sums, uint32_t **tickets);
+/* What of a transformer block is behind its attention, in one launch (block_tail.hip): out = r + SwiGLU(RMSNorm(r)) * down
+ * with r = x + comb * proj.  All row-major and dense; out may be x. */
+struct BlockTailArgs {
+    const float *comb, *x, *proj, *norm_w, *up, *gate, *down;
+    float *out, *resid; /* resid: room for r */
+    uint32_t rows, hidden;
+    uint64_t *sums; /* set by the launcher */
+    uint32_t *tickets;
+};
+/* false: not for this shape, nothing was launched */
+bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s);
 /* g0 (plain) and g1 (two weight matrices, two outputs) in one launch; only when matmul_pair_ok says so */
 bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1);
 void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStream_t s);

@@ -57,11 +57,6 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int TM = 64, TN = 64, TK = 32; /* smallest workgroup tile of the mfma kernel */
 
-__device__ __forceinline__ float silu_times(float gate, float up) {
-    const float silu = gate / (1.0f + expf(-gate));
-    return silu * up;
-}
-
 /* Four consecutive results of output row `row` starting at column `col`:
  * optional rotation, optional residual, store with bounds. */
 template <bool ROPE>
@@ -764,8 +759,6 @@ Path choose_path(const MatmulArgs &g) {
     return PATH_MFMA;
 }
 
-/* Sums and tickets of the K slices, per (thread, stream) like the scratch of the KV step: launches
- * on one stream follow each other, launches on two streams never share them. */
 struct SliceScratch {
     float *sums = nullptr;
     size_t sum_floats = 0;
@@ -776,28 +769,31 @@ __global__ void clear_words_kernel(uint32_t *w, size_t n) {
     const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
     if (i < n) w[i] = 0u;
 }
-/* false: the scratch would have to grow while a graph capture is open (the launch then runs unsliced) */
-bool slice_scratch(MatmulArgs &g, size_t tiles, hipStream_t s) {
+
+} // namespace
+
+bool matmul_slice_scratch(size_t floats, size_t count, hipStream_t s, float **sums, uint32_t **tickets) {
     static thread_local std::map<hipStream_t, SliceScratch> by_stream;
     SliceScratch &sc = by_stream[blt_stream_key()];
-    const size_t floats = tiles * g.slices * 1024u;
-    if (blt_stream_capturing() && (floats > sc.sum_floats || tiles > sc.ticket_count)) return false;
+    if (blt_stream_capturing() && (floats > sc.sum_floats || count > sc.ticket_count)) return false;
     /* outgrown buffers are left to the process: a launch still in flight may be using them */
     if (floats > sc.sum_floats) {
         sc.sum_floats = std::max(floats, 2 * sc.sum_floats);
         HIP_CHECK(hipMalloc((void **)&sc.sums, sc.sum_floats * sizeof(float)));
     }
-    if (tiles > sc.ticket_count) {
-        sc.ticket_count = std::max<size_t>(2 * tiles, 1024);
+    if (count > sc.ticket_count) {
+        sc.ticket_count = std::max<size_t>(2 * count, 1024);
         HIP_CHECK(hipMalloc((void **)&sc.tickets, sc.ticket_count * sizeof(uint32_t)));
         /* a fill kernel, not a memset, on the stream the launches follow */
         blt_launch("matmul_clear_words", clear_words_kernel, dim3((unsigned)((sc.ticket_count + 255) / 256)), dim3(256), 0,
                    s ? s : blt_stream(), sc.tickets, sc.ticket_count);
     }
-    g.slice_sums = sc.sums;
-    g.slice_tickets = sc.tickets;
+    *sums = sc.sums;
+    *tickets = sc.tickets;
     return true;
 }
+
+namespace {
 
 /* Slices of K per output tile: long K over few tiles leaves most of the chip idle and every wave
  * with a serial chain of chunk loads (2048 x 512 weights under 118 rows: 64 tiles, eight chunks per
@@ -819,7 +815,8 @@ void launch_splitk(const MatmulArgs &g_in, dim3 grid, hipStream_t s) {
     const bool eight = g_in.k >= 256u && (uint64_t)grid.x * grid.y <= 512u;
     MatmulArgs g = g_in;
     g.slices = slices_for(g, grid, eight);
-    if (g.slices > 1u && slice_scratch(g, (size_t)grid.x * grid.y, s)) grid.z = g.slices;
+    const size_t tiles = (size_t)grid.x * grid.y;
+    if (g.slices > 1u && matmul_slice_scratch(tiles * g.slices * 1024u, tiles, s, &g.slice_sums, &g.slice_tickets)) grid.z = g.slices;
     else g.slices = 1u;
     if (g.cross_k) {
         if constexpr (VEC && !ROPE)

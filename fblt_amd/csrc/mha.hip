@@ -39,9 +39,11 @@ namespace {
 /* The attention block; with norm_w the rows of `input` are RMS-normalised first (in the packed
  * projection's own pass where that kernel takes it, csrc/models/transformer.c:60-66), with
  * residual that [seq_len, embed_dim] array is added to the projected output (transformer.c:
- * 116-117) -- the two statements a transformer block wraps around its attention. */
-void mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_tensor *weight_proj, blt_tensor *output,
-             const blt_attention_config *config, blt_arena *arena, const float *norm_w, const float *residual) {
+ * 116-117) -- the two statements a transformer block wraps around its attention.  With tail the rest of
+ * the block follows in the launch of the projection where that takes the shape; true: it did. */
+bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_tensor *weight_proj, blt_tensor *output,
+             const blt_attention_config *config, blt_arena *arena, const float *norm_w, const float *residual,
+             const BlockTailArgs *tail = nullptr) {
     BLT_REQUIRE(config != NULL && arena != NULL, "blt_multihead_attention: config and arena cannot be NULL");
     BLT_REQUIRE(arena->backend == BLT_BACKEND_HIP, "blt_multihead_attention: HIP implementation needs a device arena");
     const size_t E = config->embed_dim, H = config->num_heads;
@@ -66,7 +68,7 @@ void mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
         BLT_REQUIRE(config->rope_theta > 0.0f,
                     "blt_multihead_attention: rope_theta must be positive when use_rope is true");
     }
-    if (T == 0) return;
+    if (T == 0) return false;
     BLT_REQUIRE(T <= 0x7FFFFFFFu && E <= 0x3FFFFFFFu, "blt_multihead_attention: dimensions exceed 2^31-1");
 
     float *qkv = (float *)blt_arena_alloc(arena, T * 3 * E * sizeof(float), 64);
@@ -226,6 +228,11 @@ void mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
     blt_attention_batch_hip(pr.data(), pr.size());
 
     /* 3. output projection (+ residual) */
+    if (tail != nullptr) {
+        BlockTailArgs t = *tail;
+        t.comb = combined, t.x = residual, t.proj = (const float *)weight_proj->data, t.rows = (uint32_t)T;
+        if (block_tail_launch(t, (uint32_t)E, 0)) return true;
+    }
     std::memset(&g, 0, sizeof(g));
     g.a = combined;
     g.b = (const float *)weight_proj->data;
@@ -235,6 +242,7 @@ void mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
     g.lda = g.ldb = g.ldo = (uint32_t)E;
     matmul_f32_launch(g, 0);
     HIP_CHECK_LAUNCH("blt_multihead_attention");
+    return false;
 }
 
 } // namespace
@@ -256,7 +264,9 @@ extern "C" void blt_multihead_attention_hip(const blt_tensor *input, const blt_t
  *   2. all heads in one attention launch (mask as a descriptor or as row ranges);
  *   3. attn_residual = input + combined * attn_proj_w;
  *   4. act = silu(RMSNorm(attn_residual) * ffn_gate_w) .* (RMSNorm(attn_residual) * ffn_up_w);
- *   5. output = attn_residual + act * ffn_down_w.
+ *   5. output = attn_residual + act * ffn_down_w
+ *
+ * -- or three, with 3 to 5 in one (block_tail.hip), for more than 32 rows of narrow blocks.
  *
  * RMSNorm + SwiGLU blocks with FP32 weights (what every BLT block is, csrc/models/
  * local_common.c:99-115); LayerNorm / GELU blocks and BF16 weight copies end with a message.
@@ -292,10 +302,20 @@ extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_t
 
     const size_t embed_shape[2] = {T, E}, hidden_shape[2] = {T, hidden};
     blt_tensor attn_residual = blt_tensor_create_uninit(arena, embed_shape, 2, BLT_DTYPE_FP32);
-    mha_run(input, w->attn_qkv_w, w->attn_proj_w, &attn_residual, &config->attn_config, arena,
-            (const float *)w->norm1_weight->data, (const float *)input->data);
-
+    BlockTailArgs tail;
+    std::memset(&tail, 0, sizeof(tail));
+    tail.norm_w = (const float *)w->norm2_weight->data;
+    tail.up = (const float *)w->ffn_up_w->data, tail.gate = (const float *)w->ffn_gate_w->data;
+    tail.down = (const float *)w->ffn_down_w->data, tail.out = (float *)output->data, tail.resid = (float *)attn_residual.data;
+    tail.hidden = (uint32_t)hidden;
+    /* up to 32 rows the products keep the reference's order of sums */
+    const bool done = mha_run(input, w->attn_qkv_w, w->attn_proj_w, &attn_residual, &config->attn_config, arena,
+                              (const float *)w->norm1_weight->data, (const float *)input->data, T > 32 ? &tail : nullptr);
     blt_tensor act = blt_tensor_create_uninit(arena, hidden_shape, 2, BLT_DTYPE_FP32);
+    if (done) {
+        HIP_CHECK_LAUNCH("blt_transformer_forward");
+        return;
+    }
     MatmulArgs g;
     std::memset(&g, 0, sizeof(g));
     g.a = (const float *)attn_residual.data;

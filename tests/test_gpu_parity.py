@@ -1679,6 +1679,74 @@ def test_transformer_block(shape, impl, oracle, dev):
         lib.blt_arena_destroy(arena)
 
 
+@pytest.mark.parametrize("T,E,H,hidden,shift,fused", [(33, 64, 2, 64, 0, True), (48, 64, 2, 320, 0, True), (49, 128, 4, 64, 0, True),
+                                                      (65, 128, 4, 576, 0, True), (1024, 128, 4, 512, 0, True),
+                                                      (1025, 128, 4, 512, 0, False), (34, 256, 8, 192, 0, True),
+                                                      (256, 256, 4, 1024, 0, True), (50, 128, 4, 96, 0, False),
+                                                      (50, 128, 4, 512, 1, False), (50, 96, 3, 384, 0, False)])
+def test_block_behind_its_attention(T, E, H, hidden, shift, fused, dev):
+    """The launch behind the attention of a narrow block, at the edges of its row tiles, hidden slices and of its dispatch
+    (shift: weights one float off a 16-byte boundary), in place and again: against float64, and the same bits each time."""
+    import torch
+    from tests.golden.block_cases import transformer_case
+    lib = api.load()
+    x, w, cfg, _keep = transformer_case(np.random.RandomState(T + E + hidden), T, E, H, hidden, "causal")
+    hd = E // H
+    pos = torch.arange(T, dtype=torch.float64)[:, None] * 500000.0 ** (-torch.arange(0, hd, 2, dtype=torch.float64) / hd)
+    cos, sin = pos.cos().float(), pos.sin().float()
+    d = {n: torch.from_numpy(t).double() for n, t in w.items()}
+    norm = lambda t, s: t / (t.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * s
+    xs = torch.from_numpy(x).double()
+    q, k, v = (norm(xs, d["norm1"]) @ d["qkv"]).view(T, 3, H, hd).permute(1, 2, 0, 3)
+
+    def turn(t):
+        a, b = t[..., 0::2], t[..., 1::2]
+        c, s = cos.double(), sin.double()
+        return torch.stack([a * c - b * s, b * c + a * s], -1).flatten(-2)
+    att = (turn(q) @ turn(k).transpose(1, 2) / hd ** 0.5).masked_fill(torch.ones(T, T).triu(1).bool(), float("-inf")).softmax(-1) @ v
+    resid = xs + att.transpose(0, 1).reshape(T, E) @ d["proj"]
+    n2 = norm(resid, d["norm2"])
+    want = resid + (torch.nn.functional.silu(n2 @ d["gate"]) * (n2 @ d["up"])) @ d["down"]
+
+    order = ("norm1", "qkv", "proj", "norm2", "up", "gate", "down")
+    tens = {}
+    for n in order:
+        room = torch.zeros(w[n].size + 4, device="cuda")
+        tens[n] = room[shift:shift + w[n].size].view(w[n].shape)
+        tens[n].copy_(torch.from_numpy(w[n]))
+    tv = {n: _dev_tensor(t) for n, t in tens.items()}
+    wt = abi.BltTransformerWeights()
+    wt.norm1_weight, wt.attn_qkv_w, wt.attn_proj_w = C.pointer(tv["norm1"]), C.pointer(tv["qkv"]), C.pointer(tv["proj"])
+    wt.norm2_weight, wt.ffn_up_w, wt.ffn_gate_w = C.pointer(tv["norm2"]), C.pointer(tv["up"]), C.pointer(tv["gate"])
+    wt.ffn_down_w = C.pointer(tv["down"])
+    tc = abi.BltTransformerConfig()
+    ac = tc.attn_config
+    ac.embed_dim, ac.num_heads, ac.head_dim, ac.is_causal, ac.use_rope, ac.rope_theta = E, H, hd, True, True, 500000.0
+    tcos, tsin = cos.cuda(), sin.cuda()
+    vc, vs = _dev_tensor(tcos), _dev_tensor(tsin)
+    ac.rope_cos_cache, ac.rope_sin_cache, ac.mask_config = C.pointer(vc), C.pointer(vs), C.pointer(cfg)
+    tc.hidden_dim, tc.norm_type, tc.activation_type = hidden, abi.BLT_NORM_RMSNORM, abi.BLT_ACTIVATION_SWIGLU
+    rows = [torch.from_numpy(x).cuda() for _ in range(3)]
+    outs = [torch.full((T, E), 7.0, device="cuda"), torch.full((T, E), 7.0, device="cuda"), rows[2]]   # the last one in place
+    arena = lib.blt_arena_create(64 << 20, abi.BLT_BACKEND_HIP)
+    try:
+        torch.cuda.synchronize()
+        lib.blt_hip_profile_begin()
+        for r, o in zip(rows, outs):
+            arena.contents.offset = 0
+            vx, vo = _dev_tensor(r), _dev_tensor(o)
+            lib.blt_transformer_forward(C.byref(vx), C.byref(wt), C.byref(vo), C.byref(tc), arena)
+        launched = api.profile_end()
+    finally:
+        lib.blt_arena_destroy(arena)
+    assert launched.get("block_tail", (0,))[0] == (3 if fused else 0), launched
+    got = [o.cpu().numpy() for o in outs]
+    # each of the four products rounds a sum of at most 1024 terms: 2^-24 sqrt(1024) of it in the 2-norm, were it one chain of
+    # independent roundings, and the four add up as independent errors
+    assert _relative(outs[0].cpu(), want) <= 2 * 2 ** -24 * 1024 ** 0.5
+    assert got[0].tobytes() == got[1].tobytes() == got[2].tobytes()
+
+
 @pytest.mark.parametrize("P,E,H,hidden,L,docs", [(128, 512, 8, 1024, 2, [40, 90]),   # C2's caller: one window of patches
                                                  (50, 64, 2, 96, 3, []), (200, 128, 4, 256, 1, [7, 8, 150])])
 def test_global_transformer_on_the_fused_block(P, E, H, hidden, L, docs, oracle, dev):
