@@ -2045,6 +2045,17 @@ def test_kv_decode_step_in_one_launch(batch, n, case, oracle, dev):
     assert in_one_launch(_decode_steps(batch, n, RESIDENT_CASES[case], 600 + case, oracle))
 
 
+@pytest.mark.parametrize("n,case", [(2, 1), (16, 1), (2, 3), (16, 3), (15, 5), (16, 5)])
+def test_kv_decode_step_of_one_sequence_with_wide_heads(n, case, oracle, dev):
+    """Several rows of one sequence at heads of 64 columns take the one-launch form, up to one row tile."""
+    assert in_one_launch(_decode_steps(1, n, RESIDENT_CASES[case], 640 + case, oracle))
+
+
+def test_kv_decode_step_of_wide_heads_past_one_row_tile(oracle, dev):
+    launched = _decode_steps(1, 17, RESIDENT_CASES[1], 641, oracle)
+    assert all("kv_step_resident" not in names for names in launched), launched
+
+
 @pytest.mark.parametrize("batch,n,case", [(1, 17, 2), (1, 32, 4), (9, 2, 3), (40, 1, 5), (9, 17, 0)])
 def test_kv_decode_step_past_one_launch(batch, n, case, oracle, dev):
     """One row more than the one-launch form takes: the launches, against the restated step."""
