@@ -48,7 +48,7 @@
  * in which it signs in, and who finds the time up before everybody has signs the others out.  If all are in, each has the
  * role its index gives it.  Else those that are in take all the work among them, stage by stage in the same order (any
  * number can: the first unfinished stage waits for nothing unfinished), and who finds itself signed out leaves.  The
- * fewer are in, the longer it is worth waiting: 20 us for the last one, 1.3 ms for the second.
+ * fewer are in, the longer it is worth waiting: 10 us for the last one, 0.3 ms for the second.
  *
  * Every wait is bounded all the same (SPIN_LIMIT polls, then the wave raises a word in pinned host memory, stops
  * waiting for the rest of the launch, takes NaN for what it did not get and runs to its end; the host turns the word
@@ -91,7 +91,9 @@ constexpr uint32_t MAX_GROUP_ROWS = 32;
 constexpr uint32_t MAX_ROWS = GROUPS * MAX_GROUP_ROWS;
 constexpr uint32_t MAX_SPLITS_R = 2; /* shares of a (sequence, head)'s keys */
 constexpr uint32_t SPIN_LIMIT = 1u << 22; /* polls, about half a microsecond each */
-constexpr uint32_t ROLL_LIMIT = 2000; /* ticks of 10 ns */
+/* Ticks of 10 ns for the last one.  Steps on one or two streams never come to it; four streams of 16 / 64 sequences, whose launches
+ * take each other's compute units: 77 / 81 us a step at 40 us, 58 / 62 at 20, 48 / 53 at 10, 46 / 52 at 5. */
+constexpr uint32_t ROLL_LIMIT = 1000;
 constexpr uint32_t MAX_HIDDEN = 1024;
 
 struct ResidentLayer {
