@@ -6,9 +6,9 @@
  * Work item = 128 (or 256) consecutive query rows of one (sequence, head) problem.
  * The wavefronts of the workgroup own one 32-row query tile each and
  * walk the key tiles (32 keys) TOGETHER: every K and V tile is brought from
- * global memory once per workgroup, taken apart into three bf16 parts
- * (split_bf16.h), parked in a double-buffered LDS area and read from there by all
- * waves as MFMA fragments.  Nothing is split along the keys, so there is no merge: a wave
+ * global memory once per workgroup, taken apart into two f16 parts
+ * (split_f16.h) or, out of their range, three bf16 parts (split_bf16.h), parked in a double-buffered LDS area and read
+ * from there by all waves as MFMA fragments.  Nothing is split along the keys, so there is no merge: a wave
  * keeps its own running (max, sum, output) from the first key tile to the
  * last and writes its 32 output rows itself.  Against the latency-oriented
  * kernel in attn_mfma.hip this removes the per-tile query load, the
@@ -18,9 +18,8 @@
  *   S^T[key, query] = K Q^T,  O^T[d, query] = V^T P^T
  * so a lane's softmax statistics, P^T operands and output accumulators all
  * belong to one query and the only cross-lane step per tile is one exchange
- * with lane L^32 for the maximum.  Scores live in log2 units (the query
- * fragment is pre-multiplied by scale*log2(e)); the accumulator is rescaled
- * only on tiles where some row's maximum actually moved.
+ * with lane L^32 for the maximum.  Weights are powers of two of scores in log2 units; the accumulator is rescaled
+ * only on tiles where some row's maximum moved (as f16: by more than 2).
  *
  * Causal problems: the workgroup walks the union of its four tiles' key
  * ranges; a wave skips the arithmetic (not the loads or barriers) of key
@@ -36,13 +35,20 @@
  * Shapes: head_dim 32 or 64 exactly, 16-byte aligned rows, no weights
  * output, any visibility except per-row ranges.
  *
- * Bound: vector ALU and matrix unit together.  A 32x32 tile of heads of 32 is 768 cycles of bf16 matrix
- * instructions and about 215 vector instructions (5.5 per value to take apart weights, K and V, three per
- * weight for the softmax); within a wave the two run side by side where they are mixed (twelve matrix instructions 179 ns,
- * 192 fused multiply-adds 386, both 384), less so with a second wave on the SIMD (330, 399, 637).  On fp32 matrix
- * instructions the same tile took 2048 cycles that nothing ran beside.  Causal self-attention, 32 problems of 4096
- * rows: 323 -> 209 us for heads of 32 (106 -> 164 TFLOP/s; matrix unit busy 0.44 of the time, vector issue 0.60);
- * 48 problems of 2048 rows, heads of 64: 299 -> 180.
+ * f16 or bf16: a group starts as f16 and looks at every run of K and V values that a thread takes apart; if one is out of
+ * range, the group is run again as bf16 (seen before the first score if all of K or V is so, as it mostly is: then the
+ * second run is all there is).
+ *
+ * Bound: vector ALU and matrix unit, whose times add up: on a SIMD a 32x32 tile of heads of 32 is 12 matrix instructions
+ * (384 cycles) and about 165 vector instructions (4.3 cycles each by the counters), 1090 cycles in all where it takes 1140.
+ * As bf16 it was 24 and 215, and the matrix unit drew so much power that the clock gave way: the same launch took 201 us on
+ * random values and 172 on constant ones (now 3 us apart).  Four waves a SIMD instead of two (two to a row tile, on even and
+ * odd key tiles) gained nothing with either: 206 against 206 us, 174 against 168.  Causal self-attention, 32 problems of
+ * 4096 rows, heads of 32: 197 us as bf16, 158 as f16, 150 with two tiles between barriers, 139 with every fragment read at
+ * the top of a tile (a read sunk to its use waited for LDS four times a tile).  48 problems of 2048 rows, heads of 64:
+ * 168 -> 130.  Short problems gain less: two workgroups of four waves fit a compute unit where three did
+ * (64 x 8 problems of 256 rows 28.8 -> 26.9 us, of 200 rows 25.4 -> 27.1, 64 x 4 of 300 rows in windows of 75 17.6 -> 19.0).
+ * Held to 168 registers for three, the compiler spills 24: 33.4 us against 26.4 for 40 x 8 problems of 300 rows.
  */
 #include "attn_device.h"
 #include "attn_launch.h"
@@ -51,6 +57,7 @@
 #include "lane_ops.h"
 #include "launch.h"
 #include "split_bf16.h"
+#include "split_f16.h"
 
 #include <algorithm>
 
@@ -132,28 +139,42 @@ __device__ __forceinline__ void wide_group_checked(const AttnProb &p, uint32_t g
     }
 }
 
-/* Bytes of LDS of one buffer: three parts of a K tile, rows of HD (+ 8) values; three of a V tile, a row of 32 (+ 8) keys
+/* One slot of LDS: the parts of a K tile, rows of HD (+ 8) values, and of a V tile, a row of 32 (+ 8) keys
  * per column.  The padding puts the 16-byte reads of eight consecutive rows into different banks. */
-template <int HD>
+template <int HD, bool F16>
 struct WideTiles {
+    static constexpr int PARTS = F16 ? 2 : 3;
+    /* tiles an iteration: two where a tile's work is short against the way from memory (heads of 32) */
+    static constexpr int STEP = F16 && HD == 32 ? 2 : 1;
+    static constexpr int SLOTS = 2 * STEP;
     static constexpr int KROW = HD + 8, VROW = 32 + 8;
     static constexpr int KPART = 32 * KROW, VPART = HD * VROW;
-    __bf16 k[3][KPART], v[3][VPART];
+    __bf16 k[PARTS][KPART], v[PARTS][VPART];
 };
 
+template <int HD>
+union WideLds {
+    WideTiles<HD, true> f16[WideTiles<HD, true>::SLOTS];
+    WideTiles<HD, false> bf16[WideTiles<HD, false>::SLOTS];
+};
+
+/* K and V are taken times this as f16: 2^-17 .. 4094 is the range that a run's largest value may lie in.  Of the 4 or 8 normal
+ * deviates of a run none comes near its lower end unless their deviation is below 1e-3. */
+constexpr float WIDE_UP = 16.0f;
 /* One group of 32 WV rows of problem p, WV waves.  Returns whether any of its rows met something that is not finite;
  * nothing is stored then.
  *
  * The keys of a V tile lie in the order in which a lane half holds its scores (accumulator register r of half h
  * is key acc_key(r, h)): position 16 j + 8 h + i is the key of register 8 j + i, so the weights of a lane are the
  * second operand as they are. */
-template <int HD, int WV, bool DENSE>
-__device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, WideTiles<HD> (&sm)[2]) {
-    using Tiles = WideTiles<HD>;
+template <int HD, int WV, bool DENSE, bool F16>
+__device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, WideTiles<HD, F16> (&sm)[WideTiles<HD, F16>::SLOTS]) {
+    using Tiles = WideTiles<HD, F16>;
+    constexpr int STEP = Tiles::STEP, PARTS = Tiles::PARTS;
     constexpr int KS = HD / 16;  /* steps of a score's contraction */
     constexpr int DB = HD / 32;
     constexpr int EPT = HD / 8;  /* values of K and of V a thread carries per tile */
-    typedef __bf16 piece __attribute__((ext_vector_type(EPT)));
+    typedef __bf16 piece __attribute__((ext_vector_type(EPT))); /* of either type */
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
@@ -186,31 +207,49 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
     flo = __builtin_amdgcn_readfirstlane(flo);
     fhi = __builtin_amdgcn_readfirstlane(fhi);
 
-    const float scale2 = p.scale * LOG2E * SPLIT_FAR;
     const float *mrow = DENSE ? p.mask + (size_t)i * p.nk : nullptr;
     const bool mvec = DENSE && (p.nk % 4u == 0u) && ((reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0u);
 
     /* ---- query fragment: row c, floats 16 s + 8 h ..., pre-scaled ---- */
     bf16x8 qf[KS][3];
+    float unit = SPLIT_DOWN; /* of a score as it is accumulated */
     {
         const float *qrow = p.q + (size_t)i * p.q_stride + 8u * h;
+        float x[KS][8], scale2 = p.scale * LOG2E * SPLIT_FAR;
 #pragma unroll
         for (int s = 0; s < KS; s++) {
             const float4 a = *reinterpret_cast<const float4 *>(qrow + 16 * s), b = *reinterpret_cast<const float4 *>(qrow + 16 * s + 4);
-            const float x[8] = {a.x * scale2, a.y * scale2, a.z * scale2, a.w * scale2,
-                                b.x * scale2, b.y * scale2, b.z * scale2, b.w * scale2};
-            split_bf16<8>(x, qf[s][0], qf[s][1], qf[s][2]);
+            x[s][0] = a.x, x[s][1] = a.y, x[s][2] = a.z, x[s][3] = a.w, x[s][4] = b.x, x[s][5] = b.y, x[s][6] = b.z, x[s][7] = b.w;
+        }
+        if (F16) { /* a power of two that brings the row's largest value to 2^14 .. 2^15; the rest of the scale is the score's */
+            float top = 0x1p-100f;
+#pragma unroll
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) top = fmaxf(top, fabsf(x[s][e]));
+            const int up = 15 - __builtin_amdgcn_frexp_expf(swap32(top, OpMax()));
+            scale2 = copysignf(ldexpf(1.0f, up), p.scale);
+            unit = fabsf(p.scale) * LOG2E * ldexpf(1.0f / WIDE_UP, -up);
+        }
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[s][e] *= scale2;
+            if (F16) split_f16_down<8>(x[s], qf[s][0], qf[s][1], qf[s][2]);
+            else split_bf16<8>(x[s], qf[s][0], qf[s][1], qf[s][2]);
         }
     }
 
-    floatx16 oacc[DB];
+    floatx16 oacc[DB], osml[DB]; /* F16: the small products by themselves, times HALF_UP */
 #pragma unroll
     for (int b = 0; b < DB; b++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) oacc[b][r] = 0.f;
-    float m = neg_inf(), l = 0.f;
+        for (int r = 0; r < 16; r++) oacc[b][r] = osml[b][r] = 0.f;
+    /* F16: m follows `top`, the largest score, only once that is LAZY above it (weights up to 2^LAZY then): most tiles of a
+     * long row leave its accumulators alone */
+    constexpr float LAZY = 2.0f;
+    float m = neg_inf(), l = 0.f, top = neg_inf();
     bool bad = false;
-    constexpr float unit = DENSE ? 1.0f : SPLIT_DOWN; /* of the score registers */
 
     /* ---- tile movement: 256 threads carry EPT values of one K row each, 256 EPT keys of one V column each (of eight
      * waves the first four K and the others V) ---- */
@@ -223,9 +262,18 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
 #pragma unroll
     for (int u = 0; u < EPT; u++) voff[u] = 4u * ((vkey + (uint32_t)(u < 4 ? u : u + 4)) * p.v_stride + vcol);
     const uint32_t last_tile = (p.nk - 1u) / 32u;
-    float pk[EPT], pv[EPT];
-    /* K tile kk and V tile kv; past the last tile: the last one again, past the last row: that row again */
-    auto request = [&](uint32_t kk, uint32_t kv) __attribute__((always_inline)) {
+    constexpr float K_FACTOR = F16 ? WIDE_UP : 1.0f, V_FACTOR = F16 ? WIDE_UP : SPLIT_FAR;
+    auto take_apart = [&](const float (&x)[EPT], piece (&a)[3]) __attribute__((always_inline)) {
+        if (F16) {
+            bad |= !half_range(x);
+            split_f16<EPT>(x, a[0], a[1]);
+        } else {
+            split_bf16<EPT>(x, a[0], a[1], a[2]);
+        }
+    };
+    float pk[STEP][EPT], pv[STEP][EPT];
+    /* K tile kk and V tile kv, to set `at`; past the last tile: the last one again, past the last row: that row again */
+    auto request = [&](int at, uint32_t kk, uint32_t kv) __attribute__((always_inline)) {
         kk = min(kk, last_tile), kv = min(kv, last_tile);
         if (for_k) {
             const char *base = reinterpret_cast<const char *>(p.k + (size_t)(kk * 32u) * p.k_stride);
@@ -233,7 +281,7 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
 #pragma unroll
             for (int u = 0; u < EPT; u += 4) {
                 const float4 a = *reinterpret_cast<const float4 *>(base + koff + 4 * u);
-                pk[u + 0] = a.x, pk[u + 1] = a.y, pk[u + 2] = a.z, pk[u + 3] = a.w;
+                pk[at][u + 0] = a.x, pk[at][u + 1] = a.y, pk[at][u + 2] = a.z, pk[at][u + 3] = a.w;
             }
         }
         if (for_v) {
@@ -244,157 +292,191 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
                     voff[u] = 4u * (min(vkey + (uint32_t)(u < 4 ? u : u + 4), p.nk - 1u - kv * 32u) * p.v_stride + vcol);
             }
 #pragma unroll
-            for (int u = 0; u < EPT; u++) pv[u] = *reinterpret_cast<const float *>(base + voff[u]);
+            for (int u = 0; u < EPT; u++) pv[at][u] = *reinterpret_cast<const float *>(base + voff[u]);
         }
     };
-    /* pieces of K to buffer kbuf, of V to buffer vbuf */
-    auto park = [&](uint32_t kbuf, uint32_t vbuf, bool k_too, bool v_too) __attribute__((always_inline)) {
+    /* what set `at` holds: pieces of K to slot kbuf, of V to slot vbuf */
+    auto park = [&](int at, uint32_t kbuf, uint32_t vbuf, bool k_too, bool v_too) __attribute__((always_inline)) {
         if (WV == 8) { /* the same instructions for either: two addresses and a choice */
             piece a[3];
             float x[EPT];
 #pragma unroll
-            for (int u = 0; u < EPT; u++) x[u] = for_k ? pk[u] : pv[u] * SPLIT_FAR;
-            split_bf16<EPT>(x, a[0], a[1], a[2]);
+            for (int u = 0; u < EPT; u++) x[u] = F16 ? (for_k ? pk[at][u] : pv[at][u]) * WIDE_UP : for_k ? pk[at][u] : pv[at][u] * SPLIT_FAR;
+            take_apart(x, a);
             __bf16 *to = for_k ? &sm[kbuf].k[0][krow * Tiles::KROW + kcol] : &sm[vbuf].v[0][vcol * Tiles::VROW + vgrp * EPT];
             const uint32_t part = for_k ? Tiles::KPART : Tiles::VPART;
             if (for_k ? k_too : v_too) {
 #pragma unroll
-                for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(to + part * t) = a[t];
+                for (int t = 0; t < PARTS; t++) *reinterpret_cast<piece *>(to + part * t) = a[t];
             }
             return;
         }
         piece a[3];
+        float x[EPT];
         if (k_too) {
-            split_bf16<EPT>(pk, a[0], a[1], a[2]);
 #pragma unroll
-            for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&sm[kbuf].k[t][krow * Tiles::KROW + kcol]) = a[t];
+            for (int u = 0; u < EPT; u++) x[u] = pk[at][u] * K_FACTOR;
+            take_apart(x, a);
+#pragma unroll
+            for (int t = 0; t < PARTS; t++) *reinterpret_cast<piece *>(&sm[kbuf].k[t][krow * Tiles::KROW + kcol]) = a[t];
         }
         if (v_too) {
-            float x[EPT];
 #pragma unroll
-            for (int u = 0; u < EPT; u++) x[u] = pv[u] * SPLIT_FAR;
-            split_bf16<EPT>(x, a[0], a[1], a[2]);
+            for (int u = 0; u < EPT; u++) x[u] = pv[at][u] * V_FACTOR;
+            take_apart(x, a);
 #pragma unroll
-            for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&sm[vbuf].v[t][vcol * Tiles::VROW + vgrp * EPT]) = a[t];
+            for (int t = 0; t < PARTS; t++) *reinterpret_cast<piece *>(&sm[vbuf].v[t][vcol * Tiles::VROW + vgrp * EPT]) = a[t];
         }
     };
     /* ---- S^T = K Q^T ---- */
     auto scores = [&](uint32_t buf) __attribute__((always_inline)) {
         floatx16 s;
+        bf16x8 kh[KS];
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = 0.f;
 #pragma unroll
         for (int k = 0; k < KS; k++) {
-            bf16x8 kf[3];
+            bf16x8 kf[PARTS];
 #pragma unroll
-            for (int t = 0; t < 3; t++) kf[t] = *reinterpret_cast<const bf16x8 *>(&sm[buf].k[t][c * Tiles::KROW + 16 * k + 8 * h]);
-            s = mfma_split(kf, qf[k], s);
+            for (int t = 0; t < PARTS; t++) kf[t] = *reinterpret_cast<const bf16x8 *>(&sm[buf].k[t][c * Tiles::KROW + 16 * k + 8 * h]);
+            if constexpr (F16) s = mfma_f16(kf[0], qf[k][1], mfma_f16(kf[1], qf[k][2], s)), kh[k] = kf[0];
+            else s = mfma_split(kf, qf[k], s);
+        }
+        if constexpr (F16) {
+#pragma unroll
+            for (int k = 0; k < KS; k++) s = mfma_f16(kh[k], qf[k][0], s);
         }
         return s;
     };
 
     /* The loop runs one score tile ahead: while tile kt's weights are made and applied, the matrix unit has the
      * scores of tile kt + 1 to work on.  K is in LDS one tile ahead of V. */
-    floatx16 sacc;
+    floatx16 score[2]; /* of this tile and of the next one, in turn if an iteration is two tiles */
+    constexpr int TURN = STEP - 1;
 #pragma unroll
-    for (int r = 0; r < 16; r++) sacc[r] = 0.f;
+    for (int r = 0; r < 16; r++) score[0][r] = score[1][r] = 0.f;
     if (gt_lo < gt_hi) {
-        request(gt_lo, gt_lo);
-        park(0, 0, true, true);
-        request(gt_lo + 1u, gt_lo);
-        park(1, 0, true, false);
-        __syncthreads();
-        if (gt_lo == kt_lo) sacc = scores(0);
+#pragma unroll
+        for (int n = 0; n < STEP; n++) request(n, gt_lo + n, gt_lo + n);
+#pragma unroll
+        for (int n = 0; n < STEP; n++) park(n, n, n, true, true);
+        request(0, gt_lo + STEP, gt_lo);
+        park(0, STEP, 0, true, false);
+        if (F16) { /* where K or V is out of range, that is seen here as a rule */
+            if (__syncthreads_or(bad)) return true;
+        } else {
+            __syncthreads();
+        }
+        if (gt_lo == kt_lo) score[0] = scores(0);
         __syncthreads();
     }
 
-    for (uint32_t kt = gt_lo; kt < gt_hi; kt++) {
-        const uint32_t buf = (kt - gt_lo) & 1u;
-        request(kt + 2u, kt + 1u); /* travels while this tile is worked on */
-
-        if (kt >= kt_lo && kt < kt_hi) {
-            const uint32_t k0 = kt * 32u;
-
-            /* ---- mask, tile maximum ----
-             * Interior tiles (no row masks any key) take the scores as they
-             * are; edge tiles compare the key's offset into the row's range
-             * with one unsigned test.  No per-element branches. */
-            float mt = neg_inf();
-            const bool all_seen = !DENSE && k0 >= flo && k0 + 32u <= fhi; /* wave-uniform */
-            if (!all_seen) {
-                float mk[16];
-                if (DENSE) {
+    for (uint32_t g = gt_lo; g < gt_hi; g += STEP) {
 #pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        const uint32_t j0 = k0 + 8u * g + 4u * h;
-                        if (mvec) {
-                            float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-                            if (j0 < p.nk) t = *reinterpret_cast<const float4 *>(mrow + j0);
-                            mk[4 * g + 0] = t.x, mk[4 * g + 1] = t.y, mk[4 * g + 2] = t.z, mk[4 * g + 3] = t.w;
+        for (int n = 0; n < STEP; n++) request(n, g + STEP + 1 + n, g + STEP + n); /* travel while these tiles are worked on */
+#pragma unroll
+        for (int n = 0; n < STEP; n++) {
+            const uint32_t kt = g + n;
+            floatx16 &sacc = score[n & TURN], &after = score[(n + 1) & TURN];
+            const uint32_t buf = (kt - gt_lo) % Tiles::SLOTS, next = (kt - gt_lo + 1u) % Tiles::SLOTS;
+            const uint32_t kfree = (kt - gt_lo + STEP + 1u) % Tiles::SLOTS, vfree = (kt - gt_lo + STEP) % Tiles::SLOTS;
+            if (kt >= kt_lo && kt < kt_hi) {
+                const uint32_t k0 = kt * 32u;
+
+                /* ---- mask, tile maximum ----
+                 * Interior tiles (no row masks any key) take the scores as they
+                 * are; edge tiles compare the key's offset into the row's range
+                 * with one unsigned test.  No per-element branches. */
+                float mt = neg_inf();
+                const bool all_seen = !DENSE && k0 >= flo && k0 + 32u <= fhi; /* wave-uniform */
+                if (!all_seen) {
+                    float mk[16];
+                    if (DENSE) {
+#pragma unroll
+                        for (int g = 0; g < 4; g++) {
+                            const uint32_t j0 = k0 + 8u * g + 4u * h;
+                            if (mvec) {
+                                float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+                                if (j0 < p.nk) t = *reinterpret_cast<const float4 *>(mrow + j0);
+                                mk[4 * g + 0] = t.x, mk[4 * g + 1] = t.y, mk[4 * g + 2] = t.z, mk[4 * g + 3] = t.w;
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < 4; e++) mk[4 * g + e] = mrow[min(j0 + e, p.nk - 1u)];
+                            }
+                        }
+                    }
+                    const uint32_t rel = k0 + 4u * h - lo, len = hi - lo;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        if (DENSE) {
+                            bad |= !isfinite(sacc[r]); /* behind the mask a score that overflowed downwards looks masked */
+                            sacc[r] = sacc[r] * unit + mk[r] * LOG2E;
+                        }
+                        sacc[r] = rel + (8u * (r >> 2) + (r & 3u)) < len ? sacc[r] : neg_inf();
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 16; r++) mt = fmaxf(mt, sacc[r]);
+                mt = swap32(mt, OpMax()) * (DENSE ? 1.0f : unit);
+                const float mn = F16 && !(mt > m + LAZY) ? m : fmaxf(m, mt);
+                if (F16) top = fmaxf(top, mt);
+                const float ms = mn == neg_inf() ? 0.f : mn; /* nothing seen yet: keep the differences finite */
+                if (__any(mn > m)) {
+                    const float alpha = fast_exp2(m - ms);
+                    l *= alpha;
+#pragma unroll
+                    for (int b = 0; b < DB; b++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            oacc[b][r] *= alpha;
+                            if (F16) osml[b][r] *= alpha;
+                        }
+                    m = mn;
+                }
+                floatx16 ahead;
+                (TURN ? after : ahead) = scores(next); /* past the wave's last tile: not used */
+
+                /* ---- O^T += V^T P^T ---- */
+                float ps = 0.f;
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    float x[8];
+#pragma unroll
+                    for (int r = 0; r < 8; r++) {
+                        x[r] = fast_exp2(sacc[8 * j + r] * (DENSE ? 1.0f : unit) - ms);
+                        ps += x[r];
+                    }
+                    bf16x8 pf[3];
+                    if (F16) split_f16<8>(x, pf[0], pf[1]);
+                    else split_bf16<8>(x, pf[0], pf[1], pf[2]);
+#pragma unroll
+                    for (int b = 0; b < DB; b++) {
+                        bf16x8 vf[PARTS];
+#pragma unroll
+                        for (int t = 0; t < PARTS; t++)
+                            vf[t] = *reinterpret_cast<const bf16x8 *>(&sm[buf].v[t][(32 * b + c) * Tiles::VROW + 16 * j + 8 * h]);
+                        if constexpr (F16) {
+                            osml[b] = mfma_f16(vf[0], pf[1], mfma_f16(vf[1], pf[0], osml[b]));
+                            oacc[b] = mfma_f16(vf[0], pf[0], oacc[b]);
                         } else {
-#pragma unroll
-                            for (int e = 0; e < 4; e++) mk[4 * g + e] = mrow[min(j0 + e, p.nk - 1u)];
+                            oacc[b] = mfma_split(vf, pf, oacc[b]);
                         }
                     }
                 }
-                const uint32_t rel = k0 + 4u * h - lo, len = hi - lo;
+                l += ps;
+                if (!TURN) after = ahead;
+                park(n, kfree, vfree, true, true);
+                /* all fragments first: left to itself the compiler reads one before each use and waits for it */
+                if (F16 && HD == 32) __builtin_amdgcn_sched_group_barrier(0x100, 2 * (KS + 2 * DB), 0);
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    if (DENSE) {
-                        bad |= !isfinite(sacc[r]); /* behind the mask a score that overflowed downwards looks masked */
-                        sacc[r] = sacc[r] * SPLIT_DOWN + mk[r] * LOG2E;
-                    }
-                    sacc[r] = rel + (8u * (r >> 2) + (r & 3u)) < len ? sacc[r] : neg_inf();
+                for (int i = 0; i < (F16 ? 3 : 6) * (KS + 2 * DB); i++) { /* a matrix instruction, its time in vector instructions */
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, F16 ? (HD == 32 ? 10 : 8) : HD == 32 ? 6 : 4, 0);
                 }
+            } else {
+                if (kt + 1u == kt_lo) after = scores(next);
+                park(n, kfree, vfree, true, true);
             }
-#pragma unroll
-            for (int r = 0; r < 16; r++) mt = fmaxf(mt, sacc[r]);
-            mt = swap32(mt, OpMax()) * unit;
-            const float mn = fmaxf(m, mt);
-            const float ms = mn == neg_inf() ? 0.f : mn; /* nothing seen yet: keep the differences finite */
-            if (__any(mn > m)) {
-                const float alpha = fast_exp2(m - ms);
-                l *= alpha;
-#pragma unroll
-                for (int b = 0; b < DB; b++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) oacc[b][r] *= alpha;
-                m = mn;
-            }
-            const floatx16 ahead = scores(buf ^ 1u); /* past the wave's last tile: not used */
-
-            /* ---- O^T += V^T P^T ---- */
-            float ps = 0.f;
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                float x[8];
-#pragma unroll
-                for (int r = 0; r < 8; r++) {
-                    x[r] = fast_exp2(sacc[8 * j + r] * unit - ms);
-                    ps += x[r];
-                }
-                bf16x8 pf[3];
-                split_bf16<8>(x, pf[0], pf[1], pf[2]);
-#pragma unroll
-                for (int b = 0; b < DB; b++) {
-                    bf16x8 vf[3];
-#pragma unroll
-                    for (int t = 0; t < 3; t++)
-                        vf[t] = *reinterpret_cast<const bf16x8 *>(&sm[buf].v[t][(32 * b + c) * Tiles::VROW + 16 * j + 8 * h]);
-                    oacc[b] = mfma_split(vf, pf, oacc[b]);
-                }
-            }
-            l += ps;
-            sacc = ahead;
-            park(buf, buf ^ 1u, true, true);
-#pragma unroll
-            for (int n = 0; n < 6 * KS + 12 * DB; n++) { /* a matrix instruction, its time in vector instructions */
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, HD == 32 ? 6 : 4, 0);
-            }
-        } else {
-            if (kt + 1u == kt_lo) sacc = scores(buf ^ 1u);
-            park(buf, buf ^ 1u, true, true);
         }
         __syncthreads();
     }
@@ -406,12 +488,15 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
 #pragma unroll
     for (int b = 0; b < DB; b++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) bad |= !isfinite(oacc[b][r]);
+        for (int r = 0; r < 16; r++) {
+            if (F16) oacc[b][r] += osml[b][r] * HALF_DOWN;
+            bad |= !isfinite(oacc[b][r]);
+        }
     /* together, before anything is stored: the output may lie in place of the queries, which the second run reads */
     if (__syncthreads_or(bad)) return true;
     if (!live) return false;
 
-    const float inv = l > 0.f ? SPLIT_DOWN / l : 0.f;
+    const float inv = l > 0.f ? 1.0f / V_FACTOR / l : 0.f;
     float *orow = p.out + (size_t)i * p.out_stride;
 #pragma unroll
     for (int b = 0; b < DB; b++)
@@ -421,8 +506,8 @@ __device__ __forceinline__ bool wide_group(const AttnProb &p, uint32_t group, Wi
                 make_float4(oacc[b][4 * g + 0] * inv, oacc[b][4 * g + 1] * inv, oacc[b][4 * g + 2] * inv,
                             oacc[b][4 * g + 3] * inv);
     if (h == 0 && p.lse) {
-        p.lse[2 * (size_t)i + 0] = m * LN2; /* back to natural units */
-        p.lse[2 * (size_t)i + 1] = l;
+        p.lse[2 * (size_t)i + 0] = (F16 ? top : m) * LN2; /* back to natural units */
+        p.lse[2 * (size_t)i + 1] = F16 && l > 0.f ? l * exp2f(m - top) : l;
     }
     return false;
 }
@@ -440,7 +525,7 @@ __device__ __forceinline__ void wide_pair(uint32_t t, uint32_t G, uint32_t &ga, 
 template <int HD, int WV, int SRC, bool DENSE>
 __global__ __launch_bounds__(64 * WV, 2) void attn_wide_kernel(const AttnProb *__restrict__ probs,
                                                            const AttnTile *__restrict__ tiles, AttnAffine aff) {
-    __shared__ __attribute__((aligned(16))) WideTiles<HD> sm[2];
+    __shared__ __attribute__((aligned(16))) WideLds<HD> sm;
 
     uint32_t ga, gb = WIDE_NO_GROUP;
     AttnProb p;
@@ -465,7 +550,8 @@ __global__ __launch_bounds__(64 * WV, 2) void attn_wide_kernel(const AttnProb *_
     for (int pass = 0; pass < 2; pass++) {
         const uint32_t group = pass == 0 ? ga : gb;
         if (group == WIDE_NO_GROUP) break;
-        if (wide_group<HD, WV, DENSE>(p, group, sm)) wide_group_checked<HD, WV, DENSE>(p, group);
+        if (wide_group<HD, WV, DENSE, true>(p, group, sm.f16) && wide_group<HD, WV, DENSE, false>(p, group, sm.bf16))
+            wide_group_checked<HD, WV, DENSE>(p, group);
     }
 }
 

@@ -834,6 +834,47 @@ def test_attention_on_split_operands(kernel, batch, H, hd, nq, nk, window, dev):
         d.close()
 
 
+@pytest.mark.parametrize("batch,H,hd,nq,nk", [(24, 4, 32, 1025, 1025), (64, 2, 32, 513, 600), (24, 8, 64, 300, 300)])
+def test_attention_on_halves_out_of_range(batch, H, hd, nq, nk, dev):
+    """The large-batch kernel takes K and V apart into f16 parts where runs of them lie within 2^-17 .. 4094, and a group of rows
+    whose keys do not is run again on bf16 parts: below, above, at zero, with one value or one column outside, within at both
+    ends.  Each column against float64 in the 2-norm: a value is within 2^-23, a product within 2^-21, scores of at most 8 in
+    log2 units double that in a weight; 2^-19 in all."""
+    import torch
+    w = workloads.offset_causal(batch=batch, nq=nq, nk=nk, H=H, hd=hd)
+    d = dev.DeviceWorkload(w)
+    lib = api.load()
+    try:
+        q, k, v = (d.dev[n].view(batch, -1, H, hd) for n in ("q", "k", "v"))
+        v[1] *= 1e-7                                 # all of V below
+        q[2] *= 1e-5
+        k[2] *= 1e5                                  # all of K above
+        v[3, nk // 2, :, 1] = 3e4                    # one value above, met half way
+        k[4] = 0.0
+        v[5, :, :, 2] *= 1e-8                        # a column below, the others not
+        k[6] *= 2.0 ** -6
+        v[6] *= 2.0 ** -8                            # within
+        v[7] *= 500.0
+        k[8, :, 1] *= 1e-9                           # the keys of one head below
+        torch.cuda.synchronize()
+        d.zero_outputs()
+        plan = d.make_plan("descriptor")
+        assert lib.blt_attention_plan_kernel_hip(plan) == b"wide"
+        lib.blt_attention_plan_run_hip(plan)
+        lib.blt_backend_pass_sync_hip()
+        lib.blt_attention_plan_destroy_hip(plan)
+        got = torch.from_numpy(d.output("out").copy()).cuda().view(batch, nq, H, hd).double()
+        i, j = torch.arange(nq, device="cuda")[:, None], torch.arange(nk, device="cuda")[None, :]
+        for b in range(10):
+            for head in (0, 1):
+                s = (q[b, :, head].double() @ k[b, :, head].double().T.contiguous()) * w.heads[0].scale
+                want = torch.softmax(s.masked_fill(j > i + nk - nq, float("-inf")), dim=1) @ v[b, :, head].double()
+                error = (got[b, :, head] - want).norm(dim=0) / want.norm(dim=0)
+                assert error.max().item() < 2.0 ** -19, (b, head, error.max().item())
+    finally:
+        d.close()
+
+
 @pytest.mark.parametrize("family", ["auto", "rows", "mfma", "wide", "fine", "fine16", "fine128", "once"])
 def test_attention_random_shapes(family):
     """72 randomly shaped strided batches per routing (automatic, and every family / workgroup shape
