@@ -13,9 +13,9 @@
  *    is bit-identical to blt_matmul_cpu.
  *
  *  - "mfma" (everything else; from three terms a sum on): 64x64 or 128x128 output tiles per workgroup of eight
- *    wavefronts, K in steps of 32 through double-buffered LDS tiles, on the bf16
- *    matrix instructions with both operands taken apart into three exact parts on the
- *    way to LDS (split_bf16.h).  The product is accumulated
+ *    wavefronts, K in steps of 32 or 64 through double-buffered LDS tiles, on the f16 or bf16
+ *    matrix instructions with both operands taken apart on the way to LDS
+ *    (split_f16.h, split_bf16.h).  The product is accumulated
  *    TRANSPOSED (MFMA A operand = b tile, B operand = a tile), which puts one
  *    output ROW in each lane with four consecutive columns per register
  *    group: rows are stored with 16-byte stores, and an optional epilogue can
@@ -23,11 +23,8 @@
  *    embedding of the Q and K blocks of a packed QKV projection
  *    (csrc/models/attention.c:76-90) -- without a second pass over the
  *    result.  Summation order differs from the reference's (fp32 tolerance).
- *    Bound: matrix and vector instructions share the time about evenly for the 64x64 tile
- *    (384 and about 500 cycles of a step), the matrix ones and the barrier of every step for the 128x128 tile
- *    (8192 x 512 . 512 x 1536: matrix unit busy 0.40 of the time, vector issue 0.34).  On fp32 instructions -> on
- *    parts: 2048 x 512 . 512 x 2048 41.0 -> 30.4 us, 2048 x 2048 . 2048 x 512 45.3 -> 37.0, 8192 x 512 . 512 x 512
- *    42.8 -> 30.2, 4096 x 1024 . 1024 x 4096 274 -> 197 (174 TFLOP/s).
+ *    On fp32 instructions -> on bf16 parts -> on f16 parts: 2048 x 512 . 512 x 2048 41.0 -> 30.4 -> 20.6 us, 2048 x 2048 .
+ *    2048 x 512 45.3 -> 37.0 -> 28.6, 8192 x 512 . 512 x 1536 84.2 as bf16 -> 65.2.
  *
  *  - "splitk" (outputs too small to give every compute unit a 64x64 tile,
  *    e.g. 512x128 * 128x384; sums of one or two terms; more than 2^25 columns): one 32x32 output tile per workgroup, its four
@@ -43,6 +40,7 @@
 #include "launch.h"
 #include "matmul.h"
 #include "split_bf16.h"
+#include "split_f16.h"
 #include "cross_rows_device.h"
 
 #include <stdint.h>
@@ -86,9 +84,14 @@ __device__ __forceinline__ void store4(const MatmulArgs &g, uint32_t row, uint32
 
 /* One (64*WT)x(64*WT) output tile per workgroup of eight wavefronts: four quadrants of WT x WT MFMA tiles, and for each
  * quadrant two waves that take half of every K step (16 of 32); their sums meet in LDS at the end.  The
- * operands are taken apart into three bf16 parts (split_bf16.h) once per workgroup, on the way from registers
- * to the double-buffered LDS tiles: rows of a as [row][k], columns of b as [column][k], so that a fragment is one
+ * operands are taken apart into two f16 parts (split_f16.h) or three bf16 parts (split_bf16.h) once per workgroup, on the
+ * way from registers to the double-buffered LDS tiles: rows of a as [row][k], columns of b as [column][k], so that a fragment is one
  * 16-byte read.  WT = 2 halves the split and the LDS reads per output.
+ * f16 first, if K is long enough; a workgroup that meets operands out of its range, before the first product as a rule,
+ * starts again as bf16.  Half the matrix instructions, four fifths of the vector ones, half the error (K = 2048: 2.2e-7
+ * against 4.9e-7), and a clock that gives way less (8192 x 2048 . 2048 x 1536, random operands against ones: 268 and 210 us
+ * as bf16, 196 and 160 as f16).  Bound: in a step of the large tile the matrix unit takes 770 cycles of a SIMD, the vector
+ * unit about 720, which add up, the LDS 770 beside them, of 2000 in all; the rest is the barrier.
  * VEC: a 16-byte aligned with lda and K multiples of 4.  ROPE: rotate pairs of the first g.rope_cols columns in
  * the epilogue.
  * NORM: the row statistic comes from the values on their way to LDS, the norm weight is multiplied in there, the row's
@@ -97,27 +100,40 @@ __device__ __forceinline__ void store4(const MatmulArgs &g, uint32_t row, uint32
  * GATED: the left quadrants are columns of a*b, the right ones the same columns of a*b2; the gates pass through LDS to
  * the waves that hold the other factor (2048 x 512 . 512 x (2 x 2048): two products and the activation 71 us,
  * this way 63). */
-template <int WT>
+template <int WT, bool NORM, bool F16>
 struct MfmaShape {
     static constexpr int BT = 64 * WT;          /* rows and columns of the tile */
-    static constexpr int EPT = 4 * WT;          /* values of each operand a thread carries per step */
-    static constexpr int LP = TK + 8;           /* LDS row: 16-byte reads of eight consecutive rows hit different banks */
-    static constexpr int PART = BT * LP;
+    static constexpr int STEP = F16 && WT == 1 && !NORM ? 64 : 32; /* of K: the small tile's work in 32 is short against a barrier */
+    static constexpr int EPT = BT * STEP / 512; /* values of each operand a thread carries per step */
+    static constexpr int LP = STEP + 8;         /* LDS row: 16-byte reads of eight consecutive rows hit different banks */
+    static constexpr int PART = BT * LP, PARTS = F16 ? 2 : 3;
     struct Tiles {
-        __bf16 a[3][PART], b[3][PART];
+        __bf16 a[PARTS][PART], b[PARTS][PART]; /* of either type */
     };
     static constexpr size_t LDS_BYTES = 2 * sizeof(Tiles);
     static_assert(4 * WT * WT * 16 * 64 * sizeof(float) <= LDS_BYTES, "the second waves' sums pass through the tile buffers");
 };
+template <int WT, bool NORM>
+constexpr size_t MFMA_LDS_BYTES = std::max(MfmaShape<WT, NORM, true>::LDS_BYTES, MfmaShape<WT, NORM, false>::LDS_BYTES);
 
-template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED>
-__global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
-    using Shape = MfmaShape<WT>;
-    constexpr int BT = Shape::BT, EPT = Shape::EPT, LP = Shape::LP;
-    typedef __bf16 piece __attribute__((ext_vector_type(EPT)));
-    extern __shared__ __attribute__((aligned(16))) unsigned char mm_lds[];
-    auto *tiles = reinterpret_cast<typename Shape::Tiles *>(mm_lds);
-    __shared__ float row_ss[NORM ? BT : 1];
+/* Operands of the f16 form are taken times these: runs of a whose largest value lies in 2^-17 .. 4094, of b in 2^-19 .. 1023. */
+constexpr float HALF_A = 16.0f, HALF_B = 64.0f;
+
+/* K from which the f16 form is taken, by WT: the error of its parts is that of the longer chain of roundings of the bf16 form
+ * at K = 100 and less from there on; 64x64 tiles lose their first two steps of 64 to filling and draining (2048 x 128 . 128 x 1024
+ * 7.8 us as bf16, 9.1 as f16; K = 256 10.9 and 11.4; K = 512 19.2 and 16.8), 128x128 ones gain from the start (8192 x 128 .
+ * 128 x 1536 36.4 -> 33.0). */
+constexpr uint32_t HALF_K[2] = {384, 128};
+
+/* The sums of a wave over its half of K, scaled (by HALF_A HALF_B, or 2^32), and a thread's share of its row's sum of squares.
+ * F16: as f16 parts; returns true, the same for all threads and with nothing of use in acc, if a run of values is out of
+ * their range. */
+template <bool VEC, int WT, bool NORM, bool GATED, bool F16>
+__device__ __forceinline__ bool mfma_sums(const MatmulArgs &g, unsigned char *lds, floatx16 (&acc)[WT][WT], float &ss) {
+    using Shape = MfmaShape<WT, NORM, F16>;
+    constexpr int BT = Shape::BT, EPT = Shape::EPT, LP = Shape::LP, PARTS = Shape::PARTS, TK = Shape::STEP;
+    auto *tiles = reinterpret_cast<typename Shape::Tiles *>(lds);
+    typedef __bf16 piece __attribute__((ext_vector_type(EPT))); /* of either type */
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -165,50 +181,68 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
             }
         }
     };
-    float ss = 0.f; /* this thread's share of its row's sum of squares */
+    ss = 0.f;
+    bool bad = false;
+    constexpr float UP_A = F16 ? HALF_A : SPLIT_UP, UP_B = F16 ? HALF_B : SPLIT_UP;
     auto park = [&](const Values &v, uint32_t buf, bool counts) __attribute__((always_inline)) {
         float pa[EPT], pb[EPT], squares = 0.f;
 #pragma unroll
         for (int i = 0; i < EPT; i++) {
-            if constexpr (NORM) squares = fmaf(v.a[i], v.a[i], squares), pa[i] = v.a[i] * v.w[i] * SPLIT_UP;
-            else pa[i] = v.a[i] * SPLIT_UP;
-            pb[i] = v.b[i] * SPLIT_UP;
+            if constexpr (NORM) squares = fmaf(v.a[i], v.a[i], squares), pa[i] = v.a[i] * v.w[i] * UP_A;
+            else pa[i] = v.a[i] * UP_A;
+            pb[i] = v.b[i] * UP_B;
         }
         if constexpr (NORM) ss += counts ? squares : 0.f;
         piece parts[3];
-        split_bf16<EPT>(pa, parts[0], parts[1], parts[2]);
+        if constexpr (F16) bad |= !half_range(pa) | !half_range(pb), split_f16<EPT>(pa, parts[0], parts[1]);
+        else split_bf16<EPT>(pa, parts[0], parts[1], parts[2]);
 #pragma unroll
-        for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&tiles[buf].a[t][a_row * LP + a_k]) = parts[t];
-        split_bf16<EPT>(pb, parts[0], parts[1], parts[2]);
+        for (int t = 0; t < PARTS; t++) *reinterpret_cast<piece *>(&tiles[buf].a[t][a_row * LP + a_k]) = parts[t];
+        if constexpr (F16) split_f16<EPT>(pb, parts[0], parts[1]);
+        else split_bf16<EPT>(pb, parts[0], parts[1], parts[2]);
 #pragma unroll
-        for (int t = 0; t < 3; t++) *reinterpret_cast<piece *>(&tiles[buf].b[t][b_col * LP + b_k]) = parts[t];
+        for (int t = 0; t < PARTS; t++) *reinterpret_cast<piece *>(&tiles[buf].b[t][b_col * LP + b_k]) = parts[t];
     };
 
-    floatx16 acc[WT][WT];
+    floatx16 small[WT][WT]; /* F16: the products with a low part, times HALF_UP */
 #pragma unroll
     for (int i = 0; i < WT; i++)
 #pragma unroll
         for (int j = 0; j < WT; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+            for (int r = 0; r < 16; r++) acc[i][j][r] = small[i][j][r] = 0.f;
 
     struct Fragments {
-        bf16x8 a[WT][3], b[WT][3];
+        bf16x8 a[WT][PARTS][TK / 32], b[WT][PARTS][TK / 32];
     };
     auto read = [&](uint32_t buf, Fragments &f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < 3; t++)
+        for (int t = 0; t < PARTS; t++)
 #pragma unroll
-            for (int i = 0; i < WT; i++) {
-                f.a[i][t] = *reinterpret_cast<const bf16x8 *>(&tiles[buf].a[t][(wr * (32u * WT) + 32u * i + c) * LP + 16u * kg + 8u * h]);
-                f.b[i][t] = *reinterpret_cast<const bf16x8 *>(&tiles[buf].b[t][(wc * (32u * WT) + 32u * i + c) * LP + 16u * kg + 8u * h]);
-            }
+            for (int i = 0; i < WT; i++)
+#pragma unroll
+                for (int k = 0; k < TK / 32; k++) {
+                    const uint32_t at = TK / 2u * kg + 16u * k + 8u * h;
+                    f.a[i][t][k] = *reinterpret_cast<const bf16x8 *>(&tiles[buf].a[t][(wr * (32u * WT) + 32u * i + c) * LP + at]);
+                    f.b[i][t][k] = *reinterpret_cast<const bf16x8 *>(&tiles[buf].b[t][(wc * (32u * WT) + 32u * i + c) * LP + at]);
+                }
     };
     auto multiply = [&](const Fragments &f) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < WT; i++)
 #pragma unroll
-            for (int j = 0; j < WT; j++) acc[i][j] = mfma_split(f.b[j], f.a[i], acc[i][j]);
+            for (int j = 0; j < WT; j++)
+#pragma unroll
+                for (int k = 0; k < TK / 32; k++) {
+                    if constexpr (F16) {
+                        small[i][j] = mfma_f16(f.b[j][1][k], f.a[i][0][k], small[i][j]);
+                        acc[i][j] = mfma_f16(f.b[j][0][k], f.a[i][0][k], acc[i][j]);
+                        small[i][j] = mfma_f16(f.b[j][0][k], f.a[i][1][k], small[i][j]);
+                    } else {
+                        const bf16x8 a[3] = {f.a[i][0][k], f.a[i][1][k], f.a[i][2][k]}, b[3] = {f.b[j][0][k], f.b[j][1][k], f.b[j][2][k]};
+                        acc[i][j] = mfma_split(b, a, acc[i][j]);
+                    }
+                }
     };
     /* Whole steps: two register sets take turns, the values of step s+1 and s+2 are on their way while step s
      * runs, so a request has two steps of matrix work to arrive in.  Past the last one it is requested and
@@ -221,17 +255,22 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
         request(v1, of_step(1u));
         park(v0, 0, true);
         request(v0, of_step(2u));
-        __syncthreads();
+        if (F16) { /* an operand that is out of range is so everywhere, as a rule */
+            if (__syncthreads_or(bad)) return true;
+        } else {
+            __syncthreads();
+        }
         auto step = [&](uint32_t s, Values &v) __attribute__((always_inline)) {
             /* v holds the values of step s+1 */
             Fragments f;
             read(s & 1u, f);
             multiply(f);
             park(v, (s & 1u) ^ 1u, s + 1u < steps);
+            if (F16) __builtin_amdgcn_sched_group_barrier(0x100, 4 * WT * TK / 32, 0); /* fragments first */
 #pragma unroll
-            for (int n = 0; n < 6 * WT * WT; n++) { /* a matrix instruction, its time in vector instructions */
+            for (int n = 0; n < (F16 ? 3 : 6) * WT * WT * TK / 32; n++) { /* a matrix instruction, its time in vector instructions */
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, WT == 2 ? 4 : 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (F16 ? 2 : 1) * (WT == 2 ? 4 : 8), 0);
             }
             request(v, of_step(s + 3u));
             __syncthreads();
@@ -258,10 +297,43 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
         multiply(f);
         __syncthreads();
     }
-    if constexpr (NORM) { /* the threads of a row are neighbours */
+    if (F16) {
 #pragma unroll
-        for (uint32_t d = 1u; d < TK / EPT; d *= 2u) ss += __shfl_xor(ss, (int)d, 64);
-        if (tid % (TK / EPT) == 0u) row_ss[a_row] = ss;
+        for (int i = 0; i < WT; i++)
+#pragma unroll
+            for (int j = 0; j < WT; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf(small[i][j][r], HALF_DOWN, acc[i][j][r]);
+        return __syncthreads_or(bad);
+    }
+    return false;
+}
+
+template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED>
+__global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(MatmulArgs g) {
+    constexpr int BT = MfmaShape<WT, NORM, true>::BT;
+    extern __shared__ __attribute__((aligned(16))) unsigned char mm_lds[];
+    __shared__ float row_ss[NORM ? BT : 1];
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t h = lane >> 5, c = lane & 31u;
+    const uint32_t wr = (wave & 3u) >> 1, wc = wave & 1u; /* wave's quadrant of the tile */
+    const uint32_t kg = wave >> 2;                         /* its half of a K step */
+    constexpr uint32_t COLS = GATED ? BT / 2 : BT; /* columns of a product */
+    const uint32_t row0 = blockIdx.y * BT, col0 = blockIdx.x * COLS;
+
+    floatx16 acc[WT][WT];
+    float ss, down = 1.0f / (HALF_A * HALF_B);
+    if (g.k < HALF_K[WT - 1] || mfma_sums<VEC, WT, NORM, GATED, true>(g, mm_lds, acc, ss)) {
+        mfma_sums<VEC, WT, NORM, GATED, false>(g, mm_lds, acc, ss);
+        down = SPLIT_DOWN;
+    }
+    if constexpr (NORM) { /* the threads of a row are neighbours */
+        constexpr uint32_t SHARE = 512u / BT;
+#pragma unroll
+        for (uint32_t d = 1u; d < SHARE; d *= 2u) ss += __shfl_xor(ss, (int)d, 64);
+        if (tid % SHARE == 0u) row_ss[tid / SHARE] = ss;
     }
 
     /* the tile buffers are free */
@@ -281,7 +353,7 @@ __global__ __launch_bounds__(512, 2) void matmul_mfma_kernel(MatmulArgs g) {
         for (int r = 0; r < 16; r++) {
             acc[i / WT][i % WT][r] += meet[(i * 16 + r) * 64];
             bad |= !isfinite(acc[i / WT][i % WT][r]);
-            acc[i / WT][i % WT][r] *= SPLIT_DOWN;
+            acc[i / WT][i % WT][r] *= down;
         }
     const bool gate_wave = GATED && wc == 1u;
     const uint32_t wave_col = col0 + (GATED ? 0u : wc * (32u * WT));
@@ -868,9 +940,9 @@ void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStrea
 namespace {
 template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED>
 void launch_mfma_as(const MatmulArgs &g, hipStream_t s) {
-    constexpr uint32_t BT = MfmaShape<WT>::BT, COLS = GATED ? BT / 2u : BT;
+    constexpr uint32_t BT = MfmaShape<WT, NORM, true>::BT, COLS = GATED ? BT / 2u : BT;
     const dim3 grid((g.n + COLS - 1u) / COLS, (g.m + BT - 1u) / BT);
-    constexpr size_t lds = MfmaShape<WT>::LDS_BYTES;
+    constexpr size_t lds = MFMA_LDS_BYTES<WT, NORM>;
     const auto kernel = matmul_mfma_kernel<VEC, ROPE, WT, NORM, GATED>;
     if constexpr (lds > 64u * 1024u - 512u) { /* from 64 KB on a kernel has to ask for its LDS first */
         static const hipError_t asked =
@@ -927,13 +999,13 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
         }
         return;
     }
-    /* One 128x128 workgroup lives on a compute unit, 256 at a time, and takes 3.3 times as long as a 64x64 one, which
-     * splits and reads twice as much per output: the large tile once its rounds are at least three quarters full
-     * (2048 x 512 . 512 x 1536, 192 tiles: 27.9 us against 28.6; 2048 columns, 256 tiles: 31.2 against 36.9; 1024
-     * columns, 128 tiles of K = 256: 15.2 against 11.4). */
+    /* One 128x128 workgroup lives on a compute unit, 256 at a time; of the 64x64 ones, which split and read twice as much per
+     * output, two, 512 at a time: the large tile once its rounds are at least nine sixteenths full, four and a half rounds
+     * of the small one for two (K = 512, small against large: 128 large tiles 16.8 us against 19.4, 144 23.0 against
+     * 20.0, 176 23.0 against 20.4, 256 26.9 against 20.6, 288 37.5 against 38.6, 352 43.1 against 39.4). */
     const uint32_t big_cols = g.b2 ? 64u : 128u;
     const uint64_t big_tiles = (uint64_t)((g.n + big_cols - 1u) / big_cols) * ((g.m + 127u) / 128u);
-    const bool big = big_tiles >= (big_tiles + 255u) / 256u * 192u;
+    const bool big = big_tiles >= (big_tiles + 255u) / 256u * 144u;
     if (big) {
         if (vec) launch_mfma<true, 2>(g, rope, s);
         else launch_mfma<false, 2>(g, rope, s);

@@ -1066,6 +1066,63 @@ def test_matmul_over_the_range_of_fp32(m, k, n, scale_a, scale_b, dev):
     assert _relative(out, a.double() @ b.double()) <= 3 * 2.0 ** -24 * max(k, 4) ** 0.5
 
 
+@pytest.mark.parametrize("m,k,n", [(300, 400, 500), (2048, 160, 1290), (70, 384, 4000), (1500, 385, 700)])
+def test_matmul_on_halves_out_of_range(m, k, n, dev):
+    """The matrix-core product takes its operands apart into f16 parts where runs of them lie within 2^-17 .. 4094 (a) and
+    2^-19 .. 1023 (b), and a tile that meets others starts again on bf16 parts: below, above, at zero, one value outside in
+    the last step, NaN and infinity.  Each against float64 in the 2-norm of a row: 2^-24 for each of at most
+    sqrt(K) roundings that count, and 2^-22 for the parts."""
+    import ctypes as C
+    import torch
+    lib = api.load()
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    view = lambda t: abi.tensor_view(t.data_ptr(), tuple(t.shape), abi.BLT_BACKEND_HIP)
+    bound = 2.0 ** -24 * k ** 0.5 + 2.0 ** -22
+
+    def product(a, b):
+        out = torch.zeros(m, n, device="cuda")
+        va, vb, vo = view(a), view(b), view(out)
+        lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+        torch.cuda.synchronize()
+        return out.double()
+
+    a0 = torch.randn(m, k, device="cuda", generator=gen)
+    b0 = torch.randn(k, n, device="cuda", generator=gen)
+    for what in ("as drawn", "a below", "b above", "a zero", "one late", "rows apart", "ends"):
+        a, b = a0.clone(), b0.clone()
+        if what == "a below":
+            a *= 1e-9
+        elif what == "b above":
+            b *= 1e4
+        elif what == "a zero":
+            a.zero_()
+        elif what == "one late":
+            a[m // 2, k - 1] = 1e5
+        elif what == "rows apart":
+            a[::3] *= 1e-8
+            b[:, ::5] *= 1e6
+        elif what == "ends":
+            a *= 2.0 ** -7
+            b *= 100.0
+        want = a.double() @ b.double()
+        error = (product(a, b) - want).norm(dim=1)
+        if what == "rows apart":                     # columns of two scales: each by itself
+            for cols in (slice(0, None, 5), slice(1, None, 5)):
+                part = (product(a, b) - want)[:, cols].norm(dim=1) / want[:, cols].norm(dim=1)
+                assert part.max().item() < 4 * bound, (what, part.max().item())
+        else:
+            assert (error <= 4 * bound * want.norm(dim=1)).all(), (what, (error / want.norm(dim=1)).max().item())
+    a, b = a0.clone(), b0.clone()
+    a[3, 5] = float("nan")
+    b[k - 2, 9] = float("inf")
+    got, clean = product(a, b), product(a0, b0)
+    assert torch.isnan(got[3]).all()
+    rows = torch.arange(m, device="cuda") != 3
+    assert torch.equal(got[rows, 9], a0[rows, k - 2].double().sign() * float("inf"))
+    cols = torch.arange(n, device="cuda") != 9
+    assert ((got - clean)[rows][:, cols].norm() / clean.norm()).item() < 4 * bound
+
+
 @pytest.mark.parametrize("m,k,n", [(1024, 1, 1024), (1500, 2, 700), (2048, 3, 2048), (1024, 4, 1024)])
 def test_matmul_of_few_products(m, k, n, dev):
     """One and two products an element are as close as fp32 makes them: a single one correctly rounded (uniform rounding
