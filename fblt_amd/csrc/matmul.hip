@@ -97,9 +97,10 @@ __device__ __forceinline__ void store4(const MatmulArgs &g, uint32_t row, uint32
  * NORM: the row statistic comes from the values on their way to LDS, the norm weight is multiplied in there, the row's
  * scale after the product: two vector instructions per value of a against a pass over a of its own (2048 rows of
  * 512: 14 us with sums in the reference's order).
- * GATED: the left quadrants are columns of a*b, the right ones the same columns of a*b2; the gates pass through LDS to
- * the waves that hold the other factor (2048 x 512 . 512 x (2 x 2048): two products and the activation 71 us,
- * this way 63). */
+ * GATED: the left quadrants are columns of a*b, the right ones the same columns of a*b2; they meet in LDS
+ * (2048 x 512 . 512 x (2 x 2048): two products and the activation 71 us, this way 63, with eight waves finishing 52).
+ * The end is shared by all eight waves and stores rows: a layer of 2048 rows and width 512 took 132.5 us with four waves
+ * storing from registers, of which the rotation alone 5.6, and takes 124.0. */
 template <int WT, bool NORM, bool F16>
 struct MfmaShape {
     static constexpr int BT = 64 * WT;          /* rows and columns of the tile */
@@ -111,7 +112,6 @@ struct MfmaShape {
         __bf16 a[PARTS][PART], b[PARTS][PART]; /* of either type */
     };
     static constexpr size_t LDS_BYTES = 2 * sizeof(Tiles);
-    static_assert(4 * WT * WT * 16 * 64 * sizeof(float) <= LDS_BYTES, "the second waves' sums pass through the tile buffers");
 };
 template <int WT, bool NORM>
 constexpr size_t MFMA_LDS_BYTES = std::max(MfmaShape<WT, NORM, true>::LDS_BYTES, MfmaShape<WT, NORM, false>::LDS_BYTES);
@@ -336,98 +336,103 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
         if (tid % SHARE == 0u) row_ss[tid / SHARE] = ss;
     }
 
-    /* the tile buffers are free */
-    float *meet = reinterpret_cast<float *>(mm_lds) + (wave & 3u) * (WT * WT * 16u * 64u) + lane;
-    if (kg == 1u) {
+    /* The tile buffers are free.  The two waves of a quadrant add their sums through one area, row by row: of the large tile each
+     * the half that it finishes (row tile `mine`), of the small one all to the first.  The finished quadrant goes back there,
+     * and all waves store rows of it: a lane holds a column's worth of rows, so from registers a store (and a load of the
+     * rotation or of the residual) would touch 32 rows with 32 bytes each. */
+    constexpr uint32_t SIDE = 32u * WT, PITCH = SIDE + 4u;
+    static_assert(4 * SIDE * PITCH * sizeof(float) <= MFMA_LDS_BYTES<WT, NORM>, "the results pass through the tile buffers");
+    const auto area = [&](uint32_t quadrant) { return reinterpret_cast<float *>(mm_lds) + quadrant * (SIDE * PITCH); };
+    const auto place = [&](uint32_t tile, int j, int q) {
+        return reinterpret_cast<float4 *>(area(wave & 3u) + (32u * tile + c) * PITCH + 32u * j + 8u * q + 4u * h);
+    };
+    const uint32_t mine = WT == 2 ? kg : 0u;
+    const bool finishes = WT == 2 || kg == 0u;
+    floatx16 sum[WT];
 #pragma unroll
-        for (int i = 0; i < WT * WT; i++)
+    for (int j = 0; j < WT; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) meet[(i * 16 + r) * 64] = acc[i / WT][i % WT][r];
-    }
-    __syncthreads();
-    if (kg == 1u) return;
-    bool bad = false;
+        for (int q = 0; q < 4; q++) {
+            float4 give;
+            float *const g4 = &give.x;
 #pragma unroll
-    for (int i = 0; i < WT * WT; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            acc[i / WT][i % WT][r] += meet[(i * 16 + r) * 64];
-            bad |= !isfinite(acc[i / WT][i % WT][r]);
-            acc[i / WT][i % WT][r] *= down;
+            for (int e = 0; e < 4; e++) {
+                g4[e] = WT == 2 && kg != 0u ? acc[0][j][4 * q + e] : acc[WT - 1][j][4 * q + e];
+                sum[j][4 * q + e] = WT == 2 && kg != 0u ? acc[WT - 1][j][4 * q + e] : acc[0][j][4 * q + e];
+            }
+            if (WT == 2 || kg == 1u) *place(WT == 2 ? 1u - kg : 0u, j, q) = give;
         }
+    __syncthreads();
     const bool gate_wave = GATED && wc == 1u;
-    const uint32_t wave_col = col0 + (GATED ? 0u : wc * (32u * WT));
-    if (__any(bad)) {
-        /* something is not finite, or too large for the scaled sums: the quadrant again on the fp32 instructions, which
-         * tell infinities from NaN */
+    const uint32_t wave_col = col0 + (GATED ? 0u : wc * SIDE);
+    if (finishes) {
+        bool bad = false;
 #pragma unroll
-        for (int i = 0; i < WT; i++)
+        for (int j = 0; j < WT; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float4 got = *place(mine, j, q);
+                const float *const g4 = &got.x;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    sum[j][4 * q + e] += g4[e];
+                    bad |= !isfinite(sum[j][4 * q + e]);
+                    sum[j][4 * q + e] *= down;
+                }
+            }
+        if (__any(bad)) {
+            /* something is not finite, or too large for the scaled sums: these rows again on the fp32 instructions, which
+             * tell infinities from NaN */
+            const float *ar = g.a + (size_t)min(row0 + SIDE * wr + 32u * mine + c, g.m - 1u) * g.lda;
 #pragma unroll
             for (int j = 0; j < WT; j++) {
-                const float *ar = g.a + (size_t)min(row0 + 32u * (WT * wr + i) + c, g.m - 1u) * g.lda;
                 const float *bc = (gate_wave ? g.b2 : g.b) + min(wave_col + 32u * j + c, g.n - 1u);
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-                for (uint32_t k0 = 0; k0 < g.k; k0 += 64u) { /* sums of 64, then their sum: closer than one chain (K = 512: 1.5e-7 against 4.1e-7) */
-                    floatx16 sum;
+                for (int r = 0; r < 16; r++) sum[j][r] = 0.f;
+                /* sums of 64, then their sum: closer than one chain (K = 512: 1.5e-7 against 4.1e-7) */
+                for (uint32_t k0 = 0; k0 < g.k; k0 += 64u) {
+                    floatx16 part;
 #pragma unroll
-                    for (int r = 0; r < 16; r++) sum[r] = 0.f;
+                    for (int r = 0; r < 16; r++) part[r] = 0.f;
                     for (uint32_t k = k0 + h; k < min(k0 + 64u, g.k) + h; k += 2u) { /* an odd K ends with a product of zeros */
                         float x = k < g.k ? ar[k] : 0.f;
                         const float y = k < g.k ? bc[(size_t)k * g.ldb] : 0.f;
                         if (NORM && k < g.k) x *= g.norm_w[k];
-                        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(y, x, sum, 0, 0, 0);
+                        part = __builtin_amdgcn_mfma_f32_32x32x2f32(y, x, part, 0, 0, 0);
                     }
-                    acc[i][j] += sum;
+                    sum[j] += part;
                 }
             }
-    }
-    if constexpr (NORM) {
-#pragma unroll
-        for (int i = 0; i < WT; i++) {
-            const float scale = 1.0f / sqrtf(row_ss[32u * (WT * wr + i) + c] / (float)g.k + 1e-6f); /* reductions_cpu.c:345-346 */
-#pragma unroll
-            for (int j = 0; j < WT; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][j][r] *= scale;
         }
-    }
-    MatmulArgs to = g;
-    if constexpr (GATED) {
-        if (g.out2 == nullptr) { /* the waves of the second group have left: these four meet */
-            if (gate_wave) {
-#pragma unroll
-                for (int i = 0; i < WT * WT; i++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) meet[(i * 16 + r) * 64] = acc[i / WT][i % WT][r];
-            }
-            __syncthreads();
-            if (gate_wave) return;
-            const float *gates = meet + WT * WT * 16u * 64u; /* of the wave to the right */
-#pragma unroll
-            for (int i = 0; i < WT * WT; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[i / WT][i % WT][r] = silu_times(gates[(i * 16 + r) * 64], acc[i / WT][i % WT][r]);
-        } else if (gate_wave) {
-            to.out = g.out2, to.residual = nullptr;
-        }
-    }
-
-    /* lane (h, c) holds out[row0 + 32*(WT*wr + i) + c][wave_col + 32*j + 8*q + 4*h + 0..3] in acc[i][j][4q..4q+3] */
-    const bool vst = VEC && g.n % 4u == 0u && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(to.out) & 15u) == 0u) &&
-                     ((reinterpret_cast<uintptr_t>(to.residual) & 15u) == 0u);
-#pragma unroll
-    for (int i = 0; i < WT; i++) {
-        const uint32_t row = row0 + 32u * (WT * wr + i) + c;
-        if (row >= g.m) continue;
+        const float scale = NORM ? 1.0f / sqrtf(row_ss[SIDE * wr + 32u * mine + c] / (float)g.k + 1e-6f) : 1.0f; /* reductions_cpu.c:345-346 */
 #pragma unroll
         for (int j = 0; j < WT; j++)
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                store4<ROPE>(to, row, wave_col + 32u * j + 8u * q + 4u * h,
-                             make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                                         acc[i][j][4 * q + 3]),
-                             vst);
+                *place(mine, j, q) = make_float4(sum[j][4 * q + 0] * scale, sum[j][4 * q + 1] * scale, sum[j][4 * q + 2] * scale,
+                                                 sum[j][4 * q + 3] * scale);
+    }
+    __syncthreads();
+
+    MatmulArgs to = g;
+    const bool joined = GATED && g.out2 == nullptr; /* four waves a pair of quadrants then, two a quadrant else */
+    if (gate_wave && !joined) to.out = g.out2, to.residual = nullptr;
+    const bool vst = VEC && g.n % 4u == 0u && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(to.out) & 15u) == 0u) &&
+                     ((reinterpret_cast<uintptr_t>(to.residual) & 15u) == 0u);
+    constexpr uint32_t PER = SIDE / 4u, ROWS = 64u / PER; /* lanes a row, rows at once */
+    const uint32_t share = joined ? SIDE / 4u : SIDE / 2u, first = (joined ? 2u * wc + kg : kg) * share;
+    const float *const from = area(joined ? 2u * wr : wave & 3u), *const gates = area(2u * wr + 1u);
+#pragma unroll
+    for (uint32_t r = 0; r < SIDE / 2u; r += ROWS) {
+        if (r >= share) break;
+        const uint32_t at = first + r + lane / PER, col = lane % PER * 4u;
+        const uint32_t row = row0 + SIDE * wr + at;
+        float4 v = *reinterpret_cast<const float4 *>(from + at * PITCH + col);
+        if (joined) {
+            const float4 gate = *reinterpret_cast<const float4 *>(gates + at * PITCH + col);
+            v.x = silu_times(gate.x, v.x), v.y = silu_times(gate.y, v.y), v.z = silu_times(gate.z, v.z), v.w = silu_times(gate.w, v.w);
+        }
+        if (row < g.m) store4<ROPE>(to, row, wave_col + col, v, vst);
     }
 }
 
