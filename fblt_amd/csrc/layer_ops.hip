@@ -229,43 +229,31 @@ extern "C" void blt_swiglu_forward_hip(const blt_tensor *gate, const blt_tensor 
 namespace {
 
 /* Prompt prefill through the step: `n` (> 32) new rows per sequence, causal.  The step kernels take
- * 32 rows at a time, one slice after the other with few workgroups each; here the rows are staged
- * once -- Q rotated into a scratch buffer, K rotated and V written through to the slabs, one small
- * launch -- and the attention of all of them runs as one batch of (sequence, head) problems of the
- * prefill kernels with the causal diagonal moved by the cached length (csrc/infer/kv_cache.c:
- * 229-236: j <= base + r, base + r - j < window).  Needs the lengths on the host. */
-__global__ __launch_bounds__(256) void kv_chunk_stage_kernel(const float *__restrict__ qkv, float *__restrict__ q_rot,
-                                                             float *__restrict__ cache_k, float *__restrict__ cache_v,
-                                                             const uint32_t *__restrict__ self_len,
-                                                             const float *__restrict__ rope_cos,
-                                                             const float *__restrict__ rope_sin, uint32_t n, uint32_t E,
-                                                             uint32_t hd, uint64_t max_seq_len) {
-    const uint32_t row = blockIdx.x, b = row / n, r = row % n;
-    const uint32_t pos = self_len[b] + r;
-    const float *src = qkv + (size_t)row * 3u * E;
-    float *kd = cache_k + ((size_t)b * max_seq_len + pos) * E;
-    float *vd = cache_v + ((size_t)b * max_seq_len + pos) * E;
-    for (uint32_t col = 4u * threadIdx.x; col < E; col += 1024u) {
-        const size_t at = (size_t)pos * (hd / 2u) + (col % hd) / 2u;
-        const float4 q4 = *reinterpret_cast<const float4 *>(src + col);
-        const float4 k4 = *reinterpret_cast<const float4 *>(src + E + col);
-        *reinterpret_cast<float4 *>(q_rot + (size_t)row * E + col) = rope_rotate4(q4, rope_cos + at, rope_sin + at);
-        *reinterpret_cast<float4 *>(kd + col) = rope_rotate4(k4, rope_cos + at, rope_sin + at);
-        *reinterpret_cast<float4 *>(vd + col) = *reinterpret_cast<const float4 *>(src + 2u * E + col);
-    }
-}
-
-void long_chunk_attention(const blt_kv_attn_cache *cache, const float *qkv, const float *rope_cos,
-                          const float *rope_sin, size_t rope_positions, size_t n, const size_t *host_base,
-                          float *combined, blt_arena *arena) {
-    const size_t E = cache->embed_dim, H = cache->num_heads, hd = E / H, rows = cache->batch * n;
-    float *q_rot = (float *)blt_arena_alloc(arena, rows * E * sizeof(float), 64);
+ * 32 rows at a time, one slice after the other with few workgroups each; here the QKV product of all rows leaves Q rotated
+ * in a scratch buffer and writes K, rotated, and V through to the slabs, and the attention runs as one batch of (sequence,
+ * head) problems of the prefill kernels with the causal diagonal moved by the cached length (csrc/infer/kv_cache.c:
+ * 229-236: j <= base + r, base + r - j < window).  Needs the lengths on the host, and in cache->self_len.
+ * (A launch of its own between the product and the attention took 2.8 us and a gap of 0.8 for 512 rows of 128.) */
+void long_chunk_qkv(const blt_kv_attn_cache *cache, const float *rows_in, const float *qkv_w, const float *norm_w, float *q_rot,
+                    const float *rope_cos, const float *rope_sin, size_t rope_positions, size_t n, const size_t *host_base) {
+    const size_t E = cache->embed_dim;
     for (size_t b = 0; b < cache->batch; b++)
         BLT_REQUIRE(host_base[b] + n <= rope_positions && host_base[b] + n <= cache->max_seq_len,
                     "blt_kv_decode_step: positions exceed the rotary tables or the cache");
-    blt_launch("kv_chunk_stage", kv_chunk_stage_kernel, dim3((unsigned)rows), dim3(256), 0, 0, qkv, q_rot, cache->self_k,
-               cache->self_v, cache->self_len, rope_cos, rope_sin, (uint32_t)n, (uint32_t)E, (uint32_t)hd,
-               (uint64_t)cache->max_seq_len);
+    MatmulArgs g;
+    std::memset(&g, 0, sizeof(g));
+    g.a = rows_in, g.b = qkv_w, g.norm_w = norm_w, g.out = q_rot;
+    g.m = (uint32_t)(cache->batch * n), g.k = (uint32_t)E, g.n = (uint32_t)(3 * E);
+    g.lda = g.ldo = (uint32_t)E, g.ldb = (uint32_t)(3 * E);
+    g.rope_cos = rope_cos, g.rope_sin = rope_sin, g.rope_cols = (uint32_t)(2 * E), g.head_dim = (uint32_t)(E / cache->num_heads);
+    g.stage_k = cache->self_k, g.stage_v = cache->self_v, g.stage_len = cache->self_len;
+    g.stage_slab_rows = cache->max_seq_len, g.stage_n = (uint32_t)n;
+    g.tolerant = step_tolerant();
+    matmul_f32_launch(g, 0);
+}
+
+void long_chunk_attention(const blt_kv_attn_cache *cache, const float *q_rot, size_t n, const size_t *host_base, float *combined) {
+    const size_t E = cache->embed_dim, H = cache->num_heads, hd = E / H;
     std::vector<blt_attention_problem> pr(cache->batch * H);
     const float scale = 1.0f / sqrtf((float)hd);
     for (size_t b = 0; b < cache->batch; b++) {
@@ -348,32 +336,36 @@ void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_wei
     probe.tolerant = step_tolerant();
     /* self-attention block, kv_cache.c:326-394 */
     probe.n = (uint32_t)(3 * E);
-    if (matmul_takes_norm(probe)) {
-        gemm(rows_in, f32(w->attn_qkv_w), qkv, rows, E, 3 * E, nullptr, nullptr, f32(w->norm1_weight));
-    } else {
-        rmsnorm_launch(rows_in, f32(w->norm1_weight), normed, rows, E);
-        gemm(normed, f32(w->attn_qkv_w), qkv, rows, E, 3 * E);
+    const bool chunk = host_base != nullptr && n > 32 && step_kind == BLT_KV_STEP_CAUSAL && commit == 0 && dev_positions == nullptr &&
+                       (E / cache->num_heads) % 4 == 0;
+    const float *qkv_in = rows_in, *qkv_norm = f32(w->norm1_weight);
+    if (!matmul_takes_norm(probe)) {
+        rmsnorm_launch(rows_in, qkv_norm, normed, rows, E);
+        qkv_in = normed, qkv_norm = nullptr;
     }
-    if (host_base != nullptr && n > 32 && step_kind == BLT_KV_STEP_CAUSAL && commit == 0 && dev_positions == nullptr &&
-        (E / cache->num_heads) % 4 == 0) {
-        long_chunk_attention(cache, qkv, rope_cos, rope_sin, rope_positions, n, host_base, combined, arena);
-    } else if (host_base != nullptr && commit == 0) {
-        /* the caller keeps the lengths: they go into the kernel arguments */
-        std::vector<uint32_t> lens(cache->batch);
-        for (size_t b = 0; b < cache->batch; b++) lens[b] = (uint32_t)host_base[b];
-        if (dev_positions != nullptr) { /* rows rotated at their own positions first, then a plain step */
-            BLT_REQUIRE((E / cache->num_heads) % 4 == 0, "blt_kv_block_step: explicit row positions need head_dim %% 4 == 0");
-            blt_launch("rope_rows_at", rope_rows_at_kernel, dim3((unsigned)rows), dim3(256), 0, 0, qkv, dev_positions,
-                       rope_cos, rope_sin, (uint32_t)E, (uint32_t)(E / cache->num_heads));
-            blt_kv_attend_step_lens_hip(cache, lens.data(), qkv, 3 * E, qkv + E, 3 * E, qkv + 2 * E, 3 * E, nullptr,
-                                        nullptr, 0, combined, E, n, step_kind);
-        } else {
-            blt_kv_attend_step_lens_hip(cache, lens.data(), qkv, 3 * E, qkv + E, 3 * E, qkv + 2 * E, 3 * E, rope_cos,
-                                        rope_sin, rope_positions, combined, E, n, step_kind);
-        }
+    if (chunk) {
+        long_chunk_qkv(cache, qkv_in, f32(w->attn_qkv_w), qkv_norm, qkv, rope_cos, rope_sin, rope_positions, n, host_base);
+        long_chunk_attention(cache, qkv, n, host_base, combined);
     } else {
-        blt_kv_rope_attend_step_hip(cache, qkv, 3 * E, qkv + E, 3 * E, qkv + 2 * E, 3 * E, rope_cos, rope_sin,
-                                    rope_positions, combined, E, n, step_kind, commit, max_len_hint);
+        gemm(qkv_in, f32(w->attn_qkv_w), qkv, rows, E, 3 * E, nullptr, nullptr, qkv_norm);
+        if (host_base != nullptr && commit == 0) {
+            /* the caller keeps the lengths: they go into the kernel arguments */
+            std::vector<uint32_t> lens(cache->batch);
+            for (size_t b = 0; b < cache->batch; b++) lens[b] = (uint32_t)host_base[b];
+            if (dev_positions != nullptr) { /* rows rotated at their own positions first, then a plain step */
+                BLT_REQUIRE((E / cache->num_heads) % 4 == 0, "blt_kv_block_step: explicit row positions need head_dim %% 4 == 0");
+                blt_launch("rope_rows_at", rope_rows_at_kernel, dim3((unsigned)rows), dim3(256), 0, 0, qkv, dev_positions,
+                           rope_cos, rope_sin, (uint32_t)E, (uint32_t)(E / cache->num_heads));
+                blt_kv_attend_step_lens_hip(cache, lens.data(), qkv, 3 * E, qkv + E, 3 * E, qkv + 2 * E, 3 * E, nullptr,
+                                            nullptr, 0, combined, E, n, step_kind);
+            } else {
+                blt_kv_attend_step_lens_hip(cache, lens.data(), qkv, 3 * E, qkv + E, 3 * E, qkv + 2 * E, 3 * E, rope_cos,
+                                            rope_sin, rope_positions, combined, E, n, step_kind);
+            }
+        } else {
+            blt_kv_rope_attend_step_hip(cache, qkv, 3 * E, qkv + E, 3 * E, qkv + 2 * E, 3 * E, rope_cos, rope_sin,
+                                        rope_positions, combined, E, n, step_kind, commit, max_len_hint);
+        }
     }
     if (rows > 32 || step_tolerant()) { /* up to 32 rows the products keep the reference's order of sums unless told otherwise */
         BlockTailArgs t;

@@ -44,6 +44,15 @@ struct MatmulArgs {
     const uint32_t *cross_hi;
     uint32_t cross_rows_per_seq, cross_slab_rows, cross_head_dim;
     float cross_scale;
+    /* Optional destination of a packed QKV product (n = 3 E, rope_cols = 2 E): row stage_n * b + r is the new row r of
+     * sequence b, at position stage_len[b] + r of the rotary tables (which then have a row per position, not per row).  The
+     * rotated Q rows go to out (ldo = E), the rotated K rows and the V rows to the slabs [batch, stage_slab_rows, E]; all
+     * 16-byte aligned. */
+    float *stage_k;
+    float *stage_v;
+    const uint32_t *stage_len;
+    uint64_t stage_slab_rows;
+    uint32_t stage_n;
     /* Products of up to 32 rows normally run on the thread-per-column kernel, whose sums follow the
      * reference's order (bit-identical results) at the price of a serial chain of k additions.
      * tolerant != 0: the caller accepts fp32-tolerance results for such shapes too, and they go to

@@ -59,6 +59,17 @@ constexpr int TM = 64, TN = 64, TK = 32; /* smallest workgroup tile of the mfma 
  * optional rotation, optional residual, store with bounds. */
 template <bool ROPE>
 __device__ __forceinline__ void store4(const MatmulArgs &g, uint32_t row, uint32_t col, float4 v, bool vec_ok) {
+    if (ROPE && g.stage_k) { /* new rows of a cache: no residual */
+        if (col >= g.n) return;
+        const uint32_t E = g.n / 3u, part = col / E, at = col % E, b = row / g.stage_n, pos = g.stage_len[b] + row % g.stage_n;
+        if (part < 2u) {
+            const size_t turn = (size_t)pos * (g.head_dim / 2u) + (at % g.head_dim) / 2u;
+            v = rope_rotate4(v, g.rope_cos + turn, g.rope_sin + turn);
+        }
+        float *const to = part == 0u ? g.out + (size_t)row * E : (part == 1u ? g.stage_k : g.stage_v) + ((size_t)b * g.stage_slab_rows + pos) * E;
+        *reinterpret_cast<float4 *>(to + at) = v;
+        return;
+    }
     if (ROPE && col < g.rope_cols) {
         /* columns col..col+3 are pairs (col % head_dim)/2 and the next one of the row's position */
         const size_t at = (size_t)row * (g.head_dim / 2u) + (col % g.head_dim) / 2u;

@@ -2161,6 +2161,13 @@ def test_kv_decode_step_past_one_launch(batch, n, case, oracle, dev):
     assert all("kv_step_resident" not in names for names in launched), launched
 
 
+@pytest.mark.parametrize("batch,n,case,product", [(2, 33, 2, "matmul_splitk"), (24, 64, 4, "matmul_mfma")])
+def test_kv_decode_step_of_chunks_staged_by_their_product(batch, n, case, product, oracle, dev):
+    """Chunks of more than 32 rows: the QKV product leaves Q rotated and writes K and V to the slabs, from either kernel."""
+    launched = _decode_steps(batch, n, RESIDENT_CASES[case], 660 + case, oracle)
+    assert all(product in names and "kv_chunk_stage" not in names for names in launched), launched
+
+
 @pytest.mark.parametrize("batch,n,case", [(1, 1, 2), (9, 8, 2), (33, 1, 0)])
 def test_kv_decode_step_of_rows_whose_norm_overflows(batch, n, case, oracle, dev):
     """Input rows of 1e20: their sum of squares is infinite and the normalised row zero, in the one-launch form as in
