@@ -638,6 +638,8 @@ void refresh_cross_seq(blt_kv_cache *cache, size_t seq, const blt_tensor *patch_
     const blt_local_decoder *dec = cache->decoder;
     const size_t E = cache->embed_dim, L = dec->config.num_layers;
     const size_t first = from_patch * cache->k, count = (num_patches - from_patch) * cache->k;
+    MatmulArgs waiting; /* two layers share a launch where they can */
+    bool waits = false;
     for (size_t l = 0; l < L; l++) {
         if (!cross_fires(&dec->config, l)) continue;
         const blt_local_layer_storage *s = &dec->layers[l];
@@ -654,8 +656,17 @@ void refresh_cross_seq(blt_kv_cache *cache, size_t seq, const blt_tensor *patch_
         g.b2 = (const float *)s->cross_weight_v.data;
         g.out2 = (float *)cache->cross_v[l].data + row0 * E;
         g.tolerant = step_tolerant();
-        matmul_f32_launch(g, 0); /* K and V in one pass over the patch rows */
+        if (waits) { /* K and V in one pass over the patch rows */
+            if (matmul_pair_ok(waiting, g)) {
+                matmul_f32_launch_pair(waiting, g, 0);
+            } else {
+                matmul_f32_launch(waiting, 0);
+                matmul_f32_launch(g, 0);
+            }
+        }
+        waiting = g, waits = !waits;
     }
+    if (waits) matmul_f32_launch(waiting, 0);
     std::memcpy(&cache->cached_patches[seq * cache->max_seq_len + from_patch], &patches[from_patch],
                 (num_patches - from_patch) * sizeof(blt_patch_info)); /* kv_cache.c:154-157 */
     HIP_CHECK_LAUNCH("blt_kv_cache_refresh_cross");

@@ -88,7 +88,7 @@ struct BlockTailArgs {
 };
 /* false: not for this shape, nothing was launched */
 bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s);
-/* g0 (plain) and g1 (two weight matrices, two outputs) in one launch; only when matmul_pair_ok says so */
+/* g0 (plain, or like g1) and g1 (two weight matrices, two outputs) in one launch; only when matmul_pair_ok says so */
 bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1);
 void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStream_t s);
 /* the cross-attention epilogue for this shape and g.cross_head_dim, no other epilogue set */

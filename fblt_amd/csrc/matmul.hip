@@ -669,16 +669,16 @@ __global__ __launch_bounds__(64 * NW, 2) void matmul_splitk_kernel(MatmulArgs g)
 }
 
 /* Two independent products in one launch: the tile rows of the second are
- * stacked under those of the first (rows0 tile rows); the second may carry a
- * second weight matrix.  For pairs of small products whose launches would
+ * stacked under those of the first (rows0 tile rows); the second carries a
+ * second weight matrix, the first too if BOTH.  For pairs of small products whose launches would
  * otherwise each pay the fixed launch cost. */
-template <bool VEC>
+template <bool VEC, bool BOTH>
 __global__ __launch_bounds__(256, 2) void matmul_splitk_pair_kernel(MatmulArgs g0, MatmulArgs g1, uint32_t rows0) {
     __shared__ float part[8][16][64];
     __shared__ float part_ss[4][32];
     if (blockIdx.y < rows0) { /* uniform per workgroup */
         if (blockIdx.x * 32u >= g0.n) return;
-        splitk_tile<VEC, false, false>(g0, blockIdx.x, blockIdx.y, part, part_ss);
+        splitk_tile<VEC, false, BOTH>(g0, blockIdx.x, blockIdx.y, part, part_ss);
     } else {
         if (blockIdx.x * 32u >= g1.n) return;
         splitk_tile<VEC, false, true>(g1, blockIdx.x, blockIdx.y - rows0, part, part_ss);
@@ -940,7 +940,7 @@ bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1) {
                !(g.rope_cos != nullptr && g.rope_cols > 0);
     };
     /* the first product may normalise its rows on the way (four waves: the tile code's own sums) */
-    return plain(g0) && plain(g1) && g0.b2 == nullptr && g1.b2 != nullptr && g1.out2 != nullptr && !g1.norm_w;
+    return plain(g0) && plain(g1) && (g0.b2 == nullptr || g0.out2 != nullptr) && g1.b2 != nullptr && g1.out2 != nullptr && !g1.norm_w;
 }
 
 void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStream_t s) {
@@ -948,9 +948,10 @@ void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStrea
     const uint32_t rows0 = (g0.m + 31u) / 32u, rows1 = (g1.m + 31u) / 32u;
     const uint32_t cols = (std::max(g0.n, g1.n) + 31u) / 32u;
     const dim3 grid(cols, rows0 + rows1);
-    if (vec_ok(g0) && vec_ok(g1))
-        blt_launch("matmul_splitk", matmul_splitk_pair_kernel<true>, grid, dim3(256), 0, s, g0, g1, rows0);
-    else blt_launch("matmul_splitk", matmul_splitk_pair_kernel<false>, grid, dim3(256), 0, s, g0, g1, rows0);
+    const auto launch = [&](auto kernel) { blt_launch("matmul_splitk", kernel, grid, dim3(256), 0, s, g0, g1, rows0); };
+    const bool vec = vec_ok(g0) && vec_ok(g1);
+    if (g0.b2) launch(vec ? matmul_splitk_pair_kernel<true, true> : matmul_splitk_pair_kernel<false, true>);
+    else launch(vec ? matmul_splitk_pair_kernel<true, false> : matmul_splitk_pair_kernel<false, false>);
 }
 
 namespace {

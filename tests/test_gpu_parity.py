@@ -2037,6 +2037,35 @@ def test_kv_decode_step_long_prefill(window, oracle, dev):
         lib.blt_arena_destroy(arena)
 
 
+@pytest.mark.parametrize("L,P,launches", [(3, 40, 2), (2, 70, 1), (2, 32, 2)])   # 33 rows and more: two layers a launch
+def test_refresh_of_two_layers_in_one_launch(L, P, launches, oracle, dev):
+    import torch
+    from fblt_amd import decoder
+    lib = api.load()
+    c = dict(E=128, H=4, XH=4, L=L, hidden=64, V=16, max_len=160, k=1, window=0, all_layers=True, placement=0)
+    rs = np.random.RandomState(77 + P)
+    host, device = _decoders(oracle, c, 78)
+    mine = decoder.HostCache(host, c["max_len"])
+    arena = lib.blt_arena_create(64 << 20, abi.BLT_BACKEND_HIP)
+    try:
+        cache = lib.blt_kv_cache_create(arena, device.ptr, c["max_len"])
+        patches = decoder.patch_table([2] * P)
+        patch_in = rs.randn(P, c["E"]).astype(np.float32)
+        tp = torch.from_numpy(patch_in).cuda()
+        vp = _dev_tensor(tp)
+        lib.blt_hip_profile_begin()
+        lib.blt_kv_cache_refresh_cross(cache, C.byref(vp), patches, P, 0, arena)
+        assert sum(e[0] for e in api.profile_end().values()) == launches
+        lib.blt_backend_pass_sync_hip()
+        assert oracle.orc_kv_cache_refresh_cross(mine.ptr, 0, binding.fptr(patch_in.reshape(-1)), P, 0) == 0
+        for name in ("cross_k", "cross_v"):
+            for l in range(L):
+                assert_close(_tier(lib, cache, name, l, P, c["E"]), mine.tiers[name][l][:P], "%s[%d]" % (name, l))
+        lib.blt_kv_cache_destroy(cache)
+    finally:
+        lib.blt_arena_destroy(arena)
+
+
 def _decode_steps(batch, n, c, seed, oracle, row_scale=1.0, before_sync=None):
     """Two steps of a batched cache against the restated step run sequence by sequence; the kernels each step launched.
     before_sync(logits): called after each step, before the library synchronises."""
