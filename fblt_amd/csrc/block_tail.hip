@@ -18,8 +18,8 @@
  * bf16 parts costs more than the matrix time it saves.
  *
  * Bound: latency.  E = 128, hidden 512, 512 rows: 10.9 us in the kernel trace, of which (parts left out, one after the other)
- * an empty launch with all requests 3, the barriers and the partial sums through LDS 2.5 (0 would need a whole row's
- * product in one wave), fp32 matrix time of the compute unit 2.2, the ticket 1.9.  Whole blocks, three launches -> this: 128 rows
+ * an empty launch with all requests 3, the barriers and the partial sums through LDS 2.5, fp32 matrix time of the compute
+ * unit 2.2, the ticket 1.9.  Whole blocks, three launches -> this: 128 rows
  * 25.0 -> 17.3 us, 512 rows 29.5 -> 21.6; E = 64 22.7 -> 13.9 and 26.1 -> 17.2; E = 256, 128 rows 31.5 -> 28.4.
  * Relative error of the block against float64: 1.57e-7 -> 1.45e-7 (E = 128, 128 rows), 1.64e-7 -> 1.47e-7 (256 of 256).
  */
@@ -39,8 +39,8 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 /* Columns go in groups of 64, a wave per (group, share of the terms): lane (g, c) loads four consecutive columns
  * 4 c .. 4 c + 3 of row 4 g + t of every block of 16 terms, 16 bytes, and column j of the four is the tile of every fourth
  * column from j on.  A load instruction costs a compute unit's vector memory path about the same whatever it
- * brings: with a tile of 16 consecutive columns a wave and 4 bytes a lane the 690 loads of a workgroup were what the launch
- * waited for. */
+ * brings: with a tile of 16 consecutive columns a wave and 4 bytes a lane, four times the loads, a block of 512 rows took
+ * 23.3 us instead of 21.6. */
 template <int E_, int NW_, bool PROJ_>
 struct TailShape {
     static constexpr int E = E_, HS = 64, NW = NW_, THREADS = 64 * NW;
@@ -215,6 +215,116 @@ __global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArg
     if (row0 + f_row < a.rows) *reinterpret_cast<rowpart *>(a.out + f_at) = out;
 }
 
+/* A cross block of 16 rows a workgroup: norm, query projection, the rows' attention, output projection, residual
+ * (csrc/models/cross_attention.c:101-157, csrc/infer/kv_cache.c:303-324).  A row sees few keys, a handful of bytes or the
+ * patches of its own window, so the rows of K and V come straight from memory, eight keys in flight, the first before there
+ * is a query, to the threads that hold the query: EPT columns each, a head's threads neighbours.  Running maximum over
+ * finite scores; a score that is not finite weighs nothing, a row without keys gives zeros.
+ *
+ * Bound: latency: weights and keys on their way, two products with their partial sums through LDS; 7.2 us in the kernel trace
+ * for 512 rows of 128 that see a patch each, 9.4 for 128 rows of up to 16 bytes (a further trip to memory for every eight
+ * keys past the first), against 5.6 + 4.3 and 6.1 + 4.2 with a gap as two launches. */
+constexpr uint32_t CROSS_ROWS = 16384; /* the most measured: a prompt of 32 x 512 rows 375.7 -> 343.1 us, of 1 x 64 68.8 -> 62.9 */
+constexpr uint32_t CROSS_KEYS = 4;
+
+template <typename Shape>
+__global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockArgs a) {
+    using Proj = typename Shape::Proj;
+    constexpr int E = Shape::E, ROW = Shape::ROW, EPT = Shape::EPT;
+    static_assert(EPT == 4, "a thread holds 16 bytes of a row");
+    __shared__ __attribute__((aligned(16))) float rows[16 * ROW], part[Proj::PART];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr uint32_t TPR = E / EPT;
+    const uint32_t row0 = 16u * blockIdx.x, f_row = tid / TPR, f_col = EPT * (tid % TPR);
+    const uint32_t row = min(row0 + f_row, a.rows - 1u);
+    const size_t f_at = (size_t)row * E + f_col;
+    const uint32_t group = wave % Proj::GROUPS, term = wave / Proj::GROUPS * (16 * Proj::BLOCKS);
+    float *const mine = part + wave / Proj::GROUPS * (16 * Proj::PITCH) + 64u * group;
+
+    floatx4 wq[4 * Proj::BLOCKS], wp[4 * Proj::BLOCKS];
+    floatx4 x = *reinterpret_cast<const floatx4 *>(a.x + f_at), norm_w = {1.f, 1.f, 1.f, 1.f}, resid = {0.f, 0.f, 0.f, 0.f};
+    if (a.norm_w) norm_w = *reinterpret_cast<const floatx4 *>(a.norm_w + f_col);
+    request<Proj::BLOCKS>(wq, a.wq + 64u * group, E, term);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t lo = a.lo[row], hi = a.hi[row];
+    constexpr uint32_t KEYS = CROSS_KEYS;
+    const uint32_t lanes = a.head_dim / EPT; /* of a head: a power of two up to TPR */
+    const size_t slab = (size_t)(row / a.rows_per_seq) * a.slab_rows * E + f_col;
+    struct Keys {
+        floatx4 k[KEYS], v[KEYS];
+    } even, odd; /* taking turns */
+    const auto fetch = [&](Keys &to, uint32_t j) __attribute__((always_inline)) { /* past the last key: that one again */
+        if (j >= hi) return;
+#pragma unroll
+        for (uint32_t u = 0; u < KEYS; u++) to.k[u] = *reinterpret_cast<const floatx4 *>(a.k + slab + (size_t)min(j + u, hi - 1u) * E);
+#pragma unroll
+        for (uint32_t u = 0; u < KEYS; u++) to.v[u] = *reinterpret_cast<const floatx4 *>(a.v + slab + (size_t)min(j + u, hi - 1u) * E);
+    };
+    if (a.residual) resid = *reinterpret_cast<const floatx4 *>(a.residual + f_at);
+    request<Proj::BLOCKS>(wp, a.proj + 64u * group, E, term);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(even, lo); /* the keys do not wait for the query */
+    fetch(odd, lo + KEYS);
+    __builtin_amdgcn_sched_barrier(0);
+
+    if (a.norm_w) {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < EPT; i++) ss += x[i] * x[i];
+        ss = key_sum<TPR>(ss);
+        x *= 1.0f / sqrtf(ss / (float)E + 1e-6f) * norm_w; /* reductions_cpu.c:345-346 */
+    }
+    *reinterpret_cast<floatx4 *>(rows + f_row * ROW + f_col) = x;
+    __syncthreads();
+    multiply<Proj::BLOCKS, Proj::PITCH>(rows, ROW, term, wq, mine);
+    __syncthreads();
+    float q[EPT];
+    gather<Proj::SHARES, Proj::PITCH, EPT>(part + f_row * Proj::PITCH + f_col, q);
+
+    float m = -__builtin_huge_valf(), l = 0.f;
+    floatx4 o = {0.f, 0.f, 0.f, 0.f};
+    const auto attend = [&](const Keys &from, uint32_t j) __attribute__((always_inline)) {
+        float s[KEYS], top = m;
+#pragma unroll
+        for (uint32_t u = 0; u < KEYS; u++) s[u] = q[0] * from.k[u][0] + q[1] * from.k[u][1] + q[2] * from.k[u][2] + q[3] * from.k[u][3];
+        for (uint32_t d = 1u; d < lanes; d *= 2u)
+#pragma unroll
+            for (uint32_t u = 0; u < KEYS; u++) s[u] += __shfl_xor(s[u], (int)d, 64);
+#pragma unroll
+        for (uint32_t u = 0; u < KEYS; u++) {
+            s[u] *= a.scale;
+            if (j + u >= hi || !isfinite(s[u])) s[u] = -__builtin_huge_valf();
+            top = fmaxf(top, s[u]);
+        }
+        if (top == -__builtin_huge_valf()) return; /* nothing of weight yet */
+        const float fade = expf(m - top);
+        m = top, l *= fade, o *= fade;
+#pragma unroll
+        for (uint32_t u = 0; u < KEYS; u++) {
+            const float e = expf(s[u] - top);
+            if (e == 0.f) continue; /* its value row may be anything */
+            l += e, o += e * from.v[u];
+        }
+    };
+    for (uint32_t j = lo; j < hi; j += 2u * KEYS) { /* the same for a row's threads */
+        attend(even, j);
+        fetch(even, j + 2u * KEYS);
+        if (j + KEYS < hi) attend(odd, j + KEYS);
+        fetch(odd, j + 3u * KEYS);
+    }
+    o *= l > 0.f ? 1.0f / l : 0.f;
+    *reinterpret_cast<floatx4 *>(rows + f_row * ROW + f_col) = o;
+    __syncthreads();
+    multiply<Proj::BLOCKS, Proj::PITCH>(rows, ROW, term, wp, mine);
+    __syncthreads();
+    float sum[EPT];
+    gather<Proj::SHARES, Proj::PITCH, EPT>(part + f_row * Proj::PITCH + f_col, sum);
+#pragma unroll
+    for (int i = 0; i < EPT; i++) resid[i] += sum[i];
+    if (row0 + f_row < a.rows) *reinterpret_cast<floatx4 *>(a.out + f_at) = resid;
+}
+
 template <typename Shape>
 void launch_tail(const BlockTailArgs &a, dim3 grid, hipStream_t s) {
     blt_launch("block_tail", block_tail_kernel<Shape>, grid, dim3(Shape::THREADS), 0, s, a);
@@ -260,5 +370,23 @@ bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s) {
         a.x = a.resid;
         launch_tail<TailShape<256, 16, false>>(a, grid, s);
     }
+    return true;
+}
+
+bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim) {
+    if ((embed_dim != 64u && embed_dim != 128u) || a.rows == 0u) return false;
+    /* a head's columns are spread over neighbouring threads, four each */
+    if (a.head_dim < 4u || a.head_dim > embed_dim || (a.head_dim & (a.head_dim - 1u)) != 0u) return false;
+    for (const void *p : {(const void *)a.x, (const void *)a.norm_w, (const void *)a.wq, (const void *)a.k, (const void *)a.v,
+                          (const void *)a.proj, (const void *)a.residual, (const void *)a.out})
+        if ((reinterpret_cast<uintptr_t>(p) & 15u) != 0u) return false;
+    return a.rows <= CROSS_ROWS;
+}
+
+bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t s) {
+    if (!cross_block_ok(a, embed_dim)) return false;
+    const dim3 grid((a.rows + 15u) / 16u);
+    if (embed_dim == 64u) blt_launch("cross_block", cross_block_kernel<TailShape<64, 4, true>>, grid, dim3(256), 0, s, a);
+    else blt_launch("cross_block", cross_block_kernel<TailShape<128, 8, true>>, grid, dim3(512), 0, s, a);
     return true;
 }

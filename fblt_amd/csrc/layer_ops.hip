@@ -552,11 +552,22 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
             check_weight(&s->cross_weight_q, E, E, "blt_kv_decode_step: cross_weight_q must be [embed_dim, embed_dim]");
             check_weight(&s->cross_weight_proj, E, E,
                          "blt_kv_decode_step: cross_weight_proj must be [embed_dim, embed_dim]");
+            CrossBlockArgs whole;
+            std::memset(&whole, 0, sizeof(whole));
+            whole.x = whole.residual = cur, whole.out = mid, whole.norm_w = (const float *)s->cross_norm_weight.data;
+            whole.wq = (const float *)s->cross_weight_q.data, whole.proj = (const float *)s->cross_weight_proj.data;
+            whole.k = (const float *)cache->cross_k[l].data, whole.v = (const float *)cache->cross_v[l].data;
+            whole.lo = dev + batch, whole.hi = dev + batch + rows, whole.slab_rows = cache->max_subtokens;
+            whole.rows = (uint32_t)rows, whole.rows_per_seq = (uint32_t)n, whole.head_dim = (uint32_t)xhd;
+            whole.scale = 1.0f / sqrtf((float)xhd);
             MatmulArgs probe;
             std::memset(&probe, 0, sizeof(probe));
             probe.m = (uint32_t)rows, probe.k = (uint32_t)E, probe.n = (uint32_t)E;
             probe.cross_head_dim = (uint32_t)xhd;
             probe.tolerant = step_tolerant();
+            if (rows > 32 && cross_block_launch(whole, (uint32_t)E, 0)) {
+                in = mid;
+            } else {
             if (matmul_takes_norm(probe) && matmul_takes_cross(probe)) {
                 /* norm, Q projection and the rows' cross attention in one launch: with more than 32
                  * rows a 32x32 tile of the projection is one 32-wide head of 32 rows; up to 32 rows
@@ -594,6 +605,7 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
             }
             gemm(xcomb, (const float *)s->cross_weight_proj.data, mid, rows, E, E, cur); /* + residual */
             in = mid;
+            }
         }
         blt_kv_attn_cache view;
         view.self_k = (float *)cache->self_k[l].data;

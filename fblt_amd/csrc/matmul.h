@@ -88,6 +88,20 @@ struct BlockTailArgs {
 };
 /* false: not for this shape, nothing was launched */
 bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s);
+/* A cross block past its K and V rows, in one launch (block_tail.hip): out = residual + combined * proj, where row r of
+ * `combined` attends, head by head, from RMSNorm(x) * wq (x * wq without norm_w) over rows lo[r] .. hi[r] - 1 of k and v,
+ * counted from slab_rows * (r / rows_per_seq); no rows: zeros.  All dense rows of embed_dim; out may be x. */
+struct CrossBlockArgs {
+    const float *x, *norm_w, *wq, *k, *v, *proj, *residual; /* norm_w, residual: optional */
+    float *out;
+    const uint32_t *lo, *hi;
+    uint64_t slab_rows;
+    uint32_t rows, rows_per_seq, head_dim;
+    float scale;
+};
+/* false: not for this shape, nothing was launched.  cross_block_ok: the same answer before lo and hi are there. */
+bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim);
+bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t s);
 /* g0 (plain, or like g1) and g1 (two weight matrices, two outputs) in one launch; only when matmul_pair_ok says so */
 bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1);
 void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStream_t s);

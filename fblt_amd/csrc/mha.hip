@@ -343,6 +343,10 @@ extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_t
     HIP_CHECK_LAUNCH("blt_transformer_forward");
 }
 
+/* Keys of a row up to which the launch of block_tail.hip is taken: it reads eight at a time and needs a trip to memory for
+ * every eight, where the attention kernels spread a row's keys over a wave. */
+constexpr uint32_t CROSS_SPAN = 64;
+
 /*
  * blt_cross_attention_forward on the device (reference: csrc/models/
  * cross_attention.c:101-157): patch queries against byte keys and values under
@@ -359,6 +363,9 @@ extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_t
  *      a configuration that does not reduce falls back to the dense mask
  *      built by the device mask builder;
  *   4. output = combined * weight_proj.
+ *
+ * 1, 3 and 4 are one launch behind that of 2 for narrow blocks of more than 32 rows whose rows see few keys (block_tail.hip):
+ * a forward pass of 512 bytes 248.6 -> 240.1 us, of 2048 504.8 -> 419.2.
  *
  * A patch that owns no byte is fatal, as in the reference's mask builder.
  */
@@ -392,45 +399,7 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     BLT_REQUIRE(P <= 0x7FFFFFFFu && T <= 0x7FFFFFFFu && E <= 0x3FFFFFFFu,
                 "blt_cross_attention: dimensions exceed 2^31-1");
 
-    float *q = (float *)blt_arena_alloc(arena, P * E * sizeof(float), 64);
-    float *k = (float *)blt_arena_alloc(arena, (T ? T : 1) * E * sizeof(float), 64);
-    float *v = (float *)blt_arena_alloc(arena, (T ? T : 1) * E * sizeof(float), 64);
-    float *combined = (float *)blt_arena_alloc(arena, P * E * sizeof(float), 64);
-
-    /* 1, 2. projections */
-    MatmulArgs g;
-    std::memset(&g, 0, sizeof(g));
-    g.a = (const float *)query_in->data;
-    g.b = (const float *)weights->weight_q->data;
-    g.out = q;
-    g.m = (uint32_t)P, g.k = (uint32_t)E, g.n = (uint32_t)E;
-    g.lda = g.ldb = g.ldo = (uint32_t)E;
-    MatmulArgs gkv = g;
-    g.norm_w = norm_w; /* the query rows only */
-    if (norm_w != nullptr && !matmul_takes_norm(g)) { /* shapes the fused norm does not cover: a pass of its own */
-        blt_tensor normed = blt_tensor_create_uninit(arena, query_in->shape, 2, BLT_DTYPE_FP32);
-        blt_tensor wt;
-        std::memset(&wt, 0, sizeof(wt));
-        wt.data = const_cast<float *>(norm_w), wt.ndim = 1, wt.shape[0] = E, wt.strides[0] = 1, wt.numel = E;
-        wt.dtype = BLT_DTYPE_FP32, wt.backend = BLT_BACKEND_HIP, wt.is_view = true;
-        blt_rmsnorm_forward_hip(query_in, &wt, &normed);
-        g.a = (const float *)normed.data;
-        g.norm_w = nullptr;
-    }
-    gkv.a = (const float *)kv_in->data;
-    gkv.b = (const float *)weights->weight_k->data;
-    gkv.out = k;
-    gkv.m = (uint32_t)T;
-    gkv.b2 = (const float *)weights->weight_v->data;
-    gkv.out2 = v;
-    if (T != 0 && matmul_pair_ok(g, gkv)) {
-        matmul_f32_launch_pair(g, gkv, 0); /* all three in one launch */
-    } else {
-        matmul_f32_launch(g, 0);
-        if (T != 0) matmul_f32_launch(gkv, 0);
-    }
-
-    /* 3. mask as row ranges when it reduces, then every head in one launch */
+    /* the mask as row ranges when it reduces */
     const uint32_t *row_lo = nullptr, *row_hi = nullptr;
     const float *dense = nullptr;
     uint32_t row_span = 0;
@@ -451,6 +420,59 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
             dense = (const float *)mask_tensor.data;
         }
     }
+    float *k = (float *)blt_arena_alloc(arena, (T ? T : 1) * E * sizeof(float), 64);
+    float *v = (float *)blt_arena_alloc(arena, (T ? T : 1) * E * sizeof(float), 64);
+
+    MatmulArgs g;
+    std::memset(&g, 0, sizeof(g));
+    g.m = (uint32_t)P, g.k = (uint32_t)E, g.n = (uint32_t)E;
+    g.lda = g.ldb = g.ldo = (uint32_t)E;
+    MatmulArgs gkv = g;
+    gkv.a = (const float *)kv_in->data;
+    gkv.b = (const float *)weights->weight_k->data;
+    gkv.out = k;
+    gkv.m = (uint32_t)T;
+    gkv.b2 = (const float *)weights->weight_v->data;
+    gkv.out2 = v;
+    CrossBlockArgs whole;
+    std::memset(&whole, 0, sizeof(whole));
+    whole.x = (const float *)query_in->data, whole.norm_w = norm_w, whole.residual = residual, whole.out = (float *)output->data;
+    whole.wq = (const float *)weights->weight_q->data, whole.proj = (const float *)weights->weight_proj->data;
+    whole.k = k, whole.v = v, whole.lo = row_lo, whole.hi = row_hi;
+    whole.rows = whole.rows_per_seq = (uint32_t)P, whole.head_dim = (uint32_t)hd, whole.scale = 1.0f / sqrtf((float)hd);
+    /* up to 32 rows the products keep the reference's order of sums */
+    if (row_lo != nullptr && P > 32 && T != 0 && row_span <= CROSS_SPAN && cross_block_ok(whole, (uint32_t)E)) {
+        matmul_f32_launch(gkv, 0);
+        cross_block_launch(whole, (uint32_t)E, 0);
+        HIP_CHECK_LAUNCH("blt_cross_attention_forward");
+        return;
+    }
+
+    float *q = (float *)blt_arena_alloc(arena, P * E * sizeof(float), 64);
+    float *combined = (float *)blt_arena_alloc(arena, P * E * sizeof(float), 64);
+    /* 1, 2. projections */
+    g.a = (const float *)query_in->data;
+    g.b = (const float *)weights->weight_q->data;
+    g.out = q;
+    g.norm_w = norm_w; /* the query rows only */
+    if (norm_w != nullptr && !matmul_takes_norm(g)) { /* shapes the fused norm does not cover: a pass of its own */
+        blt_tensor normed = blt_tensor_create_uninit(arena, query_in->shape, 2, BLT_DTYPE_FP32);
+        blt_tensor wt;
+        std::memset(&wt, 0, sizeof(wt));
+        wt.data = const_cast<float *>(norm_w), wt.ndim = 1, wt.shape[0] = E, wt.strides[0] = 1, wt.numel = E;
+        wt.dtype = BLT_DTYPE_FP32, wt.backend = BLT_BACKEND_HIP, wt.is_view = true;
+        blt_rmsnorm_forward_hip(query_in, &wt, &normed);
+        g.a = (const float *)normed.data;
+        g.norm_w = nullptr;
+    }
+    if (T != 0 && matmul_pair_ok(g, gkv)) {
+        matmul_f32_launch_pair(g, gkv, 0); /* all three in one launch */
+    } else {
+        matmul_f32_launch(g, 0);
+        if (T != 0) matmul_f32_launch(gkv, 0);
+    }
+
+    /* 3. every head in one launch */
     std::vector<blt_attention_problem> pr(H);
     const float scale = 1.0f / sqrtf((float)hd);
     for (size_t head = 0; head < H; head++) {

@@ -1475,6 +1475,74 @@ def test_cross_attention_block(P, T, E, H, kind, impl, oracle, dev):
     assert_close(got, ref, "cross attention P=%d T=%d E=%d H=%d %s" % (P, T, E, H, kind))
 
 
+@pytest.mark.parametrize("P,T,E,H,longest,fused", [
+    (33, 60, 64, 16, 4, True), (40, 300, 64, 1, 17, True), (50, 90, 128, 32, 9, True), (63, 1500, 128, 1, 64, True),
+    (65, 400, 128, 4, 33, True),
+    (40, 300, 128, 4, 65, False), (32, 60, 128, 4, 4, False), (40, 60, 96, 3, 4, False)])   # each past one of its limits
+def test_cross_attention_in_one_launch_past_its_keys(P, T, E, H, longest, fused, oracle, dev):
+    """The launch from the query's norm to the residual at the edges of its shapes, against the restated block; then with a key
+    that is not finite, which drops out of its own patch's softmax and changes no other row."""
+    import torch
+    lib = api.load()
+    rs = np.random.RandomState(P + T + H)
+    xq, xkv = rs.randn(P, E).astype(np.float32), rs.randn(T, E).astype(np.float32)
+    ws = [(rs.randn(E, E) / np.sqrt(E)).astype(np.float32) for _ in range(4)]
+    sizes = np.ones(P, dtype=int)
+    sizes[P // 2] = longest
+    while sizes.sum() < T:                          # the rest at random, none past the longest
+        sizes[rs.choice(np.flatnonzero(sizes < min(longest, T)))] += 1
+        if (sizes >= longest).all():
+            break
+    T = int(sizes.sum())
+    xkv = np.ascontiguousarray(np.resize(xkv, (T, E)))
+    cfg = abi.BltMaskConfig()
+    cfg.seq_len_q, cfg.seq_len_kv = P, T
+    keep = (abi.size_array(list(range(P))), abi.size_array(np.repeat(np.arange(P), sizes).tolist()))
+    cfg.query_group_ids, cfg.kv_group_ids = keep
+    cfg.bidirectional_within_group = True
+
+    def run(kv):
+        tensors = [torch.from_numpy(a).cuda() for a in (xq, kv, *ws)]
+        to = torch.full((P, E), 7.0, dtype=torch.float32, device="cuda")
+        views = [_dev_tensor(t) for t in tensors]
+        vo = _dev_tensor(to)
+        wts = abi.BltCrossAttentionWeights(*(C.pointer(v) for v in views[2:]))
+        cc = abi.BltCrossAttentionConfig()
+        cc.embed_dim, cc.num_heads, cc.head_dim = E, H, 0
+        cc.mask_config = C.pointer(cfg)
+        arena = lib.blt_arena_create(64 << 20, abi.BLT_BACKEND_HIP)
+        try:
+            lib.blt_hip_profile_begin()
+            lib.blt_cross_attention_forward(C.byref(views[0]), C.byref(views[1]), C.byref(wts), C.byref(vo), C.byref(cc), arena)
+            assert ("cross_block" in api.profile_end()) == fused
+            lib.blt_backend_pass_sync_hip()
+            return to.cpu().numpy()
+        finally:
+            lib.blt_arena_destroy(arena)
+
+    ref = np.zeros((P, E), dtype=np.float32)
+    assert oracle.orc_cross_attention_forward(*(binding.fptr(a.reshape(-1)) for a in (xq, xkv, *ws, ref)), P, T, E, H,
+                                              C.byref(cfg)) == 0
+    got = run(xkv)
+    assert_close(got, ref, "cross block")
+    if fused:
+        bad = xkv.copy()
+        patch = P // 2
+        bad[int(sizes[:patch].sum()) + longest - 1] = np.nan      # the last byte of the longest patch
+        out = run(bad)
+        others = np.arange(P) != patch
+        assert np.array_equal(out[others], got[others])
+        short = sizes.copy()
+        short[patch] -= 1
+        cut = np.delete(xkv, int(sizes[:patch].sum()) + longest - 1, axis=0)
+        cfg.seq_len_kv = T - 1
+        keep2 = (keep[0], abi.size_array(np.repeat(np.arange(P), short).tolist()))
+        cfg.query_group_ids, cfg.kv_group_ids = keep2
+        assert oracle.orc_cross_attention_forward(*(binding.fptr(np.ascontiguousarray(a).reshape(-1)) for a in (xq, cut, *ws)),
+                                                  binding.fptr(ref.reshape(-1)), P, T - 1, E, H, C.byref(cfg)) == 0
+        assert_close(out[patch], ref[patch], "without the key that is not finite")
+
+
 def test_row_ops(oracle, dev):
     """blt_rmsnorm_forward and blt_add bit-identical to the reference loops, blt_swiglu_forward in tolerance."""
     import torch
