@@ -27,9 +27,11 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix, published
-# fp32 products taken as six bf16 ones (split_bf16.h) on the dense bf16 rate, published 2500
+# fp32 products taken as six bf16 ones (split_bf16.h) or three f16 ones (split_f16.h) on their dense rate, published 2500
 SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 6.0
-SPLIT_KERNELS = {"wide", "mfma", "attn_wide", "attn_mfma", "matmul_mfma"}
+SPLIT_KERNELS = {"mfma", "attn_mfma"}
+HALF_MFMA_PEAK_TFLOPS = 2500.0 / 3.0
+HALF_KERNELS = {"wide", "attn_wide", "matmul_mfma"}
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.md")
 DETAIL_FILE = os.path.join(ROOT, "gpurun_out", "bench_detail.json")
@@ -69,7 +71,9 @@ def roofline(bound, work, avg_s, traffic=None, kernel=""):
     if bound == "hbm":
         achieved, peak, unit = work / avg_s / 1e9, HBM_PEAK_GBS, "GB/s"
     else:
-        peak = SPLIT_MFMA_PEAK_TFLOPS if SPLIT_KERNELS & set(kernel.split("+")) else FP32_MFMA_PEAK_TFLOPS
+        used = set(kernel.split("+"))
+        peak = (HALF_MFMA_PEAK_TFLOPS if HALF_KERNELS & used else
+                SPLIT_MFMA_PEAK_TFLOPS if SPLIT_KERNELS & used else FP32_MFMA_PEAK_TFLOPS)
         achieved, unit = work / avg_s / 1e12, "TFLOP/s"
     return {"bound": bound, "achieved": achieved, "peak": peak, "unit": unit, "frac": achieved / peak,
             "traffic": traffic}

@@ -40,9 +40,9 @@
  * second run is all there is).
  *
  * Bound: vector ALU and matrix unit, whose times add up: on a SIMD a 32x32 tile of heads of 32 is 12 matrix instructions
- * (384 cycles) and about 165 vector instructions (4.3 cycles each by the counters), 1090 cycles in all where it takes 1140.
+ * (384 cycles) and about 165 vector instructions (4.3 cycles each by the counters), 1090 cycles in all, most of what it takes.
  * As bf16 it was 24 and 215, and the matrix unit drew so much power that the clock gave way: the same launch took 201 us on
- * random values and 172 on constant ones (now 3 us apart).  Four waves a SIMD instead of two (two to a row tile, on even and
+ * random values and 172 on constant ones (the f16 form 159 and 153).  Four waves a SIMD instead of two (two to a row tile, on even and
  * odd key tiles) gained nothing with either: 206 against 206 us, 174 against 168.  Causal self-attention, 32 problems of
  * 4096 rows, heads of 32: 197 us as bf16, 158 as f16, 150 with two tiles between barriers, 139 with every fragment read at
  * the top of a tile (a read sunk to its use waited for LDS four times a tile).  48 problems of 2048 rows, heads of 64:
