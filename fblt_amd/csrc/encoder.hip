@@ -20,6 +20,7 @@
 #include "blt_fatal.h"
 #include "hip_check.h"
 #include "launch.h"
+#include "matmul.h"
 
 #include <cstdlib>
 #include <cstring>
@@ -27,11 +28,12 @@
 
 /* blt_cross_attention_forward_hip with the steps either side of it in a caller's layer folded in
  * (mha.hip): norm_w, when set, is the weight of the RMSNorm that makes query_in's rows the queries
- * (taken inside the query projection), residual [rows, embed] is added to the projected output. */
+ * (taken inside the query projection), residual [rows, embed] is added to the projected output.
+ * ranges: kept between the layers of one forward pass, whose cross blocks share a mask. */
 void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in,
                              const blt_cross_attention_weights *weights, blt_tensor *output,
                              const blt_cross_attention_config *config, blt_arena *arena, const float *norm_w,
-                             const float *residual);
+                             const float *residual, CrossRanges *ranges);
 
 namespace {
 
@@ -340,6 +342,7 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
     cross_cfg.mask_config = &cross_mask;
 
     /* ---- layers; the last results land in the caller's tensors ---- */
+    CrossRanges cross_ranges; /* in the arena, like everything else of the pass (a launch of its own per layer before: 2 … 4 us) */
     size_t last_cross = cfg.num_layers; /* none */
     for (size_t l = 0; l < cfg.num_layers; l++)
         if (blt_local_cross_attn_fires(cfg.cross_attn_placement, cfg.cross_attn_all_layers, cfg.num_layers, l)) last_cross = l;
@@ -366,7 +369,7 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
                                             : blt_tensor_create_uninit(arena, patch_shape, 2, BLT_DTYPE_FP32);
         blt_tensor next_rows = view_2d(p_next.data, num_patches * k, E);
         blt_cross_attention_run(&p_rows, &h, &xw, &next_rows, &cross_cfg, arena,
-                                (const float *)s->cross_norm_weight.data, (const float *)p.data);
+                                (const float *)s->cross_norm_weight.data, (const float *)p.data, &cross_ranges);
         p = p_next;
     }
     if (last_cross == cfg.num_layers) /* no cross block fired: P_0 is the result */
@@ -462,6 +465,7 @@ extern "C" void blt_local_decoder_forward_ext_hip(const blt_local_decoder *model
     cross_cfg.mask_config = &cross_mask;
 
     /* ---- layers ---- */
+    CrossRanges cross_ranges;
     const size_t byte_shape[2] = {seq_len, E};
     blt_tensor latents = view_2d(patch_in->data, num_patches * k, E);
     blt_tensor d = view_2d(byte_hidden_in->data, seq_len, E);
@@ -474,7 +478,7 @@ extern "C" void blt_local_decoder_forward_ext_hip(const blt_local_decoder *model
             xw.weight_proj = &s->cross_weight_proj;
             b = blt_tensor_create_uninit(arena, byte_shape, 2, BLT_DTYPE_FP32);
             blt_cross_attention_run(&d, &latents, &xw, &b, &cross_cfg, arena, (const float *)s->cross_norm_weight.data,
-                                    (const float *)d.data);
+                                    (const float *)d.data, &cross_ranges);
         }
         blt_transformer_weights w;
         std::memset(&w, 0, sizeof(w));

@@ -99,6 +99,12 @@ struct CrossBlockArgs {
     uint32_t rows, rows_per_seq, head_dim;
     float scale;
 };
+/* The key ranges of a cross mask on the device, for the calls of one forward pass that share the mask; lo null: not there
+ * (yet). */
+struct CrossRanges {
+    const uint32_t *lo = nullptr, *hi = nullptr;
+    uint32_t span = 0;
+};
 /* false: not for this shape, nothing was launched.  cross_block_ok: the same answer before lo and hi are there. */
 bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim);
 bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t s);

@@ -372,7 +372,7 @@ constexpr uint32_t CROSS_SPAN = 64;
 void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in,
                              const blt_cross_attention_weights *weights, blt_tensor *output,
                              const blt_cross_attention_config *config, blt_arena *arena, const float *norm_w,
-                             const float *residual) {
+                             const float *residual, CrossRanges *ranges) {
     BLT_REQUIRE(config != NULL && arena != NULL, "blt_cross_attention: config and arena cannot be NULL");
     BLT_REQUIRE(config->mask_config != NULL,
                 "blt_cross_attention: mask_config is required (block-diagonal patch mask)");
@@ -403,7 +403,9 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     const uint32_t *row_lo = nullptr, *row_hi = nullptr;
     const float *dense = nullptr;
     uint32_t row_span = 0;
-    {
+    if (ranges != nullptr && ranges->lo != nullptr) {
+        row_lo = ranges->lo, row_hi = ranges->hi, row_span = ranges->span;
+    } else {
         std::vector<uint32_t> lohi(2 * P);
         if (blt_mask_config_row_ranges(mc, lohi.data(), lohi.data() + P) == 1) {
             for (size_t i = 0; i < P; i++) { /* the dense builder refuses such a mask (mask_builder_cpu.c:93) */
@@ -413,6 +415,7 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
             uint32_t *dev = (uint32_t *)blt_arena_alloc(arena, 2 * P * sizeof(uint32_t), 64);
             blt_upload_staged(dev, lohi.data(), 2 * P * sizeof(uint32_t));
             row_lo = dev, row_hi = dev + P;
+            if (ranges != nullptr) ranges->lo = row_lo, ranges->hi = row_hi, ranges->span = row_span;
         } else {
             blt_tensor mask_tensor;
             std::memset(&mask_tensor, 0, sizeof(mask_tensor));
@@ -516,5 +519,5 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
 extern "C" void blt_cross_attention_forward_hip(const blt_tensor *query_in, const blt_tensor *kv_in,
                                                 const blt_cross_attention_weights *weights, blt_tensor *output,
                                                 const blt_cross_attention_config *config, blt_arena *arena) {
-    blt_cross_attention_run(query_in, kv_in, weights, output, config, arena, nullptr, nullptr);
+    blt_cross_attention_run(query_in, kv_in, weights, output, config, arena, nullptr, nullptr, nullptr);
 }
