@@ -923,6 +923,50 @@ def test_attention_whose_small_values_carry_the_result(batch, H, hd, nq, nk, dev
         d.close()
 
 
+@pytest.mark.parametrize("batch,H,hd,nq,nk,window", [
+    (32, 4, 32, 1025, 1025, 0), (64, 4, 32, 300, 333, 0), (64, 4, 32, 520, 520, 65),       # eight waves, four, windows
+    (48, 4, 64, 510, 510, 0), (48, 4, 64, 512, 512, 0), (32, 2, 64, 1030, 1061, 0),        # both sides of the line for heads of 64
+    (48, 4, 64, 640, 640, 319), (48, 4, 64, 640, 640, 320)])
+def test_attention_weighed_before_its_maximum(batch, H, hd, nq, nk, window, dev):
+    """The large-batch kernel weighs a tile against the maximum so far and looks for a new one only where the weights add up to
+    too much: scores that rise all along a row, stand still, fall, jump near its end, or are the same everywhere; a window that
+    some rows of a tile enter later than others; and a column of V that is nothing but zeros until values too small for f16
+    parts come.  Against float64, column by column in the 2-norm, relative to the sum of the terms' magnitudes: scores of up to 42 in
+    log2 units that fp32 rounds twelve times are off by 42 sqrt(12) 2^-24 typically and three times that at most, 2^-16 in a weight."""
+    import torch
+    w = workloads.offset_causal(batch=batch, nq=nq, nk=nk, H=H, hd=hd, window=window)
+    d = dev.DeviceWorkload(w)
+    lib = api.load()
+    scale = w.heads[0].scale
+    try:
+        q, k, v = (d.dev[n].view(batch, -1, H, hd) for n in ("q", "k", "v"))
+        ramp = torch.arange(nk, device="cuda", dtype=torch.float32)[:, None] / nk
+        for b, column in ((1, ramp * 40), (2, -ramp * 40), (3, torch.zeros_like(ramp)), (4, (ramp > 0.7) * 30.0), (5, (ramp > 0.98) * 3.5)):
+            q[b, :, :, 0], k[b, :, :, 0] = 1.0, column * (0.6931 / scale)
+            q[b, :, :, 1:] *= 0.0 if b == 3 else 0.3
+        v[6, : nk - 50, :, 3] = 0.0
+        v[6, nk - 50 :, :, 3] *= 1e-8
+        torch.cuda.synchronize()
+        d.zero_outputs()
+        plan = d.make_plan("descriptor")
+        assert lib.blt_attention_plan_kernel_hip(plan) == b"wide"
+        lib.blt_attention_plan_run_hip(plan)
+        lib.blt_backend_pass_sync_hip()
+        lib.blt_attention_plan_destroy_hip(plan)
+        got = torch.from_numpy(d.output("out").copy()).cuda().view(batch, nq, H, hd).double()
+        i, j = torch.arange(nq, device="cuda")[:, None] + nk - nq, torch.arange(nk, device="cuda")[None, :]
+        keep = (j <= i) & (j > i - window) if window else j <= i
+        for b in range(8):
+            for head in (0, H - 1):
+                s = (q[b, :, head].double() @ k[b, :, head].double().T.contiguous()) * scale
+                p, x = torch.softmax(s.masked_fill(~keep, float("-inf")), dim=1), v[b, :, head].double()
+                off, size = (got[b, :, head] - p @ x).norm(dim=0), (p @ x.abs()).norm(dim=0)
+                worst = (off / size.clamp_min(1e-300)).max().item()
+                assert worst <= 2.0 ** -16, (b, head, worst)
+    finally:
+        d.close()
+
+
 @pytest.mark.parametrize("batch,T,window,hd,mixed,kernel", [
     (65, 129, 0, 32, False, "attn_wide_brief"), (64, 129, 0, 32, False, "attn_wide"), (65, 129, 0, 64, False, "attn_wide"),
     (22, 700, 128, 32, False, "attn_wide_brief"), (22, 700, 129, 32, False, "attn_wide"), (44, 383, 0, 32, True, "attn_wide_brief"),
