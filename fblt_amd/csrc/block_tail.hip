@@ -100,17 +100,23 @@ __device__ __forceinline__ void gather(const float *part, float (&out)[N]) {
 }
 
 template <typename Shape>
-__global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArgs a) {
+struct TailLds {
+    __attribute__((aligned(16))) float rows[16 * Shape::ROW], part[Shape::AREA], act[16 * Shape::ACT];
+    uint32_t ticket;
+};
+
+/* slice `slice` of row tile `tile` */
+template <typename Shape>
+__device__ __forceinline__ void tail_tile(const BlockTailArgs &a, uint32_t slices, uint32_t slice, uint32_t tile, TailLds<Shape> &lds) {
     using Proj = typename Shape::Proj;
     using Gated = typename Shape::Gated;
     using Down = typename Shape::Down;
     constexpr int E = Shape::E, HS = Shape::HS, ROW = Shape::ROW, ACT = Shape::ACT, EPT = Shape::EPT, APT = Shape::APT;
     typedef float rowpart __attribute__((ext_vector_type(EPT)));
-    __shared__ __attribute__((aligned(16))) float rows[16 * ROW], part[Shape::AREA], act[16 * ACT];
-    __shared__ uint32_t ticket;
+    float *const rows = lds.rows, *const part = lds.part, *const act = lds.act;
     const uint32_t tid = threadIdx.x;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t slices = gridDim.x, slice = blockIdx.x, row0 = 16u * blockIdx.y;
+    const uint32_t row0 = 16u * tile;
     /* what this thread finishes of the 16 rows */
     constexpr uint32_t TPR = E / EPT; /* threads of a row: neighbours in one wave */
     static_assert(TPR <= 64, "a row's threads are in one wave");
@@ -179,7 +185,7 @@ __global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArg
         /* device-scope stores and loads, and an explicit wait for the stores' completion before the barrier that
          * precedes the workgroup's ticket */
         constexpr uint32_t WORDS = 16 * E / 2; /* a slice's sums, two a word */
-        uint64_t *mine = a.sums + (size_t)blockIdx.y * slices * WORDS + tid;
+        uint64_t *mine = a.sums + (size_t)tile * slices * WORDS + tid;
 #pragma unroll
         for (int i = 0; i < EPT / 2; i++)
             __hip_atomic_store(mine + (size_t)slice * WORDS + i * Shape::THREADS,
@@ -188,10 +194,10 @@ __global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArg
         blt_vector_memory_done();
         __syncthreads();
         if (tid == 0u)
-            ticket = __hip_atomic_fetch_add(&a.tickets[blockIdx.y], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            lds.ticket = __hip_atomic_fetch_add(&a.tickets[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
-        if (ticket != slices - 1u) return;
-        if (tid == 0u) a.tickets[blockIdx.y] = 0u; /* re-armed for the next launch */
+        if (lds.ticket != slices - 1u) return;
+        if (tid == 0u) a.tickets[tile] = 0u; /* re-armed for the next launch */
 #pragma unroll
         for (int i = 0; i < EPT; i++) sum[i] = 0.f;
         for (uint32_t z = 0; z < slices; z += 8u) { /* slice order, whoever comes last */
@@ -215,6 +221,12 @@ __global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArg
     if (row0 + f_row < a.rows) *reinterpret_cast<rowpart *>(a.out + f_at) = out;
 }
 
+template <typename Shape>
+__global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArgs a) {
+    __shared__ TailLds<Shape> lds;
+    tail_tile<Shape>(a, gridDim.x, blockIdx.x, blockIdx.y, lds);
+}
+
 /* A cross block of 16 rows a workgroup: norm, query projection, the rows' attention, output projection, residual
  * (csrc/models/cross_attention.c:101-157, csrc/infer/kv_cache.c:303-324).  A row sees few keys, a handful of bytes or the
  * patches of its own window, so the rows of K and V come straight from memory, eight keys in flight, the first before there
@@ -229,16 +241,15 @@ __global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArg
 constexpr uint32_t CROSS_ROWS = 16384;
 constexpr uint32_t CROSS_KEYS = 4;
 
-template <typename Shape>
-__global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockArgs a) {
+template <typename Shape, uint32_t KEYS = CROSS_KEYS>
+__device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, uint32_t tile, float *rows, float *part) {
     using Proj = typename Shape::Proj;
     constexpr int E = Shape::E, ROW = Shape::ROW, EPT = Shape::EPT;
     static_assert(EPT == 4, "a thread holds 16 bytes of a row");
-    __shared__ __attribute__((aligned(16))) float rows[16 * ROW], part[Proj::PART];
     const uint32_t tid = threadIdx.x;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr uint32_t TPR = E / EPT;
-    const uint32_t row0 = 16u * blockIdx.x, f_row = tid / TPR, f_col = EPT * (tid % TPR);
+    const uint32_t row0 = 16u * tile, f_row = tid / TPR, f_col = EPT * (tid % TPR);
     const uint32_t row = min(row0 + f_row, a.rows - 1u);
     const size_t f_at = (size_t)row * E + f_col;
     const uint32_t group = wave % Proj::GROUPS, term = wave / Proj::GROUPS * (16 * Proj::BLOCKS);
@@ -250,7 +261,6 @@ __global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockA
     request<Proj::BLOCKS>(wq, a.wq + 64u * group, E, term);
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t lo = a.lo[row], hi = a.hi[row];
-    constexpr uint32_t KEYS = CROSS_KEYS;
     const uint32_t lanes = a.head_dim / EPT; /* of a head: a power of two up to TPR */
     const size_t slab = (size_t)(row / a.rows_per_seq) * a.slab_rows * E + f_col;
     struct Keys {
@@ -342,13 +352,41 @@ __global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockA
 }
 
 template <typename Shape>
-void launch_tail(const BlockTailArgs &a, dim3 grid, hipStream_t s) {
+__global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockArgs a) {
+    __shared__ __attribute__((aligned(16))) float rows[16 * Shape::ROW], part[Shape::Proj::PART];
+    cross_tile<Shape>(a, blockIdx.x, rows, part);
+}
+
+/* A block's tail and a cross block that neither reads nor writes anything of it, in the first `first` rows of workgroups: the
+ * encoder's, whose patches take up a layer's bytes while the next layer goes on with them.  Its few workgroups fit beside the tail's, so
+ * it costs nothing of its own (128 patches of 512 bytes, 128 columns: 9.6 us as a launch).  Half the keys in flight: more registers than the
+ * tail has would halve the workgroups of a compute unit. */
+template <typename Shape>
+__global__ __launch_bounds__(Shape::THREADS, 4) void block_tail_beside_kernel(BlockTailArgs a, CrossBlockArgs c, uint32_t first) {
+    __shared__ TailLds<Shape> lds;
+    if (blockIdx.y < first) {
+        const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
+        if (tile < (c.rows + 15u) / 16u) cross_tile<Shape, CROSS_KEYS / 2>(c, tile, lds.rows, lds.part);
+    } else {
+        tail_tile<Shape>(a, gridDim.x, blockIdx.x, blockIdx.y - first, lds);
+    }
+}
+
+template <typename Shape>
+void launch_tail(const BlockTailArgs &a, dim3 grid, hipStream_t s, const CrossBlockArgs *beside = nullptr) {
+    if constexpr (Shape::PROJ) {
+        if (beside) {
+            const uint32_t first = ((beside->rows + 15u) / 16u + grid.x - 1u) / grid.x;
+            blt_launch("block_tail", block_tail_beside_kernel<Shape>, dim3(grid.x, grid.y + first), dim3(Shape::THREADS), 0, s, a, *beside, first);
+            return;
+        }
+    }
     blt_launch("block_tail", block_tail_kernel<Shape>, grid, dim3(Shape::THREADS), 0, s, a);
 }
 
 } // namespace
 
-bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s) {
+bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s, CrossLater *later) {
     if (a.rows == 0u || a.hidden == 0u || (embed_dim != 64u && embed_dim != 128u && embed_dim != 256u) || a.hidden % 64u != 0u)
         return false;
     for (const void *p : {(const void *)a.comb, (const void *)a.x, (const void *)a.proj, (const void *)a.norm_w, (const void *)a.up,
@@ -378,10 +416,16 @@ bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s) {
     if (slices > 1u && !matmul_slice_scratch((size_t)tiles * slices * 16u * embed_dim, tiles, s, (float **)&a.sums, &a.tickets))
         return false;
     const dim3 grid(slices, tiles);
+    /* with a cross block that waits, as long as all workgroups have a place at once */
+    const CrossBlockArgs *beside = nullptr;
+    if (later != nullptr && later->cross_waits && embed_dim != 256u && workgroups + (later->cross.rows + 15u) / 16u <= most) {
+        matmul_later_launch(*later, s); /* its keys */
+        beside = &later->cross, later->cross_waits = false;
+    }
     if (embed_dim == 64u) {
-        launch_tail<TailShape<64, 4, true>>(a, grid, s);
+        launch_tail<TailShape<64, 4, true>>(a, grid, s, beside);
     } else if (embed_dim == 128u) {
-        launch_tail<TailShape<128, 8, true>>(a, grid, s);
+        launch_tail<TailShape<128, 8, true>>(a, grid, s, beside);
     } else { /* 1024 threads leave a wave 128 registers, and its share of proj is 64 of them */
         MatmulArgs g;
         std::memset(&g, 0, sizeof(g));
@@ -403,6 +447,12 @@ bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim) {
                           (const void *)a.proj, (const void *)a.residual, (const void *)a.out})
         if ((reinterpret_cast<uintptr_t>(p) & 15u) != 0u) return false;
     return a.rows <= CROSS_ROWS;
+}
+
+void cross_later_launch(CrossLater &later, uint32_t embed_dim, hipStream_t s) {
+    matmul_later_launch(later, s);
+    if (later.cross_waits) cross_block_launch(later.cross, embed_dim, s);
+    later.cross_waits = false;
 }
 
 bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t s) {

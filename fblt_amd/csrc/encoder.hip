@@ -29,11 +29,14 @@
 /* blt_cross_attention_forward_hip with the steps either side of it in a caller's layer folded in
  * (mha.hip): norm_w, when set, is the weight of the RMSNorm that makes query_in's rows the queries
  * (taken inside the query projection), residual [rows, embed] is added to the projected output.
- * ranges: kept between the layers of one forward pass, whose cross blocks share a mask. */
+ * pass: kept between the layers of one forward pass, whose cross blocks share a mask. */
 void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in,
                              const blt_cross_attention_weights *weights, blt_tensor *output,
                              const blt_cross_attention_config *config, blt_arena *arena, const float *norm_w,
-                             const float *residual, CrossRanges *ranges);
+                             const float *residual, CrossPass *pass);
+/* blt_transformer_forward_hip (mha.hip); later: a cross block that waits for launches to go along with, all of it launched on return */
+void blt_transformer_run(const blt_tensor *input, const blt_transformer_weights *w, blt_tensor *output,
+                         const blt_transformer_config *config, blt_arena *arena, CrossLater *later);
 
 namespace {
 
@@ -342,7 +345,11 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
     cross_cfg.mask_config = &cross_mask;
 
     /* ---- layers; the last results land in the caller's tensors ---- */
-    CrossRanges cross_ranges; /* in the arena, like everything else of the pass (a launch of its own per layer before: 2 … 4 us) */
+    /* A layer's cross block takes nothing from the next layer and gives nothing to it: but for the last one it goes along with that
+     * layer's launches.  512 bytes through an encoder and a decoder of two layers of 128 columns with four patch layers between them, us: with
+     * the decoder's keys in pairs 240 -> 230, three layers each 256 -> 239. */
+    CrossPass cross_pass; /* in the arena, like everything else of the pass (a launch of its own per layer before: 2 … 4 us) */
+    CrossLater later;
     size_t last_cross = cfg.num_layers; /* none */
     for (size_t l = 0; l < cfg.num_layers; l++)
         if (blt_local_cross_attn_fires(cfg.cross_attn_placement, cfg.cross_attn_all_layers, cfg.num_layers, l)) last_cross = l;
@@ -355,7 +362,7 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
         w.ffn_down_w = &s->ffn_down_w;
         blt_tensor h_next = l + 1 == cfg.num_layers ? view_2d(byte_hidden_out->data, seq_len, E)
                                                     : blt_tensor_create_uninit(arena, byte_shape, 2, BLT_DTYPE_FP32);
-        blt_transformer_forward_hip(&h, &w, &h_next, &layer_cfg, arena);
+        blt_transformer_run(&h, &w, &h_next, &layer_cfg, arena, &later);
         h = h_next;
         if (!blt_local_cross_attn_fires(cfg.cross_attn_placement, cfg.cross_attn_all_layers, cfg.num_layers, l)) continue;
 
@@ -368,8 +375,9 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
         blt_tensor p_next = l == last_cross ? view_2d(patch_out->data, num_patches, patch_dim)
                                             : blt_tensor_create_uninit(arena, patch_shape, 2, BLT_DTYPE_FP32);
         blt_tensor next_rows = view_2d(p_next.data, num_patches * k, E);
+        cross_pass.later = l + 1 < cfg.num_layers ? &later : nullptr;
         blt_cross_attention_run(&p_rows, &h, &xw, &next_rows, &cross_cfg, arena,
-                                (const float *)s->cross_norm_weight.data, (const float *)p.data, &cross_ranges);
+                                (const float *)s->cross_norm_weight.data, (const float *)p.data, &cross_pass);
         p = p_next;
     }
     if (last_cross == cfg.num_layers) /* no cross block fired: P_0 is the result */
@@ -465,7 +473,7 @@ extern "C" void blt_local_decoder_forward_ext_hip(const blt_local_decoder *model
     cross_cfg.mask_config = &cross_mask;
 
     /* ---- layers ---- */
-    CrossRanges cross_ranges;
+    CrossPass cross_pass;
     const size_t byte_shape[2] = {seq_len, E};
     blt_tensor latents = view_2d(patch_in->data, num_patches * k, E);
     blt_tensor d = view_2d(byte_hidden_in->data, seq_len, E);
@@ -477,8 +485,13 @@ extern "C" void blt_local_decoder_forward_ext_hip(const blt_local_decoder *model
             xw.weight_q = &s->cross_weight_q, xw.weight_k = &s->cross_weight_k, xw.weight_v = &s->cross_weight_v;
             xw.weight_proj = &s->cross_weight_proj;
             b = blt_tensor_create_uninit(arena, byte_shape, 2, BLT_DTYPE_FP32);
+            /* every layer's keys and values come from the same latents: those of two layers in one launch */
+            cross_pass.next_k = cross_pass.next_v = nullptr;
+            for (size_t n = l + 1; n < cfg.num_layers && cross_pass.next_k == nullptr; n++)
+                if (blt_local_cross_attn_fires(cfg.cross_attn_placement, cfg.cross_attn_all_layers, cfg.num_layers, n))
+                    cross_pass.next_k = &model->layers[n].cross_weight_k, cross_pass.next_v = &model->layers[n].cross_weight_v;
             blt_cross_attention_run(&d, &latents, &xw, &b, &cross_cfg, arena, (const float *)s->cross_norm_weight.data,
-                                    (const float *)d.data, &cross_ranges);
+                                    (const float *)d.data, &cross_pass);
         }
         blt_transformer_weights w;
         std::memset(&w, 0, sizeof(w));

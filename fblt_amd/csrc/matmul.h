@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "blt_abi.h"
 #include "rope_device.h"
 
 /* out[m, n] = a[m, k] * b[k, n], leading dimensions in elements.  With
@@ -86,8 +87,6 @@ struct BlockTailArgs {
     uint64_t *sums; /* set by the launcher */
     uint32_t *tickets;
 };
-/* false: not for this shape, nothing was launched */
-bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s);
 /* A cross block past its K and V rows, in one launch (block_tail.hip): out = residual + combined * proj, where row r of
  * `combined` attends, head by head, from RMSNorm(x) * wq (x * wq without norm_w) over rows lo[r] .. hi[r] - 1 of k and v,
  * counted from slab_rows * (r / rows_per_seq); no rows: zeros.  All dense rows of embed_dim; out may be x. */
@@ -99,16 +98,31 @@ struct CrossBlockArgs {
     uint32_t rows, rows_per_seq, head_dim;
     float scale;
 };
-/* The key ranges of a cross mask on the device, for the calls of one forward pass that share the mask; lo null: not there
- * (yet). */
-struct CrossRanges {
-    const uint32_t *lo = nullptr, *hi = nullptr;
-    uint32_t span = 0;
-};
 /* false: not for this shape, nothing was launched.  cross_block_ok: the same answer before lo and hi are there. */
 bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim);
 bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t s);
-/* g0 (plain, or like g1) and g1 (two weight matrices, two outputs) in one launch; only when matmul_pair_ok says so */
+/* A cross block put off until launches of the next layer, which has nothing to do with it, can take it along: the product of its
+ * keys and values beside that layer's first product, the rest beside its tail. */
+struct CrossLater {
+    MatmulArgs kv;
+    CrossBlockArgs cross;
+    bool kv_waits = false, cross_waits = false;
+};
+/* What the cross blocks of one forward pass, which have their mask in common, leave each other. */
+struct CrossPass {
+    const uint32_t *lo = nullptr, *hi = nullptr; /* the mask's key ranges on the device; lo null: not there (yet) */
+    uint32_t span = 0;
+    CrossLater *later = nullptr; /* a block may be left there instead of launched */
+    /* K and V weights of the next block over the same rows: its keys and values may be made in this block's launch ... */
+    const blt_tensor *next_k = nullptr, *next_v = nullptr;
+    float *made_k = nullptr, *made_v = nullptr; /* ... and are here then */
+};
+/* what still waits, in launches of its own: the product only, or both */
+void matmul_later_launch(CrossLater &later, hipStream_t s);
+void cross_later_launch(CrossLater &later, uint32_t embed_dim, hipStream_t s);
+/* false: not for this shape, nothing was launched.  later: what waits may go along. */
+bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s, CrossLater *later = nullptr);
+/* g0 (plain, rotated, or like g1) and g1 (two weight matrices, two outputs) in one launch; only when matmul_pair_ok says so */
 bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1);
 void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStream_t s);
 /* the cross-attention epilogue for this shape and g.cross_head_dim, no other epilogue set */

@@ -801,15 +801,15 @@ __global__ __launch_bounds__(64 * NW, 2) void matmul_splitk_kernel(MatmulArgs g)
 
 /* Two independent products in one launch: the tile rows of the second are
  * stacked under those of the first (rows0 tile rows); the second carries a
- * second weight matrix, the first too if BOTH.  For pairs of small products whose launches would
+ * second weight matrix, the first too if BOTH, or the first is rotated if ROPE.  For pairs of small products whose launches would
  * otherwise each pay the fixed launch cost. */
-template <bool VEC, bool BOTH>
+template <bool VEC, bool BOTH, bool ROPE = false>
 __global__ __launch_bounds__(256, 2) void matmul_splitk_pair_kernel(MatmulArgs g0, MatmulArgs g1, uint32_t rows0) {
     __shared__ float part[8][16][64];
     __shared__ float part_ss[4][32];
     if (blockIdx.y < rows0) { /* uniform per workgroup */
         if (blockIdx.x * 32u >= g0.n) return;
-        splitk_tile<VEC, false, BOTH>(g0, blockIdx.x, blockIdx.y, part, part_ss);
+        splitk_tile<VEC, ROPE, BOTH>(g0, blockIdx.x, blockIdx.y, part, part_ss);
     } else {
         if (blockIdx.x * 32u >= g1.n) return;
         splitk_tile<VEC, false, true>(g1, blockIdx.x, blockIdx.y - rows0, part, part_ss);
@@ -1066,12 +1066,12 @@ bool vec_ok(const MatmulArgs &g) {
 } // namespace
 
 bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1) {
+    const auto rotated = [](const MatmulArgs &g) { return g.rope_cos != nullptr && g.rope_cols > 0; };
     const auto plain = [](const MatmulArgs &g) {
-        return g.m != 0 && g.n != 0 && g.k != 0 && g.m > 32u && choose_path(g) == PATH_SPLITK && !g.residual &&
-               !(g.rope_cos != nullptr && g.rope_cols > 0);
+        return g.m != 0 && g.n != 0 && g.k != 0 && g.m > 32u && choose_path(g) == PATH_SPLITK && !g.residual;
     };
     /* the first product may normalise its rows on the way (four waves: the tile code's own sums) */
-    return plain(g0) && plain(g1) && (g0.b2 == nullptr || g0.out2 != nullptr) && g1.b2 != nullptr && g1.out2 != nullptr && !g1.norm_w;
+    return plain(g0) && plain(g1) && !rotated(g1) && !(rotated(g0) && g0.b2 != nullptr) && (g0.b2 == nullptr || g0.out2 != nullptr) && g1.b2 != nullptr && g1.out2 != nullptr && !g1.norm_w;
 }
 
 void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStream_t s) {
@@ -1081,7 +1081,8 @@ void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStrea
     const dim3 grid(cols, rows0 + rows1);
     const auto launch = [&](auto kernel) { blt_launch("matmul_splitk", kernel, grid, dim3(256), 0, s, g0, g1, rows0); };
     const bool vec = vec_ok(g0) && vec_ok(g1);
-    if (g0.b2) launch(vec ? matmul_splitk_pair_kernel<true, true> : matmul_splitk_pair_kernel<false, true>);
+    if (g0.rope_cos != nullptr && g0.rope_cols > 0) launch(vec ? matmul_splitk_pair_kernel<true, false, true> : matmul_splitk_pair_kernel<false, false, true>);
+    else if (g0.b2) launch(vec ? matmul_splitk_pair_kernel<true, true> : matmul_splitk_pair_kernel<false, true>);
     else launch(vec ? matmul_splitk_pair_kernel<true, false> : matmul_splitk_pair_kernel<false, false>);
 }
 
@@ -1161,6 +1162,11 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
         if (vec) launch_mfma<true, 1>(g, rope, s);
         else launch_mfma<false, 1>(g, rope, s);
     }
+}
+
+void matmul_later_launch(CrossLater &later, hipStream_t s) {
+    if (later.kv_waits) matmul_f32_launch(later.kv, s);
+    later.kv_waits = false;
 }
 
 extern "C" void blt_matmul_hip(const blt_tensor *a, const blt_tensor *b, blt_tensor *out) {

@@ -40,10 +40,11 @@ namespace {
  * projection's own pass where that kernel takes it, csrc/models/transformer.c:60-66), with
  * residual that [seq_len, embed_dim] array is added to the projected output (transformer.c:
  * 116-117) -- the two statements a transformer block wraps around its attention.  With tail the rest of
- * the block follows in the launch of the projection where that takes the shape; true: it did. */
+ * the block follows in the launch of the projection where that takes the shape; true: it did.  What waits in later goes along where
+ * it can. */
 bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_tensor *weight_proj, blt_tensor *output,
              const blt_attention_config *config, blt_arena *arena, const float *norm_w, const float *residual,
-             const BlockTailArgs *tail = nullptr) {
+             const BlockTailArgs *tail = nullptr, CrossLater *later = nullptr) {
     BLT_REQUIRE(config != NULL && arena != NULL, "blt_multihead_attention: config and arena cannot be NULL");
     BLT_REQUIRE(arena->backend == BLT_BACKEND_HIP, "blt_multihead_attention: HIP implementation needs a device arena");
     const size_t E = config->embed_dim, H = config->num_heads;
@@ -126,7 +127,12 @@ bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
             g.a = (const float *)normed.data;
         }
     }
-    matmul_f32_launch(g, 0);
+    if (later != nullptr && later->kv_waits && matmul_pair_ok(g, later->kv)) {
+        matmul_f32_launch_pair(g, later->kv, 0);
+        later->kv_waits = false;
+    } else {
+        matmul_f32_launch(g, 0);
+    }
     if (config->use_rope && !fuse_rope) {
         for (size_t head = 0; head < H; head++) {
             blt_rope_apply_packed_hip(qkv, 3 * E, head * hd, T, hd, rope_cos, rope_sin);
@@ -231,7 +237,7 @@ bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
     if (tail != nullptr) {
         BlockTailArgs t = *tail;
         t.comb = combined, t.x = residual, t.proj = (const float *)weight_proj->data, t.rows = (uint32_t)T;
-        if (block_tail_launch(t, (uint32_t)E, 0)) return true;
+        if (block_tail_launch(t, (uint32_t)E, 0, later)) return true;
     }
     std::memset(&g, 0, sizeof(g));
     g.a = combined;
@@ -271,8 +277,8 @@ extern "C" void blt_multihead_attention_hip(const blt_tensor *input, const blt_t
  * RMSNorm + SwiGLU blocks with FP32 weights (what every BLT block is, csrc/models/
  * local_common.c:99-115); LayerNorm / GELU blocks and BF16 weight copies end with a message.
  */
-extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_transformer_weights *w, blt_tensor *output,
-                                            const blt_transformer_config *config, blt_arena *arena) {
+void blt_transformer_run(const blt_tensor *input, const blt_transformer_weights *w, blt_tensor *output,
+                         const blt_transformer_config *config, blt_arena *arena, CrossLater *later) {
     BLT_REQUIRE(input != NULL && w != NULL && output != NULL && config != NULL,
                 "Transformer: input, weights, output, and config cannot be NULL");
     BLT_REQUIRE(arena != NULL, "Transformer: arena cannot be NULL");
@@ -310,9 +316,10 @@ extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_t
     tail.hidden = (uint32_t)hidden;
     /* up to 32 rows the products keep the reference's order of sums */
     const bool done = mha_run(input, w->attn_qkv_w, w->attn_proj_w, &attn_residual, &config->attn_config, arena,
-                              (const float *)w->norm1_weight->data, (const float *)input->data, T > 32 ? &tail : nullptr);
+                              (const float *)w->norm1_weight->data, (const float *)input->data, T > 32 ? &tail : nullptr, later);
     blt_tensor act = blt_tensor_create_uninit(arena, hidden_shape, 2, BLT_DTYPE_FP32);
     if (done) {
+        if (later != nullptr) cross_later_launch(*later, (uint32_t)E, 0);
         HIP_CHECK_LAUNCH("blt_transformer_forward");
         return;
     }
@@ -340,7 +347,13 @@ extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_t
     g.m = (uint32_t)T, g.k = (uint32_t)hidden, g.n = (uint32_t)E;
     g.lda = (uint32_t)hidden, g.ldb = g.ldo = (uint32_t)E;
     matmul_f32_launch(g, 0);
+    if (later != nullptr) cross_later_launch(*later, (uint32_t)E, 0);
     HIP_CHECK_LAUNCH("blt_transformer_forward");
+}
+
+extern "C" void blt_transformer_forward_hip(const blt_tensor *input, const blt_transformer_weights *w, blt_tensor *output,
+                                            const blt_transformer_config *config, blt_arena *arena) {
+    blt_transformer_run(input, w, output, config, arena, nullptr);
 }
 
 /* Keys of a row up to which the launch of block_tail.hip is taken: what the tests state.  It reads eight at a time and needs a trip
@@ -374,7 +387,7 @@ constexpr uint32_t CROSS_SPAN = 64;
 void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in,
                              const blt_cross_attention_weights *weights, blt_tensor *output,
                              const blt_cross_attention_config *config, blt_arena *arena, const float *norm_w,
-                             const float *residual, CrossRanges *ranges) {
+                             const float *residual, CrossPass *pass) {
     BLT_REQUIRE(config != NULL && arena != NULL, "blt_cross_attention: config and arena cannot be NULL");
     BLT_REQUIRE(config->mask_config != NULL,
                 "blt_cross_attention: mask_config is required (block-diagonal patch mask)");
@@ -405,8 +418,8 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     const uint32_t *row_lo = nullptr, *row_hi = nullptr;
     const float *dense = nullptr;
     uint32_t row_span = 0;
-    if (ranges != nullptr && ranges->lo != nullptr) {
-        row_lo = ranges->lo, row_hi = ranges->hi, row_span = ranges->span;
+    if (pass != nullptr && pass->lo != nullptr) {
+        row_lo = pass->lo, row_hi = pass->hi, row_span = pass->span;
     } else {
         std::vector<uint32_t> lohi(2 * P);
         if (blt_mask_config_row_ranges(mc, lohi.data(), lohi.data() + P) == 1) {
@@ -417,7 +430,7 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
             uint32_t *dev = (uint32_t *)blt_arena_alloc(arena, 2 * P * sizeof(uint32_t), 64);
             blt_upload_staged(dev, lohi.data(), 2 * P * sizeof(uint32_t));
             row_lo = dev, row_hi = dev + P;
-            if (ranges != nullptr) ranges->lo = row_lo, ranges->hi = row_hi, ranges->span = row_span;
+            if (pass != nullptr) pass->lo = row_lo, pass->hi = row_hi, pass->span = row_span;
         } else {
             blt_tensor mask_tensor;
             std::memset(&mask_tensor, 0, sizeof(mask_tensor));
@@ -425,8 +438,11 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
             dense = (const float *)mask_tensor.data;
         }
     }
-    float *k = (float *)blt_arena_alloc(arena, (T ? T : 1) * E * sizeof(float), 64);
-    float *v = (float *)blt_arena_alloc(arena, (T ? T : 1) * E * sizeof(float), 64);
+    const auto rows_of_keys = [&]() { return (float *)blt_arena_alloc(arena, (T ? T : 1) * E * sizeof(float), 64); };
+    bool made = pass != nullptr && pass->made_k != nullptr; /* K and V are there */
+    float *const k = made ? pass->made_k : rows_of_keys();
+    float *const v = made ? pass->made_v : rows_of_keys();
+    if (made) pass->made_k = pass->made_v = nullptr;
 
     MatmulArgs g;
     std::memset(&g, 0, sizeof(g));
@@ -447,7 +463,23 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     whole.rows = whole.rows_per_seq = (uint32_t)P, whole.head_dim = (uint32_t)hd, whole.scale = 1.0f / sqrtf((float)hd);
     /* up to 32 rows the products keep the reference's order of sums */
     if (row_lo != nullptr && P > 32 && T != 0 && row_span <= CROSS_SPAN && cross_block_ok(whole, (uint32_t)E)) {
-        matmul_f32_launch(gkv, 0);
+        if (pass != nullptr && pass->later != nullptr) {
+            pass->later->kv = gkv, pass->later->cross = whole;
+            pass->later->kv_waits = !made, pass->later->cross_waits = true;
+            return;
+        }
+        if (!made && pass != nullptr && pass->next_k != nullptr) {
+            check_2d_fp32(pass->next_k, E, E, "blt_cross_attention: weight_k must be [embed_dim, embed_dim] FP32");
+            check_2d_fp32(pass->next_v, E, E, "blt_cross_attention: weight_v must be [embed_dim, embed_dim] FP32");
+            MatmulArgs more = gkv;
+            more.b = (const float *)pass->next_k->data, more.b2 = (const float *)pass->next_v->data;
+            if (matmul_pair_ok(gkv, more)) {
+                more.out = pass->made_k = rows_of_keys(), more.out2 = pass->made_v = rows_of_keys();
+                matmul_f32_launch_pair(gkv, more, 0);
+                made = true;
+            }
+        }
+        if (!made) matmul_f32_launch(gkv, 0);
         cross_block_launch(whole, (uint32_t)E, 0);
         HIP_CHECK_LAUNCH("blt_cross_attention_forward");
         return;
@@ -470,11 +502,11 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
         g.a = (const float *)normed.data;
         g.norm_w = nullptr;
     }
-    if (T != 0 && matmul_pair_ok(g, gkv)) {
+    if (T != 0 && !made && matmul_pair_ok(g, gkv)) {
         matmul_f32_launch_pair(g, gkv, 0); /* all three in one launch */
     } else {
         matmul_f32_launch(g, 0);
-        if (T != 0) matmul_f32_launch(gkv, 0);
+        if (T != 0 && !made) matmul_f32_launch(gkv, 0);
     }
 
     /* 3. every head in one launch */

@@ -2935,6 +2935,46 @@ def test_local_encoder_forward(name, impl, oracle, dev):
 
 
 
+@pytest.mark.parametrize("T,E,L,k,mean_patch,all_layers,placement", [
+    (300, 128, 3, 1, 4, True, 0), (170, 64, 4, 1, 5, True, 0),      # a cross block behind every layer, all but the last beside the next one
+    (133, 64, 2, 2, 8, True, 0), (1040, 128, 2, 1, 3, True, 0),     # sub-tokens; more workgroups than go along
+    (260, 128, 3, 1, 4, False, 4), (90, 64, 3, 1, 30, True, 0),     # behind the first layer only; too few patches for the launch
+    (230, 256, 2, 1, 5, True, 0), (2300, 64, 2, 1, 64, True, 0)])   # wide; patches of more bytes
+def test_cross_blocks_beside_the_next_layer(T, E, L, k, mean_patch, all_layers, placement, oracle, dev):
+    """The encoder leaves a layer's cross block to the next layer's launches, the decoder makes two layers' keys and values in one:
+    every layer's block against the restated forwards, for shapes that share the launches and shapes that cannot."""
+    import torch
+    from fblt_amd import decoder
+    from tests import encoder_runs
+    from tests.golden import block_cases
+    lib = api.load()
+    c = dict(T=T, E=E, H=E // 32, XH=E // 32, L=L, hidden=2 * E, ngrams=(3,), vocab=64, k=k, window=0, placement=placement,
+             all_layers=all_layers, pool="mean", docs=None, normalize=True, mean_patch=mean_patch)
+    data, lengths, weights = block_cases.encoder_case(np.random.RandomState(T), c)
+    want_p, want_h = encoder_runs.run_oracle(oracle, c, data, lengths, weights)
+    got_p, got_h = encoder_runs.run_device(lib.blt_local_encoder_forward, lib, oracle, c, data, lengths, weights)
+    assert_close(got_h, want_h, "byte_hidden_out")
+    assert_close(got_p, want_p, "patch_out")
+
+    host, device = _decoders(oracle, dict(E=E, H=E // 32, XH=E // 32, L=L, hidden=2 * E, V=64, k=k, window=0, placement=placement,
+                                          all_layers=all_layers, max_len=T), T)
+    P, patches = len(lengths), decoder.patch_table(lengths)
+    want = np.zeros((T, 64), dtype=np.float32)
+    assert oracle.orc_local_decoder_forward(host.ptr, binding.fptr(want_h.reshape(-1)), T, binding.fptr(want_p.reshape(-1)), patches,
+                                            P, None, 0, 0, binding.fptr(want.reshape(-1))) == 0
+    th, tp = torch.from_numpy(want_h).cuda(), torch.from_numpy(want_p).cuda()
+    tl = torch.full((T, 64), 7.0, dtype=torch.float32, device="cuda")
+    vh, vp, vl = _dev_tensor(th), _dev_tensor(tp), _dev_tensor(tl)
+    arena = lib.blt_arena_create(256 << 20, abi.BLT_BACKEND_HIP)
+    try:
+        lib.blt_local_decoder_forward_ext(device.ptr, C.byref(vh), C.byref(vp), patches, P, None, None, None, 0, None, 0,
+                                          C.byref(vl), None, arena)
+        lib.blt_backend_pass_sync_hip()
+    finally:
+        lib.blt_arena_destroy(arena)
+    assert_close(tl.cpu().numpy(), want, "logits")
+
+
 @pytest.mark.parametrize("driver", ["reference_encoder", "library_encoder", "library_stages"])
 @pytest.mark.parametrize("name", ["model_T96", "model_T200_docs_window"])
 def test_model_forward_on_the_library(name, driver, oracle, dev):
