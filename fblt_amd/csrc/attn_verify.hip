@@ -455,7 +455,12 @@ __global__ __launch_bounds__(64 * WAVES, 1) void kv_block16_mfma_kernel(StepArgs
             b = lens.order[at / gridDim.z];
         }
     }
-    const uint32_t split = blockIdx.x;
+    uint32_t split = blockIdx.x;
+    if (a.halves == 2u) { /* the first half stores the new rows, both attend them */
+        split = 0u;
+        a.q0 += 16u * blockIdx.x;
+        a.write_through = a.write_through && blockIdx.x == 0u;
+    }
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); /* uniform, and known to be */
     const uint32_t hshift = (uint32_t)__builtin_ctz(a.hpb);                 /* heads per workgroup: a power of two */
@@ -999,7 +1004,7 @@ void launch_block_as(StepArgs a, uint32_t batch, const uint32_t *host_lens, hipS
         }
     }
     a.slices = std::max(1u, std::min<uint32_t>((uint32_t)WAVES / a.hpb, subs));
-    dim3 grid(a.splits, batch, (a.num_heads + a.hpb - 1) / a.hpb);
+    dim3 grid(a.splits * a.halves, batch, (a.num_heads + a.hpb - 1) / a.hpb);
     const dim3 block(64 * a.hpb * a.slices);
     if (host_lens) {
         for (uint32_t b = 0; b < batch; b++) lens.v[b] = host_lens[b];
@@ -1082,8 +1087,10 @@ uint32_t kv_block_heads_per_group(uint32_t batch, uint32_t subs, uint32_t num_he
 /* Takes head_dim 32 and 64 (the K tiles of four waves fit the static LDS
  * budget); the caller falls back to the VALU kernel otherwise.  Handles up to
  * 32 query rows per launch: a.q0 .. a.q0 + 31. */
-bool kv_block_mfma_launch(const StepArgs &a, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
+bool kv_block_mfma_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
                           hipStream_t s) {
+    StepArgs a = a_in;
+    a.halves = 1u;
     /* the per-wave K tiles bound the workgroups: 8 waves of 4.6 KB or 4 of 8.7 KB */
     /* BLT_HIP_BLOCK_TILE=16 keeps blocks of up to four rows on the 16-wide tiles, =4 keeps the looping
      * kernels (4x4x1 tiles up to four rows, 16-wide above), =once takes the all-at-once kernel wherever
@@ -1098,6 +1105,26 @@ bool kv_block_mfma_launch(const StepArgs &a, uint32_t batch, uint32_t head_dim, 
      * of head width 32 the 4x4x1 kernel, which has no padding rows to multiply, stays ahead (6.4 against
      * 6.9 us). */
     const bool small = head_dim == 32u && a.n - a.q0 <= 4u;
+    /* 17 to 32 rows: as two halves of the 16-wide kernels, a workgroup each, where the compute units would idle or all keys are
+     * requested at once anyway; a workgroup that reads its keys for all rows (32-wide) is ahead again where two would wait
+     * for each other's traffic.  us, 4 heads, 32 rows, 32-wide / halves.  Heads of 32: 1 sequence of up to 300 keys 13.5 / 6.3, 16 of 500
+     * 16.0 / 7.8, 16 of 2000 32.3 / 17.5, 64 of 500 16.5 / 14.3, 200 of 500 43.4 / 33.9, 250 of 100 26.8 / 19.7; 50 of 900 21.8 /
+     * 22.7, 100 of 900 32.6 / 39.8, 64 of 2000 35.2 / 39.2.  Of 64: 1 of 300 21.9 / 9.0, 16 of 2000 58.4 / 34.8, 64 of 400 27.1 / 24.7,
+     * 250 of 60 34.5 / 26.1; 200 of 200 44.9 / 50.6, 128 of 500 44.1 / 49.5.  17 rows of 100 sequences of 500: 21.5 / 20.7. */
+    if (a.n > 16u && a.q0 == 0u && a.splits == 1u && (pin == 0 || pin == 1)) {
+        const uint64_t pairs = (uint64_t)batch * a.num_heads;
+        const uint32_t tiles = (a.span + 15u) / 16u + 2u;
+        const bool idle = 2u * pairs <= 256u;
+        a.halves = 2u;
+        if (pin == 1 || idle || (head_dim == 32u ? tiles <= 48u : pairs <= 256u || tiles <= 8u))
+            if (kv_block_once_launch(a, batch, head_dim, host_lens, s)) return true;
+        if (idle && (head_dim == 32u || head_dim == 64u)) {
+            if (head_dim == 32u) launch_block_as<32, 8, true>(a, batch, host_lens, s);
+            else launch_block_as<64, 4, true>(a, batch, host_lens, s);
+            return true;
+        }
+        a.halves = 1u;
+    }
     if ((pin == 1 || (pin == 0 && !small)) && kv_block_once_launch(a, batch, head_dim, host_lens, s)) return true;
     if (head_dim == 32u) {
         if (a.n - a.q0 <= 4u && !no_tile4) launch_block4(a, batch, host_lens, s);

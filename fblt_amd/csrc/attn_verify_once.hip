@@ -1,5 +1,5 @@
 /*
- * Block step of the KV cache for blocks of at most 16 rows over a prefix short
+ * Block step of the KV cache for blocks of at most 16 rows (32 as two halves, a workgroup each) over a prefix short
  * enough to be in flight all at once (BLT-D/DV draft and verify blocks of 4 ...
  * 16 rows over a few hundred cached keys, csrc/infer/block_generation.c:156-266;
  * chunks of a prompt, csrc/infer/kv_cache.c:229-236).  The attention statements
@@ -10,8 +10,8 @@
  *
  *   - one workgroup per (sequence, head), W = 4, 8, 12 or 16 waves (the launch's
  *     choice: as few as give the longest sequence's tiles a slot); the sequence
- *     is walked as ceil(len / 16) tiles of cached rows followed by ONE tile that
- *     holds the step's new rows, wave w owning tiles w, w + W, ... (T at most).
+ *     is walked as ceil(len / 16) tiles of cached rows followed by the tile (of
+ *     halves two) that holds the step's new rows, wave w owning tiles w, w + W, ... (T at most).
  *     Which of the two a tile is, is uniform over the wave: base pointer, pitch
  *     and row limit are scalar selects;
  *   - every row the wave will need is requested at entry, Q, K and V rows alike
@@ -79,6 +79,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 
     const uint32_t b = blockIdx.y;
     const uint32_t head = blockIdx.z;
+    const uint32_t q0 = 16u * blockIdx.x; /* first query row */
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -91,7 +92,8 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
     if (!KARG && kv_over_capacity(a, nk)) return; /* uniform over the sequence's workgroups */
     const size_t slab = (size_t)b * a.max_seq_len;
     const size_t newrow0 = (size_t)b * a.n_seq;
-    const uint32_t cached_tiles = (len + 15u) / 16u; /* then the tile with the new rows */
+    const uint32_t cached_tiles = (len + 15u) / 16u; /* then the tile or two with the new rows */
+    const uint32_t last_tile = cached_tiles + (a.n - 1u) / 16u;
 
     const float *const cache_k = a.cache_k + slab * a.embed_dim + head * HD;
     const float *const cache_v = a.cache_v + slab * a.embed_dim + head * HD;
@@ -106,28 +108,28 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
         const char *qb = reinterpret_cast<const char *>(a.q_rows + newrow0 * a.q_stride + head * HD);
 #pragma unroll
         for (int v = 0; v < NV; v++)
-            qg[v] = *reinterpret_cast<const floatx4 *>(qb + min(prow + (uint32_t)(RPI * v), last_new) * (a.q_stride * 4u) + 16u * pf);
+            qg[v] = *reinterpret_cast<const floatx4 *>(qb + min(q0 + prow + (uint32_t)(RPI * v), last_new) * (a.q_stride * 4u) + 16u * pf);
     }
     floatx4 vg[T][NV];
 #pragma unroll
     for (int u = 0; u < T; u++) {
         /* a tile past the sequence's last repeats it: the loads hit the cache, nothing is computed */
-        const uint32_t ti = min(wave + W * u, cached_tiles);
-        const bool fresh = ti == cached_tiles; /* wave-uniform: scalar selects */
+        const uint32_t ti = min(wave + W * u, last_tile);
+        const bool fresh = ti >= cached_tiles; /* wave-uniform: scalar selects */
         const char *kb = reinterpret_cast<const char *>(fresh ? new_k : cache_k);
         const uint32_t kp = fresh ? newk_pitch : cache_pitch;
-        const uint32_t row0 = fresh ? 0u : ti * 16u, limit = fresh ? last_new : last_cached;
+        const uint32_t row0 = 16u * (fresh ? ti - cached_tiles : ti), limit = fresh ? last_new : last_cached;
 #pragma unroll
         for (int v = 0; v < NV; v++)
             kg[u][v] = *reinterpret_cast<const floatx4 *>(kb + min(row0 + prow + (uint32_t)(RPI * v), limit) * kp + 16u * pf);
     }
 #pragma unroll
     for (int u = 0; u < T; u++) {
-        const uint32_t ti = min(wave + W * u, cached_tiles);
-        const bool fresh = ti == cached_tiles;
+        const uint32_t ti = min(wave + W * u, last_tile);
+        const bool fresh = ti >= cached_tiles;
         const char *vb = reinterpret_cast<const char *>(fresh ? new_v : cache_v);
         const uint32_t vp = fresh ? newv_pitch : cache_pitch;
-        const uint32_t row0 = fresh ? 0u : ti * 16u, limit = fresh ? last_new : last_cached;
+        const uint32_t row0 = 16u * (fresh ? ti - cached_tiles : ti), limit = fresh ? last_new : last_cached;
 #pragma unroll
         for (int v = 0; v < NV; v++)
             vg[u][v] = *reinterpret_cast<const floatx4 *>(vb + min(row0 + prow + (uint32_t)(RPI * v), limit) * vp + 16u * pf);
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
     if (a.rope_cos) {
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            const size_t at = (size_t)(len + min(prow + (uint32_t)(RPI * v), last_new)) * HALF + 2u * pf;
+            const size_t at = (size_t)(len + min(q0 + prow + (uint32_t)(RPI * v), last_new)) * HALF + 2u * pf;
             const float4 t = rope_rotate4(make_float4(qg[v][0], qg[v][1], qg[v][2], qg[v][3]), a.rope_cos + at, a.rope_sin + at);
             qg[v][0] = t.x, qg[v][1] = t.y, qg[v][2] = t.z, qg[v][3] = t.w;
         }
@@ -156,10 +158,12 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 #pragma unroll
     for (int u = 0; u < T; u++) {
         const uint32_t ti = wave + W * u;
-        if (ti == cached_tiles) { /* this wave holds the new rows */
+        if (ti >= cached_tiles) { /* new rows; of two tiles a half stores its own */
+            const uint32_t row0 = 16u * (ti - cached_tiles);
+            const bool store = a.write_through && row0 == q0;
 #pragma unroll
             for (int v = 0; v < NV; v++) {
-                const uint32_t r = prow + (uint32_t)(RPI * v);
+                const uint32_t r = row0 + prow + (uint32_t)(RPI * v);
                 const bool real = r < a.n;
                 if (a.rope_cos && real) {
                     const size_t at = (size_t)(len + r) * HALF + 2u * pf;
@@ -167,7 +171,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
                                                   a.rope_cos + at, a.rope_sin + at);
                     kg[u][v][0] = t.x, kg[u][v][1] = t.y, kg[u][v][2] = t.z, kg[u][v][3] = t.w;
                 }
-                if (a.write_through && real) {
+                if (store && real) {
                     const size_t at = (slab + len + r) * a.embed_dim + head * HD + 4u * pf;
                     *reinterpret_cast<floatx4 *>(a.cache_k + at) = kg[u][v];
                     *reinterpret_cast<floatx4 *>(a.cache_v + at) = vg[u][v];
@@ -189,11 +193,11 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
      * (kv_cache.c:229-236), padding rows nothing */
     uint32_t vis_lo = 0, vis_hi = nk;
     if (!a.block_kind) {
-        const uint32_t qpos = len + c;
+        const uint32_t qpos = len + q0 + c;
         vis_hi = min(vis_hi, qpos + 1u);
         if (a.window > 0u && qpos + 1u > a.window) vis_lo = qpos + 1u - a.window;
     }
-    if (c >= a.n) vis_hi = 0;
+    if (q0 + c >= a.n) vis_hi = 0;
     const float scale2 = a.scale * LOG2E; /* log2 units: weights are 2^(x - max) */
 
     /* ---- phase 1: scores of the wave's tiles, the wave's maximum per query ---- */
@@ -202,7 +206,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
     bool on[T], all_on = true;
 #pragma unroll
     for (int u = 0; u < T; u++) {
-        on[u] = wave + W * u <= cached_tiles;
+        on[u] = wave + W * u <= last_tile;
         all_on = all_on & on[u];
 #pragma unroll
         for (int k = 0; k < NA; k++) sa[u][k] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -254,8 +258,8 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 #pragma unroll
     for (int u = 0; u < T; u++) {
         const uint32_t ti = wave + W * u;
-        const bool fresh = ti == cached_tiles;
-        const uint32_t j0 = fresh ? len : ti * 16u; /* absolute position of the tile's first key */
+        const bool fresh = ti >= cached_tiles;
+        const uint32_t j0 = fresh ? len + 16u * (ti - cached_tiles) : ti * 16u; /* absolute position of the tile's first key */
         const uint32_t j_end = fresh ? nk : len;    /* rows past it are clamped repeats */
         const uint32_t hi = min(vis_hi, j_end);
         const uint32_t span = on[u] && hi > vis_lo ? hi - vis_lo : 0u;
@@ -335,9 +339,9 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
             o.x += t.x * f, o.y += t.y * f, o.z += t.z * f, o.w += t.w * f;
         }
         L = key_sum<4>(L), o.x = key_sum<4>(o.x), o.y = key_sum<4>(o.y), o.z = key_sum<4>(o.z), o.w = key_sum<4>(o.w);
-        if (part == 0u && mr < a.n) {
+        if (part == 0u && q0 + mr < a.n) {
             const float inv = L > 0.f ? 1.0f / L : 0.f;
-            *reinterpret_cast<float4 *>(a.combined + (newrow0 + mr) * a.out_stride + head * HD + 4u * mf) =
+            *reinterpret_cast<float4 *>(a.combined + (newrow0 + q0 + mr) * a.out_stride + head * HD + 4u * mf) =
                 make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
         }
     }
@@ -347,7 +351,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 template <int HD, int T>
 void block_once_launch_as(const StepArgs &a, uint32_t batch, uint32_t waves, const uint32_t *host_lens, hipStream_t s) {
     using Shape = BlockOnceShape<HD>;
-    const dim3 grid(1, batch, a.num_heads), block(64 * waves);
+    const dim3 grid(a.halves, batch, a.num_heads), block(64 * waves);
     const size_t lds = Shape::bytes(waves);
     if (host_lens) {
         static const bool raised = [] {
@@ -372,13 +376,13 @@ void block_once_launch_as(const StepArgs &a, uint32_t batch, uint32_t waves, con
 
 } // namespace
 
-/* Launch of the once block kernel: at most 16 rows per sequence from row 0 on, one split, and a prefix
- * whose 16-key tiles (plus the one with the new rows) fit the waves' registers; false when it does
+/* Launch of the once block kernel: at most 16 rows per sequence from row 0 on, 32 by halves, one split, and a prefix
+ * whose 16-key tiles (plus those with the new rows) fit the waves' registers; false when it does
  * not take the shape.  host_lens: NULL (device lengths) or `batch` <= KARG_SEQS lengths. */
 bool kv_block_once_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
                           hipStream_t s) {
-    if (a_in.q0 != 0u || a_in.n > 16u || a_in.n == 0u || a_in.splits != 1u) return false;
-    const uint32_t tiles = (a_in.span + 15u) / 16u + 1u; /* what the longest sequence of the launch may need */
+    if (a_in.q0 != 0u || a_in.n > 16u * a_in.halves || a_in.n == 0u || a_in.splits != 1u) return false;
+    const uint32_t tiles = (a_in.span + 15u) / 16u + a_in.halves; /* what the longest sequence of the launch may need */
     const uint32_t per_wave = (tiles + 15u) / 16u;       /* tiles a wave holds at once */
     /* as few waves as give every tile a slot, in fours: a slot without a tile still costs its requests */
     const uint32_t waves = std::min(16u, ((tiles + per_wave - 1u) / per_wave + 3u) / 4u * 4u);

@@ -36,7 +36,8 @@ struct StepArgs {
     uint32_t len_bias; /* rows of the same step already written through by earlier launches:
                           the sequence's length for this launch is self_len[b] + len_bias */
     uint32_t q0;       /* first query row this launch handles */
-    uint32_t splits;   /* gridDim.x */
+    uint32_t splits;   /* gridDim.x, but for launches by halves */
+    uint32_t halves;   /* 2: workgroup x of a sequence's (one split) takes the 16 query rows from q0 + 16 x on */
     uint32_t span;     /* keys per split, a multiple of SUB */
     uint32_t cap;      /* most keys (cached + new) a sequence may attend in this launch: what the slab, the
                           launch's splits * span and the rotation tables all hold */
@@ -137,7 +138,7 @@ __device__ __forceinline__ float observe(const float *p) {
  * for its own stores to complete before the barrier that precedes the
  * workgroup's ticket. */
 /* The step commits, has one split per sequence but several workgroups (head
- * groups): all that has to be known is when every workgroup of the sequence
+ * groups, halves): all that has to be known is when every workgroup of the sequence
  * has read the old length.  Thread 0 of each workgroup draws its ticket at a
  * point where all its waves have done that read (after the barrier that ends
  * the key loop) -- the reply travels while the workgroup merges and stores --
@@ -145,7 +146,7 @@ __device__ __forceinline__ float observe(const float *p) {
  * the ticket (thread 0 only; KV_NO_TICKET when this scheme does not apply). */
 constexpr uint32_t KV_NO_TICKET = 0xFFFFFFFFu;
 __device__ __forceinline__ bool kv_early_ticket_applies(const StepArgs &a) {
-    return a.splits == 1u && gridDim.z > 1u && a.commit;
+    return a.splits == 1u && gridDim.x * gridDim.z > 1u && a.commit;
 }
 __device__ __forceinline__ uint32_t kv_draw_early_ticket(const StepArgs &a, uint32_t b) {
     if (!kv_early_ticket_applies(a) || threadIdx.x != 0) return KV_NO_TICKET;
@@ -155,14 +156,14 @@ __device__ __forceinline__ uint32_t kv_draw_early_ticket(const StepArgs &a, uint
 template <int HD>
 __device__ __forceinline__ void kv_finish_sequence(const StepArgs &a, uint32_t slots, uint32_t b, uint32_t nk,
                                                    uint32_t *sm_ticket, uint32_t early_ticket) {
-    if (a.splits == 1u && (gridDim.z == 1u || !a.commit)) {
+    if (a.splits == 1u && (gridDim.x * gridDim.z == 1u || !a.commit)) {
         /* the output rows are written; the ticket is only needed to tell when the
          * last workgroup of the sequence has read the old length */
         if (a.commit && threadIdx.x == 0) a.self_len[b] = nk;
         return;
     }
     if (kv_early_ticket_applies(a)) {
-        if (threadIdx.x == 0 && early_ticket == gridDim.z - 1u) {
+        if (threadIdx.x == 0 && early_ticket == gridDim.x * gridDim.z - 1u) {
             a.tickets[b] = 0u; /* re-armed for the next launch */
             a.self_len[b] = nk;
         }

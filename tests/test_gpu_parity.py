@@ -735,6 +735,34 @@ def test_rope_position_gather(dev):
     assert (got_c == cos[pos]).all() and (got_s == sin[pos]).all()
 
 
+@pytest.mark.parametrize("lens", ["host", "device"])
+@pytest.mark.parametrize("batch,H,hd,n,lo,hi,kind,window,kernel", [
+    (3, 4, 32, 17, 1, 3, "block", 0, "kv_block_once"), (9, 4, 32, 32, 0, 150, "causal", 0, "kv_block_once"),
+    (5, 1, 32, 31, 20, 300, "causal", 40, "kv_block_once"), (9, 4, 32, 18, 0, 150, "causal", 9, "kv_block_once"),
+    (2, 2, 64, 25, 100, 380, "block", 0, "kv_block_once"), (70, 4, 64, 17, 10, 70, "causal", 0, "kv_block_once"),
+    (33, 4, 32, 20, 500, 690, "block", 0, "kv_block_once"), (33, 4, 32, 20, 500, 760, "block", 0, "kv_block_mfma"),   # past 48 tiles
+    (32, 4, 32, 20, 500, 960, "block", 0, "kv_block_once"), (32, 4, 32, 17, 500, 1100, "causal", 700, "kv_block16_mfma"),
+    (3, 1, 64, 32, 300, 700, "causal", 0, "kv_block16_mfma"), (33, 4, 64, 32, 400, 600, "block", 0, "kv_block_mfma"),
+    (66, 4, 64, 32, 150, 200, "causal", 0, "kv_block_mfma"), (1, 3, 32, 32, 2000, 2300, "causal", 0, "kv_block_mfma")])
+def test_kv_steps_of_two_row_tiles(batch, H, hd, n, lo, hi, kind, window, kernel, lens, dev, oracle):
+    """Steps of 17 to 32 rows: a sequence's rows as two halves, a workgroup each, or all in one, by the rule's lines.  Two steps that
+    commit, rows rotated inside; outputs against the restated step, the cache's rows bit for bit (either half stores), and the
+    lengths that the last of a sequence's workgroups advances."""
+    kw = workloads.config5(batch=batch, B=n, H=H, hd=hd, len_lo=lo, len_hi=hi, max_seq_len=hi + 2 * n, steps=2, rope=True)
+    kw.kind, kw.window, kw.commit = kind, window, True
+    ref_out, ref_k, ref_v = orunner.run_kv(kw, lib=oracle)
+    d = dev.DeviceKvWorkload(kw, lens=lens)
+    lib = api.load()
+    lib.blt_hip_profile_begin()
+    d.run()
+    names = [name for name in api.profile_end() if name.startswith("kv_block")]
+    out, ck, cv, got_lens = d.results()
+    assert kernel in names, names  # the second step sees more keys
+    assert_close(out, ref_out, "step rows")
+    assert ck.tobytes() == ref_k.tobytes() and cv.tobytes() == ref_v.tobytes()
+    assert (np.asarray(got_lens).astype(np.int64) == kw.lens.astype(np.int64) + 2 * n).all()
+
+
 @pytest.mark.parametrize("kernel", ["valu", "mfma", "mfma_once", "mfma_loop", "mfma32"])
 def test_kv_step_kernel_families_agree(kernel):
     """The kernels behind the KV step entry points (VALU; matrix-core as routed; the all-at-once kernel
