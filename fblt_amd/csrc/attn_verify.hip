@@ -423,7 +423,8 @@ __device__ __forceinline__ void kv_merge_slices(const StepArgs &a, const float (
  *     between counts exactly the newer requests;
  *   - cross-lane maxima and sums use the row swaps of the vector ALU, not the LDS crossbar;
  *   - the slices meet once in LDS; the merge issues all of a cell's reads before it adds. */
-template <int HD, int WAVES, bool KARG>
+/* HALVES: two workgroups for 16 query rows each of up to 32, one split */
+template <int HD, int WAVES, bool KARG, bool HALVES>
 __global__ __launch_bounds__(64 * WAVES, 1) void kv_block16_mfma_kernel(StepArgs a, LensArg<KARG> lens) {
     kv_fetch_arguments(a);
     constexpr int HALF = HD / 2;
@@ -455,9 +456,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void kv_block16_mfma_kernel(StepArgs
             b = lens.order[at / gridDim.z];
         }
     }
-    uint32_t split = blockIdx.x;
-    if (a.halves == 2u) { /* the first half stores the new rows, both attend them */
-        split = 0u;
+    const uint32_t split = HALVES ? 0u : blockIdx.x;
+    if constexpr (HALVES) { /* the first half stores the new rows, both attend them */
         a.q0 += 16u * blockIdx.x;
         a.write_through = a.write_through && blockIdx.x == 0u;
     }
@@ -683,11 +683,11 @@ __global__ __launch_bounds__(64 * WAVES, 1) void kv_block16_mfma_kernel(StepArgs
     }
     if (g == 0) *reinterpret_cast<float2 *>(mine + c * LPR + HD) = make_float2(m * LN2, l); /* merges work in natural units */
     __syncthreads();
-    const uint32_t early_ticket = kv_draw_early_ticket(a, b); /* as in the 32-wide kernel */
+    const uint32_t early_ticket = kv_draw_early_ticket(a, b, HALVES ? 2u * gridDim.z : gridDim.z); /* as in the 32-wide kernel */
 
     kv_merge_slices<HD, WAVES, LPR, (int)ROWS, 32 * KROW>(a, sm_o, hshift, wave, b, split, newrow0, zblock);
 
-    kv_finish_sequence<HD>(a, (uint32_t)SLOTS, b, nk, &sm_ticket, early_ticket);
+    kv_finish_sequence<HD>(a, (uint32_t)SLOTS, b, nk, &sm_ticket, early_ticket, HALVES ? 2u * gridDim.z : gridDim.z);
 }
 
 /* The same step for blocks of at most 4 rows and head width 32 on 4x4x1 tiles
@@ -976,7 +976,7 @@ __global__ __launch_bounds__(64 * MAXW, 1) void kv_block4_mfma_kernel(StepArgs a
     kv_finish_sequence<HD>(a, (uint32_t)SLOTS, b, nk, &sm_ticket, early_ticket);
 }
 
-template <int HD, int WAVES, bool NARROW>
+template <int HD, int WAVES, bool NARROW, bool HALVES = false>
 void launch_block_as(StepArgs a, uint32_t batch, const uint32_t *host_lens, hipStream_t s) {
     /* a.hpb heads per workgroup (the caller's choice, see kv_block_heads_per_group; a power of two);
      * the other waves are slices */
@@ -1004,15 +1004,15 @@ void launch_block_as(StepArgs a, uint32_t batch, const uint32_t *host_lens, hipS
         }
     }
     a.slices = std::max(1u, std::min<uint32_t>((uint32_t)WAVES / a.hpb, subs));
-    dim3 grid(a.splits * a.halves, batch, (a.num_heads + a.hpb - 1) / a.hpb);
+    dim3 grid(HALVES ? 2u : a.splits, batch, (a.num_heads + a.hpb - 1) / a.hpb);
     const dim3 block(64 * a.hpb * a.slices);
     if (host_lens) {
         for (uint32_t b = 0; b < batch; b++) lens.v[b] = host_lens[b];
-        if constexpr (NARROW) blt_launch("kv_block16_mfma", kv_block16_mfma_kernel<HD, WAVES, true>, grid, block, 0, s, a, lens);
+        if constexpr (NARROW) blt_launch("kv_block16_mfma", kv_block16_mfma_kernel<HD, WAVES, true, HALVES>, grid, block, 0, s, a, lens);
         else blt_launch("kv_block_mfma", kv_block_mfma_kernel<HD, WAVES, true>, grid, block, 0, s, a, lens);
     } else {
         const DeviceLens lens{0u};
-        if constexpr (NARROW) blt_launch("kv_block16_mfma", kv_block16_mfma_kernel<HD, WAVES, false>, grid, block, 0, s, a, lens);
+        if constexpr (NARROW) blt_launch("kv_block16_mfma", kv_block16_mfma_kernel<HD, WAVES, false, HALVES>, grid, block, 0, s, a, lens);
         else blt_launch("kv_block_mfma", kv_block_mfma_kernel<HD, WAVES, false>, grid, block, 0, s, a, lens);
     }
 }
@@ -1119,8 +1119,8 @@ bool kv_block_mfma_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_di
         if (pin == 1 || idle || (head_dim == 32u ? tiles <= 48u : pairs <= 256u || tiles <= 8u))
             if (kv_block_once_launch(a, batch, head_dim, host_lens, s)) return true;
         if (idle && (head_dim == 32u || head_dim == 64u)) {
-            if (head_dim == 32u) launch_block_as<32, 8, true>(a, batch, host_lens, s);
-            else launch_block_as<64, 4, true>(a, batch, host_lens, s);
+            if (head_dim == 32u) launch_block_as<32, 8, true, true>(a, batch, host_lens, s);
+            else launch_block_as<64, 4, true, true>(a, batch, host_lens, s);
             return true;
         }
         a.halves = 1u;

@@ -57,7 +57,8 @@ struct BlockOnceShape {
     static constexpr size_t bytes(uint32_t waves) { return (size_t)(STATS + waves * 16 * ROW) * sizeof(float); }
 };
 
-template <int HD, int T, bool KARG>
+/* HALVES: two workgroups a (sequence, head), 16 query rows each, and two tiles of new rows */
+template <int HD, int T, bool KARG, bool HALVES>
 __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg<KARG> lens) {
     kv_fetch_arguments(a);
     using Shape = BlockOnceShape<HD>;
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 
     const uint32_t b = blockIdx.y;
     const uint32_t head = blockIdx.z;
-    const uint32_t q0 = 16u * blockIdx.x; /* first query row */
+    const uint32_t q0 = HALVES ? 16u * blockIdx.x : 0u; /* first query row */
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
     const size_t slab = (size_t)b * a.max_seq_len;
     const size_t newrow0 = (size_t)b * a.n_seq;
     const uint32_t cached_tiles = (len + 15u) / 16u; /* then the tile or two with the new rows */
-    const uint32_t last_tile = cached_tiles + (a.n - 1u) / 16u;
+    const uint32_t last_tile = HALVES ? cached_tiles + 1u : cached_tiles;
 
     const float *const cache_k = a.cache_k + slab * a.embed_dim + head * HD;
     const float *const cache_v = a.cache_v + slab * a.embed_dim + head * HD;
@@ -115,10 +116,10 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
     for (int u = 0; u < T; u++) {
         /* a tile past the sequence's last repeats it: the loads hit the cache, nothing is computed */
         const uint32_t ti = min(wave + W * u, last_tile);
-        const bool fresh = ti >= cached_tiles; /* wave-uniform: scalar selects */
+        const bool fresh = HALVES ? ti >= cached_tiles : ti == cached_tiles; /* wave-uniform: scalar selects */
         const char *kb = reinterpret_cast<const char *>(fresh ? new_k : cache_k);
         const uint32_t kp = fresh ? newk_pitch : cache_pitch;
-        const uint32_t row0 = 16u * (fresh ? ti - cached_tiles : ti), limit = fresh ? last_new : last_cached;
+        const uint32_t row0 = fresh ? (HALVES ? 16u * (ti - cached_tiles) : 0u) : ti * 16u, limit = fresh ? last_new : last_cached;
 #pragma unroll
         for (int v = 0; v < NV; v++)
             kg[u][v] = *reinterpret_cast<const floatx4 *>(kb + min(row0 + prow + (uint32_t)(RPI * v), limit) * kp + 16u * pf);
@@ -126,10 +127,10 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 #pragma unroll
     for (int u = 0; u < T; u++) {
         const uint32_t ti = min(wave + W * u, last_tile);
-        const bool fresh = ti >= cached_tiles;
+        const bool fresh = HALVES ? ti >= cached_tiles : ti == cached_tiles;
         const char *vb = reinterpret_cast<const char *>(fresh ? new_v : cache_v);
         const uint32_t vp = fresh ? newv_pitch : cache_pitch;
-        const uint32_t row0 = 16u * (fresh ? ti - cached_tiles : ti), limit = fresh ? last_new : last_cached;
+        const uint32_t row0 = fresh ? (HALVES ? 16u * (ti - cached_tiles) : 0u) : ti * 16u, limit = fresh ? last_new : last_cached;
 #pragma unroll
         for (int v = 0; v < NV; v++)
             vg[u][v] = *reinterpret_cast<const floatx4 *>(vb + min(row0 + prow + (uint32_t)(RPI * v), limit) * vp + 16u * pf);
@@ -158,8 +159,8 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 #pragma unroll
     for (int u = 0; u < T; u++) {
         const uint32_t ti = wave + W * u;
-        if (ti >= cached_tiles) { /* new rows; of two tiles a half stores its own */
-            const uint32_t row0 = 16u * (ti - cached_tiles);
+        if (HALVES ? ti == cached_tiles || ti == last_tile : ti == cached_tiles) { /* new rows; of two tiles a half stores its own */
+            const uint32_t row0 = HALVES ? 16u * (ti - cached_tiles) : 0u;
             const bool store = a.write_through && row0 == q0;
 #pragma unroll
             for (int v = 0; v < NV; v++) {
@@ -258,8 +259,8 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 #pragma unroll
     for (int u = 0; u < T; u++) {
         const uint32_t ti = wave + W * u;
-        const bool fresh = ti >= cached_tiles;
-        const uint32_t j0 = fresh ? len + 16u * (ti - cached_tiles) : ti * 16u; /* absolute position of the tile's first key */
+        const bool fresh = HALVES ? ti >= cached_tiles : ti == cached_tiles;
+        const uint32_t j0 = fresh ? (HALVES ? len + 16u * (ti - cached_tiles) : len) : ti * 16u; /* absolute position of the tile's first key */
         const uint32_t j_end = fresh ? nk : len;    /* rows past it are clamped repeats */
         const uint32_t hi = min(vis_hi, j_end);
         const uint32_t span = on[u] && hi > vis_lo ? hi - vis_lo : 0u;
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
     }
     __syncthreads();
     /* every wave of the workgroup has read the old length: draw the sequence's ticket now, look at it last */
-    const uint32_t early_ticket = kv_draw_early_ticket(a, b);
+    const uint32_t early_ticket = kv_draw_early_ticket(a, b, HALVES ? 2u * gridDim.z : gridDim.z);
 
     /* ---- phase 3: four threads per (row, 16-byte piece of the row), each folds every fourth wave's
      * partial, scaled to the row's maximum over all waves; the four meet inside their quad of lanes ---- */
@@ -345,33 +346,39 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
                 make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
         }
     }
-    kv_finish_sequence<HD>(a, 16u, b, nk, &sm_ticket, early_ticket);
+    kv_finish_sequence<HD>(a, 16u, b, nk, &sm_ticket, early_ticket, HALVES ? 2u * gridDim.z : gridDim.z);
 }
 
-template <int HD, int T>
-void block_once_launch_as(const StepArgs &a, uint32_t batch, uint32_t waves, const uint32_t *host_lens, hipStream_t s) {
+template <int HD, int T, bool HALVES>
+void block_once_launch_with(const StepArgs &a, uint32_t batch, uint32_t waves, const uint32_t *host_lens, hipStream_t s) {
     using Shape = BlockOnceShape<HD>;
     const dim3 grid(a.halves, batch, a.num_heads), block(64 * waves);
     const size_t lds = Shape::bytes(waves);
     if (host_lens) {
         static const bool raised = [] {
-            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&kv_block_once_kernel<HD, T, true>),
+            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&kv_block_once_kernel<HD, T, true, HALVES>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)Shape::bytes(Shape::WMAX)));
             return true;
         }();
         (void)raised;
         KargLens lens;
         for (uint32_t b = 0; b < batch; b++) lens.v[b] = host_lens[b];
-        blt_launch("kv_block_once", kv_block_once_kernel<HD, T, true>, grid, block, lds, s, a, lens);
+        blt_launch("kv_block_once", kv_block_once_kernel<HD, T, true, HALVES>, grid, block, lds, s, a, lens);
     } else {
         static const bool raised = [] {
-            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&kv_block_once_kernel<HD, T, false>),
+            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&kv_block_once_kernel<HD, T, false, HALVES>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)Shape::bytes(Shape::WMAX)));
             return true;
         }();
         (void)raised;
-        blt_launch("kv_block_once", kv_block_once_kernel<HD, T, false>, grid, block, lds, s, a, DeviceLens{0u});
+        blt_launch("kv_block_once", kv_block_once_kernel<HD, T, false, HALVES>, grid, block, lds, s, a, DeviceLens{0u});
     }
+}
+
+template <int HD, int T>
+void block_once_launch_as(const StepArgs &a, uint32_t batch, uint32_t waves, const uint32_t *host_lens, hipStream_t s) {
+    if (a.halves == 2u) block_once_launch_with<HD, T, true>(a, batch, waves, host_lens, s);
+    else block_once_launch_with<HD, T, false>(a, batch, waves, host_lens, s);
 }
 
 } // namespace

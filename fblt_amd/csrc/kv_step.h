@@ -37,7 +37,6 @@ struct StepArgs {
                           the sequence's length for this launch is self_len[b] + len_bias */
     uint32_t q0;       /* first query row this launch handles */
     uint32_t splits;   /* gridDim.x, but for launches by halves */
-    uint32_t halves;   /* 2: workgroup x of a sequence's (one split) takes the 16 query rows from q0 + 16 x on */
     uint32_t span;     /* keys per split, a multiple of SUB */
     uint32_t cap;      /* most keys (cached + new) a sequence may attend in this launch: what the slab, the
                           launch's splits * span and the rotation tables all hold */
@@ -49,6 +48,7 @@ struct StepArgs {
     int commit;        /* advance self_len when the sequence is done */
     int by_length;     /* block step with the lengths in the arguments: workgroups take the (sequence, head
                           group) pairs in the order of KargLens::order, longest sequences first */
+    uint32_t halves;   /* 2: (launcher) workgroup x of a sequence's (one split) takes the 16 query rows from q0 + 16 x on */
 };
 
 
@@ -142,28 +142,28 @@ __device__ __forceinline__ float observe(const float *p) {
  * has read the old length.  Thread 0 of each workgroup draws its ticket at a
  * point where all its waves have done that read (after the barrier that ends
  * the key loop) -- the reply travels while the workgroup merges and stores --
- * and the one that drew the last ticket writes the new length when it is done.  Returns
- * the ticket (thread 0 only; KV_NO_TICKET when this scheme does not apply). */
+ * and the one that drew the last of the sequence's `workgroups` tickets (twice gridDim.z by halves) writes the new length when it is
+ * done.  Returns the ticket (thread 0 only; KV_NO_TICKET when this scheme does not apply). */
 constexpr uint32_t KV_NO_TICKET = 0xFFFFFFFFu;
-__device__ __forceinline__ bool kv_early_ticket_applies(const StepArgs &a) {
-    return a.splits == 1u && gridDim.x * gridDim.z > 1u && a.commit;
+__device__ __forceinline__ bool kv_early_ticket_applies(const StepArgs &a, uint32_t workgroups) {
+    return a.splits == 1u && workgroups > 1u && a.commit;
 }
-__device__ __forceinline__ uint32_t kv_draw_early_ticket(const StepArgs &a, uint32_t b) {
-    if (!kv_early_ticket_applies(a) || threadIdx.x != 0) return KV_NO_TICKET;
+__device__ __forceinline__ uint32_t kv_draw_early_ticket(const StepArgs &a, uint32_t b, uint32_t workgroups = gridDim.z) {
+    if (!kv_early_ticket_applies(a, workgroups) || threadIdx.x != 0) return KV_NO_TICKET;
     return __hip_atomic_fetch_add(&a.tickets[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <int HD>
 __device__ __forceinline__ void kv_finish_sequence(const StepArgs &a, uint32_t slots, uint32_t b, uint32_t nk,
-                                                   uint32_t *sm_ticket, uint32_t early_ticket) {
-    if (a.splits == 1u && (gridDim.x * gridDim.z == 1u || !a.commit)) {
+                                                   uint32_t *sm_ticket, uint32_t early_ticket, uint32_t workgroups = gridDim.z) {
+    if (a.splits == 1u && (workgroups == 1u || !a.commit)) {
         /* the output rows are written; the ticket is only needed to tell when the
          * last workgroup of the sequence has read the old length */
         if (a.commit && threadIdx.x == 0) a.self_len[b] = nk;
         return;
     }
-    if (kv_early_ticket_applies(a)) {
-        if (threadIdx.x == 0 && early_ticket == gridDim.x * gridDim.z - 1u) {
+    if (kv_early_ticket_applies(a, workgroups)) {
+        if (threadIdx.x == 0 && early_ticket == workgroups - 1u) {
             a.tickets[b] = 0u; /* re-armed for the next launch */
             a.self_len[b] = nk;
         }
