@@ -166,18 +166,6 @@ void check_weight(const blt_tensor *t, size_t rows, size_t cols, const char *wha
                 "%s (the HIP backend takes FP32 device weights only)", what);
 }
 
-/* The decoder step and layer take their projections on the matrix cores whatever the row count
- * (fp32 tolerance, as they always did above 32 rows).  BLT_HIP_EXACT_STEP=1 keeps the exact
- * thread-per-column kernel for steps of up to 32 rows (results bit-identical to the CPU
- * reference, about 1.5 times the time). */
-uint32_t step_tolerant() {
-    static const uint32_t on = [] {
-        const char *e = getenv("BLT_HIP_EXACT_STEP");
-        return (e && atoi(e) == 1) ? 0u : 1u;
-    }();
-    return on;
-}
-
 /* out = a * b (+ residual), or silu(a * gate_w) .* (a * b) with gate_w set */
 void gemm(const float *a, const float *b, float *out, size_t m, size_t k, size_t n, const float *residual = nullptr,
           const float *gate_w = nullptr, const float *norm_w = nullptr) {
@@ -187,7 +175,7 @@ void gemm(const float *a, const float *b, float *out, size_t m, size_t k, size_t
     g.residual = residual, g.b2 = gate_w, g.norm_w = norm_w;
     g.m = (uint32_t)m, g.k = (uint32_t)k, g.n = (uint32_t)n;
     g.lda = (uint32_t)k, g.ldb = (uint32_t)n, g.ldo = (uint32_t)n;
-    g.tolerant = step_tolerant();
+    g.tolerant = matmul_tolerant();
     matmul_f32_launch(g, 0);
 }
 
@@ -248,7 +236,7 @@ void long_chunk_qkv(const blt_kv_attn_cache *cache, const float *rows_in, const 
     g.rope_cos = rope_cos, g.rope_sin = rope_sin, g.rope_cols = (uint32_t)(2 * E), g.head_dim = (uint32_t)(E / cache->num_heads);
     g.stage_k = cache->self_k, g.stage_v = cache->self_v, g.stage_len = cache->self_len;
     g.stage_slab_rows = cache->max_seq_len, g.stage_n = (uint32_t)n;
-    g.tolerant = step_tolerant();
+    g.tolerant = matmul_tolerant();
     matmul_f32_launch(g, 0);
 }
 
@@ -333,7 +321,7 @@ void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_wei
     MatmulArgs probe;
     std::memset(&probe, 0, sizeof(probe));
     probe.m = (uint32_t)rows, probe.k = (uint32_t)E;
-    probe.tolerant = step_tolerant();
+    probe.tolerant = matmul_tolerant();
     /* self-attention block, kv_cache.c:326-394 */
     probe.n = (uint32_t)(3 * E);
     const bool chunk = host_base != nullptr && n > 32 && step_kind == BLT_KV_STEP_CAUSAL && commit == 0 && dev_positions == nullptr &&
@@ -367,7 +355,7 @@ void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_wei
                                         rope_positions, combined, E, n, step_kind, commit, max_len_hint);
         }
     }
-    if (rows > 32 || step_tolerant()) { /* up to 32 rows the products keep the reference's order of sums unless told otherwise */
+    if (rows > 32 || matmul_tolerant()) { /* up to 32 rows the products keep the reference's order of sums unless told otherwise */
         BlockTailArgs t;
         std::memset(&t, 0, sizeof(t));
         t.comb = combined, t.x = rows_in, t.proj = f32(w->attn_proj_w), t.norm_w = f32(w->norm2_weight);
@@ -497,7 +485,7 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
                 BLT_REQUIRE(positions[b * n + r] < cfg->max_seq_len, "rope_position_gather: position index out of range");
                 own_positions = own_positions || positions[b * n + r] != base[b] + r;
             }
-    if (step_tolerant()) {
+    if (matmul_tolerant()) {
         check_layers(dec, E);
         bool crosses[64];
         StepResident st;
@@ -564,7 +552,7 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
             std::memset(&probe, 0, sizeof(probe));
             probe.m = (uint32_t)rows, probe.k = (uint32_t)E, probe.n = (uint32_t)E;
             probe.cross_head_dim = (uint32_t)xhd;
-            probe.tolerant = step_tolerant();
+            probe.tolerant = matmul_tolerant();
             /* however many sub-tokens a patch has: a prompt of 512 rows, two layers of 128 columns, as launches / this, of one 69 /
              * 66 us, 16 96 / 71, 128 319 / 120 */
             if (rows > 32 && cross_block_launch(whole, (uint32_t)E, 0)) {
@@ -584,7 +572,7 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
                 g.cross_out = xcomb, g.cross_lo = dev + batch, g.cross_hi = dev + batch + rows;
                 g.cross_rows_per_seq = (uint32_t)n, g.cross_slab_rows = (uint32_t)cache->max_subtokens;
                 g.cross_scale = 1.0f / sqrtf((float)xhd), g.cross_head_dim = (uint32_t)xhd;
-                g.tolerant = step_tolerant();
+                g.tolerant = matmul_tolerant();
                 matmul_f32_launch(g, 0);
             } else {
             if (matmul_takes_norm(probe)) {
@@ -669,7 +657,7 @@ void refresh_cross_seq(blt_kv_cache *cache, size_t seq, const blt_tensor *patch_
         g.lda = g.ldb = g.ldo = (uint32_t)E;
         g.b2 = (const float *)s->cross_weight_v.data;
         g.out2 = (float *)cache->cross_v[l].data + row0 * E;
-        g.tolerant = step_tolerant();
+        g.tolerant = matmul_tolerant();
         if (waits) { /* K and V in one pass over the patch rows */
             if (matmul_pair_ok(waiting, g)) {
                 matmul_f32_launch_pair(waiting, g, 0);

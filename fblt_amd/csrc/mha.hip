@@ -40,11 +40,12 @@ namespace {
  * projection's own pass where that kernel takes it, csrc/models/transformer.c:60-66), with
  * residual that [seq_len, embed_dim] array is added to the projected output (transformer.c:
  * 116-117) -- the two statements a transformer block wraps around its attention.  With tail the rest of
- * the block follows in the launch of the projection where that takes the shape; true: it did.  What waits in later goes along where
+ * the block follows in the launch of the projection where that takes the shape; true: it did.  block: up to 32 rows
+ * too the sums may be taken in another order than the reference's.  What waits in later goes along where
  * it can. */
 bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_tensor *weight_proj, blt_tensor *output,
              const blt_attention_config *config, blt_arena *arena, const float *norm_w, const float *residual,
-             const BlockTailArgs *tail = nullptr, CrossLater *later = nullptr) {
+             bool block = false, const BlockTailArgs *tail = nullptr, CrossLater *later = nullptr) {
     BLT_REQUIRE(config != NULL && arena != NULL, "blt_multihead_attention: config and arena cannot be NULL");
     BLT_REQUIRE(arena->backend == BLT_BACKEND_HIP, "blt_multihead_attention: HIP implementation needs a device arena");
     const size_t E = config->embed_dim, H = config->num_heads;
@@ -108,7 +109,8 @@ bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
     g.out = qkv;
     g.m = (uint32_t)T, g.k = (uint32_t)E, g.n = (uint32_t)(3 * E);
     g.lda = (uint32_t)E, g.ldb = (uint32_t)(3 * E), g.ldo = (uint32_t)(3 * E);
-    const bool fuse_rope = config->use_rope && hd % 4 == 0 && T > 32;
+    g.tolerant = block ? matmul_tolerant() : 0u;
+    const bool fuse_rope = config->use_rope && hd % 4 == 0 && (T > 32 || g.tolerant);
     if (fuse_rope) {
         g.rope_cos = rope_cos, g.rope_sin = rope_sin;
         g.rope_cols = (uint32_t)(2 * E), g.head_dim = (uint32_t)hd;
@@ -246,6 +248,7 @@ bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
     g.residual = residual;
     g.m = (uint32_t)T, g.k = (uint32_t)E, g.n = (uint32_t)E;
     g.lda = g.ldb = g.ldo = (uint32_t)E;
+    g.tolerant = block ? matmul_tolerant() : 0u;
     matmul_f32_launch(g, 0);
     HIP_CHECK_LAUNCH("blt_multihead_attention");
     return false;
@@ -272,7 +275,7 @@ extern "C" void blt_multihead_attention_hip(const blt_tensor *input, const blt_t
  *   4. act = silu(RMSNorm(attn_residual) * ffn_gate_w) .* (RMSNorm(attn_residual) * ffn_up_w);
  *   5. output = attn_residual + act * ffn_down_w
  *
- * -- or three, with 3 to 5 in one (block_tail.hip), for more than 32 rows of narrow blocks.
+ * -- or three, with 3 to 5 in one (block_tail.hip), for narrow blocks.
  *
  * RMSNorm + SwiGLU blocks with FP32 weights (what every BLT block is, csrc/models/
  * local_common.c:99-115); LayerNorm / GELU blocks and BF16 weight copies end with a message.
@@ -314,9 +317,9 @@ void blt_transformer_run(const blt_tensor *input, const blt_transformer_weights 
     tail.up = (const float *)w->ffn_up_w->data, tail.gate = (const float *)w->ffn_gate_w->data;
     tail.down = (const float *)w->ffn_down_w->data, tail.out = (float *)output->data, tail.resid = (float *)attn_residual.data;
     tail.hidden = (uint32_t)hidden;
-    /* up to 32 rows the products keep the reference's order of sums */
+    const uint32_t tolerant = matmul_tolerant();
     const bool done = mha_run(input, w->attn_qkv_w, w->attn_proj_w, &attn_residual, &config->attn_config, arena,
-                              (const float *)w->norm1_weight->data, (const float *)input->data, T > 32 ? &tail : nullptr, later);
+                              (const float *)w->norm1_weight->data, (const float *)input->data, true, T > 32 || tolerant ? &tail : nullptr, later);
     blt_tensor act = blt_tensor_create_uninit(arena, hidden_shape, 2, BLT_DTYPE_FP32);
     if (done) {
         if (later != nullptr) cross_later_launch(*later, (uint32_t)E, 0);
@@ -331,6 +334,7 @@ void blt_transformer_run(const blt_tensor *input, const blt_transformer_weights 
     g.m = (uint32_t)T, g.k = (uint32_t)E, g.n = (uint32_t)hidden;
     g.lda = (uint32_t)E, g.ldb = g.ldo = (uint32_t)hidden;
     g.b2 = (const float *)w->ffn_gate_w->data;
+    g.tolerant = tolerant;
     if (matmul_takes_norm(g)) { /* norm, up, gate and the activation in one pass */
         g.norm_w = (const float *)w->norm2_weight->data;
     } else {
@@ -346,6 +350,7 @@ void blt_transformer_run(const blt_tensor *input, const blt_transformer_weights 
     g.residual = (const float *)attn_residual.data;
     g.m = (uint32_t)T, g.k = (uint32_t)hidden, g.n = (uint32_t)E;
     g.lda = (uint32_t)hidden, g.ldb = g.ldo = (uint32_t)E;
+    g.tolerant = tolerant;
     matmul_f32_launch(g, 0);
     if (later != nullptr) cross_later_launch(*later, (uint32_t)E, 0);
     HIP_CHECK_LAUNCH("blt_transformer_forward");
@@ -444,10 +449,12 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     float *const v = made ? pass->made_v : rows_of_keys();
     if (made) pass->made_k = pass->made_v = nullptr;
 
+    const uint32_t tolerant = pass != nullptr ? matmul_tolerant() : 0u;
     MatmulArgs g;
     std::memset(&g, 0, sizeof(g));
     g.m = (uint32_t)P, g.k = (uint32_t)E, g.n = (uint32_t)E;
     g.lda = g.ldb = g.ldo = (uint32_t)E;
+    g.tolerant = tolerant;
     MatmulArgs gkv = g;
     gkv.a = (const float *)kv_in->data;
     gkv.b = (const float *)weights->weight_k->data;
@@ -461,8 +468,8 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     whole.wq = (const float *)weights->weight_q->data, whole.proj = (const float *)weights->weight_proj->data;
     whole.k = k, whole.v = v, whole.lo = row_lo, whole.hi = row_hi;
     whole.rows = whole.rows_per_seq = (uint32_t)P, whole.head_dim = (uint32_t)hd, whole.scale = 1.0f / sqrtf((float)hd);
-    /* up to 32 rows the products keep the reference's order of sums */
-    if (row_lo != nullptr && P > 32 && T != 0 && row_span <= CROSS_SPAN && cross_block_ok(whole, (uint32_t)E)) {
+    /* up to 32 rows the products of a block by itself keep the reference's order of sums */
+    if (row_lo != nullptr && (P > 32 || tolerant) && T != 0 && row_span <= CROSS_SPAN && cross_block_ok(whole, (uint32_t)E)) {
         if (pass != nullptr && pass->later != nullptr) {
             pass->later->kv = gkv, pass->later->cross = whole;
             pass->later->kv_waits = !made, pass->later->cross_waits = true;
@@ -546,6 +553,7 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     g.residual = residual;
     g.m = (uint32_t)P, g.k = (uint32_t)E, g.n = (uint32_t)E;
     g.lda = g.ldb = g.ldo = (uint32_t)E;
+    g.tolerant = tolerant;
     matmul_f32_launch(g, 0);
     HIP_CHECK_LAUNCH("blt_cross_attention_forward");
 }

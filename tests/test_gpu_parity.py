@@ -2172,6 +2172,34 @@ def test_block_behind_its_attention(T, E, H, hidden, shift, fused, dev):
     assert got[0].tobytes() == got[1].tobytes() == got[2].tobytes()
 
 
+@pytest.mark.parametrize("T,E,H,hidden,shift,fused", [(1, 64, 2, 64, 0, True), (15, 128, 4, 512, 0, True), (16, 128, 4, 512, 0, True),
+                                                      (17, 256, 4, 1024, 0, True), (32, 128, 4, 512, 0, True), (30, 512, 8, 2048, 0, False),
+                                                      (2, 96, 3, 96, 0, False), (31, 128, 4, 512, 1, False), (9, 64, 2, 100, 0, False),
+                                                      (25, 40, 2, 72, 0, False)])
+def test_block_of_few_rows(T, E, H, hidden, shift, fused, dev):
+    """Blocks of up to 32 rows run on the matrix cores like larger ones; widths, hidden layers and weights of every alignment, in place
+    and again, against float64."""
+    outs, launched, want = _transformer_block(T, E, H, hidden, shift)
+    assert launched.get("block_tail", (0,))[0] == (3 if fused else 0) and "matmul_skinny" not in launched, launched
+    # four products, each of which rounds a sum of at most max(E, hidden) terms, as above
+    assert _relative(outs[0].cpu(), want) <= 2 * 2 ** -24 * max(E, hidden) ** 0.5
+    assert outs[0].cpu().numpy().tobytes() == outs[1].cpu().numpy().tobytes() == outs[2].cpu().numpy().tobytes()
+
+
+def test_block_of_few_rows_in_the_reference_order():
+    """BLT_HIP_EXACT_STEP=1 keeps the exact kernel for them (read once a process)."""
+    import os
+    import subprocess
+    import sys
+    code = ("from tests.test_gpu_parity import _transformer_block, _relative\n"
+            "outs, launched, want = _transformer_block(17, 128, 4, 512)\n"
+            "assert 'matmul_skinny' in launched and 'block_tail' not in launched, launched\n"
+            "assert _relative(outs[0].cpu(), want) < 1e-5\nprint('OK')\n")
+    p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, env=dict(os.environ, BLT_HIP_EXACT_STEP="1"),
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert p.returncode == 0 and "OK" in p.stdout, p.stdout[-2000:] + p.stderr[-2000:]
+
+
 @pytest.mark.parametrize("T,E,H,hidden,fused", [(304, 64, 2, 2112, True), (305, 64, 2, 2112, False), (112, 128, 4, 2112, True),
                                                 (113, 128, 4, 2112, False), (112, 256, 8, 1088, True), (113, 256, 8, 1088, False)])
 def test_block_behind_its_attention_of_many_slices(T, E, H, hidden, fused, dev):
