@@ -241,8 +241,10 @@ __global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArg
 constexpr uint32_t CROSS_ROWS = 16384;
 constexpr uint32_t CROSS_KEYS = 4;
 
-template <typename Shape, uint32_t KEYS = CROSS_KEYS>
-__device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, uint32_t tile, float *rows, float *part) {
+/* then(): further requests, behind the first keys'.  Returns the thread's columns of its row; rows and part are free for the taking
+ * behind a barrier. */
+template <typename Shape, uint32_t KEYS, typename Then>
+__device__ __forceinline__ floatx4 cross_rows(const CrossBlockArgs &a, uint32_t tile, float *rows, float *part, Then then) {
     using Proj = typename Shape::Proj;
     constexpr int E = Shape::E, ROW = Shape::ROW, EPT = Shape::EPT;
     static_assert(EPT == 4, "a thread holds 16 bytes of a row");
@@ -278,6 +280,7 @@ __device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, uint32_t til
     __builtin_amdgcn_sched_barrier(0);
     fetch(even, lo); /* the keys do not wait for the query */
     fetch(odd, lo + KEYS);
+    then();
     __builtin_amdgcn_sched_barrier(0);
 
     if (a.norm_w) {
@@ -348,7 +351,48 @@ __device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, uint32_t til
     gather<Proj::SHARES, Proj::PITCH, EPT>(part + f_row * Proj::PITCH + f_col, sum);
 #pragma unroll
     for (int i = 0; i < EPT; i++) resid[i] += sum[i];
-    if (row0 + f_row < a.rows) *reinterpret_cast<floatx4 *>(a.out + f_at) = resid;
+    return resid;
+}
+
+template <typename Shape, uint32_t KEYS = CROSS_KEYS>
+__device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, uint32_t tile, float *rows, float *part) {
+    const floatx4 out = cross_rows<Shape, KEYS>(a, tile, rows, part, [] {});
+    const uint32_t row = 16u * tile + threadIdx.x / (Shape::E / 4);
+    if (row < a.rows) *reinterpret_cast<floatx4 *>(a.out + (size_t)row * Shape::E + 4u * (threadIdx.x % (Shape::E / 4))) = out;
+}
+
+/* A cross block and the QKV product of its rows: workgroup x of a row tile takes the columns of Q, K or V, each with the cross block
+ * of its own -- again, as in the tail --, and the first stores that block's rows.
+ * Bound: latency, a chain of two products behind each other and the norm between; for 512 rows of 128 that see a patch each 9.9 us in
+ * the kernel trace, against 6.9 and 5.6 and the gap as two launches (a prompt of 512 bytes, two layers: 70.2 / 66.6 us). */
+template <typename Shape>
+__global__ __launch_bounds__(Shape::THREADS) void cross_qkv_kernel(CrossBlockArgs a, MatmulArgs g) {
+    using Proj = typename Shape::Proj;
+    constexpr int E = Shape::E, ROW = Shape::ROW;
+    constexpr uint32_t TPR = E / 4;
+    __shared__ __attribute__((aligned(16))) float rows[16 * ROW], part[Proj::PART];
+    const uint32_t tid = threadIdx.x, third = blockIdx.x, tile = blockIdx.y;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t group = wave % Proj::GROUPS, share = wave / Proj::GROUPS, term = share * (16 * Proj::BLOCKS);
+    const uint32_t f_row = tid / TPR, f_col = 4u * (tid % TPR), row = 16u * tile + f_row;
+    floatx4 w[4 * Proj::BLOCKS], norm_w;
+    floatx4 x = cross_rows<Shape, CROSS_KEYS>(a, tile, rows, part, [&]() __attribute__((always_inline)) {
+        norm_w = *reinterpret_cast<const floatx4 *>(g.norm_w + f_col);
+        request<Proj::BLOCKS>(w, g.b + third * E + 64u * group, g.ldb, term);
+    });
+    if (third == 0u && row < a.rows) *reinterpret_cast<floatx4 *>(a.out + (size_t)row * E + f_col) = x;
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) ss += x[i] * x[i];
+    ss = key_sum<TPR>(ss);
+    x *= 1.0f / sqrtf(ss / (float)E + 1e-6f) * norm_w; /* reductions_cpu.c:345-346 */
+    *reinterpret_cast<floatx4 *>(rows + f_row * ROW + f_col) = x;
+    __syncthreads();
+    multiply<Proj::BLOCKS, Proj::PITCH>(rows, ROW, term, w, part + share * (16 * Proj::PITCH) + 64u * group);
+    __syncthreads();
+    float v[4];
+    gather<Proj::SHARES, Proj::PITCH, 4>(part + f_row * Proj::PITCH + f_col, v);
+    if (row < a.rows) matmul_store4<true>(g, row, third * E + f_col, make_float4(v[0], v[1], v[2], v[3]), true);
 }
 
 template <typename Shape>
@@ -460,5 +504,21 @@ bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t
     const dim3 grid((a.rows + 15u) / 16u);
     if (embed_dim == 64u) blt_launch("cross_block", cross_block_kernel<TailShape<64, 4, true>>, grid, dim3(256), 0, s, a);
     else blt_launch("cross_block", cross_block_kernel<TailShape<128, 8, true>>, grid, dim3(512), 0, s, a);
+    return true;
+}
+
+bool cross_qkv_launch(const CrossBlockArgs &a, const MatmulArgs &g, uint32_t embed_dim, hipStream_t s) {
+    /* Three workgroups a row tile, as long as the chip holds them all at once (registers: one a CU for 128 columns, three for 64):
+     * prompts of 1000 / 1360 / 1500 rows of 128 89.2 / 124.4 / 126.6 us as two launches a layer, 85.0 / 114.3 / 131.4 as one. */
+    const uint32_t tiles = (a.rows + 15u) / 16u, most = embed_dim == 64u ? 768u : 256u;
+    if (!cross_block_ok(a, embed_dim) || 3u * tiles > most || a.out == a.x || a.out == a.residual) return false; /* a row is read three times */
+    if (g.norm_w == nullptr || g.b2 != nullptr || g.residual != nullptr || g.cross_k != nullptr || g.m != a.rows || g.k != embed_dim ||
+        g.n != 3u * embed_dim || g.ldb % 4u != 0u || g.ldo % 4u != 0u || g.head_dim % 4u != 0u)
+        return false;
+    for (const void *p : {(const void *)g.b, (const void *)g.norm_w, (const void *)g.out, (const void *)g.stage_k, (const void *)g.stage_v})
+        if ((reinterpret_cast<uintptr_t>(p) & 15u) != 0u) return false;
+    const dim3 grid(3u, tiles);
+    if (embed_dim == 64u) blt_launch("cross_qkv", cross_qkv_kernel<TailShape<64, 4, true>>, grid, dim3(256), 0, s, a, g);
+    else blt_launch("cross_qkv", cross_qkv_kernel<TailShape<128, 8, true>>, grid, dim3(512), 0, s, a, g);
     return true;
 }

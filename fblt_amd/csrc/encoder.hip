@@ -474,6 +474,9 @@ extern "C" void blt_local_decoder_forward_ext_hip(const blt_local_decoder *model
 
     /* ---- layers ---- */
     CrossPass cross_pass;
+    CrossLater first; /* a layer's cross block, for the launch of its QKV product */
+    first.feeds = true;
+    cross_pass.later = &first;
     const size_t byte_shape[2] = {seq_len, E};
     blt_tensor latents = view_2d(patch_in->data, num_patches * k, E);
     blt_tensor d = view_2d(byte_hidden_in->data, seq_len, E);
@@ -499,7 +502,7 @@ extern "C" void blt_local_decoder_forward_ext_hip(const blt_local_decoder *model
         w.attn_qkv_w = &s->attn_qkv_w, w.attn_proj_w = &s->attn_proj_w;
         w.ffn_up_w = &s->ffn_up_w, w.ffn_gate_w = &s->ffn_gate_w, w.ffn_down_w = &s->ffn_down_w;
         blt_tensor d_next = blt_tensor_create_uninit(arena, byte_shape, 2, BLT_DTYPE_FP32);
-        blt_transformer_forward_hip(&b, &w, &d_next, &layer_cfg, arena);
+        blt_transformer_run(&b, &w, &d_next, &layer_cfg, arena, &first);
         d = d_next;
     }
     blt_matmul_hip(&d, &model->lm_head_weight, logits_out);

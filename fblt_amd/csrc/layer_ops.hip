@@ -222,8 +222,8 @@ namespace {
  * head) problems of the prefill kernels with the causal diagonal moved by the cached length (csrc/infer/kv_cache.c:
  * 229-236: j <= base + r, base + r - j < window).  Needs the lengths on the host, and in cache->self_len.
  * (A launch of its own between the product and the attention took 2.8 us and a gap of 0.8 for 512 rows of 128.) */
-void long_chunk_qkv(const blt_kv_attn_cache *cache, const float *rows_in, const float *qkv_w, const float *norm_w, float *q_rot,
-                    const float *rope_cos, const float *rope_sin, size_t rope_positions, size_t n, const size_t *host_base) {
+MatmulArgs long_chunk_qkv(const blt_kv_attn_cache *cache, const float *rows_in, const float *qkv_w, const float *norm_w, float *q_rot,
+                          const float *rope_cos, const float *rope_sin, size_t rope_positions, size_t n, const size_t *host_base) {
     const size_t E = cache->embed_dim;
     for (size_t b = 0; b < cache->batch; b++)
         BLT_REQUIRE(host_base[b] + n <= rope_positions && host_base[b] + n <= cache->max_seq_len,
@@ -237,7 +237,7 @@ void long_chunk_qkv(const blt_kv_attn_cache *cache, const float *rows_in, const 
     g.stage_k = cache->self_k, g.stage_v = cache->self_v, g.stage_len = cache->self_len;
     g.stage_slab_rows = cache->max_seq_len, g.stage_n = (uint32_t)n;
     g.tolerant = matmul_tolerant();
-    matmul_f32_launch(g, 0);
+    return g;
 }
 
 void long_chunk_attention(const blt_kv_attn_cache *cache, const float *q_rot, size_t n, const size_t *host_base, float *combined) {
@@ -285,11 +285,12 @@ __global__ __launch_bounds__(256) void rope_rows_at_kernel(float *__restrict__ q
 
 /* host_base: the sequences' lengths where the caller keeps them (NULL: device lengths in
  * cache->self_len); they then travel in the step kernels' arguments.  dev_positions: device array
- * [rows] of rotary positions when they are not base + r (NULL otherwise). */
+ * [rows] of rotary positions when they are not base + r (NULL otherwise).  cross: the cross block that makes rows_in, which it
+ * launches (NULL: there already). */
 void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_weights *w, const float *rows_in,
                        float *rows_out, const float *rope_cos, const float *rope_sin, size_t rope_positions, size_t n,
                        int step_kind, int commit, size_t max_len_hint, blt_arena *arena, const size_t *host_base,
-                       const uint32_t *dev_positions = nullptr) {
+                       const uint32_t *dev_positions = nullptr, const CrossBlockArgs *cross = nullptr) {
     BLT_REQUIRE(cache != NULL && w != NULL && rows_in != NULL && rows_out != NULL && arena != NULL,
                 "blt_kv_decode_layer: arguments must not be NULL");
     BLT_REQUIRE(arena->backend == BLT_BACKEND_HIP, "blt_kv_decode_layer: needs a device arena");
@@ -327,15 +328,31 @@ void decode_layer_impl(const blt_kv_attn_cache *cache, const blt_transformer_wei
     const bool chunk = host_base != nullptr && n > 32 && step_kind == BLT_KV_STEP_CAUSAL && commit == 0 && dev_positions == nullptr &&
                        (E / cache->num_heads) % 4 == 0;
     const float *qkv_in = rows_in, *qkv_norm = f32(w->norm1_weight);
-    if (!matmul_takes_norm(probe)) {
+    const auto chunk_product = [&]() {
+        return long_chunk_qkv(cache, qkv_in, f32(w->attn_qkv_w), qkv_norm, qkv, rope_cos, rope_sin, rope_positions, n, host_base);
+    };
+    bool taken = false; /* the QKV product, with the cross block */
+    if (cross != nullptr) {
+        MatmulArgs g;
+        if (chunk) {
+            g = chunk_product();
+        } else {
+            std::memset(&g, 0, sizeof(g));
+            g.b = f32(w->attn_qkv_w), g.norm_w = qkv_norm, g.out = qkv;
+            g.m = (uint32_t)rows, g.k = (uint32_t)E, g.n = g.ldb = g.ldo = (uint32_t)(3 * E);
+        }
+        taken = cross_qkv_launch(*cross, g, (uint32_t)E, 0);
+        if (!taken) cross_block_launch(*cross, (uint32_t)E, 0);
+    }
+    if (!taken && !matmul_takes_norm(probe)) {
         rmsnorm_launch(rows_in, qkv_norm, normed, rows, E);
         qkv_in = normed, qkv_norm = nullptr;
     }
     if (chunk) {
-        long_chunk_qkv(cache, qkv_in, f32(w->attn_qkv_w), qkv_norm, qkv, rope_cos, rope_sin, rope_positions, n, host_base);
+        if (!taken) matmul_f32_launch(chunk_product(), 0);
         long_chunk_attention(cache, qkv, n, host_base, combined);
     } else {
-        gemm(qkv_in, f32(w->attn_qkv_w), qkv, rows, E, 3 * E, nullptr, nullptr, qkv_norm);
+        if (!taken) gemm(qkv_in, f32(w->attn_qkv_w), qkv, rows, E, 3 * E, nullptr, nullptr, qkv_norm);
         if (host_base != nullptr && commit == 0) {
             /* the caller keeps the lengths: they go into the kernel arguments */
             std::vector<uint32_t> lens(cache->batch);
@@ -535,12 +552,13 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
     for (size_t l = 0; l < L; l++) {
         const blt_local_layer_storage *s = &dec->layers[l];
         const float *in = cur;
+        CrossBlockArgs whole;
+        bool waits = false; /* for the layer's QKV product */
         if (cross_fires(cfg, l)) { /* kv_cache.c:303-341 */
             check_vec(s->cross_norm_weight, E, "blt_kv_decode_step: cross_norm_weight must be [embed_dim] FP32");
             check_weight(&s->cross_weight_q, E, E, "blt_kv_decode_step: cross_weight_q must be [embed_dim, embed_dim]");
             check_weight(&s->cross_weight_proj, E, E,
                          "blt_kv_decode_step: cross_weight_proj must be [embed_dim, embed_dim]");
-            CrossBlockArgs whole;
             std::memset(&whole, 0, sizeof(whole));
             whole.x = whole.residual = cur, whole.out = mid, whole.norm_w = (const float *)s->cross_norm_weight.data;
             whole.wq = (const float *)s->cross_weight_q.data, whole.proj = (const float *)s->cross_weight_proj.data;
@@ -555,8 +573,8 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
             probe.tolerant = matmul_tolerant();
             /* however many sub-tokens a patch has: a prompt of 512 rows, two layers of 128 columns, as launches / this, of one 69 /
              * 66 us, 16 96 / 71, 128 319 / 120 */
-            if (rows > 32 && cross_block_launch(whole, (uint32_t)E, 0)) {
-                in = mid;
+            if (rows > 32 && cross_block_ok(whole, (uint32_t)E)) {
+                in = mid, waits = true;
             } else {
             if (matmul_takes_norm(probe) && matmul_takes_cross(probe)) {
                 /* norm, Q projection and the rows' cross attention in one launch: with more than 32
@@ -615,7 +633,7 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
         arena->offset = arena_mark; /* the layer's work buffers are reused by the next layer */
         decode_layer_impl(&view, &w, in, next, (const float *)dec->rope_cos_cache.data,
                           (const float *)dec->rope_sin_cache.data, cfg->max_seq_len, n, step_kind, 0, max_total, arena,
-                          base, own_positions ? dev + batch + 2 * rows : nullptr);
+                          base, own_positions ? dev + batch + 2 * rows : nullptr, waits ? &whole : nullptr);
         cur = next;
     }
     gemm(cur, (const float *)dec->lm_head_weight.data, logits, rows, E, V); /* kv_cache.c:416 */

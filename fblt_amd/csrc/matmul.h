@@ -69,6 +69,44 @@ struct MatmulArgs {
     uint32_t *slice_tickets;
 };
 
+/* Four consecutive results of output row `row` starting at column `col`:
+ * optional rotation, optional residual, store with bounds. */
+template <bool ROPE>
+__device__ __forceinline__ void matmul_store4(const MatmulArgs &g, uint32_t row, uint32_t col, float4 v, bool vec_ok) {
+    if (ROPE && g.stage_k) { /* new rows of a cache: no residual */
+        if (col >= g.n) return;
+        const uint32_t E = g.n / 3u, part = col / E, at = col % E, b = row / g.stage_n, pos = g.stage_len[b] + row % g.stage_n;
+        if (part < 2u) {
+            const size_t turn = (size_t)pos * (g.head_dim / 2u) + (at % g.head_dim) / 2u;
+            v = rope_rotate4(v, g.rope_cos + turn, g.rope_sin + turn);
+        }
+        float *const to = part == 0u ? g.out + (size_t)row * E : (part == 1u ? g.stage_k : g.stage_v) + ((size_t)b * g.stage_slab_rows + pos) * E;
+        *reinterpret_cast<float4 *>(to + at) = v;
+        return;
+    }
+    if (ROPE && col < g.rope_cols) {
+        /* columns col..col+3 are pairs (col % head_dim)/2 and the next one of the row's position */
+        const size_t at = (size_t)row * (g.head_dim / 2u) + (col % g.head_dim) / 2u;
+        v = rope_rotate4(v, g.rope_cos + at, g.rope_sin + at);
+    }
+    float *orow = g.out + (size_t)row * g.ldo;
+    const float *rrow = g.residual ? g.residual + (size_t)row * g.ldo : nullptr;
+    if (vec_ok) {
+        if (col < g.n) {
+            if (rrow) {
+                const float4 r = *reinterpret_cast<const float4 *>(rrow + col);
+                v.x = r.x + v.x, v.y = r.y + v.y, v.z = r.z + v.z, v.w = r.w + v.w;
+            }
+            *reinterpret_cast<float4 *>(orow + col) = v;
+        }
+    } else {
+        const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (col + i < g.n) orow[col + i] = rrow ? rrow[col + i] + e[i] : e[i];
+    }
+}
+
 void matmul_f32_launch(const MatmulArgs &g, hipStream_t s);
 /* MatmulArgs::tolerant of whole steps, blocks and forward passes: their projections are taken on the matrix cores whatever the
  * row count (fp32 tolerance, as they always are above 32 rows; us, exact / this: a one-row decoder step 112 / 72, a block of 16
@@ -107,12 +145,15 @@ struct CrossBlockArgs {
 /* false: not for this shape, nothing was launched.  cross_block_ok: the same answer before lo and hi are there. */
 bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim);
 bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t s);
+/* The same, and the packed QKV product g of its output rows, RMS-normalised (g.norm_w; g.a is not looked at), in one launch. */
+bool cross_qkv_launch(const CrossBlockArgs &a, const MatmulArgs &g, uint32_t embed_dim, hipStream_t s);
 /* A cross block put off until launches of the next layer, which has nothing to do with it, can take it along: the product of its
  * keys and values beside that layer's first product, the rest beside its tail. */
 struct CrossLater {
     MatmulArgs kv;
     CrossBlockArgs cross;
     bool kv_waits = false, cross_waits = false;
+    bool feeds = false; /* unlike that, the block is what the next layer starts from: it goes along with its QKV product or before */
 };
 /* What the cross blocks of one forward pass, which have their mask in common, leave each other. */
 struct CrossPass {

@@ -56,44 +56,6 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int TM = 64, TN = 64; /* smallest workgroup tile of the mfma kernel */
 
-/* Four consecutive results of output row `row` starting at column `col`:
- * optional rotation, optional residual, store with bounds. */
-template <bool ROPE>
-__device__ __forceinline__ void store4(const MatmulArgs &g, uint32_t row, uint32_t col, float4 v, bool vec_ok) {
-    if (ROPE && g.stage_k) { /* new rows of a cache: no residual */
-        if (col >= g.n) return;
-        const uint32_t E = g.n / 3u, part = col / E, at = col % E, b = row / g.stage_n, pos = g.stage_len[b] + row % g.stage_n;
-        if (part < 2u) {
-            const size_t turn = (size_t)pos * (g.head_dim / 2u) + (at % g.head_dim) / 2u;
-            v = rope_rotate4(v, g.rope_cos + turn, g.rope_sin + turn);
-        }
-        float *const to = part == 0u ? g.out + (size_t)row * E : (part == 1u ? g.stage_k : g.stage_v) + ((size_t)b * g.stage_slab_rows + pos) * E;
-        *reinterpret_cast<float4 *>(to + at) = v;
-        return;
-    }
-    if (ROPE && col < g.rope_cols) {
-        /* columns col..col+3 are pairs (col % head_dim)/2 and the next one of the row's position */
-        const size_t at = (size_t)row * (g.head_dim / 2u) + (col % g.head_dim) / 2u;
-        v = rope_rotate4(v, g.rope_cos + at, g.rope_sin + at);
-    }
-    float *orow = g.out + (size_t)row * g.ldo;
-    const float *rrow = g.residual ? g.residual + (size_t)row * g.ldo : nullptr;
-    if (vec_ok) {
-        if (col < g.n) {
-            if (rrow) {
-                const float4 r = *reinterpret_cast<const float4 *>(rrow + col);
-                v.x = r.x + v.x, v.y = r.y + v.y, v.z = r.z + v.z, v.w = r.w + v.w;
-            }
-            *reinterpret_cast<float4 *>(orow + col) = v;
-        }
-    } else {
-        const float e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (col + i < g.n) orow[col + i] = rrow ? rrow[col + i] + e[i] : e[i];
-    }
-}
-
 /* One (64*WT)x(64*WT) output tile per workgroup of eight wavefronts: four quadrants of WT x WT MFMA tiles, and for each
  * quadrant two waves that take half of every K step (16 of 32); their sums meet in LDS at the end.  The
  * operands are taken apart into two f16 parts (split_f16.h) or three bf16 parts (split_bf16.h) once per workgroup, on the
@@ -574,7 +536,7 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
             const float4 gate = *reinterpret_cast<const float4 *>(gates + at * PITCH + col);
             v.x = silu_times(gate.x, v.x), v.y = silu_times(gate.y, v.y), v.z = silu_times(gate.z, v.z), v.w = silu_times(gate.w, v.w);
         }
-        if (row < g.m) store4<ROPE>(to, row, wave_col + col, v, vst);
+        if (row < g.m) matmul_store4<ROPE>(to, row, wave_col + col, v, vst);
     }
 }
 
@@ -782,12 +744,12 @@ __device__ __forceinline__ void splitk_tile(const MatmulArgs &g, const uint32_t 
                      ((reinterpret_cast<uintptr_t>(g.residual) & 15u) == 0u) &&
                      ((reinterpret_cast<uintptr_t>(g.out2) & 15u) == 0u);
     const uint32_t oc = bx * 32u + 8u * wave + 4u * h;
-    store4<ROPE>(g, row, oc, make_float4(v4[0], v4[1], v4[2], v4[3]), vst);
+    matmul_store4<ROPE>(g, row, oc, make_float4(v4[0], v4[1], v4[2], v4[3]), vst);
     if (GATED && g.out2) {
         MatmulArgs g2 = g;
         g2.out = g.out2;
         g2.residual = nullptr;
-        store4<false>(g2, row, oc, make_float4(second[0], second[1], second[2], second[3]), vst);
+        matmul_store4<false>(g2, row, oc, make_float4(second[0], second[1], second[2], second[3]), vst);
     }
 }
 

@@ -115,7 +115,16 @@ bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
         g.rope_cos = rope_cos, g.rope_sin = rope_sin;
         g.rope_cols = (uint32_t)(2 * E), g.head_dim = (uint32_t)hd;
     }
-    if (norm_w != nullptr) {
+    bool taken = false; /* with the cross block that makes the input */
+    if (later != nullptr && later->feeds && later->cross_waits) {
+        MatmulArgs whole = g;
+        whole.norm_w = norm_w;
+        matmul_later_launch(*later, 0);
+        taken = cross_qkv_launch(later->cross, whole, (uint32_t)E, 0);
+        if (!taken) cross_block_launch(later->cross, (uint32_t)E, 0);
+        later->cross_waits = false;
+    }
+    if (norm_w != nullptr && !taken) {
         if (matmul_takes_norm(g)) {
             g.norm_w = norm_w;
         } else { /* the row norm as a pass of its own */
@@ -129,7 +138,8 @@ bool mha_run(const blt_tensor *input, const blt_tensor *weight_qkv, const blt_te
             g.a = (const float *)normed.data;
         }
     }
-    if (later != nullptr && later->kv_waits && matmul_pair_ok(g, later->kv)) {
+    if (taken) {
+    } else if (later != nullptr && later->kv_waits && matmul_pair_ok(g, later->kv)) {
         matmul_f32_launch_pair(g, later->kv, 0);
         later->kv_waits = false;
     } else {
@@ -470,11 +480,6 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     whole.rows = whole.rows_per_seq = (uint32_t)P, whole.head_dim = (uint32_t)hd, whole.scale = 1.0f / sqrtf((float)hd);
     /* up to 32 rows the products of a block by itself keep the reference's order of sums */
     if (row_lo != nullptr && (P > 32 || tolerant) && T != 0 && row_span <= CROSS_SPAN && cross_block_ok(whole, (uint32_t)E)) {
-        if (pass != nullptr && pass->later != nullptr) {
-            pass->later->kv = gkv, pass->later->cross = whole;
-            pass->later->kv_waits = !made, pass->later->cross_waits = true;
-            return;
-        }
         if (!made && pass != nullptr && pass->next_k != nullptr) {
             check_2d_fp32(pass->next_k, E, E, "blt_cross_attention: weight_k must be [embed_dim, embed_dim] FP32");
             check_2d_fp32(pass->next_v, E, E, "blt_cross_attention: weight_v must be [embed_dim, embed_dim] FP32");
@@ -485,6 +490,11 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
                 matmul_f32_launch_pair(gkv, more, 0);
                 made = true;
             }
+        }
+        if (pass != nullptr && pass->later != nullptr) {
+            pass->later->kv = gkv, pass->later->cross = whole;
+            pass->later->kv_waits = !made, pass->later->cross_waits = true;
+            return;
         }
         if (!made) matmul_f32_launch(gkv, 0);
         cross_block_launch(whole, (uint32_t)E, 0);

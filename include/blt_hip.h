@@ -115,11 +115,11 @@ void blt_cross_attention_forward_hip(const blt_tensor *query_in, const blt_tenso
 /* Device twins of the cache-aware decoder step (csrc/infer/kv_cache.c:
  * 112-159 and 161-416) with the reference's signatures, for a cache, decoder
  * weights and rows that live in device memory.  refresh_cross: one launch per
- * firing layer computes K and V of the new sub-tokens straight into the
- * tier-2 slabs.  decode_step: per layer the cross block (RMSNorm + Q
- * projection with the rows' few sub-tokens attended in its epilogue where the
- * shape allows, projection + residual: 2-3 launches) and the self-attention /
- * feed-forward layer (5 launches), then the LM head; the dense masks, strided
+ * firing layer, or two, computes K and V of the new sub-tokens straight into
+ * the tier-2 slabs.  decode_step: per layer the cross block (one launch for 64
+ * or 128 columns and more than 32 rows, with the layer's QKV product up to
+ * 1360 rows of 128 and 4096 of 64; 2-3 otherwise) and the self-attention /
+ * feed-forward layer (3-5 launches), then the LM head; the dense masks, strided
  * copies and per-head calls of the reference are gone, the row groups follow
  * the same latent rule (kv_cache.c:199-213).  A prompt chunk of more than 32
  * rows is staged once (rotation, write-through) and attended by the prefill

@@ -2618,6 +2618,17 @@ def test_kv_decode_step_of_chunks_staged_by_their_product(batch, n, case, produc
     assert all(product in names for names in launched) and staged == [0, 0], launched
 
 
+@pytest.mark.parametrize("batch,n,E,H,XH,k,joined", [
+    (1, 33, 128, 4, 4, 1, True), (3, 40, 64, 2, 4, 2, True), (4, 12, 128, 2, 8, 1, True), (3, 15, 64, 1, 1, 3, True),   # staged, packed
+    (40, 34, 128, 4, 4, 1, True), (42, 33, 128, 4, 4, 1, False), (124, 33, 64, 2, 2, 1, True), (125, 33, 64, 2, 2, 1, False)])
+def test_kv_decode_step_whose_cross_blocks_go_with_the_qkv_product(batch, n, E, H, XH, k, joined, oracle, dev):
+    """Both products of the rows in one launch, last tiles of 1 ... 16 rows, at the most rows it takes and beyond, against the
+    restated step."""
+    c = dict(E=E, H=H, XH=XH, L=2, hidden=64, V=32, max_len=160, k=k, window=0, all_layers=True, placement=0)
+    launched = _decode_steps(batch, n, c, 670 + batch, oracle)
+    assert all(("cross_qkv" in names) == joined and ("cross_block" in names) != joined for names in launched), launched
+
+
 @pytest.mark.parametrize("batch,n,case", [(1, 1, 2), (9, 8, 2), (33, 1, 0)])
 def test_kv_decode_step_of_rows_whose_norm_overflows(batch, n, case, oracle, dev):
     """Input rows of 1e20: their sum of squares is infinite and the normalised row zero, in the one-launch form as in
