@@ -286,8 +286,8 @@ __device__ __forceinline__ void fine_merge_states(floatx4 (&oa)[DT], float &ma, 
 
 template <int HD, int SRC, int HALVES, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, 4) void attn_fine_kernel(const AttnProb *__restrict__ probs,
-                                                                  const AttnTile *__restrict__ tiles, AttnAffine aff,
-                                                                  uint32_t kc) {
+                                                                  const AttnTile *__restrict__ tiles,
+                                                                  typename AttnSource<SRC>::type aff, uint32_t kc) {
     using Shape = FineShape<HD, HALVES, WAVES>;
     constexpr uint32_t FINE_THREADS = Shape::THREADS;
     constexpr uint32_t ROWS = 16u * HALVES; /* query rows of a workgroup            */
@@ -322,6 +322,10 @@ __global__ __launch_bounds__(64 * WAVES, 4) void attn_fine_kernel(const AttnProb
     } else if (SRC == SRC_SINGLE) {
         qtile = fine_tile_order(blockIdx.x, gridDim.x);
         p = aff.first;
+    } else if constexpr (SRC == SRC_DOCS) {
+        const AttnDocs::Item item = aff.item[blockIdx.x / aff.heads];
+        qtile = item.qtile;
+        docs_problem(p, aff, item.doc, blockIdx.x % aff.heads);
     } else {
         const uint32_t prob = blockIdx.x % aff.count;
         qtile = fine_tile_order(blockIdx.x / aff.count, (aff.first.nq + ROWS - 1u) / ROWS);
@@ -681,7 +685,7 @@ uint32_t fine_fill_keys(uint32_t span) {
 }
 
 template <int HD, int SRC, int HALVES, int WAVES>
-void fine_launch_as(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nblocks, const AttnAffine &aff,
+void fine_launch_as(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nblocks, const typename AttnSource<SRC>::type &aff,
                     uint32_t span, hipStream_t s) {
     using Shape = FineShape<HD, HALVES, WAVES>;
     const uint32_t kc = fine_fill_keys<Shape>(span);
@@ -700,9 +704,9 @@ void fine_launch_as(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nbl
 
 /* tall: workgroups of one 16-row tile and sixteen waves (strided batches and single problems) */
 template <int SRC>
-void fine_launch_hd(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nblocks, const AttnAffine &aff,
+void fine_launch_hd(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nblocks, const typename AttnSource<SRC>::type &aff,
                     uint32_t hd, uint32_t span, bool tall, hipStream_t s) {
-    if constexpr (SRC != SRC_TILES) {
+    if constexpr (SRC == SRC_SINGLE || SRC == SRC_AFFINE) {
         if (tall) {
             if (hd == 32u) fine_launch_as<32, SRC, 1, 16>(dprobs, dtiles, nblocks, aff, span, s);
             else fine_launch_as<64, SRC, 1, 16>(dprobs, dtiles, nblocks, aff, span, s);
@@ -805,4 +809,8 @@ void attn_fine_launch_affine(const AttnAffine &aff, bool tall, hipStream_t s) {
     const uint32_t blocks = aff.count * ((aff.first.nq + rows - 1u) / rows);
     if (blocks == 0) return;
     fine_launch_hd<SRC_AFFINE>(nullptr, nullptr, blocks, aff, aff.first.hd, attn_fine_span(aff.first), tall, s);
+}
+
+void attn_fine_launch_docs(const AttnDocs &docs, uint32_t span, hipStream_t s) {
+    fine_launch_hd<SRC_DOCS>(nullptr, nullptr, docs.n_items * docs.heads, docs, docs.first.hd, span, false, s);
 }

@@ -157,7 +157,7 @@ struct MfmaLds {
 template <int HD, int SRC, bool EXACT, bool DENSE, int NW>
 __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(const AttnProb *__restrict__ probs,
                                                                             const AttnTile *__restrict__ tiles,
-                                                                            AttnAffine aff) {
+                                                                            typename AttnSource<SRC>::type aff) {
     constexpr uint32_t NT = 64u * NW; /* threads */
     constexpr int HALF = HD / 2;
     constexpr int DB = HD / 32; /* 32-wide blocks of the head dim */
@@ -180,6 +180,10 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
         /* block b takes query tile (last - b): later tiles of a causal problem are the long ones */
         qtile = gridDim.x - 1u - blockIdx.x;
         p = aff.first;
+    } else if constexpr (SRC == SRC_DOCS) {
+        const AttnDocs::Item item = aff.item[blockIdx.x / aff.heads];
+        qtile = item.qtile;
+        docs_problem(p, aff, item.doc, blockIdx.x % aff.heads);
     } else {
         /* consecutive blocks are different problems of the same query tile,
          * longest tiles first; all tiles of a problem sit at blockIdx = prob
@@ -620,15 +624,16 @@ __global__ __launch_bounds__(64 * NW, HD <= 64 ? 2 : 1) void attn_mfma_kernel(co
 #undef K_REQUEST
 #undef K_PARK
 
+/* fewer workgroups than the compute units can spread: eight waves each (heads of 32, whose K tiles fit LDS then); measured: ahead up
+ * to 256 workgroups, level at 512 */
+constexpr uint32_t EIGHT_WAVES_BELOW = 320u;
+
 template <int HD, int SRC>
 void launch_variant(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nblocks, const AttnAffine &aff,
                     bool exact, bool dense, hipStream_t s) {
     const dim3 grid(nblocks);
     if constexpr (HD == 32) {
-        /* fewer workgroups than the compute units can spread: eight waves each (their K tiles fit
-         * LDS at this head dim); measured: ahead up to 256 workgroups, level at 512 */
-        constexpr uint32_t below = 320u;
-        if (exact && nblocks < below) {
+        if (exact && nblocks < EIGHT_WAVES_BELOW) {
             if (dense)
                 blt_launch("attn_mfma", attn_mfma_kernel<HD, SRC, true, true, 8>, grid, dim3(512), 0, s, dprobs, dtiles,
                            aff);
@@ -655,6 +660,12 @@ void launch_hd(const AttnProb *dprobs, const AttnTile *dtiles, uint32_t nblocks,
     if (hd <= 32u) launch_variant<32, SRC>(dprobs, dtiles, nblocks, aff, vec4 && hd == 32u, dense, s);
     else if (hd <= 64u) launch_variant<64, SRC>(dprobs, dtiles, nblocks, aff, vec4 && hd == 64u, dense, s);
     else launch_variant<128, SRC>(dprobs, dtiles, nblocks, aff, vec4 && hd == 128u, dense, s);
+}
+
+template <int HD, int NW>
+void launch_docs(const AttnDocs &docs, hipStream_t s) {
+    blt_launch("attn_mfma", attn_mfma_kernel<HD, SRC_DOCS, true, false, NW>, dim3(docs.n_items * docs.heads), dim3(64 * NW), 0, s,
+               static_cast<const AttnProb *>(nullptr), static_cast<const AttnTile *>(nullptr), docs);
 }
 
 } // namespace
@@ -730,4 +741,10 @@ void attn_mfma_launch_affine(const AttnAffine &aff, hipStream_t s) {
     if (blocks == 0) return;
     launch_hd<SRC_AFFINE>(nullptr, nullptr, blocks, aff, aff.first.hd, (aff.first.flags & ATTN_FLAG_VEC4) != 0,
                           aff.first.vis == ATTN_VIS_DENSE, s);
+}
+
+void attn_mfma_launch_docs(const AttnDocs &docs, hipStream_t s) {
+    if (docs.first.hd == 64u) launch_docs<64, 4>(docs, s);
+    else if (docs.n_items * docs.heads < EIGHT_WAVES_BELOW) launch_docs<32, 8>(docs, s);
+    else launch_docs<32, 4>(docs, s);
 }

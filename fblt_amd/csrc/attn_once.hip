@@ -92,7 +92,8 @@ __device__ __forceinline__ void once_store_piece(float *wrow, uint32_t j0, uint3
 
 template <int HD, int W, int T, int SRC, bool DENSE>
 __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__restrict__ probs,
-                                                          const AttnTile *__restrict__ tiles, AttnAffine aff) {
+                                                          const AttnTile *__restrict__ tiles,
+                                                          typename AttnSource<SRC>::type aff) {
     using Shape = OnceShape<HD, W>;
     constexpr int QD = HD / 4;  /* floats of a row one lane group contracts */
     constexpr int NV = QD / 4;  /* 16-byte loads per fragment row           */
@@ -113,6 +114,10 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
     } else if (SRC == SRC_SINGLE) {
         p = aff.first;
         qtile = gridDim.x - 1u - blockIdx.x; /* the long tiles of a causal problem first */
+    } else if constexpr (SRC == SRC_DOCS) {
+        const AttnDocs::Item item = aff.item[blockIdx.x / aff.heads];
+        qtile = item.qtile;
+        docs_problem(p, aff, item.doc, blockIdx.x % aff.heads);
     } else {
         /* Workgroups are handed to the chip's eight dies in turn, each die with an L2 of its own.  A
          * batch of few problems (aff.reserved = 8: eight slots per round, the slots past the
@@ -436,7 +441,7 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
 }
 
 template <int HD, int W, int T, int SRC, bool DENSE>
-void once_launch_kernel(const AttnProb *dprobs, const AttnTile *dtiles, const AttnAffine &aff, uint32_t nblocks,
+void once_launch_kernel(const AttnProb *dprobs, const AttnTile *dtiles, const typename AttnSource<SRC>::type &aff, uint32_t nblocks,
                         bool pieces, hipStream_t s) {
     using Shape = OnceShape<HD, W>;
     static const bool raised = [] { /* more than the 64 KB a kernel may use without asking */
@@ -454,15 +459,20 @@ void once_launch_kernel(const AttnProb *dprobs, const AttnTile *dtiles, const At
 }
 
 template <int HD, int W, int T, int SRC>
-void once_launch_as(const AttnProb *dprobs, const AttnTile *dtiles, const AttnAffine &aff, uint32_t nblocks, bool dense,
+void once_launch_as(const AttnProb *dprobs, const AttnTile *dtiles, const typename AttnSource<SRC>::type &aff, uint32_t nblocks, bool dense,
                     bool pieces, hipStream_t s) {
-    if (dense) once_launch_kernel<HD, W, T, SRC, true>(dprobs, dtiles, aff, nblocks, pieces, s);
-    else once_launch_kernel<HD, W, T, SRC, false>(dprobs, dtiles, aff, nblocks, pieces, s);
+    if constexpr (SRC != SRC_DOCS) {
+        if (dense) {
+            once_launch_kernel<HD, W, T, SRC, true>(dprobs, dtiles, aff, nblocks, pieces, s);
+            return;
+        }
+    }
+    once_launch_kernel<HD, W, T, SRC, false>(dprobs, dtiles, aff, nblocks, pieces, s);
 }
 
 /* `tiles` = 16-key tiles the longest 16-row tile of the launch spans: sizes the workgroups */
 template <int SRC>
-void once_launch_shape(const AttnProb *dprobs, const AttnTile *dtiles, const AttnAffine &aff, uint32_t nblocks,
+void once_launch_shape(const AttnProb *dprobs, const AttnTile *dtiles, const typename AttnSource<SRC>::type &aff, uint32_t nblocks,
                        uint32_t hd, uint32_t tiles, bool dense, bool pieces, hipStream_t s) {
     BLT_REQUIRE(tiles <= attn_once_tiles_max(hd), "attention: internal: the once kernel was given rows it does not hold");
     if (hd == 32u) {
@@ -567,4 +577,8 @@ void attn_once_launch_affine(const AttnAffine &aff, hipStream_t s) {
     const uint32_t nblocks = (a.reserved ? a.reserved : aff.count) * nqt;
     once_launch_shape<SRC_AFFINE>(nullptr, nullptr, a, nblocks, aff.first.hd, attn_once_span_tiles(aff.first),
                                   aff.first.vis == ATTN_VIS_DENSE, aff.first.weights != nullptr, s);
+}
+
+void attn_once_launch_docs(const AttnDocs &docs, uint32_t span_tiles, hipStream_t s) {
+    once_launch_shape<SRC_DOCS>(nullptr, nullptr, docs, docs.n_items * docs.heads, docs.first.hd, span_tiles, false, false, s);
 }

@@ -142,13 +142,14 @@ __device__ __forceinline__ void rows_walk(const AttnProb &p, const float4 (&q)[T
  * before the row ranges and the rows themselves can be requested. */
 template <int G, int T, int SRC>
 __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnProb *__restrict__ probs, uint32_t prob_base,
-                                                        AttnAffine aff) {
+                                                        typename AttnSource<SRC>::type aff) {
     constexpr int ROWS_PER_WAVE = 64 / G;
     constexpr int ROWS_PER_BLOCK = 4 * ROWS_PER_WAVE;
 
     AttnProb p;
     if (SRC == SRC_TILES) p = probs[prob_base + blockIdx.y];
     else if (SRC == SRC_SINGLE) p = aff.first;
+    else if constexpr (SRC == SRC_DOCS) docs_problem(p, aff, blockIdx.y / aff.heads, blockIdx.y % aff.heads);
     else affine_problem(p, aff, prob_base + blockIdx.y, aff.first.vis == ATTN_VIS_DENSE);
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
@@ -276,4 +277,14 @@ void attn_rows_launch_affine(const AttnAffine &aff, hipStream_t s) {
         dispatch_rows(nullptr, done, n, aff.first.hd, aff.first.nq, &aff, s);
         done += n;
     }
+}
+
+void attn_rows_launch_docs(const AttnDocs &docs, uint32_t max_nq, hipStream_t s) {
+    const auto launch = [&](auto kernel, uint32_t rows_per_block) {
+        blt_launch("attn_rows", kernel, dim3((max_nq + rows_per_block - 1u) / rows_per_block, docs.docs * docs.heads), dim3(256), 0, s,
+                   static_cast<const AttnProb *>(nullptr), 0u, docs);
+    };
+    BLT_REQUIRE(docs.first.hd <= 64u, "attention: internal: heads too wide for the rows kernel over documents");
+    if (docs.first.hd <= 32u) launch(attn_rows_kernel<8, 1, SRC_DOCS>, 32u);
+    else launch(attn_rows_kernel<16, 1, SRC_DOCS>, 16u);
 }

@@ -24,7 +24,12 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 enum : int {
     SRC_TILES = 0,  /* device arrays: tiles[blockIdx.x] -> probs[tile.prob]           */
     SRC_SINGLE = 1, /* one problem in the kernel arguments                            */
-    SRC_AFFINE = 2  /* kernel arguments: first problem + (sequence, head) strides     */
+    SRC_AFFINE = 2, /* kernel arguments: first problem + (sequence, head) strides     */
+    SRC_DOCS = 3    /* kernel arguments: first problem + row runs, head strides, items */
+};
+template <>
+struct AttnSource<SRC_DOCS> {
+    typedef AttnDocs type;
 };
 
 /* Problem `prob` of a strided batch.  Field by field: a whole-struct copy
@@ -47,6 +52,24 @@ __device__ __forceinline__ void affine_problem(AttnProb &p, const AttnAffine &af
     p.causal_off = f.causal_off, p.window = f.window, p.scale = f.scale, p.flags = f.flags;
     p.range_span = f.range_span;
     p.reserved1 = 0;
+}
+
+/* The problem of a document and a head. */
+__device__ __forceinline__ void docs_problem(AttnProb &p, const AttnDocs &a, uint32_t doc, uint32_t head) {
+    const uint64_t row = a.start[doc];
+    const int64_t hh = head;
+    const AttnProb &f = a.first;
+    p.q = f.q + (row * f.q_stride + hh * a.q_head);
+    p.k = f.k + (row * f.k_stride + hh * a.k_head);
+    p.v = f.v + (row * f.v_stride + hh * a.v_head);
+    p.out = f.out + (row * f.out_stride + hh * a.o_head);
+    p.weights = nullptr, p.lse = nullptr, p.mask = nullptr;
+    p.row_lo = p.row_hi = nullptr;
+    p.q_stride = f.q_stride, p.k_stride = f.k_stride, p.v_stride = f.v_stride, p.out_stride = f.out_stride;
+    p.nq = p.nk = a.start[doc + 1u] - (uint32_t)row;
+    p.hd = f.hd, p.vis = f.vis;
+    p.causal_off = f.causal_off, p.window = f.window, p.scale = f.scale, p.flags = f.flags;
+    p.range_span = 0, p.reserved1 = 0;
 }
 
 /* Keys any of the query rows [first, last] can see, [tlo, thi), and keys all

@@ -1407,6 +1407,50 @@ def test_attention_over_rows_far_apart(dev):
     assert_close(out.cpu().numpy(), (torch.softmax(s, -1) @ v).numpy(), "rows far apart")
 
 
+@pytest.mark.parametrize("lens,H,hd,window,gap,kernel,staged", [
+    ([100, 61, 7, 1, 130], 3, 32, 0, 0, "attn_once", False), ([17, 200], 2, 64, 50, 0, "attn_once", False),
+    ([300, 211, 170], 8, 64, 0, 0, "attn_mfma", False), ([250, 131, 380], 8, 32, 0, 0, "attn_mfma", False),
+    ([900, 33, 470], 8, 32, 0, 0, "attn_mfma", False), ([60, 50, 61, 33] * 8, 8, 64, 0, 0, "attn_fine", False),
+    ([190, 131, 181], 16, 32, 0, 0, "attn_fine", False),
+    ([5, 3, 12, 9], 2, 64, 0, 0, "attn_rows", False), ([1, 2, 15], 3, 24, 4, 0, "attn_rows", False),
+    ([40, 41] * 16, 1, 32, 0, 0, "attn_once", False), ([40, 41] * 16 + [8], 1, 32, 0, 0, "attn_once", True),   # one document more
+    ([2560, 2559], 1, 32, 90, 0, "attn_once", False), ([2560, 2561], 1, 32, 90, 0, "attn_once", True),           # one item more
+    ([100, 61], 2, 32, 0, 5, "attn_once", True), ([100, 61], 2, 48, 0, 0, "attn_mfma", True)])   # rows between; heads of no own kernel
+def test_attention_over_unequal_documents(lens, H, hd, window, gap, kernel, staged, dev):
+    """Packed documents of unequal lengths in one call, at the most documents and work items that the kernel arguments hold and
+    beyond, from each kernel, against the sums in 64 bits."""
+    import torch
+    lib = api.load()
+    starts = np.concatenate([[0], np.cumsum(np.array(lens) + gap)])
+    T, E, scale = int(starts[-1]), H * hd, 1.0 / np.sqrt(hd)
+    rs = np.random.RandomState(T)
+    qkv = rs.randn(T, 3 * E).astype(np.float32)
+    rows, want = qkv.astype(np.float64), np.full((T, E), 7.0)
+    tq, to = torch.from_numpy(qkv).cuda(), torch.full((T, E), 7.0, dtype=torch.float32, device="cuda")
+    probs = []
+    for first, n in zip(starts[:-1].tolist(), lens):
+        back = np.arange(n)[:, None] - np.arange(n)[None, :]
+        hidden = (back < 0) | ((back >= window) if window else False)
+        for h in range(H):
+            q, k, v = (rows[first:first + n, i * E + h * hd:i * E + (h + 1) * hd] for i in range(3))
+            x = np.where(hidden, -np.inf, q @ k.T * scale)
+            w = np.exp(x - x.max(axis=1, keepdims=True))
+            want[first:first + n, h * hd:(h + 1) * hd] = w / w.sum(axis=1, keepdims=True) @ v
+            a = abi.BltAttentionHeadArgs()
+            a.q, a.k, a.v = (tq.data_ptr() + 4 * (first * 3 * E + i * E + h * hd) for i in range(3))
+            a.q_stride = a.k_stride = a.v_stride = 3 * E
+            a.combined, a.combined_stride, a.combined_col_offset = to.data_ptr() + 4 * first * E, E, h * hd
+            a.nq = a.nk = n
+            a.head_dim, a.scale = hd, scale
+            probs.append(api.problem(a, api.BLT_ATTN_MASK_CAUSAL, window=window))
+    lib.blt_hip_profile_begin()
+    lib.blt_attention_batch_hip(api.problem_array(probs), len(probs))
+    names = set(api.profile_end())
+    lib.blt_backend_pass_sync_hip()
+    assert names == ({kernel, "upload_words"} if staged else {kernel}), names
+    assert_close(to.cpu().numpy(), want.astype(np.float32), "documents of %s rows" % lens)
+
+
 @pytest.mark.parametrize("T,H,hd,docs", [(200, 2, 32, [0, 7, 90, 150]), (512, 4, 32, [0, 300]), (128, 8, 64, [0]),
                                          (96, 2, 64, [0, 20, 40, 60, 80])])
 def test_document_causal_ranges_take_the_matrix_cores(T, H, hd, docs, oracle, dev):
