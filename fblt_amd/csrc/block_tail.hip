@@ -241,10 +241,34 @@ __global__ __launch_bounds__(Shape::THREADS) void block_tail_kernel(BlockTailArg
 constexpr uint32_t CROSS_ROWS = 16384;
 constexpr uint32_t CROSS_KEYS = 4;
 
+/* Where rows find their key ranges: in memory ... */
+struct RangesThere {};
+__device__ __forceinline__ void find_range(const CrossBlockArgs &a, RangesThere, uint32_t row, uint32_t &lo, uint32_t &hi) {
+    lo = a.lo[row], hi = a.hi[row];
+}
+__device__ __forceinline__ void leave_ranges(RangesThere, uint32_t, uint32_t) {}
+/* ... or in the kernel arguments, and then the first of a row tile's workgroups leaves them there.  With a launch that only brings them a
+ * prompt of 512 bytes takes 66.2 us, so 64.6. */
+__device__ __forceinline__ uint32_t range_start(const CrossWords &w, uint32_t row) {
+    return (w.words[w.batch + (row >> 1)] >> (16u * (row & 1u))) & 0xFFFFu;
+}
+__device__ __forceinline__ void find_range(const CrossBlockArgs &, const CrossWords &w, uint32_t row, uint32_t &lo, uint32_t &hi) {
+    lo = range_start(w, row), hi = w.span ? lo + w.span : range_start(w, row + 1u);
+}
+__device__ __forceinline__ void leave_ranges(const CrossWords &w, uint32_t tile, uint32_t threads) {
+    const uint32_t tid = threadIdx.x, row = 16u * tile + tid;
+    if (tid < 16u && row < w.rows) {
+        const uint32_t lo = range_start(w, row);
+        w.lo[row] = lo, w.hi[row] = w.span ? lo + w.span : range_start(w, row + 1u);
+    }
+    if (tile == 0u)
+        for (uint32_t b = tid; b < w.batch; b += threads) w.lens[b] = w.words[b];
+}
+
 /* then(): further requests, behind the first keys'.  Returns the thread's columns of its row; rows and part are free for the taking
  * behind a barrier. */
-template <typename Shape, uint32_t KEYS, typename Then>
-__device__ __forceinline__ floatx4 cross_rows(const CrossBlockArgs &a, uint32_t tile, float *rows, float *part, Then then) {
+template <typename Shape, uint32_t KEYS, typename Range, typename Then>
+__device__ __forceinline__ floatx4 cross_rows(const CrossBlockArgs &a, uint32_t tile, float *rows, float *part, Range range, Then then) {
     using Proj = typename Shape::Proj;
     constexpr int E = Shape::E, ROW = Shape::ROW, EPT = Shape::EPT;
     static_assert(EPT == 4, "a thread holds 16 bytes of a row");
@@ -262,7 +286,8 @@ __device__ __forceinline__ floatx4 cross_rows(const CrossBlockArgs &a, uint32_t 
     if (a.norm_w) norm_w = *reinterpret_cast<const floatx4 *>(a.norm_w + f_col);
     request<Proj::BLOCKS>(wq, a.wq + 64u * group, E, term);
     __builtin_amdgcn_sched_barrier(0);
-    const uint32_t lo = a.lo[row], hi = a.hi[row];
+    uint32_t lo, hi;
+    range(row, lo, hi);
     const uint32_t lanes = a.head_dim / EPT; /* of a head: a power of two up to TPR */
     const size_t slab = (size_t)(row / a.rows_per_seq) * a.slab_rows * E + f_col;
     struct Keys {
@@ -354,9 +379,11 @@ __device__ __forceinline__ floatx4 cross_rows(const CrossBlockArgs &a, uint32_t 
     return resid;
 }
 
-template <typename Shape, uint32_t KEYS = CROSS_KEYS>
-__device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, uint32_t tile, float *rows, float *part) {
-    const floatx4 out = cross_rows<Shape, KEYS>(a, tile, rows, part, [] {});
+template <typename Shape, uint32_t KEYS, typename Ranges>
+__device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, const Ranges &w, uint32_t tile, float *rows, float *part) {
+    leave_ranges(w, tile, Shape::THREADS);
+    const floatx4 out = cross_rows<Shape, KEYS>(
+        a, tile, rows, part, [&](uint32_t row, uint32_t &lo, uint32_t &hi) __attribute__((always_inline)) { find_range(a, w, row, lo, hi); }, [] {});
     const uint32_t row = 16u * tile + threadIdx.x / (Shape::E / 4);
     if (row < a.rows) *reinterpret_cast<floatx4 *>(a.out + (size_t)row * Shape::E + 4u * (threadIdx.x % (Shape::E / 4))) = out;
 }
@@ -365,8 +392,8 @@ __device__ __forceinline__ void cross_tile(const CrossBlockArgs &a, uint32_t til
  * of its own -- again, as in the tail --, and the first stores that block's rows.
  * Bound: latency, a chain of two products behind each other and the norm between; for 512 rows of 128 that see a patch each 9.9 us in
  * the kernel trace, against 6.9 and 5.6 and the gap as two launches (a prompt of 512 bytes, two layers: 70.2 / 66.6 us). */
-template <typename Shape>
-__global__ __launch_bounds__(Shape::THREADS) void cross_qkv_kernel(CrossBlockArgs a, MatmulArgs g) {
+template <typename Shape, typename Ranges>
+__global__ __launch_bounds__(Shape::THREADS) void cross_qkv_kernel(CrossBlockArgs a, MatmulArgs g, Ranges w_in) {
     using Proj = typename Shape::Proj;
     constexpr int E = Shape::E, ROW = Shape::ROW;
     constexpr uint32_t TPR = E / 4;
@@ -376,7 +403,9 @@ __global__ __launch_bounds__(Shape::THREADS) void cross_qkv_kernel(CrossBlockArg
     const uint32_t group = wave % Proj::GROUPS, share = wave / Proj::GROUPS, term = share * (16 * Proj::BLOCKS);
     const uint32_t f_row = tid / TPR, f_col = 4u * (tid % TPR), row = 16u * tile + f_row;
     floatx4 w[4 * Proj::BLOCKS], norm_w;
-    floatx4 x = cross_rows<Shape, CROSS_KEYS>(a, tile, rows, part, [&]() __attribute__((always_inline)) {
+    if (third == 0u) leave_ranges(w_in, tile, Shape::THREADS);
+    const auto range = [&](uint32_t r, uint32_t &lo, uint32_t &hi) __attribute__((always_inline)) { find_range(a, w_in, r, lo, hi); };
+    floatx4 x = cross_rows<Shape, CROSS_KEYS>(a, tile, rows, part, range, [&]() __attribute__((always_inline)) {
         norm_w = *reinterpret_cast<const floatx4 *>(g.norm_w + f_col);
         request<Proj::BLOCKS>(w, g.b + third * E + 64u * group, g.ldb, term);
     });
@@ -392,25 +421,34 @@ __global__ __launch_bounds__(Shape::THREADS) void cross_qkv_kernel(CrossBlockArg
     __syncthreads();
     float v[4];
     gather<Proj::SHARES, Proj::PITCH, 4>(part + f_row * Proj::PITCH + f_col, v);
-    if (row < a.rows) matmul_store4<true>(g, row, third * E + f_col, make_float4(v[0], v[1], v[2], v[3]), true);
+    if (row >= a.rows) return;
+    const float4 result = make_float4(v[0], v[1], v[2], v[3]);
+    if constexpr (std::is_same<Ranges, CrossWords>::value) {
+        if (g.stage_k) { /* the lengths are on their way too */
+            const uint32_t b = row / g.stage_n;
+            matmul_stage4(g, row, b, w_in.words[b] + row % g.stage_n, third * E + f_col, result);
+            return;
+        }
+    }
+    matmul_store4<true>(g, row, third * E + f_col, result, true);
 }
 
-template <typename Shape>
-__global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockArgs a) {
+template <typename Shape, typename Ranges>
+__global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockArgs a, Ranges w) {
     __shared__ __attribute__((aligned(16))) float rows[16 * Shape::ROW], part[Shape::Proj::PART];
-    cross_tile<Shape>(a, blockIdx.x, rows, part);
+    cross_tile<Shape, CROSS_KEYS>(a, w, blockIdx.x, rows, part);
 }
 
 /* A block's tail and a cross block that neither reads nor writes anything of it, in the first `first` rows of workgroups: the
  * encoder's, whose patches take up a layer's bytes while the next layer goes on with them.  Its few workgroups fit beside the tail's, so
  * it costs nothing of its own (128 patches of 512 bytes, 128 columns: 9.6 us as a launch).  Half the keys in flight: more registers than the
  * tail has would halve the workgroups of a compute unit. */
-template <typename Shape>
-__global__ __launch_bounds__(Shape::THREADS, 4) void block_tail_beside_kernel(BlockTailArgs a, CrossBlockArgs c, uint32_t first) {
+template <typename Shape, typename Ranges>
+__global__ __launch_bounds__(Shape::THREADS, 4) void block_tail_beside_kernel(BlockTailArgs a, CrossBlockArgs c, uint32_t first, Ranges w) {
     __shared__ TailLds<Shape> lds;
     if (blockIdx.y < first) {
         const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
-        if (tile < (c.rows + 15u) / 16u) cross_tile<Shape, CROSS_KEYS / 2>(c, tile, lds.rows, lds.part);
+        if (tile < (c.rows + 15u) / 16u) cross_tile<Shape, CROSS_KEYS / 2>(c, w, tile, lds.rows, lds.part);
     } else {
         tail_tile<Shape>(a, gridDim.x, blockIdx.x, blockIdx.y - first, lds);
     }
@@ -421,7 +459,13 @@ void launch_tail(const BlockTailArgs &a, dim3 grid, hipStream_t s, const CrossBl
     if constexpr (Shape::PROJ) {
         if (beside) {
             const uint32_t first = ((beside->rows + 15u) / 16u + grid.x - 1u) / grid.x;
-            blt_launch("block_tail", block_tail_beside_kernel<Shape>, dim3(grid.x, grid.y + first), dim3(Shape::THREADS), 0, s, a, *beside, first);
+            const dim3 both(grid.x, grid.y + first);
+            if (beside->words)
+                blt_launch("block_tail", block_tail_beside_kernel<Shape, CrossWords>, both, dim3(Shape::THREADS), 0, s, a, *beside, first,
+                           *beside->words);
+            else
+                blt_launch("block_tail", block_tail_beside_kernel<Shape, RangesThere>, both, dim3(Shape::THREADS), 0, s, a, *beside, first,
+                           RangesThere());
             return;
         }
     }
@@ -493,6 +537,24 @@ bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim) {
     return a.rows <= CROSS_ROWS;
 }
 
+bool cross_words_fill(CrossWords &w, const uint32_t *lo, const uint32_t *hi, size_t rows, const uint32_t *lens, size_t batch) {
+    if (rows == 0 || batch + rows / 2 + 1 > CrossWords::WORDS) return false;
+    bool alike = hi[0] > lo[0], tiling = true;
+    uint32_t any = hi[rows - 1];
+    for (size_t r = 0; r < rows; r++) {
+        alike = alike && hi[r] - lo[r] == hi[0] - lo[0];
+        tiling = tiling && (r + 1 == rows || hi[r] == lo[r + 1]);
+        any |= lo[r];
+    }
+    if ((!alike && !tiling) || any > 0xFFFFu) return false;
+    BLT_REQUIRE(!blt_stream_capturing(), "host data cannot be staged to the device while a graph is captured");
+    w.rows = (uint32_t)rows, w.batch = (uint32_t)batch, w.span = alike ? hi[0] - lo[0] : 0u, w.reserved = 0;
+    for (size_t b = 0; b < batch; b++) w.words[b] = lens[b];
+    const auto start = [&](size_t r) { return r < rows ? lo[r] : hi[rows - 1]; };
+    for (size_t r = 0; r <= rows; r += 2) w.words[batch + r / 2] = start(r) | start(r + 1) << 16;
+    return true;
+}
+
 void cross_later_launch(CrossLater &later, uint32_t embed_dim, hipStream_t s) {
     matmul_later_launch(later, s);
     if (later.cross_waits) cross_block_launch(later.cross, embed_dim, s);
@@ -502,8 +564,12 @@ void cross_later_launch(CrossLater &later, uint32_t embed_dim, hipStream_t s) {
 bool cross_block_launch(const CrossBlockArgs &a, uint32_t embed_dim, hipStream_t s) {
     if (!cross_block_ok(a, embed_dim)) return false;
     const dim3 grid((a.rows + 15u) / 16u);
-    if (embed_dim == 64u) blt_launch("cross_block", cross_block_kernel<TailShape<64, 4, true>>, grid, dim3(256), 0, s, a);
-    else blt_launch("cross_block", cross_block_kernel<TailShape<128, 8, true>>, grid, dim3(512), 0, s, a);
+    const auto launch = [&](auto narrow, auto wide, const auto &ranges) {
+        if (embed_dim == 64u) blt_launch("cross_block", narrow, grid, dim3(256), 0, s, a, ranges);
+        else blt_launch("cross_block", wide, grid, dim3(512), 0, s, a, ranges);
+    };
+    if (a.words) launch(cross_block_kernel<TailShape<64, 4, true>, CrossWords>, cross_block_kernel<TailShape<128, 8, true>, CrossWords>, *a.words);
+    else launch(cross_block_kernel<TailShape<64, 4, true>, RangesThere>, cross_block_kernel<TailShape<128, 8, true>, RangesThere>, RangesThere());
     return true;
 }
 
@@ -518,7 +584,12 @@ bool cross_qkv_launch(const CrossBlockArgs &a, const MatmulArgs &g, uint32_t emb
     for (const void *p : {(const void *)g.b, (const void *)g.norm_w, (const void *)g.out, (const void *)g.stage_k, (const void *)g.stage_v})
         if ((reinterpret_cast<uintptr_t>(p) & 15u) != 0u) return false;
     const dim3 grid(3u, tiles);
-    if (embed_dim == 64u) blt_launch("cross_qkv", cross_qkv_kernel<TailShape<64, 4, true>>, grid, dim3(256), 0, s, a, g);
-    else blt_launch("cross_qkv", cross_qkv_kernel<TailShape<128, 8, true>>, grid, dim3(512), 0, s, a, g);
+    static_assert(sizeof(CrossBlockArgs) + sizeof(MatmulArgs) + sizeof(CrossWords) <= 4096, "kernel argument block");
+    const auto launch = [&](auto narrow, auto wide, const auto &ranges) {
+        if (embed_dim == 64u) blt_launch("cross_qkv", narrow, grid, dim3(256), 0, s, a, g, ranges);
+        else blt_launch("cross_qkv", wide, grid, dim3(512), 0, s, a, g, ranges);
+    };
+    if (a.words) launch(cross_qkv_kernel<TailShape<64, 4, true>, CrossWords>, cross_qkv_kernel<TailShape<128, 8, true>, CrossWords>, *a.words);
+    else launch(cross_qkv_kernel<TailShape<64, 4, true>, RangesThere>, cross_qkv_kernel<TailShape<128, 8, true>, RangesThere>, RangesThere());
     return true;
 }

@@ -538,7 +538,8 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
         }
     }
     uint32_t *dev = (uint32_t *)blt_arena_alloc(arena, host.size() * sizeof(uint32_t), 64);
-    blt_upload_staged(dev, host.data(), host.size() * sizeof(uint32_t));
+    CrossWords words; /* with the first layer's cross block, where it comes first */
+    bool carried = false;
 
     float *ping = (float *)blt_arena_alloc(arena, rows * E * sizeof(float), 64);
     float *pong = (float *)blt_arena_alloc(arena, rows * E * sizeof(float), 64);
@@ -547,6 +548,23 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
     float *xnorm = (float *)blt_arena_alloc(arena, rows * E * sizeof(float), 64);
     float *xcomb = (float *)blt_arena_alloc(arena, rows * E * sizeof(float), 64);
     const size_t arena_mark = arena->offset;
+    const auto cross_of = [&](size_t l, const float *x) {
+        const blt_local_layer_storage *s = &dec->layers[l];
+        CrossBlockArgs whole;
+        std::memset(&whole, 0, sizeof(whole));
+        whole.x = whole.residual = x, whole.out = mid, whole.norm_w = (const float *)s->cross_norm_weight.data;
+        whole.wq = (const float *)s->cross_weight_q.data, whole.proj = (const float *)s->cross_weight_proj.data;
+        whole.k = (const float *)cache->cross_k[l].data, whole.v = (const float *)cache->cross_v[l].data;
+        whole.lo = dev + batch, whole.hi = dev + batch + rows, whole.slab_rows = cache->max_subtokens;
+        whole.rows = (uint32_t)rows, whole.rows_per_seq = (uint32_t)n, whole.head_dim = (uint32_t)xhd;
+        whole.scale = 1.0f / sqrtf((float)xhd);
+        return whole;
+    };
+    if (rows > 32 && L > 0 && cross_fires(cfg, 0) && !own_positions && cross_block_ok(cross_of(0, d0_rows), (uint32_t)E)) {
+        carried = cross_words_fill(words, host.data() + batch, host.data() + batch + rows, rows, host.data(), batch);
+        words.lens = dev, words.lo = dev + batch, words.hi = dev + batch + rows;
+    }
+    if (!carried) blt_upload_staged(dev, host.data(), host.size() * sizeof(uint32_t));
 
     const float *cur = d0_rows;
     for (size_t l = 0; l < L; l++) {
@@ -559,13 +577,8 @@ void decode_step_run(const blt_kv_cache *cache, size_t batch, size_t n, const si
             check_weight(&s->cross_weight_q, E, E, "blt_kv_decode_step: cross_weight_q must be [embed_dim, embed_dim]");
             check_weight(&s->cross_weight_proj, E, E,
                          "blt_kv_decode_step: cross_weight_proj must be [embed_dim, embed_dim]");
-            std::memset(&whole, 0, sizeof(whole));
-            whole.x = whole.residual = cur, whole.out = mid, whole.norm_w = (const float *)s->cross_norm_weight.data;
-            whole.wq = (const float *)s->cross_weight_q.data, whole.proj = (const float *)s->cross_weight_proj.data;
-            whole.k = (const float *)cache->cross_k[l].data, whole.v = (const float *)cache->cross_v[l].data;
-            whole.lo = dev + batch, whole.hi = dev + batch + rows, whole.slab_rows = cache->max_subtokens;
-            whole.rows = (uint32_t)rows, whole.rows_per_seq = (uint32_t)n, whole.head_dim = (uint32_t)xhd;
-            whole.scale = 1.0f / sqrtf((float)xhd);
+            whole = cross_of(l, cur);
+            if (l == 0 && carried) whole.words = &words;
             MatmulArgs probe;
             std::memset(&probe, 0, sizeof(probe));
             probe.m = (uint32_t)rows, probe.k = (uint32_t)E, probe.n = (uint32_t)E;

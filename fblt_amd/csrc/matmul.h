@@ -71,17 +71,22 @@ struct MatmulArgs {
 
 /* Four consecutive results of output row `row` starting at column `col`:
  * optional rotation, optional residual, store with bounds. */
+/* of row `row` at position pos of sequence b: to Q or to the slabs */
+__device__ __forceinline__ void matmul_stage4(const MatmulArgs &g, uint32_t row, uint32_t b, uint32_t pos, uint32_t col, float4 v) {
+    const uint32_t E = g.n / 3u, part = col / E, at = col % E;
+    if (part < 2u) {
+        const size_t turn = (size_t)pos * (g.head_dim / 2u) + (at % g.head_dim) / 2u;
+        v = rope_rotate4(v, g.rope_cos + turn, g.rope_sin + turn);
+    }
+    float *const to = part == 0u ? g.out + (size_t)row * E : (part == 1u ? g.stage_k : g.stage_v) + ((size_t)b * g.stage_slab_rows + pos) * E;
+    *reinterpret_cast<float4 *>(to + at) = v;
+}
 template <bool ROPE>
 __device__ __forceinline__ void matmul_store4(const MatmulArgs &g, uint32_t row, uint32_t col, float4 v, bool vec_ok) {
     if (ROPE && g.stage_k) { /* new rows of a cache: no residual */
         if (col >= g.n) return;
-        const uint32_t E = g.n / 3u, part = col / E, at = col % E, b = row / g.stage_n, pos = g.stage_len[b] + row % g.stage_n;
-        if (part < 2u) {
-            const size_t turn = (size_t)pos * (g.head_dim / 2u) + (at % g.head_dim) / 2u;
-            v = rope_rotate4(v, g.rope_cos + turn, g.rope_sin + turn);
-        }
-        float *const to = part == 0u ? g.out + (size_t)row * E : (part == 1u ? g.stage_k : g.stage_v) + ((size_t)b * g.stage_slab_rows + pos) * E;
-        *reinterpret_cast<float4 *>(to + at) = v;
+        const uint32_t b = row / g.stage_n;
+        matmul_stage4(g, row, b, g.stage_len[b] + row % g.stage_n, col, v);
         return;
     }
     if (ROPE && col < g.rope_cols) {
@@ -134,6 +139,17 @@ struct BlockTailArgs {
 /* A cross block past its K and V rows, in one launch (block_tail.hip): out = residual + combined * proj, where row r of
  * `combined` attends, head by head, from RMSNorm(x) * wq (x * wq without norm_w) over rows lo[r] .. hi[r] - 1 of k and v,
  * counted from slab_rows * (r / rows_per_seq); no rows: zeros.  All dense rows of embed_dim; out may be x. */
+/* Key ranges on their way: a pass's first cross block brings them in its arguments and leaves them, and the lengths of the sequences,
+ * where later launches look for them.  words: the lengths, then the ranges' starts, two in each, and after them, if a range ends where
+ * the next one starts (span 0; else all are that long), the last one's end. */
+struct CrossWords {
+    static constexpr uint32_t WORDS = 880; /* with the other arguments of the largest launch, a block of 4096 bytes */
+    uint32_t *lo, *hi, *lens;
+    uint32_t rows, batch, span, reserved;
+    uint32_t words[WORDS];
+};
+/* false: not of this kind, the caller uploads them.  lens: batch of them (none: of no use to later launches). */
+bool cross_words_fill(CrossWords &w, const uint32_t *lo, const uint32_t *hi, size_t rows, const uint32_t *lens, size_t batch);
 struct CrossBlockArgs {
     const float *x, *norm_w, *wq, *k, *v, *proj, *residual; /* norm_w, residual: optional */
     float *out;
@@ -141,6 +157,7 @@ struct CrossBlockArgs {
     uint64_t slab_rows;
     uint32_t rows, rows_per_seq, head_dim;
     float scale;
+    const CrossWords *words; /* the launcher's: what lo and hi are to hold (null: they do) */
 };
 /* false: not for this shape, nothing was launched.  cross_block_ok: the same answer before lo and hi are there. */
 bool cross_block_ok(const CrossBlockArgs &a, uint32_t embed_dim);
@@ -159,6 +176,7 @@ struct CrossLater {
 struct CrossPass {
     const uint32_t *lo = nullptr, *hi = nullptr; /* the mask's key ranges on the device; lo null: not there (yet) */
     uint32_t span = 0;
+    CrossWords words;
     CrossLater *later = nullptr; /* a block may be left there instead of launched */
     /* K and V weights of the next block over the same rows: its keys and values may be made in this block's launch ... */
     const blt_tensor *next_k = nullptr, *next_v = nullptr;

@@ -433,17 +433,17 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     const uint32_t *row_lo = nullptr, *row_hi = nullptr;
     const float *dense = nullptr;
     uint32_t row_span = 0;
+    std::vector<uint32_t> lohi; /* the ranges, until they are on the device or on their way there */
     if (pass != nullptr && pass->lo != nullptr) {
         row_lo = pass->lo, row_hi = pass->hi, row_span = pass->span;
     } else {
-        std::vector<uint32_t> lohi(2 * P);
+        lohi.resize(2 * P);
         if (blt_mask_config_row_ranges(mc, lohi.data(), lohi.data() + P) == 1) {
             for (size_t i = 0; i < P; i++) { /* the dense builder refuses such a mask (mask_builder_cpu.c:93) */
                 BLT_REQUIRE(lohi[i] < lohi[P + i], "blt_build_attention_mask: query position has no valid key");
                 row_span = std::max(row_span, lohi[P + i] - lohi[i]);
             }
             uint32_t *dev = (uint32_t *)blt_arena_alloc(arena, 2 * P * sizeof(uint32_t), 64);
-            blt_upload_staged(dev, lohi.data(), 2 * P * sizeof(uint32_t));
             row_lo = dev, row_hi = dev + P;
             if (pass != nullptr) pass->lo = row_lo, pass->hi = row_hi, pass->span = row_span;
         } else {
@@ -479,7 +479,16 @@ void blt_cross_attention_run(const blt_tensor *query_in, const blt_tensor *kv_in
     whole.k = k, whole.v = v, whole.lo = row_lo, whole.hi = row_hi;
     whole.rows = whole.rows_per_seq = (uint32_t)P, whole.head_dim = (uint32_t)hd, whole.scale = 1.0f / sqrtf((float)hd);
     /* up to 32 rows the products of a block by itself keep the reference's order of sums */
-    if (row_lo != nullptr && (P > 32 || tolerant) && T != 0 && row_span <= CROSS_SPAN && cross_block_ok(whole, (uint32_t)E)) {
+    const bool one = row_lo != nullptr && (P > 32 || tolerant) && T != 0 && row_span <= CROSS_SPAN && cross_block_ok(whole, (uint32_t)E);
+    if (row_lo != nullptr && !lohi.empty()) {
+        if (one && pass != nullptr && cross_words_fill(pass->words, lohi.data(), lohi.data() + P, P, nullptr, 0)) {
+            pass->words.lo = const_cast<uint32_t *>(row_lo), pass->words.hi = const_cast<uint32_t *>(row_hi), pass->words.lens = nullptr;
+            whole.words = &pass->words;
+        } else {
+            blt_upload_staged(const_cast<uint32_t *>(row_lo), lohi.data(), 2 * P * sizeof(uint32_t));
+        }
+    }
+    if (one) {
         if (!made && pass != nullptr && pass->next_k != nullptr) {
             check_2d_fp32(pass->next_k, E, E, "blt_cross_attention: weight_k must be [embed_dim, embed_dim] FP32");
             check_2d_fp32(pass->next_v, E, E, "blt_cross_attention: weight_v must be [embed_dim, embed_dim] FP32");

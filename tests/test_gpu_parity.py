@@ -2673,6 +2673,18 @@ def test_kv_decode_step_whose_cross_blocks_go_with_the_qkv_product(batch, n, E, 
     assert all(("cross_qkv" in names) == joined and ("cross_block" in names) != joined for names in launched), launched
 
 
+@pytest.mark.parametrize("batch,n,E,k,every,staged", [
+    (1, 33, 128, 2, True, False), (3, 15, 64, 3, True, False), (59, 16, 128, 1, True, False), (130, 10, 64, 1, True, False),
+    (1, 1757, 64, 1, True, False), (1, 1758, 64, 1, True, True),           # as many rows as go along, and one more
+    (59, 16, 128, 1, False, True), (1, 40, 256, 1, True, True)])             # no cross block in front; none in one launch
+def test_kv_decode_step_whose_row_ranges_go_with_the_first_launch(batch, n, E, k, every, staged, oracle, dev):
+    """Lengths and row ranges in the arguments of the first layer's cross block, which the later layers find in memory, or by a
+    launch of their own, against the restated step."""
+    c = dict(E=E, H=E // 32, XH=E // 32, L=2, hidden=64, V=16, max_len=2 * n + 60, k=k, window=0, all_layers=every, placement=0)
+    launched = _decode_steps(batch, n, c, 690 + batch, oracle)
+    assert all(("upload_words" in names) == staged for names in launched), launched
+
+
 @pytest.mark.parametrize("batch,n,case", [(1, 1, 2), (9, 8, 2), (33, 1, 0)])
 def test_kv_decode_step_of_rows_whose_norm_overflows(batch, n, case, oracle, dev):
     """Input rows of 1e20: their sum of squares is infinite and the normalised row zero, in the one-launch form as in
