@@ -22,6 +22,7 @@
 #include "launch.h"
 #include "matmul.h"
 
+#include <cstddef>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -39,6 +40,8 @@ void blt_transformer_run(const blt_tensor *input, const blt_transformer_weights 
                          const blt_transformer_config *config, blt_arena *arena, CrossLater *later);
 
 namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int IDX_PER_LAUNCH = 512; /* index entries a launch carries in its arguments */
 struct IndexChunk {
@@ -91,26 +94,108 @@ __global__ __launch_bounds__(256) void patch_pool_kernel(const float *__restrict
 }
 
 constexpr int MAX_TABLES = BLT_MAX_NGRAM_SIZES;
-struct EmbedTables {
-    const float *table[MAX_TABLES];
-    const uint32_t *idx[MAX_TABLES]; /* device arrays [seq_len], sentinel = no contribution */
-    uint32_t count;
+constexpr uint32_t EMBED_RUNS = 256;   /* patches of a launch */
+constexpr uint32_t EMBED_BYTES = 2560; /* bytes of text that travel in the arguments */
+constexpr uint32_t EMBED_ROWS = 8;     /* rows of a patch at a time */
+constexpr uint32_t EMBED_COLS = 512;   /* columns of a workgroup */
+struct EmbedArgs {
+    const float *byte_table;
+    const float *table[MAX_TABLES]; /* [modulus, embed_dim] each */
+    const uint8_t *bytes;           /* null: text */
+    float *h;                       /* [all rows, embed_dim] */
+    float *pooled;                  /* of the launch's patches, copies blocks of columns of each row (null: rows only) */
+    uint64_t modulus, power[8];     /* prime^i mod modulus */
+    uint32_t ngram[MAX_TABLES], tables, embed_dim, out_stride, copies;
+    int scaled, take_max;
+    float scale;
+    uint32_t start[EMBED_RUNS + 1]; /* patches follow each other */
+    uint8_t text[EMBED_BYTES];
 };
+static_assert(sizeof(EmbedArgs) <= 4096, "kernel argument block");
 
-/* out[i, :] = (byte_table[ids[i], :] + table_0[idx_0[i], :] + ... ) * scale, the tables in order */
-__global__ __launch_bounds__(256) void embed_sum_kernel(const float *__restrict__ byte_table,
-                                                        const uint32_t *__restrict__ ids, float *__restrict__ out,
-                                                        uint32_t embed_dim, EmbedTables t, int scaled, float scale) {
-    const uint32_t i = blockIdx.x;
-    const float *base = byte_table + (uint64_t)ids[i] * embed_dim;
-    for (uint32_t d = threadIdx.x; d < embed_dim; d += 256u) {
-        float acc = base[d];
-        for (uint32_t n = 0; n < t.count; n++) {
-            const uint32_t at = t.idx[n][i];
-            if (at != BLT_IDX_SENTINEL) acc += t.table[n][(uint64_t)at * embed_dim + d];
+/* h[i, :] = (byte_table[byte i, :] + table_0[index_0 of i, :] + ...) * scale, the tables in order; an index is the reference's rolling
+ * polynomial hash (csrc/models/hash_ngram.c:16-79) in closed form: position i >= n - 1 hashes bytes b[i-n+1..i] as sum b[j] *
+ * prime^(i-j) mod modulus, earlier positions have no n-gram.  And the mean or maximum of a patch's rows, first to last (the
+ * reference's order).
+ * A workgroup is a patch, eight rows at a time: one wave hashes their n-grams while the others wait, then a thread has four columns of
+ * a row (one where VEC is false), all its table rows requested before the first is added, and the rows of the eight meet in LDS.
+ * Bound: latency (byte, hash, table row, row sums).  A forward of 512 bytes, one layer of 128 columns each: 100.4 us, from 116.1 with the
+ * indices made on the host, uploaded and the patches pooled in three launches, and 171 with the bytes on the device. */
+template <bool VEC>
+__global__ __launch_bounds__(256) void embed_pool_kernel(EmbedArgs a) {
+    constexpr uint32_t W = VEC ? 4u : 1u;
+    __shared__ uint32_t index[EMBED_ROWS][MAX_TABLES + 1];
+    __shared__ __attribute__((aligned(16))) float sum[EMBED_ROWS][EMBED_COLS];
+    const uint32_t tid = threadIdx.x, E = a.embed_dim;
+    const uint32_t first = a.start[blockIdx.x], end = a.start[blockIdx.x + 1u];
+    const uint32_t col0 = blockIdx.y * EMBED_COLS, cols = min(EMBED_COLS, E - col0), pieces = cols / W;
+    const uint8_t *const bytes = a.bytes;
+    const auto byte_at = [&](uint32_t i) -> uint64_t { return bytes ? bytes[i] : a.text[i]; };
+    float pooled[EMBED_COLS / 256u] = {0.f, 0.f};
+    for (uint32_t row0 = first; row0 < end; row0 += EMBED_ROWS) {
+        const uint32_t rows = min(EMBED_ROWS, end - row0);
+        if (tid < 8u * EMBED_ROWS) {
+            const uint32_t r = tid >> 3, t = tid & 7u, i = row0 + r; /* lane 0: the byte itself, 1 ...: the tables */
+            if (r < rows && t <= a.tables) {
+                const uint32_t n = t == 0u ? 1u : a.ngram[t - 1u];
+                uint32_t at = BLT_IDX_SENTINEL;
+                if (i + 1u >= n) {
+                    uint64_t hash = 0; /* below 8 * 255 * modulus; no table has 2^50 rows */
+                    for (uint32_t j = 0; j < n; j++) hash += byte_at(i - j) * (t == 0u ? 1u : a.power[j]);
+                    at = (uint32_t)hash;
+                    if (t != 0u) at = (hash | a.modulus) >> 32 ? (uint32_t)(hash % a.modulus) : (uint32_t)hash % (uint32_t)a.modulus;
+                }
+                index[r][t] = at;
+            }
         }
-        if (scaled) acc *= scale;
-        out[(uint64_t)i * embed_dim + d] = acc;
+        __syncthreads();
+        for (uint32_t item = tid; item < rows * pieces; item += 256u) {
+            const uint32_t r = item / pieces, d = col0 + W * (item % pieces);
+            const auto add_up = [&](auto zero) {
+                typedef decltype(zero) Vec;
+                Vec acc = *reinterpret_cast<const Vec *>(a.byte_table + (uint64_t)index[r][0] * E + d), v[MAX_TABLES];
+#pragma unroll
+                for (uint32_t t = 0; t < MAX_TABLES; t++) {
+                    if (t >= a.tables) break;
+                    const uint32_t at = index[r][t + 1u];
+                    v[t] = *reinterpret_cast<const Vec *>(a.table[t] + (uint64_t)(at == BLT_IDX_SENTINEL ? 0u : at) * E + d);
+                }
+#pragma unroll
+                for (uint32_t t = 0; t < MAX_TABLES; t++) {
+                    if (t >= a.tables) break;
+                    if (index[r][t + 1u] != BLT_IDX_SENTINEL) acc += v[t];
+                }
+                if (a.scaled) acc *= a.scale;
+                *reinterpret_cast<Vec *>(a.h + (uint64_t)(row0 + r) * E + d) = acc;
+                *reinterpret_cast<Vec *>(&sum[r][d - col0]) = acc;
+            };
+            if constexpr (VEC) add_up(floatx4{0.f, 0.f, 0.f, 0.f});
+            else add_up(0.f);
+        }
+        __syncthreads();
+        if (a.pooled) {
+#pragma unroll
+            for (uint32_t c = 0; c < EMBED_COLS / 256u; c++) {
+                const uint32_t d = tid + 256u * c;
+                if (d >= cols) break;
+                if (a.take_max) {
+                    if (row0 == first) pooled[c] = sum[0][d];
+                    for (uint32_t r = row0 == first ? 1u : 0u; r < rows; r++)
+                        if (sum[r][d] > pooled[c]) pooled[c] = sum[r][d];
+                } else {
+                    for (uint32_t r = 0; r < rows; r++) pooled[c] += sum[r][d];
+                }
+            }
+            __syncthreads(); /* before the next eight */
+        }
+    }
+    if (!a.pooled) return;
+#pragma unroll
+    for (uint32_t c = 0; c < EMBED_COLS / 256u; c++) {
+        const uint32_t d = tid + 256u * c;
+        if (d >= cols) break;
+        if (!a.take_max) pooled[c] *= 1.0f / (float)(end - first);
+        for (uint32_t copy = 0; copy < a.copies; copy++) a.pooled[(uint64_t)blockIdx.x * a.out_stride + copy * E + col0 + d] = pooled[c];
     }
 }
 
@@ -157,24 +242,17 @@ void pool_launch(const float *h, size_t seq_len, size_t embed_dim, const blt_pat
     }
 }
 
-/* The reference's rolling polynomial hash (csrc/models/hash_ngram.c:16-79), restated in closed
- * form: position i >= n - 1 hashes bytes b[i-n+1..i] as sum b[j] * prime^(i-j) mod modulus;
- * earlier positions have no n-gram.  prime * modulus fits 64 bits (checked as the reference does),
- * so no product overflows. */
-void ngram_indices(const uint8_t *bytes, size_t seq_len, size_t n, uint64_t prime, uint64_t modulus, uint32_t *idx) {
-    BLT_REQUIRE(n > 0 && n <= 8, "blt_rolling_hash_init: n must be in [1, 8]");
-    BLT_REQUIRE(modulus > 1, "blt_rolling_hash_init: modulus must be > 1");
-    BLT_REQUIRE(prime > 0 && prime <= ((UINT64_MAX - 255) / modulus),
-                "blt_rolling_hash_init: prime * modulus would overflow uint64");
-    for (size_t i = 0; i < seq_len; i++) {
-        if (i + 1 < n) {
-            idx[i] = BLT_IDX_SENTINEL;
-            continue;
-        }
-        uint64_t hash = 0;
-        for (size_t j = i + 1 - n; j <= i; j++) hash = (hash * prime + bytes[j]) % modulus;
-        idx[i] = (uint32_t)hash;
+/* Do the patches follow each other over all rows?  Then the launch that makes the rows pools them, but for long ones, whose rows it
+ * would make eight after eight: a forward of 512 bytes, some patches of 8 / 64 / 256 rows, 98.7 / 121.6 / 157.7 us so, 101.1 / 125.2 /
+ * 158.4 with the pooling as a launch. */
+bool patches_tile(const blt_patch_info *patches, size_t num_patches, size_t seq_len) {
+    size_t at = 0;
+    for (size_t j = 0; j < num_patches; j++) {
+        if (patches[j].start_idx != at || patches[j].length < 1 || patches[j].length > std::min<size_t>(256, seq_len - at))
+            return false;
+        at += patches[j].length;
     }
+    return at == seq_len;
 }
 
 } // namespace
@@ -229,9 +307,9 @@ extern "C" void blt_patch_pool_forward_hip(const blt_tensor *byte_hidden, const 
                 (float *)out->data, embed_dim, 1);
 }
 
-/* csrc/models/local_encoder.c:193-281 on device tensors.  bytes_in may live on either side (the
- * ids are consumed on the host, as in the reference); weights, outputs and the arena are device
- * memory.  Index arrays and mask metadata are host allocations of this call. */
+/* csrc/models/local_encoder.c:193-281 on device tensors.  bytes_in may live on either side (on the
+ * host it may change on return, on the device it is read in stream order); weights, outputs and the
+ * arena are device memory.  Mask metadata is a host allocation of this call. */
 extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, const blt_tensor *bytes_in,
                                               const blt_patch_info *patches, size_t num_patches,
                                               const size_t *doc_boundaries, size_t num_docs, blt_tensor *patch_out,
@@ -266,37 +344,60 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
     BLT_REQUIRE(ng.num_ngram_sizes <= BLT_MAX_NGRAM_SIZES && ng.embed_dim == E,
                 "blt_local_encoder_forward: ngram_config does not fit the encoder");
 
-    /* ---- ids and bucket indices: host work, one upload ---- */
-    std::vector<uint8_t> bytes(seq_len);
-    if (bytes_in->backend == BLT_BACKEND_HIP) blt_hip_memcpy_d2h(bytes.data(), bytes_in->data, seq_len);
-    else std::memcpy(bytes.data(), bytes_in->data, seq_len);
-    std::vector<uint32_t> host_idx((1 + (size_t)MAX_TABLES) * seq_len);
-    for (size_t i = 0; i < seq_len; i++) host_idx[i] = bytes[i];
-    EmbedTables tables;
-    std::memset(&tables, 0, sizeof(tables));
-    uint32_t *dev_idx = (uint32_t *)blt_arena_alloc(arena, host_idx.size() * sizeof(uint32_t), 64);
+    /* ---- byte rows with their n-grams, and P_0: pooled rows in every sub-token column block (local_encoder.c:237-245) ---- */
+    const hipStream_t stream = blt_stream();
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (bytes_in->backend == BLT_BACKEND_HIP && stream != nullptr) HIP_CHECK(hipStreamIsCapturing(stream, &capture));
+    BLT_REQUIRE(!blt_stream_capturing() && capture == hipStreamCaptureStatusNone,
+                "blt_local_encoder_forward: bytes and patch tables are read on the way, which a graph cannot replay");
+    const size_t byte_shape[2] = {seq_len, E}, patch_shape[2] = {num_patches, patch_dim};
+    EmbedArgs em;
+    std::memset(&em, 0, offsetof(EmbedArgs, start));
+    em.byte_table = (const float *)model->byte_embedding_weight.data;
+    em.modulus = ng.per_ngram_vocab;
     for (size_t t = 0; t < ng.num_ngram_sizes; t++) {
         const size_t n = ng.ngram_sizes[t];
         if (n == 0 || n > seq_len) continue; /* hash_ngram.c:178-180 */
         check_2d(&model->ngram_weights.tables[t], ng.per_ngram_vocab, E, "blt_hash_ngram_forward: weights->tables");
-        uint32_t *dst = host_idx.data() + (1 + (size_t)tables.count) * seq_len;
-        ngram_indices(bytes.data(), seq_len, n, ng.hash_prime, ng.per_ngram_vocab, dst);
-        tables.table[tables.count] = (const float *)model->ngram_weights.tables[t].data;
-        tables.idx[tables.count] = dev_idx + (1 + (size_t)tables.count) * seq_len;
-        tables.count++;
+        BLT_REQUIRE(n <= 8, "blt_rolling_hash_init: n must be in [1, 8]");
+        BLT_REQUIRE(em.modulus > 1, "blt_rolling_hash_init: modulus must be > 1");
+        BLT_REQUIRE(ng.hash_prime > 0 && ng.hash_prime <= ((UINT64_MAX - 255) / em.modulus),
+                    "blt_rolling_hash_init: prime * modulus would overflow uint64");
+        em.table[em.tables] = (const float *)model->ngram_weights.tables[t].data;
+        em.ngram[em.tables++] = (uint32_t)n;
     }
-    blt_hip_memcpy_h2d(dev_idx, host_idx.data(), (1 + (size_t)tables.count) * seq_len * sizeof(uint32_t));
-
-    const size_t byte_shape[2] = {seq_len, E}, patch_shape[2] = {num_patches, patch_dim};
+    if (em.tables != 0) {
+        em.power[0] = 1;
+        for (int i = 1; i < 8; i++) em.power[i] = em.power[i - 1] * ng.hash_prime % em.modulus;
+    }
+    if (bytes_in->backend == BLT_BACKEND_HIP) {
+        em.bytes = (const uint8_t *)bytes_in->data;
+    } else if (seq_len <= EMBED_BYTES) {
+        std::memcpy(em.text, bytes_in->data, seq_len);
+    } else {
+        uint8_t *dev = (uint8_t *)blt_arena_alloc(arena, seq_len, 64);
+        blt_hip_memcpy_h2d(dev, bytes_in->data, seq_len);
+        em.bytes = dev;
+    }
     blt_tensor h = blt_tensor_create_uninit(arena, byte_shape, 2, BLT_DTYPE_FP32);
-    blt_launch("embed_sum", embed_sum_kernel, dim3((unsigned)seq_len), dim3(256), 0, blt_stream(),
-               (const float *)model->byte_embedding_weight.data, (const uint32_t *)dev_idx, (float *)h.data,
-               (uint32_t)E, tables, ng.normalize ? 1 : 0, 1.0f / (float)(ng.num_ngram_sizes + 1));
-    HIP_CHECK_LAUNCH("blt_local_encoder_forward: embedding");
-
-    /* ---- P_0: pooled rows in every sub-token column block (local_encoder.c:237-245) ---- */
     blt_tensor p = blt_tensor_create_uninit(arena, patch_shape, 2, BLT_DTYPE_FP32);
-    pool_launch((const float *)h.data, seq_len, E, patches, num_patches, cfg.pool_type, (float *)p.data, patch_dim, k);
+    em.h = (float *)h.data, em.embed_dim = (uint32_t)E;
+    em.scaled = ng.normalize ? 1 : 0, em.scale = 1.0f / (float)(ng.num_ngram_sizes + 1);
+    em.out_stride = (uint32_t)patch_dim, em.copies = (uint32_t)k, em.take_max = cfg.pool_type == BLT_POOL_MAX ? 1 : 0;
+    const bool tile = patches_tile(patches, num_patches, seq_len) && (cfg.pool_type == BLT_POOL_MEAN || cfg.pool_type == BLT_POOL_MAX);
+    const size_t runs = tile ? num_patches : (seq_len + EMBED_ROWS - 1) / EMBED_ROWS;
+    bool vec = E % 4 == 0 && (reinterpret_cast<uintptr_t>(em.byte_table) & 15u) == 0;
+    for (uint32_t t = 0; t < em.tables; t++) vec = vec && (reinterpret_cast<uintptr_t>(em.table[t]) & 15u) == 0;
+    for (size_t j0 = 0; j0 < runs; j0 += EMBED_RUNS) {
+        const size_t n = std::min<size_t>(EMBED_RUNS, runs - j0);
+        for (size_t j = 0; j < n; j++) em.start[j] = (uint32_t)(tile ? patches[j0 + j].start_idx : (j0 + j) * EMBED_ROWS);
+        em.start[n] = (uint32_t)(j0 + n == runs ? seq_len : tile ? patches[j0 + n].start_idx : (j0 + n) * EMBED_ROWS);
+        em.pooled = tile ? (float *)p.data + j0 * patch_dim : nullptr;
+        const dim3 grid((unsigned)n, (unsigned)((E + EMBED_COLS - 1) / EMBED_COLS));
+        blt_launch("embed_pool", vec ? embed_pool_kernel<true> : embed_pool_kernel<false>, grid, dim3(256), 0, stream, em);
+    }
+    HIP_CHECK_LAUNCH("blt_local_encoder_forward: embedding");
+    if (!tile) pool_launch((const float *)h.data, seq_len, E, patches, num_patches, cfg.pool_type, (float *)p.data, patch_dim, k);
 
     /* ---- masks (local_encoder.c:52-113): host metadata ---- */
     std::vector<size_t> q_groups(num_patches), kv_groups(seq_len), q_groups_split;

@@ -162,12 +162,13 @@ void blt_transformer_forward_hip(const blt_tensor *input, const blt_transformer_
 /* csrc/models/local_encoder.h:71-73 (local_encoder.c:193-281): bytes -> byte embedding + hashed
  * n-gram embeddings -> P_0 = pooled patches (repeated over the k sub-token column blocks) -> per
  * layer the byte transformer block and, where it fires, P += cross_attention(RMSNorm(P), h).
- * bytes_in [seq_len] UINT8 on either side (the ids are hashed on the host, as in the reference);
- * weights, outputs and the arena are device memory; patches, doc_boundaries are HOST arrays.
+ * bytes_in [seq_len] UINT8 on either side (host bytes may change on return, device bytes are read
+ * in stream order, like the other inputs); weights, outputs and the arena are device memory; patches, doc_boundaries are HOST arrays.
  * Unlike the reference's body on a device arena, sub-token splits (patch_dim = k * embed_dim,
  * k > 1) work: the expanded group ids are host memory here. */
 /* csrc/models/local_decoder.c:233-351 on the device: per layer the cross block (when it fires)
- * in three launches and the byte block in five, then the LM head. */
+ * in one to three launches, for 64 or 128 columns with the QKV product behind it, and the byte block
+ * in three to five, then the LM head. */
 void blt_local_decoder_forward_ext_hip(const blt_local_decoder *model, const blt_tensor *byte_hidden_in,
                                        const blt_tensor *patch_in, const blt_patch_info *patches, size_t num_patches,
                                        const size_t *doc_boundaries, size_t num_docs, int trailing_closed,

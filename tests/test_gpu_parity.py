@@ -2970,6 +2970,31 @@ def test_decoder_step_with_exact_projections():
     assert p.returncode == 0, p.stdout[-3000:] + p.stderr[-2000:]
 
 
+@pytest.mark.parametrize("T,E,H,ngrams,vocab,lengths,pool,on_device", [
+    (61, 64, 2, (3, 4, 5, 6, 7, 8), 1000, [1, 7, 8, 9, 16, 17, 3], "mean", True),   # one to three rounds of rows
+    (61, 64, 2, (3, 4, 5, 6, 7, 8), 1000, [1, 7, 8, 9, 16, 17, 3], "max", False),
+    (513, 18, 3, (2,), 50, [1, 2] * 171, "mean", False),                             # single columns; two launches of patches
+    (40, 640, 10, (3, 8), 31, [30, 10], "max", True), (19, 1032, 2, (), 7, [9, 10], "mean", False),   # columns in two, three groups
+    (2560, 4, 1, (1, 8), 5000011, [10] * 256, "mean", False),                        # hashes past 32 bits; as many bytes as travel along
+    (2561, 8, 1, (3,), 97, [10] * 256 + [1], "mean", False), (300, 16, 1, (3,), 97, [257, 43], "max", True)])   # a byte more; too long
+def test_encoder_embeds_and_pools_in_one_launch(T, E, H, ngrams, vocab, lengths, pool, on_device, oracle, dev):
+    """Bytes, hashed n-grams and pooled patches at the edges of the launch, against the restated forward."""
+    from tests import encoder_runs
+    from tests.golden import block_cases
+    lib = api.load()
+    c = dict(T=T, E=E, H=H, XH=H, L=1, hidden=16, ngrams=ngrams, vocab=vocab, k=1, window=0, placement=0, all_layers=True,
+             pool=pool, docs=None, normalize=True, mean_patch=4)
+    assert sum(lengths) == T
+    data, _, weights = block_cases.encoder_case(np.random.RandomState(T), c)
+    want_p, want_h = encoder_runs.run_oracle(oracle, c, data, lengths, weights)
+    lib.blt_hip_profile_begin()
+    got_p, got_h = encoder_runs.run_device(lib.blt_local_encoder_forward, lib, oracle, c, data, lengths, weights, bytes_on_device=on_device)
+    names = set(api.profile_end())
+    assert "embed_pool" in names and ("patch_pool" in names) == (max(lengths) > 256), names
+    assert_close(got_h, want_h, "byte_hidden_out")
+    assert_close(got_p, want_p, "patch_out")
+
+
 def test_encoder_ops(oracle, dev):
     """blt_indexed_row_accumulate / blt_scale / blt_patch_pool_forward on device tensors against the
     restated ops: bit for bit (the kernels keep the reference's order of additions).  Index lists
