@@ -753,8 +753,11 @@ __device__ __forceinline__ void splitk_tile(const MatmulArgs &g, const uint32_t 
     }
 }
 
-template <bool VEC, bool ROPE, bool GATED, int NW = 4, bool CROSS = false>
-__global__ __launch_bounds__(64 * NW, 2) void matmul_splitk_kernel(MatmulArgs g) {
+/* WAVES: registers for as many on a SIMD.  Left alone the compiler takes three registers more than four allow, and then a compute unit
+ * holds one workgroup of eight waves: a product of 384 tiles (512 x 256 x 768) took 7.5 us, 6.5 with two at a time.  Where each
+ * has a compute unit to itself the limit costs a little (512 x 1024 x 256 in two slices 8.55 / 8.76). */
+template <bool VEC, bool ROPE, bool GATED, int NW = 4, bool CROSS = false, int WAVES = 2>
+__global__ __launch_bounds__(64 * NW, WAVES) void matmul_splitk_kernel(MatmulArgs g) {
     __shared__ float part[(GATED ? 2 : 1) * NW][16][64];
     __shared__ float part_ss[NW][32];
     __shared__ float qt[CROSS ? 32 * 33 : 1];
@@ -1005,6 +1008,8 @@ void launch_splitk(const MatmulArgs &g_in, dim3 grid, hipStream_t s) {
         return;
     }
     if (g.b2) blt_launch("matmul_splitk", matmul_splitk_kernel<VEC, ROPE, true>, grid, dim3(256), 0, s, g);
+    else if (eight && VEC && (uint64_t)grid.x * grid.y * grid.z > 256u)
+        blt_launch("matmul_splitk", matmul_splitk_kernel<VEC, ROPE, false, 8, false, VEC ? 4 : 2>, grid, dim3(512), 0, s, g);
     else if (eight) blt_launch("matmul_splitk", matmul_splitk_kernel<VEC, ROPE, false, 8>, grid, dim3(512), 0, s, g);
     else blt_launch("matmul_splitk", matmul_splitk_kernel<VEC, ROPE, false>, grid, dim3(256), 0, s, g);
 }

@@ -1124,6 +1124,22 @@ def test_matmul(m, k, n, exact, oracle, dev):
         assert_close(got, ref, "matmul %dx%dx%d" % (m, k, n))
 
 
+@pytest.mark.parametrize("m,k,n", [(512, 256, 512), (513, 256, 512), (511, 300, 544), (33, 256, 4064), (200, 1000, 1150), (384, 512, 1020)])
+def test_matmul_of_two_small_tiles_a_compute_unit(m, k, n, dev):
+    """Products of 256 small tiles and of more, that share compute units, against float64."""
+    import torch
+    lib = api.load()
+    a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
+    out = torch.full((m, n), 7.0, device="cuda")
+    va, vb, vo = _dev_tensor(a), _dev_tensor(b), _dev_tensor(out)
+    torch.cuda.synchronize()
+    lib.blt_hip_profile_begin()
+    lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    assert set(api.profile_end()) == {"matmul_splitk"}
+    lib.blt_backend_pass_sync_hip()
+    assert _relative(out, a.double() @ b.double()) <= 3 * 2.0 ** -24 * k ** 0.5   # as of products on parts
+
+
 @pytest.mark.parametrize("m,k,n", [(769, 1, 769), (800, 33, 772), (1025, 512, 1540), (2049, 96, 2050), (770, 130, 771)])
 def test_matmul_on_split_operands(m, k, n, dev):
     """Both tile sizes of the product on bf16 parts at ragged edges against float64, then with values that are not finite:
