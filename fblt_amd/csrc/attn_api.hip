@@ -219,8 +219,10 @@ bool choose_once(const AttnProb *p, uint32_t n, uint32_t &span) {
     if (forced != 0 && forced != 5) return false;
     uint64_t tiles = 0;
     uint32_t most = 0;
+    bool matrices = false; /* of masks or weights */
     for (uint32_t i = 0; i < n; i++) {
         if (!attn_once_can(p[i])) return false;
+        matrices = matrices || p[i].weights != nullptr || p[i].vis == ATTN_VIS_DENSE;
         most = std::max(most, attn_once_span_tiles(p[i]));
         tiles += (p[i].nq + 15u) / 16u;
     }
@@ -229,6 +231,10 @@ bool choose_once(const AttnProb *p, uint32_t n, uint32_t &span) {
      * of 256 keys 7.1, mfma 6.8, and 11.3 / 9.8).  Two of shorter rows are better off on the fine kernel, which has half the
      * workgroups (512 tiles of 64 keys 4.8, fine 4.5, and 6.5 / 5.5). */
     if (forced == 0 && tiles > (most > 4u && most <= 8u ? 512u : 256u)) return false;
+    /* Heads of 64 over 513 ... 1024 keys take their keys in two goes.  Four heads, dense mask and weights, one by one: 520 rows 148, so
+     * 60, 1024 rows 232 / 79 (mfma has half the workgroups, and sweeps twice).  Without either, fine: 520 rows 12.7 / 13.1, six
+     * heads of 640 13.8 / 14.3, four of 700 14.8 / 14.4, of 1024 19.0 / 17.0. */
+    if (forced == 0 && p[0].hd == 64u && most > 32u && most < 44u && !matrices) return false;
     span = most;
     return true;
 }

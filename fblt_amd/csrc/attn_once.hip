@@ -1,7 +1,7 @@
 /*
  * "once" kernel family: attention for a tile of 16 query rows whose keys are
  * few enough to be in flight all at once (up to 1024 at head width 32, 512 at
- * 64), for launches that are one trip to memory deep -- a single
+ * 64; up to 1024 at 64 in two goes), for launches that are one trip to memory deep -- a single
  * (sequence, head) problem issued by an unmodified reference caller
  * (csrc/models/attention.c:92-128, cross_attention.c:70-96: dense additive
  * mask, weights_out set), or a handful of long problems.  At those sizes the
@@ -169,7 +169,10 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
     float *const tile = sm_o + wave * (16 * ROW);          /* becomes the wave's partial output later */
     float *const mtile = sm_o + W * (16 * ROW) + wave * (16 * Shape::MROW);
 
-    floatx4 qg[NV], kg[T][NV], vg[T][NV], mg[T]; /* native vectors: arrays of the float4 struct were kept in scratch memory */
+    /* Four tiles of 64 columns a wave do not fit its registers all at once: keys two tiles at a time, values behind the keys. */
+    constexpr bool STAGED = HD * T > 128;
+    constexpr int FLIGHT = STAGED ? 2 : T;
+    floatx4 qg[NV], kg[FLIGHT][NV], vg[T][NV], mg[T]; /* native vectors: arrays of the float4 struct were kept in scratch memory */
 #pragma unroll
     for (int v = 0; v < NV; v++)
         qg[v] = *reinterpret_cast<const floatx4 *>(p.q + (size_t)min(q0 + prow + (uint32_t)(RPI * v), p.nq - 1u) * p.q_stride + 4u * pf);
@@ -191,28 +194,34 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
             }
         }
     }
+    const auto request_keys = [&](int u0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < T; u++) {
-        const uint32_t kt = min(t0 + wave + (uint32_t)(W * u), t1 > 0u ? t1 - 1u : 0u);
+        for (int u = 0; u < FLIGHT; u++) {
+            const uint32_t kt = min(t0 + wave + (uint32_t)(W * (u0 + u)), t1 > 0u ? t1 - 1u : 0u);
 #pragma unroll
-        for (int v = 0; v < NV; v++)
-            kg[u][v] = *reinterpret_cast<const floatx4 *>(
-                p.k + (size_t)min(16u * kt + prow + (uint32_t)(RPI * v), last_key) * p.k_stride + 4u * pf);
-    }
-#pragma unroll
-    for (int u = 0; u < T; u++) {
+            for (int v = 0; v < NV; v++)
+                kg[u][v] = *reinterpret_cast<const floatx4 *>(
+                    p.k + (size_t)min(16u * kt + prow + (uint32_t)(RPI * v), last_key) * p.k_stride + 4u * pf);
+        }
+    };
+    const auto request_values = [&](int u) __attribute__((always_inline)) {
         const uint32_t kt = min(t0 + wave + (uint32_t)(W * u), t1 > 0u ? t1 - 1u : 0u);
 #pragma unroll
         for (int v = 0; v < NV; v++)
             vg[u][v] = *reinterpret_cast<const floatx4 *>(
                 p.v + (size_t)min(16u * kt + prow + (uint32_t)(RPI * v), last_key) * p.v_stride + 4u * pf);
+    };
+    request_keys(0);
+    if constexpr (!STAGED) {
+#pragma unroll
+        for (int u = 0; u < T; u++) request_values(u);
     }
 
     /* ---- fragments: lane (g, c) holds floats [g QD, (g + 1) QD) of row c.  The tile is the wave's
      * own and LDS serves a wave's requests in order, so tile after tile goes through it without
      * a barrier. ---- */
     float qf[QD];
-    float kf[T][QD];
+    float kf[FLIGHT][QD];
     float mk[T][4];
     if (DENSE) {
 #pragma unroll
@@ -231,17 +240,20 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
         const float4 t = *reinterpret_cast<const float4 *>(tile + c * ROW + g * QD + s);
         qf[s + 0] = t.x, qf[s + 1] = t.y, qf[s + 2] = t.z, qf[s + 3] = t.w;
     }
+    const auto key_fragments = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < T; u++) {
+        for (int u = 0; u < FLIGHT; u++) {
 #pragma unroll
-        for (int v = 0; v < NV; v++)
-            *reinterpret_cast<floatx4 *>(tile + (prow + (uint32_t)(RPI * v)) * ROW + 4u * pf) = kg[u][v];
+            for (int v = 0; v < NV; v++)
+                *reinterpret_cast<floatx4 *>(tile + (prow + (uint32_t)(RPI * v)) * ROW + 4u * pf) = kg[u][v];
 #pragma unroll
-        for (int s = 0; s < QD; s += 4) {
-            const float4 t = *reinterpret_cast<const float4 *>(tile + c * ROW + g * QD + s);
-            kf[u][s + 0] = t.x, kf[u][s + 1] = t.y, kf[u][s + 2] = t.z, kf[u][s + 3] = t.w;
+            for (int s = 0; s < QD; s += 4) {
+                const float4 t = *reinterpret_cast<const float4 *>(tile + c * ROW + g * QD + s);
+                kf[u][s + 0] = t.x, kf[u][s + 1] = t.y, kf[u][s + 2] = t.z, kf[u][s + 3] = t.w;
+            }
         }
-    }
+    };
+    key_fragments();
 
     /* ---- phase 1: scores of the wave's tiles, their maximum per query ---- */
     const float scale2 = p.scale * LOG2E; /* log2 units: weights are 2^(x - max) */
@@ -272,7 +284,25 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
 #pragma unroll
         for (int a = 0; a < NA; a++) sa[u][a] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    if (all_on) {
+    if constexpr (STAGED) {
+#pragma unroll
+        for (int u0 = 0; u0 < T; u0 += FLIGHT) {
+            if (u0 > 0) key_fragments();
+            __builtin_amdgcn_sched_barrier(0);
+            if (u0 + FLIGHT < T) request_keys(u0 + FLIGHT);
+            else request_values(0), request_values(1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < FLIGHT; u++)
+                if (on[u0 + u])
+#pragma unroll
+                    for (int s = 0; s < QD; s++)
+                        sa[u0 + u][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][s], qf[s], sa[u0 + u][0], 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 2; u < T; u++) request_values(u);
+        __builtin_amdgcn_sched_barrier(0);
+    } else if (all_on) {
 #pragma unroll
         for (int s = 0; s < QD; s += NA)
 #pragma unroll
@@ -295,9 +325,8 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
     /* while the matrix cores work on the scores: the V rows -> fragments through the same tile; element
      * (d, r) of tile u is column DT c + d of row 4 g + r -- the key whose weight register r of the scores
      * holds, so P^T needs no exchange */
-    float vf[T][DT][4];
-#pragma unroll
-    for (int u = 0; u < T; u++) {
+    float vf[FLIGHT][DT][4];
+    const auto value_fragments = [&](int u, int at) __attribute__((always_inline)) {
 #pragma unroll
         for (int v = 0; v < NV; v++)
             *reinterpret_cast<floatx4 *>(tile + (prow + (uint32_t)(RPI * v)) * ROW + 4u * pf) = vg[u][v];
@@ -306,13 +335,17 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
             const float *vrow = tile + (4u * g + r) * ROW + DT * c;
             if constexpr (DT == 2) {
                 const float2 t = *reinterpret_cast<const float2 *>(vrow);
-                vf[u][0][r] = t.x, vf[u][1][r] = t.y;
+                vf[at][0][r] = t.x, vf[at][1][r] = t.y;
             } else {
                 static_assert(DT == 4, "head widths 32 and 64");
                 const float4 t = *reinterpret_cast<const float4 *>(vrow);
-                vf[u][0][r] = t.x, vf[u][1][r] = t.y, vf[u][2][r] = t.z, vf[u][3][r] = t.w;
+                vf[at][0][r] = t.x, vf[at][1][r] = t.y, vf[at][2][r] = t.z, vf[at][3][r] = t.w;
             }
         }
+    };
+    if constexpr (!STAGED) {
+#pragma unroll
+        for (int u = 0; u < T; u++) value_fragments(u, u);
     }
 #pragma unroll
     for (int u = 0; u < T; u++) {
@@ -358,12 +391,14 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
     for (int d = 0; d < DT; d++) oacc[d] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < T; u++) {
+        const int at = STAGED ? u % FLIGHT : u;
+        if constexpr (STAGED) value_fragments(u, at);
         if (on[u]) {
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
                 for (int d = 0; d < DT; d++)
-                    oacc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][d][r], x[u][r], oacc[d], 0, 0, 0);
+                    oacc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[at][d][r], x[u][r], oacc[d], 0, 0, 0);
         }
     }
     /* lane (g, c) holds columns 4 DT g ... of query row c: park them */
@@ -483,14 +518,15 @@ void once_launch_shape(const AttnProb *dprobs, const AttnTile *dtiles, const typ
     } else {
         if (tiles <= 8u) once_launch_as<64, 8, 1, SRC>(dprobs, dtiles, aff, nblocks, dense, pieces, s);
         else if (tiles <= 16u) once_launch_as<64, 16, 1, SRC>(dprobs, dtiles, aff, nblocks, dense, pieces, s);
-        else once_launch_as<64, 16, 2, SRC>(dprobs, dtiles, aff, nblocks, dense, pieces, s);
+        else if (tiles <= 32u) once_launch_as<64, 16, 2, SRC>(dprobs, dtiles, aff, nblocks, dense, pieces, s);
+        else once_launch_as<64, 16, 4, SRC>(dprobs, dtiles, aff, nblocks, dense, pieces, s);
     }
 }
 
 } // namespace
 
-/* most 16-key tiles a 16-row tile may span at head width hd (sixteen waves, four / two tiles each) */
-uint32_t attn_once_tiles_max(uint32_t hd) { return hd == 32u ? 64u : 32u; }
+/* most 16-key tiles a 16-row tile may span at head width hd (sixteen waves, four tiles each) */
+uint32_t attn_once_tiles_max(uint32_t) { return 64u; }
 
 /* 16-key tiles the longest 16-row tile of the problem spans */
 uint32_t attn_once_span_tiles(const AttnProb &d) {

@@ -1423,6 +1423,41 @@ def test_attention_over_rows_far_apart(dev):
     assert_close(out.cpu().numpy(), (torch.softmax(s, -1) @ v).numpy(), "rows far apart")
 
 
+@pytest.mark.parametrize("nq,nk,masked,weighed,kernel", [(513, 513, True, True, "attn_once"), (17, 1024, True, False, "attn_once"),
+                                                         (1000, 1001, False, True, "attn_once"), (33, 1024, False, False, "attn_once"),
+                                                         (40, 689, False, False, "attn_once"), (40, 688, False, False, "attn_mfma"),
+                                                         (16, 1025, True, True, "attn_mfma")])
+def test_wide_heads_over_many_keys(nq, nk, masked, weighed, kernel, dev):
+    """Heads of 64 over more keys than a wave's registers hold at once, with a dense mask that closes rows and whole tiles, with
+    weights, with neither (from 689 keys on), against the sums in 64 bits."""
+    import torch
+    lib = api.load()
+    rs = np.random.RandomState(nq + nk)
+    q, k, v = (rs.randn(n, 64).astype(np.float32) for n in (nq, nk, nk))
+    mask = np.where(rs.rand(nq, nk) < 0.3, -np.inf, rs.randn(nq, nk)).astype(np.float32)
+    mask[:, 32:90], mask[:, 300:333], mask[nq - 1] = -np.inf, -np.inf, -np.inf
+    x = q.astype(np.float64) @ k.T.astype(np.float64) / 8.0 + (mask if masked else 0.0)
+    if masked:
+        x[nq - 1] = 0.0
+    w = np.exp(x - x.max(axis=1, keepdims=True))
+    w /= w.sum(axis=1, keepdims=True)
+    if masked:
+        w[nq - 1] = 0.0
+    dq, dk, dv, dm = (torch.from_numpy(t).cuda() for t in (q, k, v, mask))
+    out, weights = torch.full((nq, 64), 7.0, device="cuda"), torch.full((nq, nk), 7.0, device="cuda")
+    a = api.head_args(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), out.data_ptr(), nq, nk, 64, 0.125, 64, 64, 64, 64, 0)
+    a.mask, a.weights_out = (dm.data_ptr() if masked else None), (weights.data_ptr() if weighed else None)
+    torch.cuda.synchronize()
+    lib.blt_hip_profile_begin()
+    lib.blt_attention_batch_hip(api.problem_array([api.problem(a)]), 1)
+    names = set(api.profile_end())
+    lib.blt_backend_pass_sync_hip()
+    assert kernel in names, names
+    assert_close(out.cpu().numpy(), (w @ v).astype(np.float32), "output")
+    if weighed:
+        assert_close(weights.cpu().numpy(), w.astype(np.float32), "weights")
+
+
 @pytest.mark.parametrize("lens,H,hd,window,gap,kernel,staged", [
     ([100, 61, 7, 1, 130], 3, 32, 0, 0, "attn_once", False), ([17, 200], 2, 64, 50, 0, "attn_once", False),
     ([300, 211, 170], 8, 64, 0, 0, "attn_mfma", False), ([250, 131, 380], 8, 32, 0, 0, "attn_mfma", False),
