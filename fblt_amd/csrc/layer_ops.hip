@@ -697,6 +697,10 @@ void refresh_cross_seq(blt_kv_cache *cache, size_t seq, const blt_tensor *patch_
                 matmul_f32_launch(g, 0);
             }
         }
+        if (count <= 32) { /* a launch each */
+            matmul_f32_launch(g, 0);
+            continue;
+        }
         waiting = g, waits = !waits;
     }
     if (waits) matmul_f32_launch(waiting, 0);
