@@ -10,10 +10,9 @@
  *   per layer: h = transformer_block(h); where the cross block fires,
  *              P = P + cross_attention(RMSNorm(P), h)
  *
- * Hashing is integer work on the host, as in the reference; everything that
- * touches floats runs on the device.  The three small kernels keep the
- * reference's order of additions, so they are bit-identical to the CPU ops:
- * the embedding sum adds the tables in their order and scales last, the mean
+ * Hashing runs on the device too, in the launch that embeds and pools.  The small
+ * kernels keep the reference's order of additions, so they are bit-identical to the
+ * CPU ops: the embedding sum adds the tables in their order and scales last, the mean
  * pool adds a patch's rows first to last and multiplies by 1 / len.
  */
 #include "blt_hip.h"
@@ -449,7 +448,7 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
     /* A layer's cross block takes nothing from the next layer and gives nothing to it: but for the last one it goes along with that
      * layer's launches.  512 bytes through an encoder and a decoder of two layers of 128 columns with four patch layers between them, us: with
      * the decoder's keys in pairs 240 -> 230, three layers each 256 -> 239. */
-    CrossPass cross_pass; /* in the arena, like everything else of the pass (a launch of its own per layer before: 2 … 4 us) */
+    CrossPass cross_pass;
     CrossLater later;
     size_t last_cross = cfg.num_layers; /* none */
     for (size_t l = 0; l < cfg.num_layers; l++)
