@@ -293,11 +293,16 @@ __global__ __launch_bounds__(64 * W) void attn_once_kernel(const AttnProb *__res
             else request_values(0), request_values(1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < FLIGHT; u++)
-                if (on[u0 + u])
+            for (int u = 0; u < FLIGHT; u++) { /* two chains each, as above: half the roundings behind each other */
+                if (!on[u0 + u]) continue;
+                floatx4 odd = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int s = 0; s < QD; s++)
-                        sa[u0 + u][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][s], qf[s], sa[u0 + u][0], 0, 0, 0);
+                for (int s = 0; s < QD; s += 2) {
+                    sa[u0 + u][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][s], qf[s], sa[u0 + u][0], 0, 0, 0);
+                    odd = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][s + 1], qf[s + 1], odd, 0, 0, 0);
+                }
+                sa[u0 + u][0] += odd;
+            }
         }
 #pragma unroll
         for (int u = 2; u < T; u++) request_values(u);
