@@ -64,7 +64,7 @@ constexpr int TM = 64, TN = 64; /* smallest workgroup tile of the mfma kernel */
  * f16 first, if K is long enough; a workgroup that meets operands out of its range, before the first product as a rule, or
  * finds its results too small for it (half_lost()) starts again as bf16.  Half the matrix instructions, four fifths of the vector ones, half the error (K = 2048: 2.2e-7
  * against 4.9e-7), and a clock that gives way less (8192 x 2048 . 2048 x 1536, random operands against ones: 268 and 210 us
- * as bf16, 196 and 160 as f16).  Bound: in a step of the large tile the matrix unit takes 770 cycles of a SIMD, the vector
+ * as bf16, 196 and 160 as f16, 189 random ones as the loop is now).  Bound: in a step of the large tile the matrix unit takes 770 cycles of a SIMD, the vector
  * unit about 720, which add up, the LDS 770 beside them, of 2000 in all; the rest is the barrier.
  * VEC: a 16-byte aligned with lda and K multiples of 4.  ROPE: rotate pairs of the first g.rope_cols columns in
  * the epilogue.
@@ -87,7 +87,8 @@ struct MfmaShape {
     };
     static constexpr size_t LDS_BYTES = 2 * sizeof(Tiles);
 };
-/* most columns of b whose rows of a step 32-bit byte offsets reach, whatever the form */
+/* most columns of b that the tiles take: what 32-bit byte offsets over a step's rows reach, whatever the form.  A column's own
+ * offset is all that has 32 bits now; the lines stay where they have been tested. */
 template <int WT>
 constexpr uint32_t widest_b() {
     constexpr int steps[] = {MfmaShape<WT, false, false>::STEP, MfmaShape<WT, false, true>::STEP, MfmaShape<WT, true, false>::STEP,
@@ -216,18 +217,30 @@ __device__ __forceinline__ bool mfma_sums(const MatmulArgs &g, unsigned char *ld
     const uint32_t b_col = tid % BT, b_k = (tid / BT) * EPT;
     const float *const arow = g.a + (size_t)min(row0 + a_row, g.m - 1u) * g.lda;
     /* b or b2: one of them per wave, for the small tile per half of a wave */
-    const float *const bmat = GATED && (WT == 2 ? (wave & 1u) != 0u : b_col >= COLS) ? g.b2 : g.b;
+    const bool gates = GATED && (WT == 2 ? (wave & 1u) != 0u : b_col >= COLS);
     const uint32_t b_at = min(col0 + b_col % COLS, g.n - 1u);
-    uint32_t b_off[EPT]; /* bytes within a step's rows of b */
-#pragma unroll
-    for (int i = 0; i < EPT; i++) b_off[i] = 4u * ((b_k + i) * g.ldb + b_at);
+    /* A wave takes whole rows of b: a row's address is the wave's, and the lane adds its column, one register for all of them.
+     * (Not where the lanes of a wave take from both matrices.) */
+    constexpr bool ONE = !GATED || WT == 2;
+    const float *const bmat = gates ? g.b2 : g.b;
+    const uint32_t b_first = ONE ? wave * 64u / BT * EPT : b_k;
     struct Values {
         float a[EPT], b[EPT], w[NORM ? EPT : 1];
     };
     auto request = [&](Values &v, uint32_t k0) __attribute__((always_inline)) {
-        const char *base = reinterpret_cast<const char *>(bmat + (size_t)k0 * g.ldb);
+        const float *b_row = bmat + (size_t)(k0 + b_first) * g.ldb;
+        uint32_t column = 4u * b_at;
+        asm volatile("" : "+v"(column)); /* row and column kept apart: joined they are a 64-bit sum of the lane for each row */
 #pragma unroll
-        for (int i = 0; i < EPT; i++) v.b[i] = *reinterpret_cast<const float *>(base + b_off[i]);
+        for (int i = 0; i < EPT; i++, b_row += g.ldb) {
+            if constexpr (ONE) {
+                auto row = (const __attribute__((address_space(1))) char *)b_row;
+                asm("" : "+s"(row));
+                v.b[i] = *(const __attribute__((address_space(1))) float *)(row + column);
+            } else {
+                v.b[i] = b_row[b_at];
+            }
+        }
 #pragma unroll
         for (int i = 0; i < EPT; i += 4) {
             if (VEC) {
@@ -318,9 +331,12 @@ __device__ __forceinline__ bool mfma_sums(const MatmulArgs &g, unsigned char *ld
         Values v0, v1;
         auto of_step = [&](uint32_t s) { return min(s, steps - 1u) * TK; };
         request(v0, 0);
+        __builtin_amdgcn_sched_barrier(0);
         request(v1, of_step(1u));
+        __builtin_amdgcn_sched_barrier(0);
         park(v0, 0, true);
         request(v0, of_step(2u));
+        __builtin_amdgcn_sched_barrier(0);
         if (F16) { /* an operand that is out of range is so everywhere, as a rule */
             if (__syncthreads_or(!half_range(most_a, HALF_FIRST) || !half_range(most_b, HALF_FIRST))) return true;
         } else {
@@ -333,18 +349,26 @@ __device__ __forceinline__ bool mfma_sums(const MatmulArgs &g, unsigned char *ld
             multiply(f);
             park(v, (s & 1u) ^ 1u, s + 1u < steps);
             if (F16) __builtin_amdgcn_sched_group_barrier(0x100, 4 * WT * TK / 32, 0); /* fragments first */
+            /* behind each matrix instruction its share of the step's vector instructions (75 of the large tile as f16, 90 with the
+             * norm): eight each, and the last ones had none beside them (8192 x 2048 . 2048 x 1536 193.1 -> 188.9 us) */
+            constexpr int SHARE = !F16 ? (WT == 2 ? 4 : 8) : WT == 2 ? (NORM ? 7 : 6) : (NORM ? 16 : 12);
 #pragma unroll
-            for (int n = 0; n < (F16 ? 3 : 6) * WT * WT * TK / 32; n++) { /* a matrix instruction, its time in vector instructions */
+            for (int n = 0; n < (F16 ? 3 : 6) * WT * WT * TK / 32; n++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, (F16 ? 2 : 1) * (WT == 2 ? 4 : 8), 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, SHARE, 0);
             }
             request(v, of_step(s + 3u));
             __syncthreads();
         };
-        for (uint32_t s = 0; s < steps; s += 2u) {
+        /* In pairs, an odd step behind the loop: with a branch around the second one the compiler made the first wait for all that was
+         * on its way, the values of the step after it included, and requests out of order before the loop do the same (2048 rows of a
+         * layer of 512 columns 121.4 -> 117.2 us with this and whole rows of b (above), 1500 119.4 -> 113.1, 640 95.5 -> 85.3). */
+        uint32_t s = 0;
+        for (; s + 1u < steps; s += 2u) {
             step(s, v1);
-            if (s + 1u < steps) step(s + 1u, v0);
+            step(s + 1u, v0);
         }
+        if (s < steps) step(s, v1);
     }
     if (g.k % TK != 0u) { /* what is left of K, zeros behind it */
         const uint32_t k0 = steps * TK;
@@ -934,7 +958,7 @@ Path choose_path(const MatmulArgs &g) {
      * 128 ... 132 tiles of K = 256 ... 1024 a tenth slower; pairs of 72 tiles of K = 128 faster, of 80 and 128
      * tiles of K = 256 and 512 slower (block of 200 rows of 512: 54.8 -> 49.7 us on the tile kernel). */
     const uint64_t splitk_below = g.b2 ? 80u : 112u;
-    /* the tile kernel reaches the rows of b of a step by 32-bit byte offsets, this one computes addresses in 64 bits */
+    /* the tile kernel reaches a column of b by a 32-bit byte offset, this one computes addresses in 64 bits */
     if (g.ldb > widest_b<2>()) return PATH_SPLITK;
     /* one or two products an element: three parts drop the bits that fp32 rounds them to (error against float64 3.5e-8
      * and 3.4e-8, on the fp32 instructions 2.5e-8 and 3.1e-8; from three on the parts are closer, 3.3e-8 against 3.6e-8) */

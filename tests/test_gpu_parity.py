@@ -1096,6 +1096,24 @@ def _dev_tensor(t, shape=None):
     return abi.tensor_view(t.data_ptr(), tuple(t.shape) if shape is None else shape, abi.BLT_BACKEND_HIP)
 
 
+@pytest.mark.parametrize("m,n", [(2048, 1536), (2049, 1537), (1024, 512), (1030, 515)])
+@pytest.mark.parametrize("k", [20, 32, 64, 70, 96, 128, 160, 186, 384, 448, 455, 512])
+def test_matmul_whole_steps(m, n, k):
+    """The tile kernels' loop takes whole steps of K (32 or 64) in pairs: none, one, odd and even counts, with and without a rest,
+    on both tiles and both forms of the operands.  Against float64: a sum of k fp32 products is within k 2^-24 of the
+    sum of their magnitudes whatever its order, and rounding to fp32 adds less."""
+    import torch
+    lib = api.load()
+    rs = np.random.RandomState(m + 3 * n + 7 * k)
+    a, b = rs.randn(m, k).astype(np.float32), (rs.randn(k, n) / np.sqrt(k)).astype(np.float32)
+    ta, tb, to = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda(), torch.full((m, n), 7.0, device="cuda")
+    va, vb, vo = _dev_tensor(ta), _dev_tensor(tb), _dev_tensor(to)
+    lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    off = np.abs(to.cpu().numpy() - a @ b)
+    assert (off <= (k + 1) * 2.0 ** -24 * (np.abs(a) @ np.abs(b))).all()
+
+
 @pytest.mark.parametrize("m,k,n,exact", [(1, 128, 384, True), (5, 33, 17, True), (32, 512, 512, True),
                                           (3, 1100, 70, True), (1, 7, 300, True), (9, 528, 257, True),
                                           (16, 128, 512, True), (33, 64, 64, False), (64, 128, 384, False),
