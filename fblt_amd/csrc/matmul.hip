@@ -458,6 +458,38 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
 
     const bool gate_wave = GATED && wc == 1u;
     const uint32_t wave_col = col0 + (GATED ? 0u : wc * SIDE), my_row = SIDE * wr + 32u * mine + c;
+    MatmulArgs to = g;
+    const bool joined = GATED && g.out2 == nullptr; /* four waves a pair of quadrants then, two a quadrant else */
+    if (gate_wave && !joined) to.out = g.out2, to.residual = nullptr;
+    const bool vst = VEC && g.n % 4u == 0u && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(to.out) & 15u) == 0u) &&
+                     ((reinterpret_cast<uintptr_t>(to.residual) & 15u) == 0u);
+    constexpr uint32_t PER = SIDE / 4u, ROWS = 64u / PER; /* lanes a row, rows at once */
+    const uint32_t share = joined ? SIDE / 4u : SIDE / 2u, first = (joined ? 2u * wc + kg : kg) * share;
+    const float *const from = area(joined ? 2u * wr : wave & 3u), *const gates = area(2u * wr + 1u);
+
+    /* What the end needs from memory, the rotation or the residual of this thread's pieces, asked for while the waves of a quadrant meet:
+     * asked for where it is used, piece after piece, each waits behind the store
+     * and the branch of the one before (2048 rows of a layer of 512 columns 116.3 -> 113.6 us, 1500 113.0 -> 110.5, 301 62.5 -> 61.6). */
+    constexpr int PIECES = SIDE / 2u / ROWS;
+    float4 extra[PIECES]; /* cosines and sines, or the residual */
+    const bool rotates = ROPE && !g.stage_k && wave_col < g.rope_cols;
+    const bool prompt = !GATED && vst && (ROPE ? rotates && !to.residual : to.residual != nullptr);
+    auto ask = [&]() __attribute__((always_inline)) {
+        if (!prompt) return;
+        const uint32_t col = lane % PER * 4u;
+#pragma unroll
+        for (int i = 0; i < PIECES; i++) { /* past the end: the last row or column again */
+            const uint32_t row = min(row0 + SIDE * wr + first + min(ROWS * i, share - 1u) + lane / PER, g.m - 1u);
+            if constexpr (ROPE) {
+                const size_t at = (size_t)row * (g.head_dim / 2u) + ((wave_col + col) % g.head_dim) / 2u;
+                const float2 c2 = *reinterpret_cast<const float2 *>(g.rope_cos + at), s2 = *reinterpret_cast<const float2 *>(g.rope_sin + at);
+                extra[i] = make_float4(c2.x, c2.y, s2.x, s2.y);
+            } else {
+                extra[i] = *reinterpret_cast<const float4 *>(to.residual + (size_t)row * g.ldo + min(wave_col + col, g.n - 4u));
+            }
+        }
+    };
+
     /* the finished rows, back to the area */
     auto put = [&]() __attribute__((always_inline)) {
         const float scale = NORM ? 1.0f / sqrtf(row_ss[my_row] / (float)g.k + 1e-6f) : 1.0f; /* reductions_cpu.c:345-346 */
@@ -480,6 +512,7 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
         half = !mfma_sums<VEC, WT, NORM, GATED, true>(g, mm_lds, acc, ss, most_a, most_b);
         if (half) {
             tops.note(most_a, most_b);
+            ask();
             meet(acc, ss);
             bool lost = false;
             if (finishes) {
@@ -503,6 +536,7 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
         floatx16 acc[WT][WT];
         float ss, none;
         mfma_sums<VEC, WT, NORM, GATED, false>(g, mm_lds, acc, ss, none, none);
+        ask();
         meet(acc, ss);
         if (finishes) {
             bool bad = false;
@@ -542,14 +576,6 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
         __syncthreads();
     }
 
-    MatmulArgs to = g;
-    const bool joined = GATED && g.out2 == nullptr; /* four waves a pair of quadrants then, two a quadrant else */
-    if (gate_wave && !joined) to.out = g.out2, to.residual = nullptr;
-    const bool vst = VEC && g.n % 4u == 0u && (g.ldo % 4u == 0u) && ((reinterpret_cast<uintptr_t>(to.out) & 15u) == 0u) &&
-                     ((reinterpret_cast<uintptr_t>(to.residual) & 15u) == 0u);
-    constexpr uint32_t PER = SIDE / 4u, ROWS = 64u / PER; /* lanes a row, rows at once */
-    const uint32_t share = joined ? SIDE / 4u : SIDE / 2u, first = (joined ? 2u * wc + kg : kg) * share;
-    const float *const from = area(joined ? 2u * wr : wave & 3u), *const gates = area(2u * wr + 1u);
 #pragma unroll
     for (uint32_t r = 0; r < SIDE / 2u; r += ROWS) {
         if (r >= share) break;
@@ -560,7 +586,18 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
             const float4 gate = *reinterpret_cast<const float4 *>(gates + at * PITCH + col);
             v.x = silu_times(gate.x, v.x), v.y = silu_times(gate.y, v.y), v.z = silu_times(gate.z, v.z), v.w = silu_times(gate.w, v.w);
         }
-        if (row < g.m) matmul_store4<ROPE>(to, row, wave_col + col, v, vst);
+        if (row >= g.m) continue;
+        if (!prompt) {
+            matmul_store4<ROPE>(to, row, wave_col + col, v, vst);
+            continue;
+        }
+        const float4 e = extra[r / ROWS];
+        if constexpr (ROPE) {
+            if (wave_col + col < g.rope_cols) v = rope_rotate4(v, make_float2(e.x, e.y), make_float2(e.z, e.w));
+        } else {
+            v.x = e.x + v.x, v.y = e.y + v.y, v.z = e.z + v.z, v.w = e.w + v.w;
+        }
+        if (wave_col + col < g.n) *reinterpret_cast<float4 *>(to.out + (size_t)row * g.ldo + wave_col + col) = v;
     }
 }
 

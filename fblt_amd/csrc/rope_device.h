@@ -11,16 +11,17 @@
 
 #include <hip/hip_runtime.h>
 
-__device__ __forceinline__ float4 rope_rotate4(float4 x, const float *cs, const float *sn) {
+__device__ __forceinline__ float4 rope_rotate4(float4 x, float2 c, float2 s) {
 #pragma clang fp contract(off) /* no fused multiply-add in this block, also after inlining */
-    const float2 c = *reinterpret_cast<const float2 *>(cs);
-    const float2 s = *reinterpret_cast<const float2 *>(sn);
     float4 r;
     r.x = x.x * c.x - x.y * s.x;
     r.y = x.y * c.x + x.x * s.x;
     r.z = x.z * c.y - x.w * s.y;
     r.w = x.w * c.y + x.z * s.y;
     return r;
+}
+__device__ __forceinline__ float4 rope_rotate4(float4 x, const float *cs, const float *sn) {
+    return rope_rotate4(x, *reinterpret_cast<const float2 *>(cs), *reinterpret_cast<const float2 *>(sn));
 }
 
 /* one pair */
