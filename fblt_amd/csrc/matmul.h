@@ -61,8 +61,8 @@ struct MatmulArgs {
      * step takes 72 us instead of 112). */
     uint32_t tolerant;
     /* Set by the launcher, never by callers.  slices > 1: the K range is also split over slices
-     * workgroups per output tile (grid z); each leaves its 32x32 sums in slice_sums
-     * [tile][slice][1024] and the one that draws the last of the tile's tickets adds them in slice
+     * workgroups per output tile (grid z); each leaves its tile's sums in slice_sums
+     * [tile][slice][1024, or 4096 of the 64x64 tile] and the one that draws the last of the tile's tickets adds them in slice
      * order and runs the epilogue. */
     uint32_t slices;
     float *slice_sums;

@@ -398,8 +398,19 @@ __device__ __forceinline__ bool mfma_sums(const MatmulArgs &g, unsigned char *ld
     return false;
 }
 
-template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED>
+/* of K, for each of `slices`: whole steps of either form */
+__host__ __device__ __forceinline__ uint32_t tile_slice(uint32_t k, uint32_t slices) { return ((k + slices - 1u) / slices + 63u) / 64u * 64u; }
+
+/* SLICED (small tile): gridDim.z workgroups a tile, each with its run of K as a product of its own; the one that comes last adds
+ * up what all of them left, in their order. */
+template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED, bool SLICED = false>
 __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(MatmulArgs g) {
+    static_assert(!SLICED || (WT == 1 && !ROPE && !NORM && !GATED), "plain products");
+    if constexpr (SLICED) {
+        const uint32_t per = tile_slice(g.k, g.slices), k0 = blockIdx.z * per;
+        g.a += k0, g.b += (size_t)k0 * g.ldb;
+        g.k = min(per, g.k - k0); /* the launcher leaves no slice empty */
+    }
     constexpr int BT = MfmaShape<WT, NORM, true>::BT;
     extern __shared__ __attribute__((aligned(16))) unsigned char mm_lds[];
     __shared__ float row_ss[NORM ? BT : 1];
@@ -576,12 +587,57 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
         __syncthreads();
     }
 
+    float4 total[SLICED ? PIECES : 1];
+    if constexpr (SLICED) {
+        /* device-scope stores and loads, and an explicit wait for the stores' completion before the barrier that precedes this
+         * workgroup's ticket, as for the split states of the KV step (kv_step.h) */
+        __shared__ uint32_t ticket;
+        constexpr uint32_t WORDS = BT * BT / 2; /* a slice's sums, two a word */
+        const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
+        uint64_t *const words = reinterpret_cast<uint64_t *>(g.slice_sums) + (size_t)tile * g.slices * WORDS + tid;
+        uint64_t *const own = words + (size_t)blockIdx.z * WORDS;
+#pragma unroll
+        for (int i = 0; i < PIECES; i++) {
+            const float4 v = *reinterpret_cast<const float4 *>(from + (first + ROWS * i + lane / PER) * PITCH + lane % PER * 4u);
+            __hip_atomic_store(own + (2 * i) * 512, (uint64_t)__float_as_uint(v.y) << 32 | __float_as_uint(v.x), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(own + (2 * i + 1) * 512, (uint64_t)__float_as_uint(v.w) << 32 | __float_as_uint(v.z), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        blt_vector_memory_done(); /* every wave's sums are out before thread 0 draws the ticket */
+        __syncthreads();
+        if (tid == 0u) ticket = __hip_atomic_fetch_add(&g.slice_tickets[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (ticket != g.slices - 1u) return;
+        if (tid == 0u) g.slice_tickets[tile] = 0u; /* re-armed for the next launch */
+        static_assert(4 * PIECES * 512 == BT * BT, "a thread's pieces are all of a slice's sums");
+#pragma unroll
+        for (int i = 0; i < PIECES; i++) total[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (uint32_t z = 0; z < g.slices; z += 2u) { /* slice order, whoever comes last; two on their way */
+            uint64_t t[2][2 * PIECES];
+#pragma unroll
+            for (uint32_t u = 0; u < 2u; u++)
+#pragma unroll
+                for (int i = 0; i < 2 * PIECES; i++)
+                    t[u][i] = __hip_atomic_load(words + (size_t)min(z + u, g.slices - 1u) * WORDS + i * 512, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (uint32_t u = 0; u < 2u; u++) {
+                if (z + u >= g.slices) break;
+#pragma unroll
+                for (int i = 0; i < PIECES; i++) {
+                    total[i].x += __uint_as_float((uint32_t)t[u][2 * i]), total[i].y += __uint_as_float((uint32_t)(t[u][2 * i] >> 32));
+                    total[i].z += __uint_as_float((uint32_t)t[u][2 * i + 1]), total[i].w += __uint_as_float((uint32_t)(t[u][2 * i + 1] >> 32));
+                }
+            }
+        }
+    }
 #pragma unroll
     for (uint32_t r = 0; r < SIDE / 2u; r += ROWS) {
         if (r >= share) break;
         const uint32_t at = first + r + lane / PER, col = lane % PER * 4u;
         const uint32_t row = row0 + SIDE * wr + at;
-        float4 v = *reinterpret_cast<const float4 *>(from + at * PITCH + col);
+        float4 v = SLICED ? total[SLICED ? r / ROWS : 0] : *reinterpret_cast<const float4 *>(from + at * PITCH + col);
         if (joined) {
             const float4 gate = *reinterpret_cast<const float4 *>(gates + at * PITCH + col);
             v.x = silu_times(gate.x, v.x), v.y = silu_times(gate.y, v.y), v.z = silu_times(gate.z, v.z), v.w = silu_times(gate.w, v.w);
@@ -1115,12 +1171,10 @@ void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStrea
 }
 
 namespace {
-template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED>
-void launch_mfma_as(const MatmulArgs &g, hipStream_t s) {
-    constexpr uint32_t BT = MfmaShape<WT, NORM, true>::BT, COLS = GATED ? BT / 2u : BT;
-    const dim3 grid((g.n + COLS - 1u) / COLS, (g.m + BT - 1u) / BT);
+template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED, bool SLICED = false>
+void launch_mfma_as(const MatmulArgs &g, dim3 grid, hipStream_t s) {
     constexpr size_t lds = MFMA_LDS_BYTES<WT, NORM>;
-    const auto kernel = matmul_mfma_kernel<VEC, ROPE, WT, NORM, GATED>;
+    const auto kernel = matmul_mfma_kernel<VEC, ROPE, WT, NORM, GATED, SLICED>;
     if constexpr (lds > 64u * 1024u - 512u) { /* from 64 KB on a kernel has to ask for its LDS first */
         static const hipError_t asked =
             hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1128,17 +1182,48 @@ void launch_mfma_as(const MatmulArgs &g, hipStream_t s) {
     }
     blt_launch("matmul_mfma", kernel, grid, dim3(512), lds, s, g);
 }
+/* Slices of K per 64x64 tile; 1: not taken for it.  Up to 128 tiles with a long K leave half of the chip empty, and the 32x32 tiles
+ * that fewer than 112 of them were given do their products on the fp32 instructions.  As many slices as keep to one workgroup a
+ * compute unit (two on one take turns with its LDS and vector units: 192 tiles of K = 2048 24.5 us, as 384 27.0; 256 28.8 and 30.4),
+ * of at least HALF_K each.  From 80 tiles of K = 1024 on, 40 of 2048, 20 of 4096: 32x32 tiles against this, us, 301 rows, K = 2048, 512
+ * columns 17.1 / 12.4, 640 31.4 / 15.3, 640 of K = 1024 16.8 / 11.3, 300 of 4096 to 256 15.5 / 13.7, but 200 of 2048 11.4 /
+ * 12.0, 400 of 1024 9.8 / 11.2; the 64x64 tile as it was against this, 1000 of 2048 23.7 / 18.8, 900 of 1024 14.0 / 12.3.  Error
+ * against float64 1.4e-7 for 2.2e-7 of the whole tile and 2.9e-7 of the 32x32 ones (K = 2048). */
+uint32_t tile_slices(const MatmulArgs &g, bool rope) {
+    if (g.b2 || rope || g.norm_w || g.cross_k || g.k < 1024u || g.m <= (uint32_t)TM || g.ldb > widest_b<1>()) return 1u;
+    const uint64_t tiles = (uint64_t)((g.n + TN - 1u) / TN) * ((g.m + TM - 1u) / TM);
+    if (tiles < 16u || tiles > 128u || tiles * g.k < 80u * 1024u) return 1u; /* 16: the last workgroup adds its slices one after the other */
+    for (uint32_t n = std::min(256u / (uint32_t)tiles, g.k / HALF_K[0]); n >= 2u; n--) {
+        const uint32_t before = (n - 1u) * tile_slice(g.k, n);
+        if (before < g.k && g.k - before >= HALF_K[0]) return n; /* the last one is not empty, nor bf16 for being short */
+    }
+    return 1u;
+}
+/* false: not taken, or no room for the sums while a graph capture is open */
+template <bool VEC>
+bool launch_sliced(const MatmulArgs &g_in, bool rope, hipStream_t s) {
+    MatmulArgs g = g_in;
+    g.slices = tile_slices(g, rope);
+    const dim3 grid((g.n + TN - 1u) / TN, (g.m + TM - 1u) / TM, g.slices);
+    const size_t tiles = (size_t)grid.x * grid.y;
+    if (g.slices < 2u || !matmul_slice_scratch(tiles * g.slices * (TM * TN), tiles, s, &g.slice_sums, &g.slice_tickets)) return false;
+    launch_mfma_as<VEC, false, 1, false, false, true>(g, grid, s);
+    return true;
+}
 template <bool VEC, int WT>
 void launch_mfma(const MatmulArgs &g, bool rope, hipStream_t s) {
+    constexpr uint32_t BT = MfmaShape<WT, false, true>::BT;
+    const uint32_t cols = g.b2 ? BT / 2u : BT;
+    const dim3 grid((g.n + cols - 1u) / cols, (g.m + BT - 1u) / BT);
     if (g.b2) {
-        if (g.norm_w) launch_mfma_as<VEC, false, WT, true, true>(g, s);
-        else launch_mfma_as<VEC, false, WT, false, true>(g, s);
+        if (g.norm_w) launch_mfma_as<VEC, false, WT, true, true>(g, grid, s);
+        else launch_mfma_as<VEC, false, WT, false, true>(g, grid, s);
     } else if (rope) {
-        if (g.norm_w) launch_mfma_as<VEC, true, WT, true, false>(g, s);
-        else launch_mfma_as<VEC, true, WT, false, false>(g, s);
+        if (g.norm_w) launch_mfma_as<VEC, true, WT, true, false>(g, grid, s);
+        else launch_mfma_as<VEC, true, WT, false, false>(g, grid, s);
     } else {
-        if (g.norm_w) launch_mfma_as<VEC, false, WT, true, false>(g, s);
-        else launch_mfma_as<VEC, false, WT, false, false>(g, s);
+        if (g.norm_w) launch_mfma_as<VEC, false, WT, true, false>(g, grid, s);
+        else launch_mfma_as<VEC, false, WT, false, false>(g, grid, s);
     }
 }
 } // namespace
@@ -1165,6 +1250,7 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
                         aligned16(g.cross_out),
                     "matmul: the cross-attention epilogue is not available for this shape");
     }
+    if (vec ? launch_sliced<true>(g, rope, s) : launch_sliced<false>(g, rope, s)) return;
     if (path == PATH_SPLITK) {
         const dim3 sgrid((g.n + 31u) / 32u, (g.m + 31u) / 32u);
         if (rope) {

@@ -1114,6 +1114,33 @@ def test_matmul_whole_steps(m, n, k):
     assert (off <= (k + 1) * 2.0 ** -24 * (np.abs(a) @ np.abs(b))).all()
 
 
+@pytest.mark.parametrize("m,n", [(65, 1025), (301, 512), (641, 449), (1000, 512), (1024, 515)])
+@pytest.mark.parametrize("k", [1023, 1024, 1025, 1530, 2048, 2049, 2500, 5200])
+def test_matmul_tiles_in_slices(m, n, k):
+    """16 to 128 tiles of 64 x 64 and a long K: up to sixteen workgroups a tile, each with its run of K, odd rests among them; the bound
+    of test_matmul_whole_steps (one more rounding a slice).  The same bits whoever comes last, and an infinity in one slice is
+    one in the result."""
+    import torch
+    lib = api.load()
+    rs = np.random.RandomState(m + 3 * n + 7 * k)
+    a, b = rs.randn(m, k).astype(np.float32), (rs.randn(k, n) / np.sqrt(k)).astype(np.float32)
+    ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    outs = [torch.full((m, n), 7.0, device="cuda") for _ in range(3)]
+    va, vb = _dev_tensor(ta), _dev_tensor(tb)
+    for out in outs:
+        vo = _dev_tensor(out)
+        lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    got = [out.cpu().numpy() for out in outs]
+    assert got[0].tobytes() == got[1].tobytes() == got[2].tobytes()
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert (np.abs(got[0] - a @ b) <= (k + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(b))).all()
+    ta[5, k - 3] = float("inf")
+    lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    row = outs[2].cpu().numpy()
+    assert (row[5] == np.where(tb[k - 3].cpu().numpy() > 0, np.inf, -np.inf)).all()
+    assert np.isfinite(np.delete(row, 5, 0)).all()
+
+
 @pytest.mark.parametrize("m,k,n,exact", [(1, 128, 384, True), (5, 33, 17, True), (32, 512, 512, True),
                                           (3, 1100, 70, True), (1, 7, 300, True), (9, 528, 257, True),
                                           (16, 128, 512, True), (33, 64, 64, False), (64, 128, 384, False),
