@@ -1251,7 +1251,15 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
                     "matmul: the cross-attention epilogue is not available for this shape");
     }
     if (vec ? launch_sliced<true>(g, rope, s) : launch_sliced<false>(g, rope, s)) return;
-    if (path == PATH_SPLITK) {
+    /* More than 256 of the 32x32 tiles, of eight waves each, share compute units; from HALF_K on, where the 64x64 ones are f16, those are
+     * the better ones then (32x32 / 64x64, us, K = 512: 240 tiles 6.4 / 9.0, 256 6.4 / 9.1, 288 10.2 / 9.1, 416 10.4 / 9.2; K = 768
+     * 256 8.1 / 11.4, 312 13.6 / 11.4; K = 384 320 8.5 / 8.05; but bf16, K = 256 384 6.4 / 7.0) and closer (1.35e-7 for 1.52e-7).
+     * One to three rows or columns past a block of 32 are bf16 in any case (641 rows 10.2 / 10.5; 17.4 / 11.0 where 16-byte loads do
+     * not go). */
+    const uint64_t quarters = (uint64_t)((g.n + 31u) / 32u) * ((g.m + 31u) / 32u);
+    const bool edge = vec && (g.m % 32u - 1u < 3u || g.n % 32u - 1u < 3u);
+    const bool halves = quarters > 256u && g.k >= HALF_K[0] && g.m > (uint32_t)TM && !g.b2 && !g.cross_k && g.ldb <= widest_b<1>() && !edge;
+    if (path == PATH_SPLITK && !halves) {
         const dim3 sgrid((g.n + 31u) / 32u, (g.m + 31u) / 32u);
         if (rope) {
             if (vec) launch_splitk<true, true>(g, sgrid, s);

@@ -1096,7 +1096,7 @@ def _dev_tensor(t, shape=None):
     return abi.tensor_view(t.data_ptr(), tuple(t.shape) if shape is None else shape, abi.BLT_BACKEND_HIP)
 
 
-@pytest.mark.parametrize("m,n", [(2048, 1536), (2049, 1537), (1024, 512), (1030, 515)])
+@pytest.mark.parametrize("m,n", [(2048, 1536), (2049, 1537), (1024, 512), (1030, 515), (640, 512), (577, 450)])
 @pytest.mark.parametrize("k", [20, 32, 64, 70, 96, 128, 160, 186, 384, 448, 455, 512])
 def test_matmul_whole_steps(m, n, k):
     """The tile kernels' loop takes whole steps of K (32 or 64) in pairs: none, one, odd and even counts, with and without a rest,
@@ -1169,7 +1169,7 @@ def test_matmul(m, k, n, exact, oracle, dev):
         assert_close(got, ref, "matmul %dx%dx%d" % (m, k, n))
 
 
-@pytest.mark.parametrize("m,k,n", [(512, 256, 512), (513, 256, 512), (511, 300, 544), (33, 256, 4064), (200, 1000, 1150), (384, 512, 1020)])
+@pytest.mark.parametrize("m,k,n", [(512, 256, 512), (513, 256, 512), (511, 300, 544), (33, 256, 4064), (200, 1000, 1150), (384, 380, 1020)])
 def test_matmul_of_two_small_tiles_a_compute_unit(m, k, n, dev):
     """Products of 256 small tiles and of more, that share compute units, against float64."""
     import torch
