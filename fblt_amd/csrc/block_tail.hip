@@ -495,11 +495,6 @@ bool block_tail_launch(BlockTailArgs a, uint32_t embed_dim, hipStream_t s, Cross
     const bool many = a.hidden / 64u > (embed_dim == 256u ? 16u : 32u);
     const uint32_t most = embed_dim == 64u ? (many ? 640u : 1024u) : embed_dim == 128u ? (many ? 256u : 512u) : many ? 128u : 256u;
     if (workgroups > most) return false;
-    /* recorded by the caller's own capture, a replay may run beside later launches that use the same sums and tickets */
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const hipStream_t stream = s ? s : blt_stream();
-    if (!blt_stream_capturing() && stream != nullptr) HIP_CHECK(hipStreamIsCapturing(stream, &capture));
-    if (capture != hipStreamCaptureStatusNone) return false;
     const uint32_t slices = a.hidden / 64u, tiles = (a.rows + 15u) / 16u;
     if (slices > 1u && !matmul_slice_scratch((size_t)tiles * slices * 16u * embed_dim, tiles, s, (float **)&a.sums, &a.tickets))
         return false;

@@ -18,6 +18,10 @@ bool blt_profile_is_open();
  * graph capture is open on it (stream.hip). */
 hipStream_t blt_stream();
 bool blt_stream_capturing();
+/* Is the stream (0: the current one) captured by the caller, by other means than blt_hip_capture_begin?  Nothing is known of
+ * where and when such a recording replays: beside eager work of the stream it was recorded on, or beside itself.  Launches that
+ * hand over through memory of the library are not recorded there. */
+bool blt_stream_captured_by_caller(hipStream_t s = nullptr);
 /* The stream library-owned scratch is keyed by: the current stream, or, while a capture is open,
  * the stream the thread was on when it began (the one the graph will be replayed on). */
 hipStream_t blt_stream_key();

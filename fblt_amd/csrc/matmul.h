@@ -125,7 +125,8 @@ __device__ __forceinline__ float silu_times(float gate, float up) {
 }
 /* Room for `floats` partial sums and `count` zeroed tickets of one launch on the stream, per (thread, stream): launches on one
  * stream follow each other, launches on two never share them.  Every launch leaves its tickets at zero.  false: the
- * buffers would have to grow while a graph capture is open. */
+ * buffers would have to grow while a graph capture is open, or the capture is the caller's own: a replay may run beside later
+ * launches that use the same sums and tickets. */
 bool matmul_slice_scratch(size_t floats, size_t count, hipStream_t s, float **sums, uint32_t **tickets);
 /* What of a transformer block is behind its attention, in one launch (block_tail.hip): out = r + SwiGLU(RMSNorm(r)) * down
  * with r = x + comb * proj.  All row-major and dense; out may be x. */

@@ -1074,6 +1074,7 @@ __global__ void clear_words_kernel(uint32_t *w, size_t n) {
 } // namespace
 
 bool matmul_slice_scratch(size_t floats, size_t count, hipStream_t s, float **sums, uint32_t **tickets) {
+    if (blt_stream_captured_by_caller(s)) return false;
     static thread_local std::map<hipStream_t, SliceScratch> by_stream;
     SliceScratch &sc = by_stream[blt_stream_key()];
     if (blt_stream_capturing() && (floats > sc.sum_floats || count > sc.ticket_count)) return false;
@@ -1199,7 +1200,7 @@ uint32_t tile_slices(const MatmulArgs &g, bool rope) {
     }
     return 1u;
 }
-/* false: not taken, or no room for the sums while a graph capture is open */
+/* false: not taken, or no place for the sums in a capture */
 template <bool VEC>
 bool launch_sliced(const MatmulArgs &g_in, bool rope, hipStream_t s) {
     MatmulArgs g = g_in;

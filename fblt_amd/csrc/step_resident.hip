@@ -1482,9 +1482,7 @@ bool kv_step_resident(const StepResident &st) {
     const hipStream_t s = blt_stream();
     /* recorded by the caller's own capture of the stream, a replay would find the words of the launch before it under its
      * own tag */
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (s != nullptr) HIP_CHECK(hipStreamIsCapturing(s, &capture));
-    if (capture != hipStreamCaptureStatusNone) return false;
+    if (blt_stream_captured_by_caller(s)) return false;
     const ResidentKernel kernel = folds ? kernel_of<true>(E, hd, rt) : kernel_of<false>(E, hd, rt);
     const uint32_t groups = (uint32_t)((st.batch + per_group - 1) / per_group);
     if (!can_be_resident(kernel, groups * WORKERS, dev, s)) return false;

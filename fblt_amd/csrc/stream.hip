@@ -42,6 +42,13 @@ struct blt_hip_graph {
 hipStream_t blt_stream() { return t_stream; }
 hipStream_t blt_stream_key() { return t_capturing ? t_saved : t_stream; }
 bool blt_stream_capturing() { return t_capturing; }
+bool blt_stream_captured_by_caller(hipStream_t s) {
+    if (s == nullptr) s = t_stream;
+    if (t_capturing || s == nullptr) return false; /* the null stream cannot be captured */
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(s, &status));
+    return status != hipStreamCaptureStatusNone;
+}
 void blt_stream_note_device_length_step() {
     if (t_capturing) t_captured_device_length_step = true;
 }

@@ -2936,6 +2936,71 @@ def test_step_in_a_capture_of_the_callers_own(oracle, dev):
         w.close()
 
 
+class _KernelNode(C.Structure):
+    _fields_ = [("block", C.c_uint32 * 3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", C.c_uint32 * 3), ("params", C.c_void_p),
+                ("lds", C.c_uint32)]
+
+
+def _grids_of(graph):
+    """Grids of a recorded graph's kernels (hipKernelNodeParams), from the runtime that this process has loaded."""
+    with open("/proc/self/maps") as maps:
+        hip = C.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    raw, count = C.c_void_p(graph.raw_cuda_graph()), C.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, C.byref(count)) == 0
+    nodes, kind, grids = (C.c_void_p * count.value)(), C.c_int(), []
+    assert hip.hipGraphGetNodes(raw, nodes, C.byref(count)) == 0
+    for node in nodes:
+        assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+        assert kind.value == 0, kind.value          # a kernel
+        at = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(at)) == 0
+        grids.append(tuple(at.grid))
+    return grids
+
+
+@pytest.mark.parametrize("m,k,n", [(1000, 1024, 512), (960, 2100, 512), (118, 2048, 512), (64, 4096, 256)])
+@pytest.mark.parametrize("warm", [True, False])
+def test_long_products_in_a_capture_of_the_callers_own(m, k, n, warm, dev):
+    """Products whose K is split over workgroups hand their sums over in memory of the library, which a replay may use beside other
+    work: in a capture that the library does not see begin they are recorded whole, one workgroup a tile and nothing else,
+    whether or not the stream had that memory before.  Replays between eager products of other shapes give the same bits."""
+    import torch
+    lib = api.load()
+    torch.manual_seed(m + k)
+    a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda") / k ** 0.5
+    a2, b2 = torch.randn(700, 2048, device="cuda"), torch.randn(2048, 640, device="cuda") / 45.0
+    o, o2 = torch.zeros(m, n, device="cuda"), torch.zeros(700, 640, device="cuda")
+    va, vb, vo, va2, vb2, vo2 = (_dev_tensor(t) for t in (a, b, o, a2, b2, o2))
+    want, want2 = (a.double() @ b.double()).float().cpu().numpy(), (a2.double() @ b2.double()).float().cpu().numpy()
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
+    try:
+        lib.blt_hip_set_stream(stream.cuda_stream)
+        if warm:
+            lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+            lib.blt_backend_pass_sync_hip()
+            assert_close(o.cpu().numpy(), want, "eager product")
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+            lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+        grids = _grids_of(graph)
+        assert len(grids) == 1 and grids[0][2] == 1, grids
+        graph.instantiate()
+        seen = set()
+        for _ in range(3):
+            o.fill_(7.0)
+            o2.fill_(7.0)
+            torch.cuda.synchronize()
+            lib.blt_matmul(C.byref(va2), C.byref(vb2), C.byref(vo2))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_close(o.cpu().numpy(), want, "replayed product")
+            assert_close(o2.cpu().numpy(), want2, "eager product beside it")
+            seen.add(o.cpu().numpy().tobytes())
+        assert len(seen) == 1
+    finally:
+        lib.blt_hip_set_stream(None)
+
+
 def test_profile_holds_every_launch(dev):
     """Uploads that travel in kernel arguments and the small kernels beside the main path are in the kernel-time profile."""
     import torch
