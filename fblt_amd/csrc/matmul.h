@@ -67,6 +67,7 @@ struct MatmulArgs {
     uint32_t slices;
     float *slice_sums;
     uint32_t *slice_tickets;
+    uint32_t all_bits; /* the launcher's: 64x64 tiles in slices, on parts that hold every bit of the operands */
 };
 
 /* Four consecutive results of output row `row` starting at column `col`:

@@ -516,7 +516,7 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
      * or columns are by themselves at an edge, such a one would be all of a column, and some tile of nearly every launch start again
      * (200 x 512 . 512 x 2048 10.9 -> 18.9 us): bf16 from the start. */
     const auto few = [](uint32_t left, uint32_t whole, uint32_t block) { return left < whole && left % block - 1u < 3u; };
-    bool half = g.k >= HALF_K[WT - 1] && !few(g.m - row0, BT, 32u) && !few(g.n - col0, COLS, SIDE);
+    bool half = !(SLICED && g.all_bits != 0u) && g.k >= HALF_K[WT - 1] && !few(g.m - row0, BT, 32u) && !few(g.n - col0, COLS, SIDE);
     if (half) {
         floatx16 acc[WT][WT];
         float ss, most_a, most_b;
@@ -1183,18 +1183,23 @@ void launch_mfma_as(const MatmulArgs &g, dim3 grid, hipStream_t s) {
     }
     blt_launch("matmul_mfma", kernel, grid, dim3(512), lds, s, g);
 }
-/* Slices of K per 64x64 tile; 1: not taken for it.  Up to 128 tiles with a long K leave half of the chip empty, and the 32x32 tiles
- * that fewer than 112 of them were given do their products on the fp32 instructions.  As many slices as keep to one workgroup a
- * compute unit (two on one take turns with its LDS and vector units: 192 tiles of K = 2048 24.5 us, as 384 27.0; 256 28.8 and 30.4),
- * of at least HALF_K each.  From 80 tiles of K = 1024 on, 40 of 2048, 20 of 4096: 32x32 tiles against this, us, 301 rows, K = 2048, 512
- * columns 17.1 / 12.4, 640 31.4 / 15.3, 640 of K = 1024 16.8 / 11.3, 300 of 4096 to 256 15.5 / 13.7, but 200 of 2048 11.4 /
- * 12.0, 400 of 1024 9.8 / 11.2; the 64x64 tile as it was against this, 1000 of 2048 23.7 / 18.8, 900 of 1024 14.0 / 12.3.  Error
- * against float64 1.4e-7 for 2.2e-7 of the whole tile and 2.9e-7 of the 32x32 ones (K = 2048). */
-uint32_t tile_slices(const MatmulArgs &g, bool rope) {
+/* Slices of K per 64x64 tile; 1: not taken for it.  Up to 128 tiles with a long K leave half of the chip empty.  As many slices as
+ * keep to one workgroup a compute unit (two on one take turns with its LDS and vector units: 192 tiles of K = 2048 24.5 us, as
+ * 384 27.0; 256 28.8 and 30.4), of at least HALF_K each.  The 64x64 tile whole against this, 1000 rows of 2048 to 512 columns 23.7 /
+ * 18.8 us, 900 of 1024 14.0 / 12.3, error against float64 2.2e-7 / 1.4e-7 (K = 2048).
+ * Fewer than 112 tiles are products on the fp32 instructions otherwise, and hold every bit of their operands: so they do here, on
+ * bf16 parts (all_bits).  As f16 parts a result that comes from a row's smallest values only was as far off as those parts are, another
+ * of the row being large (values of 1e-9 beside ones near 1: 2.3e-5 of their products).  bf16 parts round six times for 16 terms, so only short slices are as close as the 32x32 tiles are, eight waves
+ * to a K: error, this / 32x32 tiles, in six slices 0.70 ... 0.72, five 0.76 ... 0.80, four 0.83 ... 0.88, three of K up to 2560
+ * 0.96 ... 1.00 but of 4096 1.01, two 1.2; none up to 128 of the 32x32 tiles, which take slices of their own.  us, 32x32 tiles / this, 301
+ * rows of 2048 to 512 columns 17.2 / 13.5, 420 18.0 / 14.3, 640 31.5 / 17.3, 420 of 1536 14.3 / 12.9, 301 of 4096 32.5 / 18.1. */
+uint32_t tile_slices(const MatmulArgs &g, bool rope, bool all_bits) {
     if (g.b2 || rope || g.norm_w || g.cross_k || g.k < 1024u || g.m <= (uint32_t)TM || g.ldb > widest_b<1>()) return 1u;
     const uint64_t tiles = (uint64_t)((g.n + TN - 1u) / TN) * ((g.m + TM - 1u) / TM);
     if (tiles < 16u || tiles > 128u || tiles * g.k < 80u * 1024u) return 1u; /* 16: the last workgroup adds its slices one after the other */
-    for (uint32_t n = std::min(256u / (uint32_t)tiles, g.k / HALF_K[0]); n >= 2u; n--) {
+    if (all_bits && (uint64_t)((g.n + 31u) / 32u) * ((g.m + 31u) / 32u) <= 128u) return 1u;
+    const uint32_t least = !all_bits ? 2u : g.k <= 2560u ? 3u : 4u;
+    for (uint32_t n = std::min(256u / (uint32_t)tiles, g.k / HALF_K[0]); n >= least; n--) {
         const uint32_t before = (n - 1u) * tile_slice(g.k, n);
         if (before < g.k && g.k - before >= HALF_K[0]) return n; /* the last one is not empty, nor bf16 for being short */
     }
@@ -1202,9 +1207,10 @@ uint32_t tile_slices(const MatmulArgs &g, bool rope) {
 }
 /* false: not taken, or no place for the sums in a capture */
 template <bool VEC>
-bool launch_sliced(const MatmulArgs &g_in, bool rope, hipStream_t s) {
+bool launch_sliced(const MatmulArgs &g_in, bool rope, bool all_bits, hipStream_t s) {
     MatmulArgs g = g_in;
-    g.slices = tile_slices(g, rope);
+    g.all_bits = all_bits;
+    g.slices = tile_slices(g, rope, all_bits);
     const dim3 grid((g.n + TN - 1u) / TN, (g.m + TM - 1u) / TM, g.slices);
     const size_t tiles = (size_t)grid.x * grid.y;
     if (g.slices < 2u || !matmul_slice_scratch(tiles * g.slices * (TM * TN), tiles, s, &g.slice_sums, &g.slice_tickets)) return false;
@@ -1251,16 +1257,9 @@ void matmul_f32_launch(const MatmulArgs &g, hipStream_t s) {
                         aligned16(g.cross_out),
                     "matmul: the cross-attention epilogue is not available for this shape");
     }
-    if (vec ? launch_sliced<true>(g, rope, s) : launch_sliced<false>(g, rope, s)) return;
-    /* More than 256 of the 32x32 tiles, of eight waves each, share compute units; from HALF_K on, where the 64x64 ones are f16, those are
-     * the better ones then (32x32 / 64x64, us, K = 512: 240 tiles 6.4 / 9.0, 256 6.4 / 9.1, 288 10.2 / 9.1, 416 10.4 / 9.2; K = 768
-     * 256 8.1 / 11.4, 312 13.6 / 11.4; K = 384 320 8.5 / 8.05; but bf16, K = 256 384 6.4 / 7.0) and closer (1.35e-7 for 1.52e-7).
-     * One to three rows or columns past a block of 32 are bf16 in any case (641 rows 10.2 / 10.5; 17.4 / 11.0 where 16-byte loads do
-     * not go). */
-    const uint64_t quarters = (uint64_t)((g.n + 31u) / 32u) * ((g.m + 31u) / 32u);
-    const bool edge = vec && (g.m % 32u - 1u < 3u || g.n % 32u - 1u < 3u);
-    const bool halves = quarters > 256u && g.k >= HALF_K[0] && g.m > (uint32_t)TM && !g.b2 && !g.cross_k && g.ldb <= widest_b<1>() && !edge;
-    if (path == PATH_SPLITK && !halves) {
+    const bool all_bits = path == PATH_SPLITK;
+    if (vec ? launch_sliced<true>(g, rope, all_bits, s) : launch_sliced<false>(g, rope, all_bits, s)) return;
+    if (path == PATH_SPLITK) {
         const dim3 sgrid((g.n + 31u) / 32u, (g.m + 31u) / 32u);
         if (rope) {
             if (vec) launch_splitk<true, true>(g, sgrid, s);

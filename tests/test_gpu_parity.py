@@ -1317,6 +1317,43 @@ def test_matmul_whose_small_values_carry_the_result(m, k, n, what, dev):
         assert worst <= 2.0 ** -24 * k ** 0.5 + 2.0 ** -22, (dim, worst)
 
 
+@pytest.mark.parametrize("m,k,n", [
+    (640, 2048, 512), (301, 2048, 512), (420, 1536, 512), (577, 2309, 500), (513, 4099, 320),    # 64 x 64 tiles in slices
+    (700, 2048, 512), (513, 3071, 512), (800, 1024, 512), (300, 4096, 256), (640, 2048, 640),    # too few slices, or tiles
+    (580, 512, 512), (180, 512, 1520), (645, 386, 512), (512, 768, 540), (448, 1000, 960)])      # more than 256 tiles of 32 x 32
+def test_matmul_below_the_tiles_keeps_every_bit(m, k, n, dev):
+    """Products of fewer than 112 tiles of 64 x 64 hold every bit of their operands, whatever stands beside a value: one result of
+    sixteen terms that are a billionth of their row and column's others, a one-hot row, and the same on the other side.  A sum of
+    sixteen is sixteen roundings of products and as many of sums, at most 2^-24 of the terms' magnitudes each; the zeros
+    between them add nothing."""
+    import torch
+    assert -(-m // 64) * -(-n // 64) < 112
+    lib = api.load()
+    torch.manual_seed(m + n + k)
+    a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
+    for x, y in ((a, b), (b.T, a.T)):       # views: row 7 of a and column 9 of b, then column 7 and row 9
+        at = torch.arange(16, device="cuda") * (k // 16) + k // 32
+        few = y[at, 9].clone()
+        y[:, 9] = 0.0
+        y[at, 9] = few
+        x[7, at] *= 1e-9
+        x[11] = 0.0
+        x[11, k - 5] = 1.0
+    a[11, :], b[:, 11] = 0.0, 0.0
+    a[11, k - 5] = b[k - 5, 11] = 1.0
+    out = torch.full((m, n), 7.0, device="cuda")
+    va, vb, vo = _dev_tensor(a), _dev_tensor(b), _dev_tensor(out)
+    torch.cuda.synchronize()
+    lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    torch.cuda.synchronize()
+    for row, column in ((7, 9), (9, 7)):
+        x, y = a[row].double(), b[:, column].double()
+        assert int((x * y != 0).sum()) == 16
+        off = abs(out[row, column].item() - float(x @ y))
+        assert off <= 32 * 2.0 ** -24 * float(x.abs() @ y.abs()), (row, column, off / float(x.abs() @ y.abs()))
+    assert torch.equal(out[11], b[k - 5]) and torch.equal(out[:, 11], a[:, k - 5])
+
+
 @pytest.mark.parametrize("m,k,n", [(700, 400, 720), (2048, 160, 1290), (70, 384, 4000), (1500, 385, 700)])
 def test_matmul_on_halves_out_of_range(m, k, n, dev):
     """The matrix-core product takes its operands apart into f16 parts up to 4094 (a) and 1023 (b), and from 2^-15 and 2^-17 on in
