@@ -27,7 +27,8 @@ bool blt_stream_captured_by_caller(hipStream_t s = nullptr);
 hipStream_t blt_stream_key();
 /* Host-to-device copy that returns at once and lets the caller reuse `src`
  * right away: a few kilobytes travel in kernel arguments, more goes through a small ring of
- * pinned buffers owned by the calling thread (memory.hip).  Not usable while a graph is captured. */
+ * pinned buffers owned by the calling thread (memory.hip).  Not usable while a graph is captured, but for what travels in
+ * arguments where the caller captures the stream by other means. */
 void blt_upload_staged(void *dst, const void *src, size_t bytes);
 /* Turns a sticky error the KV step kernels raised on the device (a sequence outgrew what its
  * launch, slab or rotation tables hold) into the fatal error; costs one 4-byte read-back, and

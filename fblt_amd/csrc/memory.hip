@@ -129,6 +129,9 @@ void blt_upload_staged(void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return;
     BLT_REQUIRE(!blt_stream_capturing(), "host data cannot be staged to the device while a graph is captured");
     if (upload_in_arguments(dst, src, bytes)) return;
+    /* a replay would copy what the ring's buffer holds by then, and an event recorded there cannot be waited for */
+    BLT_REQUIRE(!blt_stream_captured_by_caller(),
+                "more host data than launch arguments hold cannot be staged to the device while the stream is captured");
     static thread_local PinnedRing ring;
     PinnedRing::Slot &s = ring.slot[ring.next];
     ring.next = (ring.next + 1) % PinnedRing::SLOTS;

@@ -3038,6 +3038,28 @@ def test_long_products_in_a_capture_of_the_callers_own(m, k, n, warm, dev):
         lib.blt_hip_set_stream(None)
 
 
+def test_long_uploads_in_a_capture_of_the_callers_own_are_refused():
+    """Host data past what launch arguments hold goes through pinned buffers that later uploads use again, so a replay would copy
+    other data: fatal in a capture of the caller's own too.  What launch arguments hold is part of the recording."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = ("import sys\nsys.path.insert(0, %r)\nimport numpy as np, torch\nfrom fblt_amd import api\nlib = api.load()\n"
+            "stream, graph, second = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()\n"
+            "words, to = np.arange(1000, dtype=np.uint32), torch.zeros(20000, dtype=torch.int32, device='cuda')\n"
+            "many = np.arange(20000, dtype=np.uint32)\ntorch.cuda.synchronize()\nlib.blt_hip_set_stream(stream.cuda_stream)\n"
+            "with torch.cuda.graph(graph, stream=stream, capture_error_mode='relaxed'):\n"
+            "    lib.blt_hip_memcpy_h2d(to.data_ptr(), words.ctypes.data, words.nbytes)\n"
+            "words[:] = 0\ngraph.replay()\ntorch.cuda.synchronize()\n"
+            "assert to[:1000].tolist() == list(range(1000))\nprint('SHORT', flush=True)\n"
+            "with torch.cuda.graph(second, stream=stream, capture_error_mode='relaxed'):\n"
+            "    lib.blt_hip_memcpy_h2d(to.data_ptr(), many.ctypes.data, many.nbytes)\nprint('SURVIVED')\n" % root)
+    p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert "SHORT" in p.stdout and "SURVIVED" not in p.stdout, p.stdout + p.stderr
+    assert p.returncode == 1 and "while the stream is captured" in p.stderr, (p.returncode, p.stderr)
+
+
 def test_profile_holds_every_launch(dev):
     """Uploads that travel in kernel arguments and the small kernels beside the main path are in the kernel-time profile."""
     import torch
