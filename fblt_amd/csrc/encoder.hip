@@ -344,11 +344,12 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
                 "blt_local_encoder_forward: ngram_config does not fit the encoder");
 
     /* ---- byte rows with their n-grams, and P_0: pooled rows in every sub-token column block (local_encoder.c:237-245) ---- */
-    const hipStream_t stream = blt_stream();
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (bytes_in->backend == BLT_BACKEND_HIP && stream != nullptr) HIP_CHECK(hipStreamIsCapturing(stream, &capture));
-    BLT_REQUIRE(!blt_stream_capturing() && capture == hipStreamCaptureStatusNone,
-                "blt_local_encoder_forward: bytes and patch tables are read on the way, which a graph cannot replay");
+    /* The patches belong to the bytes and are part of a recording, so the bytes have to be, too: host bytes in a capture of the caller's
+     * own are, device bytes would be read by the replay. */
+    BLT_REQUIRE(!blt_stream_capturing(), "blt_local_encoder_forward: mask metadata cannot be staged while a graph capture is open");
+    BLT_REQUIRE(bytes_in->backend != BLT_BACKEND_HIP || !blt_stream_captured_by_caller(),
+                "blt_local_encoder_forward: a replay would read other bytes than the recorded patches belong to; record it with the bytes "
+                "on the host");
     const size_t byte_shape[2] = {seq_len, E}, patch_shape[2] = {num_patches, patch_dim};
     EmbedArgs em;
     std::memset(&em, 0, offsetof(EmbedArgs, start));
@@ -393,7 +394,7 @@ extern "C" void blt_local_encoder_forward_hip(const blt_local_encoder *model, co
         em.start[n] = (uint32_t)(j0 + n == runs ? seq_len : tile ? patches[j0 + n].start_idx : (j0 + n) * EMBED_ROWS);
         em.pooled = tile ? (float *)p.data + j0 * patch_dim : nullptr;
         const dim3 grid((unsigned)n, (unsigned)((E + EMBED_COLS - 1) / EMBED_COLS));
-        blt_launch("embed_pool", vec ? embed_pool_kernel<true> : embed_pool_kernel<false>, grid, dim3(256), 0, stream, em);
+        blt_launch("embed_pool", vec ? embed_pool_kernel<true> : embed_pool_kernel<false>, grid, dim3(256), 0, blt_stream(), em);
     }
     HIP_CHECK_LAUNCH("blt_local_encoder_forward: embedding");
     if (!tile) pool_launch((const float *)h.data, seq_len, E, patches, num_patches, cfg.pool_type, (float *)p.data, patch_dim, k);

@@ -164,6 +164,9 @@ void blt_transformer_forward_hip(const blt_tensor *input, const blt_transformer_
  * layer the byte transformer block and, where it fires, P += cross_attention(RMSNorm(P), h).
  * bytes_in [seq_len] UINT8 on either side (host bytes may change on return, device bytes are read
  * in stream order, like the other inputs); weights, outputs and the arena are device memory; patches, doc_boundaries are HOST arrays.
+ * Not between blt_hip_capture_begin and _end.  A capture of the caller's own takes it with the bytes on the host: bytes, patches and
+ * documents are then those of the recording in every replay.  Device bytes are refused there, and so is more host data than
+ * launch arguments hold (2560 bytes of text always fit).
  * Unlike the reference's body on a device arena, sub-token splits (patch_dim = k * embed_dim,
  * k > 1) work: the expanded group ids are host memory here. */
 /* csrc/models/local_decoder.c:233-351 on the device: per layer the cross block (when it fires)

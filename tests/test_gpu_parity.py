@@ -3215,6 +3215,56 @@ def test_encoder_embeds_and_pools_in_one_launch(T, E, H, ngrams, vocab, lengths,
     assert_close(got_p, want_p, "patch_out")
 
 
+ENCODER_CAPTURE = """
+import sys
+import numpy as np, torch
+from fblt_amd import abi, api
+from oracle import binding
+from tests import encoder_runs
+from tests.golden import block_cases
+
+def run(T, lengths, on_device):
+    lib, orc = api.load(), binding.load_oracle()
+    c = dict(T=T, E=64, H=2, XH=2, L=2, hidden=64, ngrams=(3, 4), vocab=1000, k=1, window=0, placement=0, all_layers=True, pool="mean",
+             docs=None, normalize=True, mean_patch=4)
+    data, _, weights = block_cases.encoder_case(np.random.RandomState(T), c)
+    want = encoder_runs.run_oracle(orc, c, data, lengths, weights)
+    stream, graph, outs = torch.cuda.Stream(), torch.cuda.CUDAGraph(), []
+
+    def entry(*args):
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+            lib.blt_local_encoder_forward(*args)
+        data[:] = 0
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+
+    lib.blt_hip_set_stream(stream.cuda_stream)
+    got = encoder_runs.run_device(entry, lib, orc, c, data, lengths, weights, bytes_on_device=on_device)
+    lib.blt_hip_set_stream(None)
+    for a, b in zip(got, want):
+        assert (np.abs(a - b) <= 1e-5 + 1e-4 * np.abs(b)).all()
+"""
+
+
+@pytest.mark.parametrize("T", [61, 2560])
+def test_encoder_in_a_capture_of_the_callers_own(T):
+    """Bytes on the host, patches and documents are those of the recording in every replay.  Bytes on the device, which a replay would
+    read anew under the patches of the recording, and more text than launch arguments hold are fatal."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lengths = [1, 7, 8, 9, 16, 17, 3] if T == 61 else [10] * 256
+    code = "import sys\nsys.path.insert(0, %r)\n" % root + ENCODER_CAPTURE + (
+        "run(%d, %r, False)\nprint('REPLAYED', flush=True)\n" % (T, lengths) +
+        ("run(61, %r, True)\n" % lengths if T == 61 else "run(2561, [10] * 256 + [1], False)\n") + "print('SURVIVED')\n")
+    p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert "REPLAYED" in p.stdout and "SURVIVED" not in p.stdout, p.stdout + p.stderr
+    assert p.returncode == 1 and ("record it with the bytes" if T == 61 else "while the stream is captured") in p.stderr, p.stderr
+
+
 def test_encoder_ops(oracle, dev):
     """blt_indexed_row_accumulate / blt_scale / blt_patch_pool_forward on device tensors against the
     restated ops: bit for bit (the kernels keep the reference's order of additions).  Index lists
