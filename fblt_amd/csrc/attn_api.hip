@@ -563,11 +563,7 @@ struct Staging {
             plan_launch(plan, nullptr, nullptr, docs.data());
             return;
         }
-        if (need > capacity) {
-            if (device) {
-                HIP_CHECK(hipDeviceSynchronize());
-                HIP_CHECK(hipFree(device));
-            }
+        if (need > capacity) { /* the outgrown one is left to the process: a recording of the caller's own may name it */
             capacity = std::max<size_t>(2 * need, 64 * 1024);
             HIP_CHECK(hipMalloc(&device, capacity));
         }

@@ -3038,6 +3038,40 @@ def test_long_products_in_a_capture_of_the_callers_own(m, k, n, warm, dev):
         lib.blt_hip_set_stream(None)
 
 
+def test_staged_batch_in_a_capture_of_the_callers_own(dev):
+    """A batch whose descriptors are staged, recorded by the caller's own capture, still finds them where they were after a larger
+    eager batch of that stream has outgrown the buffer."""
+    import torch
+    lib = api.load()
+    qkv, out = torch.randn(3, 40, 32, device="cuda"), torch.zeros(3, 40, 32, device="cuda")
+    row = torch.randn(1200, 32, device="cuda")
+
+    def problems(count):
+        return [api.problem(api.head_args(qkv.data_ptr(), qkv.data_ptr(), qkv.data_ptr(), (out[i] if count == 3 else row[i]).data_ptr(),
+                                          (20 + i * i) if count == 3 else 1, 40 - i % 3, 32, 0.2, 32, 32, 32, 32, 0),
+                            api.BLT_ATTN_MASK_CAUSAL) for i in range(count)]
+    few, many = api.problem_array(problems(3)), api.problem_array(problems(1200))
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    try:
+        lib.blt_hip_set_stream(stream.cuda_stream)
+        lib.blt_attention_batch_hip(few, 3)
+        torch.cuda.synchronize()
+        want = out.clone()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+            lib.blt_attention_batch_hip(few, 3)
+        for _ in range(3):
+            lib.blt_attention_batch_hip(many, 1200)
+            out.fill_(7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            for i in range(3):      # the rows that the batch has
+                assert torch.equal(out[i, : 20 + i * i], want[i, : 20 + i * i])
+    finally:
+        lib.blt_hip_set_stream(None)
+
+
 def test_long_uploads_in_a_capture_of_the_callers_own_are_refused():
     """Host data past what launch arguments hold goes through pinned buffers that later uploads use again, so a replay would copy
     other data: fatal in a capture of the caller's own too.  What launch arguments hold is part of the recording."""
