@@ -1181,7 +1181,7 @@ void launch_mfma_as(const MatmulArgs &g, dim3 grid, hipStream_t s) {
             hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         HIP_CHECK(asked);
     }
-    blt_launch("matmul_mfma", kernel, grid, dim3(512), lds, s, g);
+    blt_launch(SLICED ? "matmul_mfma_slices" : "matmul_mfma", kernel, grid, dim3(512), lds, s, g);
 }
 /* Slices of K per 64x64 tile; 1: not taken for it.  Up to 128 tiles with a long K leave half of the chip empty.  As many slices as
  * keep to one workgroup a compute unit (two on one take turns with its LDS and vector units: 192 tiles of K = 2048 24.5 us, as

@@ -1100,7 +1100,7 @@ def _dev_tensor(t, shape=None):
 @pytest.mark.parametrize("k", [20, 32, 64, 70, 96, 128, 160, 186, 384, 448, 455, 512])
 def test_matmul_whole_steps(m, n, k):
     """The tile kernels' loop takes whole steps of K (32 or 64) in pairs: none, one, odd and even counts, with and without a rest,
-    on both tiles and both forms of the operands.  Against float64: a sum of k fp32 products is within k 2^-24 of the
+    on both tiles and both forms of the operands, and the 32 x 32 tiles below them.  Against float64: a sum of k fp32 products is within k 2^-24 of the
     sum of their magnitudes whatever its order, and rounding to fp32 adds less."""
     import torch
     lib = api.load()
@@ -1114,22 +1114,41 @@ def test_matmul_whole_steps(m, n, k):
     assert (off <= (k + 1) * 2.0 ** -24 * (np.abs(a) @ np.abs(b))).all()
 
 
-@pytest.mark.parametrize("m,n", [(65, 1025), (301, 512), (641, 449), (1000, 512), (1024, 515)])
+def _product_kernel(m, k, n):
+    """The kernel that a plain product of more than 64 rows is to take, and over how many slices of K."""
+    tiles, small = -(-m // 64) * -(-n // 64), -(-m // 32) * -(-n // 32)
+    whole = "matmul_mfma" if tiles >= 112 else "matmul_splitk"
+    if k < 1024 or not 16 <= tiles <= 128 or tiles * k < 80 * 1024 or (tiles < 112 and small <= 128):
+        return whole, 1
+    for slices in range(min(256 // tiles, k // 384), 1 if tiles >= 112 else 2 if k <= 2560 else 3, -1):
+        run = -(-(-(-k // slices)) // 64) * 64
+        if k - (slices - 1) * run >= 384:
+            return "matmul_mfma_slices", slices
+    return whole, 1
+
+
+@pytest.mark.parametrize("m,n", [(65, 1025), (301, 512), (641, 449), (1000, 512), (1024, 515), (577, 450), (897, 508), (290, 460)])
 @pytest.mark.parametrize("k", [1023, 1024, 1025, 1530, 2048, 2049, 2500, 5200])
 def test_matmul_tiles_in_slices(m, n, k):
-    """16 to 128 tiles of 64 x 64 and a long K: up to sixteen workgroups a tile, each with its run of K, odd rests among them; the bound
-    of test_matmul_whole_steps (one more rounding a slice).  The same bits whoever comes last, and an infinity in one slice is
-    one in the result."""
+    """16 to 128 tiles of 64 x 64 and a long K: up to six workgroups a tile, each with its run of K, odd rests among them, and the shapes
+    beside the rule's lines that stay whole; the bound of test_matmul_whole_steps (one more rounding a slice).  The same bits whoever
+    comes last and wherever the output lies, and an infinity in one slice is one in the result."""
     import torch
     lib = api.load()
     rs = np.random.RandomState(m + 3 * n + 7 * k)
     a, b = rs.randn(m, k).astype(np.float32), (rs.randn(k, n) / np.sqrt(k)).astype(np.float32)
     ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
-    outs = [torch.full((m, n), 7.0, device="cuda") for _ in range(3)]
+    outs = [torch.full((m, n), 7.0, device="cuda") for _ in range(2)]
+    outs.append(torch.full((m * n + 1,), 7.0, device="cuda")[1:].view(m, n))     # off a 16-byte boundary
     va, vb = _dev_tensor(ta), _dev_tensor(tb)
+    torch.cuda.synchronize()
+    lib.blt_hip_profile_begin()
     for out in outs:
         vo = _dev_tensor(out)
         lib.blt_matmul(C.byref(va), C.byref(vb), C.byref(vo))
+    launched = api.profile_end()
+    launched.pop("matmul_clear_words", None)
+    assert {name: v[0] for name, v in launched.items()} == {_product_kernel(m, k, n)[0]: 3}, launched
     got = [out.cpu().numpy() for out in outs]
     assert got[0].tobytes() == got[1].tobytes() == got[2].tobytes()
     a, b = a.astype(np.float64), b.astype(np.float64)
@@ -1327,7 +1346,8 @@ def test_matmul_below_the_tiles_keeps_every_bit(m, k, n, dev):
     sixteen is sixteen roundings of products and as many of sums, at most 2^-24 of the terms' magnitudes each; the zeros
     between them add nothing."""
     import torch
-    assert -(-m // 64) * -(-n // 64) < 112
+    sliced = {(640, 2048, 512): 3, (301, 2048, 512): 4, (420, 1536, 512): 4, (577, 2309, 500): 3, (513, 4099, 320): 5}
+    assert _product_kernel(m, k, n) == (("matmul_mfma_slices", sliced[m, k, n]) if (m, k, n) in sliced else ("matmul_splitk", 1))
     lib = api.load()
     torch.manual_seed(m + n + k)
     a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
@@ -2385,6 +2405,19 @@ def test_block_behind_its_attention_of_many_slices(T, E, H, hidden, fused, dev):
     assert launched.get("block_tail", (0,))[0] == (3 if fused else 0), launched
     # four products, each of which rounds a sum of at most 2112 terms
     assert _relative(outs[0].cpu(), want) <= 2 * 2 ** -24 * 2112 ** 0.5
+    assert outs[0].cpu().numpy().tobytes() == outs[1].cpu().numpy().tobytes() == outs[2].cpu().numpy().tobytes()
+
+
+@pytest.mark.parametrize("T,hidden,shift", [(301, 2048, 0), (301, 2048, 1), (640, 2048, 0), (577, 2050, 0), (1000, 2048, 0), (1000, 2048, 1),
+                                            (965, 1100, 2)])
+def test_block_whose_down_projection_is_in_slices(T, hidden, shift, dev):
+    """A sliced product with a residual, which the last slice's workgroup adds: on parts of either kind, in 16-byte pieces and in
+    single values."""
+    assert _product_kernel(T, hidden, 512)[0] == "matmul_mfma_slices"
+    outs, launched, want = _transformer_block(T, 512, 8, hidden, shift)
+    assert launched["matmul_mfma_slices"][0] == 3, launched
+    # four products, each of which rounds a sum of at most `hidden` terms
+    assert _relative(outs[0].cpu(), want) <= 2 * 2 ** -24 * hidden ** 0.5
     assert outs[0].cpu().numpy().tobytes() == outs[1].cpu().numpy().tobytes() == outs[2].cpu().numpy().tobytes()
 
 
