@@ -1191,15 +1191,17 @@ void launch_mfma_as(const MatmulArgs &g, dim3 grid, hipStream_t s) {
  * bf16 parts (all_bits).  As f16 parts a result that comes from a row's smallest values only was as far off as those parts are, another
  * of the row being large (values of 1e-9 beside ones near 1: 2.3e-5 of their products).  bf16 parts round six times for 16 terms, so only short slices are as close as the 32x32 tiles are, eight waves
  * to a K: error, this / 32x32 tiles, in six slices 0.70 ... 0.72, five 0.76 ... 0.80, four 0.83 ... 0.88, three of K up to 2560
- * 0.96 ... 1.00 but of 4096 1.01, two 1.2; none up to 128 of the 32x32 tiles, which take slices of their own.  us, 32x32 tiles / this, 301
- * rows of 2048 to 512 columns 17.2 / 13.5, 420 18.0 / 14.3, 640 31.5 / 17.3, 420 of 1536 14.3 / 12.9, 301 of 4096 32.5 / 18.1. */
+ * 0.96 ... 1.00 but of 4096 1.01, two 1.2; none up to 128 of the 32x32 tiles, which take slices of their own.  That many slices where
+ * it takes two workgroups on some compute units too.  us, 32x32 tiles / this, 301 rows of 2048 to 512 columns 17.2 / 13.5, 420
+ * 18.0 / 14.3, 640 31.5 / 17.3, 700 31.6 / 24.5, 832 31.7 / 25.1, 832 of 1280 21.8 / 18.6, 420 of 1536 14.3 / 12.9, 301 of 4096 32.5 / 18.1,
+ * 832 57.8 / 37.5. */
 uint32_t tile_slices(const MatmulArgs &g, bool rope, bool all_bits) {
     if (g.b2 || rope || g.norm_w || g.cross_k || g.k < 1024u || g.m <= (uint32_t)TM || g.ldb > widest_b<1>()) return 1u;
     const uint64_t tiles = (uint64_t)((g.n + TN - 1u) / TN) * ((g.m + TM - 1u) / TM);
     if (tiles < 16u || tiles > 128u || tiles * g.k < 80u * 1024u) return 1u; /* 16: the last workgroup adds its slices one after the other */
     if (all_bits && (uint64_t)((g.n + 31u) / 32u) * ((g.m + 31u) / 32u) <= 128u) return 1u;
-    const uint32_t least = !all_bits ? 2u : g.k <= 2560u ? 3u : 4u;
-    for (uint32_t n = std::min(256u / (uint32_t)tiles, g.k / HALF_K[0]); n >= least; n--) {
+    const uint32_t least = !all_bits ? 2u : g.k <= 2560u ? 3u : 4u, room = 256u / (uint32_t)tiles;
+    for (uint32_t n = std::min(all_bits ? std::max(room, least) : room, g.k / HALF_K[0]); n >= least; n--) {
         const uint32_t before = (n - 1u) * tile_slice(g.k, n);
         if (before < g.k && g.k - before >= HALF_K[0]) return n; /* the last one is not empty, nor bf16 for being short */
     }

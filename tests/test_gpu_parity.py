@@ -1120,7 +1120,8 @@ def _product_kernel(m, k, n):
     whole = "matmul_mfma" if tiles >= 112 else "matmul_splitk"
     if k < 1024 or not 16 <= tiles <= 128 or tiles * k < 80 * 1024 or (tiles < 112 and small <= 128):
         return whole, 1
-    for slices in range(min(256 // tiles, k // 384), 1 if tiles >= 112 else 2 if k <= 2560 else 3, -1):
+    least = 2 if tiles >= 112 else 3 if k <= 2560 else 4
+    for slices in range(min(256 // tiles if tiles >= 112 else max(256 // tiles, least), k // 384), least - 1, -1):
         run = -(-(-(-k // slices)) // 64) * 64
         if k - (slices - 1) * run >= 384:
             return "matmul_mfma_slices", slices
@@ -1338,7 +1339,8 @@ def test_matmul_whose_small_values_carry_the_result(m, k, n, what, dev):
 
 @pytest.mark.parametrize("m,k,n", [
     (640, 2048, 512), (301, 2048, 512), (420, 1536, 512), (577, 2309, 500), (513, 4099, 320),    # 64 x 64 tiles in slices
-    (700, 2048, 512), (513, 3071, 512), (800, 1024, 512), (300, 4096, 256), (640, 2048, 640),    # too few slices, or tiles
+    (700, 2048, 512), (513, 3071, 512), (640, 2048, 640), (820, 1300, 500),                      # more than 256 workgroups
+    (800, 1024, 512), (300, 4096, 256),                                                          # too few slices, too few tiles
     (580, 512, 512), (180, 512, 1520), (645, 386, 512), (512, 768, 540), (448, 1000, 960)])      # more than 256 tiles of 32 x 32
 def test_matmul_below_the_tiles_keeps_every_bit(m, k, n, dev):
     """Products of fewer than 112 tiles of 64 x 64 hold every bit of their operands, whatever stands beside a value: one result of
@@ -1346,7 +1348,8 @@ def test_matmul_below_the_tiles_keeps_every_bit(m, k, n, dev):
     sixteen is sixteen roundings of products and as many of sums, at most 2^-24 of the terms' magnitudes each; the zeros
     between them add nothing."""
     import torch
-    sliced = {(640, 2048, 512): 3, (301, 2048, 512): 4, (420, 1536, 512): 4, (577, 2309, 500): 3, (513, 4099, 320): 5}
+    sliced = {(640, 2048, 512): 3, (301, 2048, 512): 4, (420, 1536, 512): 4, (577, 2309, 500): 3, (513, 4099, 320): 5,
+              (700, 2048, 512): 3, (513, 3071, 512): 4, (640, 2048, 640): 3, (820, 1300, 500): 3}
     assert _product_kernel(m, k, n) == (("matmul_mfma_slices", sliced[m, k, n]) if (m, k, n) in sliced else ("matmul_splitk", 1))
     lib = api.load()
     torch.manual_seed(m + n + k)
