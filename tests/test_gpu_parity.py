@@ -953,6 +953,7 @@ def test_attention_whose_small_values_carry_the_result(batch, H, hd, nq, nk, dev
 
 @pytest.mark.parametrize("batch,H,hd,nq,nk,window", [
     (32, 4, 32, 1025, 1025, 0), (64, 4, 32, 300, 333, 0), (64, 4, 32, 520, 520, 65),       # eight waves, four, windows
+    (64, 4, 32, 520, 520, 255), (64, 4, 32, 520, 520, 256), (32, 4, 32, 390, 411, 64),     # both sides of the line for windows
     (48, 4, 64, 510, 510, 0), (48, 4, 64, 512, 512, 0), (32, 2, 64, 1030, 1061, 0),        # both sides of the line for heads of 64
     (48, 4, 64, 640, 640, 319), (48, 4, 64, 640, 640, 320)])
 def test_attention_weighed_before_its_maximum(batch, H, hd, nq, nk, window, dev):
