@@ -1100,10 +1100,8 @@ uint32_t kv_block_heads_per_group(uint32_t batch, uint32_t subs, uint32_t num_he
 /* Takes head_dim 32 and 64 (the K tiles of four waves fit the static LDS
  * budget); the caller falls back to the VALU kernel otherwise.  Handles up to
  * 32 query rows per launch: a.q0 .. a.q0 + 31. */
-bool kv_block_mfma_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
+bool kv_block_mfma_launch(const StepArgs &a, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
                           hipStream_t s) {
-    StepArgs a = a_in;
-    a.halves = 1u;
     /* the per-wave K tiles bound the workgroups: 8 waves of 4.6 KB or 4 of 8.7 KB */
     /* BLT_HIP_BLOCK_TILE=16 keeps blocks of up to four rows on the 16-wide tiles, =4 keeps the looping
      * kernels (4x4x1 tiles up to four rows, 16-wide above), =once takes the all-at-once kernel wherever
@@ -1128,17 +1126,15 @@ bool kv_block_mfma_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_di
         const uint64_t pairs = (uint64_t)batch * a.num_heads;
         const uint32_t tiles = (a.span + 15u) / 16u + 2u;
         const bool idle = 2u * pairs <= 256u;
-        a.halves = 2u;
         if (pin == 1 || idle || (head_dim == 32u ? tiles <= 48u : pairs <= 256u || tiles <= 8u))
-            if (kv_block_once_launch(a, batch, head_dim, host_lens, s)) return true;
+            if (kv_block_once_launch(a, batch, head_dim, host_lens, true, s)) return true;
         if (idle && (head_dim == 32u || head_dim == 64u)) {
             if (head_dim == 32u) launch_block_as<32, 8, true, true>(a, batch, host_lens, s);
             else launch_block_as<64, 4, true, true>(a, batch, host_lens, s);
             return true;
         }
-        a.halves = 1u;
     }
-    if ((pin == 1 || (pin == 0 && !small)) && kv_block_once_launch(a, batch, head_dim, host_lens, s)) return true;
+    if ((pin == 1 || (pin == 0 && !small)) && kv_block_once_launch(a, batch, head_dim, host_lens, false, s)) return true;
     if (head_dim == 32u) {
         if (a.n - a.q0 <= 4u && !no_tile4) launch_block4(a, batch, host_lens, s);
         else if (!narrow_block(a)) launch_block_as<32, 8, false>(a, batch, host_lens, s);

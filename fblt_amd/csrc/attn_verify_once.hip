@@ -352,7 +352,7 @@ __global__ __launch_bounds__(1024) void kv_block_once_kernel(StepArgs a, LensArg
 template <int HD, int T, bool HALVES>
 void block_once_launch_with(const StepArgs &a, uint32_t batch, uint32_t waves, const uint32_t *host_lens, hipStream_t s) {
     using Shape = BlockOnceShape<HD>;
-    const dim3 grid(a.halves, batch, a.num_heads), block(64 * waves);
+    const dim3 grid(HALVES ? 2u : 1u, batch, a.num_heads), block(64 * waves);
     const size_t lds = Shape::bytes(waves);
     if (host_lens) {
         static const bool raised = [] {
@@ -376,8 +376,8 @@ void block_once_launch_with(const StepArgs &a, uint32_t batch, uint32_t waves, c
 }
 
 template <int HD, int T>
-void block_once_launch_as(const StepArgs &a, uint32_t batch, uint32_t waves, const uint32_t *host_lens, hipStream_t s) {
-    if (a.halves == 2u) block_once_launch_with<HD, T, true>(a, batch, waves, host_lens, s);
+void block_once_launch_as(const StepArgs &a, uint32_t batch, uint32_t waves, const uint32_t *host_lens, bool halves, hipStream_t s) {
+    if (halves) block_once_launch_with<HD, T, true>(a, batch, waves, host_lens, s);
     else block_once_launch_with<HD, T, false>(a, batch, waves, host_lens, s);
 }
 
@@ -386,10 +386,11 @@ void block_once_launch_as(const StepArgs &a, uint32_t batch, uint32_t waves, con
 /* Launch of the once block kernel: at most 16 rows per sequence from row 0 on, 32 by halves, one split, and a prefix
  * whose 16-key tiles (plus those with the new rows) fit the waves' registers; false when it does
  * not take the shape.  host_lens: NULL (device lengths) or `batch` <= KARG_SEQS lengths. */
-bool kv_block_once_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
+bool kv_block_once_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens, bool halves,
                           hipStream_t s) {
-    if (a_in.q0 != 0u || a_in.n > 16u * a_in.halves || a_in.n == 0u || a_in.splits != 1u) return false;
-    const uint32_t tiles = (a_in.span + 15u) / 16u + a_in.halves; /* what the longest sequence of the launch may need */
+    const uint32_t fresh = halves ? 2u : 1u; /* tiles of new rows */
+    if (a_in.q0 != 0u || a_in.n > 16u * fresh || a_in.n == 0u || a_in.splits != 1u) return false;
+    const uint32_t tiles = (a_in.span + 15u) / 16u + fresh; /* what the longest sequence of the launch may need */
     const uint32_t per_wave = (tiles + 15u) / 16u;       /* tiles a wave holds at once */
     /* as few waves as give every tile a slot, in fours: a slot without a tile still costs its requests */
     const uint32_t waves = std::min(16u, ((tiles + per_wave - 1u) / per_wave + 3u) / 4u * 4u);
@@ -397,16 +398,16 @@ bool kv_block_once_launch(const StepArgs &a_in, uint32_t batch, uint32_t head_di
     a.hpb = 1, a.slices = 1, a.by_length = 0;
     if (head_dim == 32u) {
         switch (per_wave) {
-        case 1: block_once_launch_as<32, 1>(a, batch, waves, host_lens, s); break;
-        case 2: block_once_launch_as<32, 2>(a, batch, waves, host_lens, s); break;
-        case 3: block_once_launch_as<32, 3>(a, batch, waves, host_lens, s); break;
-        case 4: block_once_launch_as<32, 4>(a, batch, waves, host_lens, s); break;
+        case 1: block_once_launch_as<32, 1>(a, batch, waves, host_lens, halves, s); break;
+        case 2: block_once_launch_as<32, 2>(a, batch, waves, host_lens, halves, s); break;
+        case 3: block_once_launch_as<32, 3>(a, batch, waves, host_lens, halves, s); break;
+        case 4: block_once_launch_as<32, 4>(a, batch, waves, host_lens, halves, s); break;
         default: return false;
         }
     } else if (head_dim == 64u) {
         switch (per_wave) {
-        case 1: block_once_launch_as<64, 1>(a, batch, waves, host_lens, s); break;
-        case 2: block_once_launch_as<64, 2>(a, batch, waves, host_lens, s); break;
+        case 1: block_once_launch_as<64, 1>(a, batch, waves, host_lens, halves, s); break;
+        case 2: block_once_launch_as<64, 2>(a, batch, waves, host_lens, halves, s); break;
         default: return false;
         }
     } else {

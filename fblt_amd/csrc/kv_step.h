@@ -48,7 +48,6 @@ struct StepArgs {
     int commit;        /* advance self_len when the sequence is done */
     int by_length;     /* block step with the lengths in the arguments: workgroups take the (sequence, head
                           group) pairs in the order of KargLens::order, longest sequences first */
-    uint32_t halves;   /* 2: (launcher) workgroup x of a sequence's (one split) takes the 16 query rows from q0 + 16 x on */
 };
 
 
@@ -221,9 +220,9 @@ uint32_t kv_block_heads_per_group(uint32_t batch, uint32_t subs, uint32_t num_he
 bool kv_block_mfma_launch(const StepArgs &a, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
                           hipStream_t s);
 
-/* block steps of at most 16 rows over a prefix short enough to be requested all at once
- * (attn_verify_once.hip); false when it does not take the shape */
-bool kv_block_once_launch(const StepArgs &a, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens,
+/* block steps of at most 16 rows, or 32 by halves (workgroup x of a (sequence, head) takes the 16 rows from 16 x on), over a
+ * prefix short enough to be requested all at once (attn_verify_once.hip); false when it does not take the shape */
+bool kv_block_once_launch(const StepArgs &a, uint32_t batch, uint32_t head_dim, const uint32_t *host_lens, bool halves,
                           hipStream_t s);
 
 /* single-row steps with one workgroup per (sequence, head) (attn_decode_row.hip): lengths from
