@@ -440,9 +440,10 @@ __global__ __launch_bounds__(Shape::THREADS) void cross_block_kernel(CrossBlockA
 }
 
 /* A block's tail and a cross block that neither reads nor writes anything of it, in the first `first` rows of workgroups: the
- * encoder's, whose patches take up a layer's bytes while the next layer goes on with them.  Its few workgroups fit beside the tail's, so
- * it costs nothing of its own (128 patches of 512 bytes, 128 columns: 9.6 us as a launch).  Half the keys in flight: more registers than the
- * tail has would halve the workgroups of a compute unit. */
+ * encoder's, whose patches take up a layer's bytes while the next layer goes on with them.  Its few workgroups fit beside the tail's: 128
+ * patches of 512 bytes, 128 columns, take 9.6 us as a launch and make this one 16.2 us where the tail alone is 11.4 ... 12.2 (64 columns,
+ * 757 bytes: 7.1, and 8.9 for 6.6).  Half the keys in flight: more registers than the tail has would halve the workgroups of a compute
+ * unit. */
 template <typename Shape, typename Ranges>
 __global__ __launch_bounds__(Shape::THREADS, 4) void block_tail_beside_kernel(BlockTailArgs a, CrossBlockArgs c, uint32_t first, Ranges w) {
     __shared__ TailLds<Shape> lds;

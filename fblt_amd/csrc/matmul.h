@@ -70,9 +70,7 @@ struct MatmulArgs {
     uint32_t all_bits; /* the launcher's: 64x64 tiles in slices, on parts that hold every bit of the operands */
 };
 
-/* Four consecutive results of output row `row` starting at column `col`:
- * optional rotation, optional residual, store with bounds. */
-/* of row `row` at position pos of sequence b: to Q or to the slabs */
+/* Four consecutive results of row `row`, position pos of sequence b, rotated where they are of Q or K: to Q or to the slabs. */
 __device__ __forceinline__ void matmul_stage4(const MatmulArgs &g, uint32_t row, uint32_t b, uint32_t pos, uint32_t col, float4 v) {
     const uint32_t E = g.n / 3u, part = col / E, at = col % E;
     if (part < 2u) {
@@ -82,6 +80,8 @@ __device__ __forceinline__ void matmul_stage4(const MatmulArgs &g, uint32_t row,
     float *const to = part == 0u ? g.out + (size_t)row * E : (part == 1u ? g.stage_k : g.stage_v) + ((size_t)b * g.stage_slab_rows + pos) * E;
     *reinterpret_cast<float4 *>(to + at) = v;
 }
+/* Four consecutive results of output row `row` starting at column `col`:
+ * optional rotation, optional residual, store with bounds. */
 template <bool ROPE>
 __device__ __forceinline__ void matmul_store4(const MatmulArgs &g, uint32_t row, uint32_t col, float4 v, bool vec_ok) {
     if (ROPE && g.stage_k) { /* new rows of a cache: no residual */

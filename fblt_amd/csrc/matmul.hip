@@ -64,8 +64,11 @@ constexpr int TM = 64, TN = 64; /* smallest workgroup tile of the mfma kernel */
  * f16 first, if K is long enough; a workgroup that meets operands out of its range, before the first product as a rule, or
  * finds its results too small for it (half_lost()) starts again as bf16.  Half the matrix instructions, four fifths of the vector ones, half the error (K = 2048: 2.2e-7
  * against 4.9e-7), and a clock that gives way less (8192 x 2048 . 2048 x 1536, random operands against ones: 268 and 210 us
- * as bf16, 196 and 160 as f16, 189 random ones as the loop is now).  Bound: in a step of the large tile the matrix unit takes 770 cycles of a SIMD, the vector
- * unit about 720, which add up, the LDS 770 beside them, of 2000 in all; the rest is the barrier.
+ * as bf16, 196 and 160 as f16, 189 random ones as the loop is now).  Bound: no one unit.  A step of the large tile takes some 2000
+ * cycles, and in it a SIMD's matrix unit 770, its vector unit 320 instructions, the compute unit's LDS 800 and 150 of bank conflicts; by the
+ * counters vector instructions issue in 0.4 ... 0.5 of a launch's cycles and the matrix unit is busy in a quarter.  What is between them
+ * is eight waves that meet at a barrier a step; requests and fragments further ahead, three buffers and another order of issue changed
+ * nothing.
  * VEC: a 16-byte aligned with lda and K multiples of 4.  ROPE: rotate pairs of the first g.rope_cols columns in
  * the epilogue.
  * NORM: the row statistic comes from the values on their way to LDS, the norm weight is multiplied in there, the row's
@@ -87,8 +90,8 @@ struct MfmaShape {
     };
     static constexpr size_t LDS_BYTES = 2 * sizeof(Tiles);
 };
-/* most columns of b that the tiles take: what 32-bit byte offsets over a step's rows reach, whatever the form.  A column's own
- * offset is all that has 32 bits now; the lines stay where they have been tested. */
+/* Most columns of b that the tiles take: a tested limit, not a reach.  A lane's 32-bit offset is its column's alone, but the lines
+ * have been drawn and tested where a whole step's rows would still fit such offsets. */
 template <int WT>
 constexpr uint32_t widest_b() {
     constexpr int steps[] = {MfmaShape<WT, false, false>::STEP, MfmaShape<WT, false, true>::STEP, MfmaShape<WT, true, false>::STEP,
@@ -1051,7 +1054,7 @@ Path choose_path(const MatmulArgs &g) {
      * 128 ... 132 tiles of K = 256 ... 1024 a tenth slower; pairs of 72 tiles of K = 128 faster, of 80 and 128
      * tiles of K = 256 and 512 slower (block of 200 rows of 512: 54.8 -> 49.7 us on the tile kernel). */
     const uint64_t splitk_below = g.b2 ? 80u : 112u;
-    /* the tile kernel reaches a column of b by a 32-bit byte offset, this one computes addresses in 64 bits */
+    /* wider than the tile kernel has been tested (widest_b); this one computes every address in 64 bits */
     if (g.ldb > widest_b<2>()) return PATH_SPLITK;
     /* one or two products an element: three parts drop the bits that fp32 rounds them to (error against float64 3.5e-8
      * and 3.4e-8, on the fp32 instructions 2.5e-8 and 3.1e-8; from three on the parts are closer, 3.3e-8 against 3.6e-8) */

@@ -115,7 +115,7 @@ void blt_cross_attention_forward_hip(const blt_tensor *query_in, const blt_tenso
 /* Device twins of the cache-aware decoder step (csrc/infer/kv_cache.c:
  * 112-159 and 161-416) with the reference's signatures, for a cache, decoder
  * weights and rows that live in device memory.  refresh_cross: one launch per
- * firing layer (two from 33 sub-tokens on) computes K and V of the new ones straight into
+ * firing layer, or two from 33 sub-tokens on, computes K and V of the new ones straight into
  * the tier-2 slabs.  decode_step: per layer the cross block (one launch for 64
  * or 128 columns and more than 32 rows, with the layer's QKV product up to
  * 1360 rows of 128 and 4096 of 64; 2-3 otherwise) and the self-attention /
