@@ -67,7 +67,6 @@ struct MatmulArgs {
     uint32_t slices;
     float *slice_sums;
     uint32_t *slice_tickets;
-    uint32_t all_bits; /* the launcher's: 64x64 tiles in slices, on parts that hold every bit of the operands */
 };
 
 /* Four consecutive results of row `row`, position pos of sequence b, rotated where they are of Q or K: to Q or to the slabs. */

@@ -404,12 +404,14 @@ __device__ __forceinline__ bool mfma_sums(const MatmulArgs &g, unsigned char *ld
 /* of K, for each of `slices`: whole steps of either form */
 __host__ __device__ __forceinline__ uint32_t tile_slice(uint32_t k, uint32_t slices) { return ((k + slices - 1u) / slices + 63u) / 64u * 64u; }
 
+/* Products in slices of K; ALL_BITS: on parts that hold every bit of the operands, bf16 ones from the start */
+enum : int { WHOLE, SLICES, SLICES_ALL_BITS };
 /* SLICED (small tile): gridDim.z workgroups a tile, each with its run of K as a product of its own; the one that comes last adds
  * up what all of them left, in their order. */
-template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED, bool SLICED = false>
+template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED, int SLICED = WHOLE>
 __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(MatmulArgs g) {
-    static_assert(!SLICED || (WT == 1 && !ROPE && !NORM && !GATED), "plain products");
-    if constexpr (SLICED) {
+    static_assert(SLICED == WHOLE || (WT == 1 && !ROPE && !NORM && !GATED), "plain products");
+    if constexpr (SLICED != WHOLE) {
         const uint32_t per = tile_slice(g.k, g.slices), k0 = blockIdx.z * per;
         g.a += k0, g.b += (size_t)k0 * g.ldb;
         g.k = min(per, g.k - k0); /* the launcher leaves no slice empty */
@@ -519,7 +521,7 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
      * or columns are by themselves at an edge, such a one would be all of a column, and some tile of nearly every launch start again
      * (200 x 512 . 512 x 2048 10.9 -> 18.9 us): bf16 from the start. */
     const auto few = [](uint32_t left, uint32_t whole, uint32_t block) { return left < whole && left % block - 1u < 3u; };
-    bool half = !(SLICED && g.all_bits != 0u) && g.k >= HALF_K[WT - 1] && !few(g.m - row0, BT, 32u) && !few(g.n - col0, COLS, SIDE);
+    bool half = SLICED != SLICES_ALL_BITS && g.k >= HALF_K[WT - 1] && !few(g.m - row0, BT, 32u) && !few(g.n - col0, COLS, SIDE);
     if (half) {
         floatx16 acc[WT][WT];
         float ss, most_a, most_b;
@@ -590,8 +592,8 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
         __syncthreads();
     }
 
-    float4 total[SLICED ? PIECES : 1];
-    if constexpr (SLICED) {
+    float4 total[SLICED != WHOLE ? PIECES : 1];
+    if constexpr (SLICED != WHOLE) {
         /* device-scope stores and loads, and an explicit wait for the stores' completion before the barrier that precedes this
          * workgroup's ticket, as for the split states of the KV step (kv_step.h) */
         __shared__ uint32_t ticket;
@@ -640,7 +642,7 @@ __global__ __launch_bounds__(512, WT == 1 ? 4 : 2) void matmul_mfma_kernel(Matmu
         if (r >= share) break;
         const uint32_t at = first + r + lane / PER, col = lane % PER * 4u;
         const uint32_t row = row0 + SIDE * wr + at;
-        float4 v = SLICED ? total[SLICED ? r / ROWS : 0] : *reinterpret_cast<const float4 *>(from + at * PITCH + col);
+        float4 v = SLICED != WHOLE ? total[SLICED != WHOLE ? r / ROWS : 0] : *reinterpret_cast<const float4 *>(from + at * PITCH + col);
         if (joined) {
             const float4 gate = *reinterpret_cast<const float4 *>(gates + at * PITCH + col);
             v.x = silu_times(gate.x, v.x), v.y = silu_times(gate.y, v.y), v.z = silu_times(gate.z, v.z), v.w = silu_times(gate.w, v.w);
@@ -1175,7 +1177,7 @@ void matmul_f32_launch_pair(const MatmulArgs &g0, const MatmulArgs &g1, hipStrea
 }
 
 namespace {
-template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED, bool SLICED = false>
+template <bool VEC, bool ROPE, int WT, bool NORM, bool GATED, int SLICED = WHOLE>
 void launch_mfma_as(const MatmulArgs &g, dim3 grid, hipStream_t s) {
     constexpr size_t lds = MFMA_LDS_BYTES<WT, NORM>;
     const auto kernel = matmul_mfma_kernel<VEC, ROPE, WT, NORM, GATED, SLICED>;
@@ -1184,14 +1186,14 @@ void launch_mfma_as(const MatmulArgs &g, dim3 grid, hipStream_t s) {
             hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         HIP_CHECK(asked);
     }
-    blt_launch(SLICED ? "matmul_mfma_slices" : "matmul_mfma", kernel, grid, dim3(512), lds, s, g);
+    blt_launch(SLICED != WHOLE ? "matmul_mfma_slices" : "matmul_mfma", kernel, grid, dim3(512), lds, s, g);
 }
 /* Slices of K per 64x64 tile; 1: not taken for it.  Up to 128 tiles with a long K leave half of the chip empty.  As many slices as
  * keep to one workgroup a compute unit (two on one take turns with its LDS and vector units: 192 tiles of K = 2048 24.5 us, as
  * 384 27.0; 256 28.8 and 30.4), of at least HALF_K each.  The 64x64 tile whole against this, 1000 rows of 2048 to 512 columns 23.7 /
  * 18.8 us, 900 of 1024 14.0 / 12.3, error against float64 2.2e-7 / 1.4e-7 (K = 2048).
  * Fewer than 112 tiles are products on the fp32 instructions otherwise, and hold every bit of their operands: so they do here, on
- * bf16 parts (all_bits).  As f16 parts a result that comes from a row's smallest values only was as far off as those parts are, another
+ * bf16 parts.  As f16 parts a result that comes from a row's smallest values only was as far off as those parts are, another
  * of the row being large (values of 1e-9 beside ones near 1: 2.3e-5 of their products).  bf16 parts round six times for 16 terms, so only short slices are as close as the 32x32 tiles are, eight waves
  * to a K: error, this / 32x32 tiles, in six slices 0.70 ... 0.72, five 0.76 ... 0.80, four 0.83 ... 0.88, three of K up to 2560
  * 0.96 ... 1.00 but of 4096 1.01, two 1.2; none up to 128 of the 32x32 tiles, which take slices of their own.  That many slices where
@@ -1214,12 +1216,12 @@ uint32_t tile_slices(const MatmulArgs &g, bool rope, bool all_bits) {
 template <bool VEC>
 bool launch_sliced(const MatmulArgs &g_in, bool rope, bool all_bits, hipStream_t s) {
     MatmulArgs g = g_in;
-    g.all_bits = all_bits;
     g.slices = tile_slices(g, rope, all_bits);
     const dim3 grid((g.n + TN - 1u) / TN, (g.m + TM - 1u) / TM, g.slices);
     const size_t tiles = (size_t)grid.x * grid.y;
     if (g.slices < 2u || !matmul_slice_scratch(tiles * g.slices * (TM * TN), tiles, s, &g.slice_sums, &g.slice_tickets)) return false;
-    launch_mfma_as<VEC, false, 1, false, false, true>(g, grid, s);
+    if (all_bits) launch_mfma_as<VEC, false, 1, false, false, SLICES_ALL_BITS>(g, grid, s);
+    else launch_mfma_as<VEC, false, 1, false, false, SLICES>(g, grid, s);
     return true;
 }
 template <bool VEC, int WT>
